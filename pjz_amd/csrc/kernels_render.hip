@@ -12,10 +12,10 @@
 //             k_render_combine  per (component, x, y, z): the moments mixed
 //                               by the shares into 1 / (p aoi + (1 - p) /
 //                               avg) or the plain average (:63-99)
-//   backward: k_render_bwd_stats   dL/dstats, summed over z
-//             k_render_bwd_share   dL/d(z share, z-moment share), summed over
-//                                  chunks of x, y (workgroups per component,
-//                                  z and chunk)
+//   backward: k_render_bwd_cells   dL/dstats, summed over z, and dL/d(z share,
+//                                  z-moment share), summed over the pixels of
+//                                  a workgroup, in one pass over the cells
+//             k_render_sum_parts   the workgroups' share sums added
 //             k_render_bwd_pos     dL/d(interface positions)
 //             k_render_bwd_layers  dL/d(layer sub-pixels), gathered through
 //                                  the shifts' edge replication
@@ -26,6 +26,7 @@
 // and y components, column 1 for z (:18-24).
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "fdtd_common.h"
 
@@ -49,11 +50,13 @@ __device__ inline int src_y(int a, int j, int m) { return a != 1 ? max(j - m, 0)
 
 __global__ __launch_bounds__(256) void k_render_stats(RenderDims d, const float* __restrict__ L,
                                                       float* __restrict__ st) {
-  const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  const long long n_out = 3LL * d.ll * d.xx * d.yy;
-  if (i >= n_out) return;
-  const int y = (int)(i % d.yy), x = (int)((i / d.yy) % d.xx);
-  const int l = (int)((i / ((long long)d.yy * d.xx)) % d.ll), a = (int)(i / ((long long)d.yy * d.xx * d.ll));
+  // 3 ll xx yy < 2^31 (the arrays' bound of the C ABI): 32-bit indices
+  const unsigned i = blockIdx.x * blockDim.x + threadIdx.x;
+  const unsigned np = (unsigned)d.xx * d.yy;
+  if (i >= 3u * d.ll * np) return;
+  const unsigned al = i / np, p = i - al * np;
+  const int x = p / (unsigned)d.yy, y = p - x * (unsigned)d.yy;
+  const int a = al / (unsigned)d.ll, l = al - a * (unsigned)d.ll;
   const int n = 2 * d.m, SX = n * d.xx, SY = n * d.yy;
   const float* Ll = L + (size_t)l * SX * SY;
   float s = 0.0f, si = 0.0f, sx = 0.0f, sy = 0.0f;
@@ -122,167 +125,305 @@ __device__ inline const float* share_at(const RenderDims& d, const float* tab, i
 
 // Mixed sums of one output cell and its value.
 struct Mix {
-  float A, B, G[3], out, pii, T;
+  float A, B, g0, g1, g2, out, pii, iT, iA;
 };
 
-__device__ inline Mix mix_cell(const RenderDims& d, const float* __restrict__ st,
-                               const float* __restrict__ tab, int a, int x, int y, int z) {
-  Mix r;
-  r.A = r.B = r.G[0] = r.G[1] = r.G[2] = 0.0f;
-  for (int l = 0; l < d.ll; ++l) {
-    const float* sh = share_at(d, tab, a, l, z);
-    const float u = sh[0], uz = sh[1];
-    const float avg = st[stat_at(d, a, 0, l, x, y)];
-    r.A += avg * u;
-    r.B += st[stat_at(d, a, 1, l, x, y)] * u;
-    r.G[0] += st[stat_at(d, a, 2, l, x, y)] * u;
-    r.G[1] += st[stat_at(d, a, 3, l, x, y)] * u;
-    r.G[2] += avg * uz;
-  }
-  if (d.simple) {
+constexpr int kRenderMaxLayers = 16;
+static_assert(kRenderMaxLayers == PJZ_FDTD_RENDER_MAX_LAYERS, "layer bound of the C ABI");
+
+// The moment along the component's own axis (selected, not indexed: an array
+// here goes to scratch memory).
+__device__ inline float own_moment(const Mix& r, int a) {
+  return a == 0 ? r.g0 : (a == 1 ? r.g1 : r.g2);
+}
+
+// Finishes a cell from its mixed sums (:89-99).
+__device__ inline void mix_finish(Mix& r, int simple, int a) {
+  if (simple) {
     r.out = r.A;
-    r.pii = r.T = 0.0f;
-    return r;
+    r.pii = r.iT = r.iA = 0.0f;
+    return;
   }
-  r.T = r.G[0] * r.G[0] + r.G[1] * r.G[1] + r.G[2] * r.G[2];
-  // (the component's moment selected, not indexed: G stays in registers)
-  const float ga = a == 0 ? r.G[0] : (a == 1 ? r.G[1] : r.G[2]);
-  r.pii = ga * ga / (r.T == 0.0f ? 1.0f : r.T);  // (:92-95)
-  r.out = 1.0f / (r.pii * r.B + (1.0f - r.pii) * (1.0f / r.A));  // (:97)
-  return r;
+  const float T = r.g0 * r.g0 + r.g1 * r.g1 + r.g2 * r.g2;
+  const float ga = own_moment(r, a);
+  r.pii = ga * ga / (T == 0.0f ? 1.0f : T);  // (:92-95)
+  r.iT = T == 0.0f ? 0.0f : 1.0f / T;
+  r.iA = 1.0f / r.A;
+  r.out = 1.0f / (r.pii * r.B + (1.0f - r.pii) * r.iA);  // (:97)
 }
 
-__global__ __launch_bounds__(256) void k_render_combine(RenderDims d, const float* __restrict__ st,
-                                                        const float* __restrict__ tab,
-                                                        float* __restrict__ eps) {
-  const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  if (i >= 3LL * d.xx * d.yy * d.zz) return;
-  const int z = (int)(i % d.zz), y = (int)((i / d.zz) % d.yy), x = (int)((i / ((long long)d.zz * d.yy)) % d.xx);
-  const int a = (int)(i / ((long long)d.zz * d.yy * d.xx));
-  eps[i] = mix_cell(d, st, tab, a, x, y, z).out;
-}
-
-// Cotangents of a cell's mixed sums A, B, G[0..2] from g = dL/d(out).
+// Cotangents of a cell's mixed sums A, B, G = (g0, g1, g2) from g = dL/d(out).
 struct MixGrad {
   float gA, gB, gG[3];
 };
 
-__device__ inline MixGrad mix_grad(const RenderDims& d, const Mix& r, int a, float g) {
+__device__ inline MixGrad mix_grad(int simple, const Mix& r, int a, float g) {
   MixGrad t;
-  if (d.simple) {
+  if (simple) {
     t.gA = g;
     t.gB = t.gG[0] = t.gG[1] = t.gG[2] = 0.0f;
     return t;
   }
   // out = 1 / D, D = pii B + (1 - pii) / A, pii = G_a^2 / T (T = sum G_k^2,
-  // no gradient through T where T = 0, where every G_k and pii are 0).
+  // no gradient through T where T = 0, where every G_k and pii are 0):
+  // dpii/dG_k = (2 G_a [k = a] - 2 pii G_k) / T.
   const float gD = -g * r.out * r.out;
-  const float iA = 1.0f / r.A;
-  t.gA = gD * (1.0f - r.pii) * (-iA * iA);
+  t.gA = gD * (1.0f - r.pii) * (-r.iA * r.iA);
   t.gB = gD * r.pii;
-  const float gp = gD * (r.B - iA);
-  const float ga = a == 0 ? r.G[0] : (a == 1 ? r.G[1] : r.G[2]);
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    float dp = 0.0f;
-    if (r.T != 0.0f) {
-      dp = -ga * ga * 2.0f * r.G[k] / (r.T * r.T);
-      if (k == a) dp += 2.0f * ga / r.T;
-    }
-    t.gG[k] = gp * dp;
-  }
+  const float gp = gD * (r.B - r.iA) * (2.0f * r.iT);
+  const float ga = own_moment(r, a);
+  t.gG[0] = gp * ((a == 0 ? ga : 0.0f) - r.pii * r.g0);
+  t.gG[1] = gp * ((a == 1 ? ga : 0.0f) - r.pii * r.g1);
+  t.gG[2] = gp * ((a == 2 ? ga : 0.0f) - r.pii * r.g2);
   return t;
 }
 
-// dL/dstats (3, 4, ll, xx, yy): sum over z of the cell cotangents times the
-// shares.  One thread per (component, x, y), up to kRenderMaxLayers layers.
-constexpr int kRenderMaxLayers = 16;
-static_assert(kRenderMaxLayers == PJZ_FDTD_RENDER_MAX_LAYERS, "layer bound of the C ABI");
+// The cell kernels (k_render_combine, k_render_bwd_cells): a wave walks over
+// pixels of one component with its lanes on z, so the output (or its
+// cotangent) is read and written in whole rows of zz floats and the layers'
+// shares of the lane's cells stay in registers.  The 4 LL moments of 16
+// pixels at a time come in as 16 lanes of as many loads and reach all lanes
+// by readlane.  C cells a lane cover the z range [z0, z0 + 64 C); taller
+// stacks take several launches.  The kernels these replaced gave each
+// (component, z, pixel) a thread: they read the cotangent with the pixels on
+// the lanes (one float of every 512-byte row) and divided 64-bit indices per
+// cell.  384 x 384 x 128 cells, 3 layers: combine 342 -> 135 us, the
+// two reverse passes 972 + 622 -> 315 us in one.
+constexpr int kRenderWaves = 4;  // waves of a workgroup
 
-__global__ __launch_bounds__(256) void k_render_bwd_stats(RenderDims d, const float* __restrict__ st,
-                                                          const float* __restrict__ tab,
-                                                          const float* __restrict__ geps,
-                                                          float* __restrict__ gst) {
-  const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  if (i >= 3LL * d.xx * d.yy) return;
-  const int y = (int)(i % d.yy), x = (int)((i / d.yy) % d.xx), a = (int)(i / ((long long)d.yy * d.xx));
-  float acc[kRenderMaxLayers][4];
-  for (int l = 0; l < kRenderMaxLayers; ++l) acc[l][0] = acc[l][1] = acc[l][2] = acc[l][3] = 0.0f;
-  for (int z = 0; z < d.zz; ++z) {
-    const Mix r = mix_cell(d, st, tab, a, x, y, z);
-    const float g = geps[(((size_t)a * d.xx + x) * d.yy + y) * d.zz + z];
-    const MixGrad t = mix_grad(d, r, a, g);
+template <int LL, int C>
+struct Shares {
+  float u[C][LL], uz[C][LL];
+};
+
+template <int LL, int C>
+__device__ inline void load_shares(Shares<LL, C>& S, const RenderDims& d, const float* tab, int a,
+                                   int z0, int lane) {
 #pragma unroll
-    for (int l = 0; l < kRenderMaxLayers; ++l) {
-      if (l < d.ll) {
-        const float* sh = share_at(d, tab, a, l, z);
-        acc[l][0] += t.gA * sh[0] + t.gG[2] * sh[1];
-        acc[l][1] += t.gB * sh[0];
-        acc[l][2] += t.gG[0] * sh[0];
-        acc[l][3] += t.gG[1] * sh[0];
-      }
-    }
-  }
+  for (int c = 0; c < C; ++c) {
+    const int z = min(z0 + 64 * c + lane, d.zz - 1);
 #pragma unroll
-  for (int l = 0; l < kRenderMaxLayers; ++l) {
-    if (l < d.ll) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) gst[stat_at(d, a, q, l, x, y)] = acc[l][q];
+    for (int l = 0; l < LL; ++l) {
+      const float* sh = share_at(d, tab, a, min(l, d.ll - 1), z);
+      S.u[c][l] = l < d.ll ? sh[0] : 0.0f;
+      S.uz[c][l] = l < d.ll ? sh[1] : 0.0f;
     }
   }
 }
 
-// dL/du and dL/duz (3, ll, zz), in parts: workgroup (z, a, ch) sums chunk ch
-// of the cells of its xy plane into part[((ch * 3 + a) * ll + l) * zz + z]
-// (u) and the same after nch * 3 * ll * zz floats (uz); k_render_sum_parts
-// adds the chunks.
-__device__ inline int render_chunks(const RenderDims& d) {
-  return min(max((d.xx * d.yy + 4095) / 4096, 1), 64);
+// Moments of pixels p .. p + 15 (lane & 15) of component a; 0 past the last
+// layer, the last pixel repeated past the end.
+template <int LL>
+__device__ inline void load_moments(float (&m)[LL][4], const RenderDims& d,
+                                    const float* __restrict__ st, int a, int p, int np, int lane) {
+  const int q0 = min(p + (lane & 15), np - 1);
+#pragma unroll
+  for (int l = 0; l < LL; ++l)
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      m[l][q] = l < d.ll ? st[(((size_t)a * 4 + q) * d.ll + l) * np + q0] : 0.0f;
 }
 
-__global__ __launch_bounds__(256) void k_render_bwd_share(RenderDims d, const float* __restrict__ st,
-                                                          const float* __restrict__ tab,
-                                                          const float* __restrict__ geps,
-                                                          float* __restrict__ part) {
-  __shared__ float red[256];
-  const int z = blockIdx.x, a = blockIdx.y, ch = blockIdx.z, nch = gridDim.z;
-  const int np = d.xx * d.yy;
-  const int p0 = (int)((long long)ch * np / nch), p1 = (int)((long long)(ch + 1) * np / nch);
-  float au[kRenderMaxLayers], auz[kRenderMaxLayers];
-  for (int l = 0; l < kRenderMaxLayers; ++l) au[l] = auz[l] = 0.0f;
-  for (int p = p0 + threadIdx.x; p < p1; p += blockDim.x) {
-    const int x = p / d.yy, y = p % d.yy;
-    const Mix r = mix_cell(d, st, tab, a, x, y, z);
-    const MixGrad t = mix_grad(d, r, a, geps[(((size_t)a * d.xx + x) * d.yy + y) * d.zz + z]);
+__device__ inline float from_lane(float v, int i) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), i));
+}
+
+template <int LL, int C>
+__device__ inline void mix_sums(Mix& r, const float (&m)[LL][4], const Shares<LL, C>& S, int c) {
+  r.A = r.B = r.g0 = r.g1 = r.g2 = 0.0f;
 #pragma unroll
-    for (int l = 0; l < kRenderMaxLayers; ++l) {
-      if (l < d.ll) {
-        const float avg = st[stat_at(d, a, 0, l, x, y)];
-        au[l] += t.gA * avg + t.gB * st[stat_at(d, a, 1, l, x, y)] +
-                 t.gG[0] * st[stat_at(d, a, 2, l, x, y)] +
-                 t.gG[1] * st[stat_at(d, a, 3, l, x, y)];
-        auz[l] += t.gG[2] * avg;
+  for (int l = 0; l < LL; ++l) {
+    r.A += m[l][0] * S.u[c][l];
+    r.B += m[l][1] * S.u[c][l];
+    r.g0 += m[l][2] * S.u[c][l];
+    r.g1 += m[l][3] * S.u[c][l];
+    r.g2 += m[l][0] * S.uz[c][l];
+  }
+}
+
+// The 16-pixel groups [g0, g1) of a wave: gpw consecutive ones.
+struct GroupRange {
+  int g0, g1;
+};
+__device__ inline GroupRange wave_groups(int np, int gpw) {
+  const int wave = blockIdx.x * kRenderWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n = (np + 15) / 16;
+  return {min(wave * gpw, n), min(wave * gpw + gpw, n)};
+}
+
+template <int LL, int C>
+__global__ __launch_bounds__(64 * kRenderWaves) void k_render_combine(
+    RenderDims d, const float* __restrict__ st, const float* __restrict__ tab,
+    float* __restrict__ eps, int gpw, int z0) {
+  const int a = blockIdx.y, lane = threadIdx.x & 63, np = d.xx * d.yy;
+  const GroupRange R = wave_groups(np, gpw);
+  if (R.g0 >= R.g1) return;
+  Shares<LL, C> S;
+  load_shares(S, d, tab, a, z0, lane);
+  for (int g = R.g0; g < R.g1; ++g) {
+    float m[LL][4];
+    load_moments(m, d, st, a, 16 * g, np, lane);
+    const int n = min(16, np - 16 * g);
+    for (int i = 0; i < n; ++i) {
+      float t[LL][4];
+#pragma unroll
+      for (int l = 0; l < LL; ++l)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) t[l][q] = from_lane(m[l][q], i);
+      float* row = eps + ((size_t)a * np + 16 * g + i) * d.zz;
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        const int z = z0 + 64 * c + lane;
+        Mix r;
+        mix_sums(r, t, S, c);
+        mix_finish(r, d.simple, a);
+        if (z < d.zz) __builtin_nontemporal_store(r.out, row + z);
       }
     }
   }
+}
+
+// Sums 4 values over the 64 lanes: on return row r (16 lanes) of the result
+// holds the sum of v[0], v[2], v[1], v[3] for r = 0..3 in each of its lanes.
+// gfx950's half and row swaps fold two values into one register per add: 3
+// swaps, 3 adds and 4 row rotations for 4 values, against 24 adds one by one.
+__device__ inline float swap_add32(float a, float b) {
+  const auto t = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, a),
+                                                  __builtin_bit_cast(unsigned, b), false, false);
+  // (copied out first: a bit cast of t[1] itself reads t[0])
+  const unsigned lo = t[0], hi = t[1];
+  return __builtin_bit_cast(float, lo) + __builtin_bit_cast(float, hi);
+}
+__device__ inline float swap_add16(float a, float b) {
+  const auto t = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, a),
+                                                  __builtin_bit_cast(unsigned, b), false, false);
+  // (copied out first: a bit cast of t[1] itself reads t[0])
+  const unsigned lo = t[0], hi = t[1];
+  return __builtin_bit_cast(float, lo) + __builtin_bit_cast(float, hi);
+}
+template <int N>
+__device__ inline float row_ror_add(float v) {
+  return v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(
+                                           0, __builtin_bit_cast(int, v), 0x120 + N, 0xf, 0xf, true));
+}
+__device__ inline float sum4(float v0, float v1, float v2, float v3) {
+  float s = swap_add16(swap_add32(v0, v1), swap_add32(v2, v3));
+  s = row_ror_add<8>(s);
+  s = row_ror_add<4>(s);
+  s = row_ror_add<2>(s);
+  return row_ror_add<1>(s);
+}
+
+// One pass over the cells of a component's pixels for both reductions of the
+// reverse pass:
+//  - dL/dstats (3, 4, ll, xx, yy): a pixel's cell cotangents times the shares,
+//    summed over z across the lanes (sum4; lane 16 r + i of a layer's register
+//    keeps pixel i's sum of moment r, stored 16 pixels at a time).  `add`
+//    accumulates onto the z ranges of earlier launches.
+//  - dL/du, dL/duz of the lane's cells, summed over the wave's pixels in
+//    registers (in double once per 16 pixels), over the workgroup in LDS and
+//    written to part[((blockIdx.x * 3 + a) * 2 + w) * ll * zz + l * zz + z].
+template <int LL, int C>
+__global__ __launch_bounds__(64 * kRenderWaves) void k_render_bwd_cells(
+    RenderDims d, const float* __restrict__ st, const float* __restrict__ tab,
+    const float* __restrict__ geps, float* __restrict__ gst, double* __restrict__ part, int gpw,
+    int z0, int add) {
+  __shared__ double red[kRenderWaves][64];
+  const int a = blockIdx.y, lane = threadIdx.x & 63, w = threadIdx.x >> 6, np = d.xx * d.yy;
+  const GroupRange R = wave_groups(np, gpw);
+  Shares<LL, C> S;
+  load_shares(S, d, tab, a, z0, lane);
+  double au[C][LL], auz[C][LL];
 #pragma unroll
-  for (int l = 0; l < kRenderMaxLayers; ++l) {
-    if (l < d.ll) {
+  for (int c = 0; c < C; ++c)
 #pragma unroll
-      for (int w = 0; w < 2; ++w) {
-        red[threadIdx.x] = w == 0 ? au[l] : auz[l];
-        __syncthreads();
-        for (int h = blockDim.x / 2; h > 0; h >>= 1) {
-          if ((int)threadIdx.x < h) red[threadIdx.x] += red[threadIdx.x + h];
-          __syncthreads();
+    for (int l = 0; l < LL; ++l) au[c][l] = auz[c][l] = 0.0;
+  // Moment held by this lane's row (sum4's order).
+  const int row = lane >> 4, qrow = row == 1 ? 2 : (row == 2 ? 1 : row);
+  for (int g = R.g0; g < R.g1; ++g) {
+    float m[LL][4], keep[LL], fu[C][LL], fuz[C][LL];
+    load_moments(m, d, st, a, 16 * g, np, lane);
+#pragma unroll
+    for (int l = 0; l < LL; ++l) {
+      keep[l] = 0.0f;
+#pragma unroll
+      for (int c = 0; c < C; ++c) fu[c][l] = fuz[c][l] = 0.0f;
+    }
+    const int n = min(16, np - 16 * g);
+    const float* grow = geps + ((size_t)a * np + 16 * g) * d.zz + z0 + lane;
+    float gnext[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+      gnext[c] = z0 + 64 * c + lane < d.zz ? __builtin_nontemporal_load(grow + 64 * c) : 0.0f;
+    for (int i = 0; i < n; ++i) {
+      float gv[C], t[LL][4], v[LL][4];
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        gv[c] = gnext[c];
+        gnext[c] = i + 1 < n && z0 + 64 * c + lane < d.zz
+                       ? __builtin_nontemporal_load(grow + (size_t)(i + 1) * d.zz + 64 * c)
+                       : 0.0f;
+      }
+#pragma unroll
+      for (int l = 0; l < LL; ++l)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          t[l][q] = from_lane(m[l][q], i);
+          v[l][q] = 0.0f;
         }
-        if (threadIdx.x == 0)
-          part[(size_t)w * nch * 3 * d.ll * d.zz + (((size_t)ch * 3 + a) * d.ll + l) * d.zz + z] =
-              red[0];
-        __syncthreads();
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        Mix r;
+        mix_sums(r, t, S, c);
+        mix_finish(r, d.simple, a);
+        const MixGrad k = mix_grad(d.simple, r, a, gv[c]);
+#pragma unroll
+        for (int l = 0; l < LL; ++l) {
+          v[l][0] += k.gA * S.u[c][l] + k.gG[2] * S.uz[c][l];
+          v[l][1] += k.gB * S.u[c][l];
+          v[l][2] += k.gG[0] * S.u[c][l];
+          v[l][3] += k.gG[1] * S.u[c][l];
+          fu[c][l] += k.gA * t[l][0] + k.gB * t[l][1] + k.gG[0] * t[l][2] + k.gG[1] * t[l][3];
+          fuz[c][l] += k.gG[2] * t[l][0];
+        }
+      }
+#pragma unroll
+      for (int l = 0; l < LL; ++l) {
+        const float s = sum4(v[l][0], v[l][1], v[l][2], v[l][3]);
+        keep[l] = (lane & 15) == i ? s : keep[l];
+      }
+    }
+#pragma unroll
+    for (int l = 0; l < LL; ++l) {
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        au[c][l] += fu[c][l];
+        auz[c][l] += fuz[c][l];
+      }
+      if (l < d.ll && (lane & 15) < n) {
+        float* o = gst + (((size_t)a * 4 + qrow) * d.ll + l) * np + 16 * g + (lane & 15);
+        *o = add ? *o + keep[l] : keep[l];
       }
     }
   }
+  if (!part) return;
+#pragma unroll
+  for (int c = 0; c < C; ++c)
+#pragma unroll
+    for (int l = 0; l < LL; ++l)
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        if (l >= d.ll) continue;
+        red[w][lane] = k == 0 ? au[c][l] : auz[c][l];
+        __syncthreads();
+        const int z = z0 + 64 * c + lane;
+        if (w == 0 && z < d.zz) {
+          double s = 0.0;
+          for (int j = 0; j < kRenderWaves; ++j) s += red[j][lane];
+          part[((((size_t)blockIdx.x * 3 + a) * 2 + k) * d.ll + l) * d.zz + z] = s;
+        }
+        __syncthreads();
+      }
 }
 
 // d clip(v, lo, hi) / dv with torch's (and jax's) halves at ties.
@@ -293,56 +434,59 @@ __device__ inline float dclip(float v, float lo, float hi) {
   return a * b;
 }
 
-// dL/dpos (ll - 1): interface j is layer j's upper bound and layer j+1's
-// lower bound.  One workgroup; lane j of the first ll - 1 sums over
-// components and z.
-// Adds the chunks of k_render_bwd_share: gus[w][a][l][z] (w = 0: dL/du,
-// 1: dL/duz), one lane per entry.
-__global__ __launch_bounds__(256) void k_render_sum_parts(RenderDims d, const float* __restrict__ part,
-                                                          float* __restrict__ gus) {
-  const int n = 3 * d.ll * d.zz;
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= 2 * n) return;
-  const int w = i / n, e = i % n;
-  const int nch = render_chunks(d);
-  float t = 0.0f;
-  for (int ch = 0; ch < nch; ++ch) t += part[((size_t)w * nch + ch) * n + e];
-  gus[i] = t;
+// Adds the workgroups' parts of k_render_bwd_cells: gus[((a * 2 + w) * ll + l)
+// * zz + z] (w = 0: dL/du, 1: dL/duz).  64 entries a workgroup, its 16 waves
+// taking every 16th part.
+constexpr int kSumWaves = 16;
+__global__ __launch_bounds__(64 * kSumWaves) void k_render_sum_parts(
+    int n, int nparts, const double* __restrict__ part, double* __restrict__ gus) {
+  __shared__ double red[kSumWaves][64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int e = blockIdx.x * 64 + lane;
+  double t = 0.0;
+  if (e < n)
+    for (int j = w; j < nparts; j += kSumWaves) t += part[(size_t)j * n + e];
+  red[w][lane] = t;
+  __syncthreads();
+  if (w == 0 && e < n) {
+    for (int j = 1; j < kSumWaves; ++j) t += red[j][lane];
+    gus[e] = t;
+  }
 }
 
-__global__ __launch_bounds__(64) void k_render_bwd_pos(RenderDims d, const float* __restrict__ pos,
-                                                       const float* __restrict__ gsa,
-                                                       const float* __restrict__ gea,
-                                                       const float* __restrict__ gus,
-                                                       float* __restrict__ gpos) {
-  const size_t n = (size_t)3 * d.ll * d.zz;
-  // dL/du (w = 0) and dL/duz (w = 1) of layer l at (a, z).
+// dL/dpos (ll - 1): interface j is layer j's upper bound and layer j+1's
+// lower bound.  One workgroup an interface, its lanes over components and z
+// (one lane an interface took 86 us at zz = 128, this 8).
+__global__ __launch_bounds__(256) void k_render_bwd_pos(RenderDims d, const float* __restrict__ pos,
+                                                        const float* __restrict__ gsa,
+                                                        const float* __restrict__ gea,
+                                                        const double* __restrict__ gus,
+                                                        float* __restrict__ gpos) {
+  __shared__ double red[256];
+  const int j = blockIdx.x;
   auto sum = [&](int w, int a, int l, int z) {
-    return gus[w * n + ((size_t)a * d.ll + l) * d.zz + z];
+    return gus[(((size_t)a * 2 + w) * d.ll + l) * d.zz + z];
   };
-  for (int j = threadIdx.x; j < d.ll - 1; j += blockDim.x) {
-    float acc = 0.0f;
-    for (int a = 0; a < 3; ++a) {
-      const int col = a == 2 ? 1 : 0;
-      for (int z = 0; z < d.zz; ++z) {
-        const float gs = gsa[2 * z + col], ge = gea[2 * z + col];
-        const float dz = ge - gs, c = (gs + ge) / 2, k = 12.0f / (dz * dz * dz);
-        // layer j: hi = pos[j] -> p1
-        {
-          const Share sh = layer_share(d, pos, gsa, gea, j, z, col);
-          const float dp1 = dclip(pos[j], gs, ge);
-          acc += (sum(0, a, j, z) / dz + sum(1, a, j, z) * k * (sh.p1 - c)) * dp1;
-        }
-        // layer j + 1: lo = pos[j] -> p0
-        {
-          const Share sh = layer_share(d, pos, gsa, gea, j + 1, z, col);
-          const float dp0 = dclip(pos[j], gs, ge);
-          acc += (-sum(0, a, j + 1, z) / dz + sum(1, a, j + 1, z) * k * (c - sh.p0)) * dp0;
-        }
-      }
-    }
-    gpos[j] = acc;
+  double acc = 0.0;
+  for (int i = threadIdx.x; i < 3 * d.zz; i += blockDim.x) {
+    const int a = i / d.zz, z = i - a * d.zz;
+    const int col = a == 2 ? 1 : 0;
+    const float gs = gsa[2 * z + col], ge = gea[2 * z + col];
+    const float dz = ge - gs, c = (gs + ge) / 2, k = 12.0f / (dz * dz * dz);
+    const float dp = dclip(pos[j], gs, ge);
+    // layer j: hi = pos[j] -> p1;  layer j + 1: lo = pos[j] -> p0
+    const Share s1 = layer_share(d, pos, gsa, gea, j, z, col);
+    const Share s0 = layer_share(d, pos, gsa, gea, j + 1, z, col);
+    acc += ((sum(0, a, j, z) - sum(0, a, j + 1, z)) / dz +
+            (sum(1, a, j, z) * (s1.p1 - c) + sum(1, a, j + 1, z) * (c - s0.p0)) * k) * dp;
   }
+  red[threadIdx.x] = acc;
+  __syncthreads();
+  for (int h = 128; h > 0; h >>= 1) {
+    if ((int)threadIdx.x < h) red[threadIdx.x] += red[threadIdx.x + h];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) gpos[j] = (float)red[0];
 }
 
 // dL/dlayers (ll, SX, SY): each source sub-pixel gathers, for every
@@ -350,16 +494,26 @@ __global__ __launch_bounds__(64) void k_render_bwd_pos(RenderDims d, const float
 // from it, or the first m + 1 along a shifted edge; none for the last m of a
 // shifted axis) with their tile's moment cotangents: d mean = 1 / n^2,
 // d mean of inverse = -1 / (v^2 n^2), d moments = 12 n w / n^2.
+// A workgroup takes 256 sub-pixels of one source row: the row's part of the
+// index is uniform and nothing is divided but the 32-bit column.  (One lane
+// a sub-pixel over a flat 64-bit index, with a division by v^2 for every
+// position read: 98 us for 3 x 1536 x 1536 sub-pixels, this 58.)
 __global__ __launch_bounds__(256) void k_render_bwd_layers(RenderDims d, const float* __restrict__ L,
                                                            const float* __restrict__ gst,
                                                            float* __restrict__ gL) {
-  const int n = 2 * d.m, SX = n * d.xx, SY = n * d.yy;
-  const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  if (i >= (long long)d.ll * SX * SY) return;
-  const int sj = (int)(i % SY), si = (int)((i / SY) % SX), l = (int)(i / ((long long)SY * SX));
+  const int n = 2 * d.m, SX = n * d.xx, SY = n * d.yy, np = d.xx * d.yy;
+  const int nblk = (SY + 255) / 256;
+  const int rowid = blockIdx.x / nblk;  // (layer, source row)
+  const int l = rowid / SX, si = rowid - l * SX;
+  const int sj = (blockIdx.x - rowid * nblk) * 256 + (int)threadIdx.x;
+  if (sj >= SY) return;
+  const size_t i = ((size_t)l * SX + si) * SY + sj;
   const float v = L[i];
   const float inv = 1.0f / (float)(n * n);
+  const float iv2 = 1.0f / (v * v);
+  const float k12 = 12.0f * n;
   float acc = 0.0f;
+#pragma unroll
   for (int a = 0; a < 3; ++a) {
     // shifted positions along x reading source row si
     int i0, i1;
@@ -382,15 +536,16 @@ __global__ __launch_bounds__(256) void k_render_bwd_layers(RenderDims d, const f
       j0 = j1 = sj + d.m;
       if (j0 >= SY) continue;
     }
+    const float* g0 = gst + ((size_t)a * 4 * d.ll + l) * np;
+    const size_t q = (size_t)d.ll * np;  // from one moment to the next
     for (int ii = i0; ii <= i1; ++ii) {
-      const int x = ii / n, di = ii % n;
+      const int x = ii / n, di = ii - x * n;
       const float wx = (di - (d.m - 0.5f)) / (float)(n * n);
       for (int jj = j0; jj <= j1; ++jj) {
-        const int y = jj / n, dj = jj % n;
+        const int y = jj / n, dj = jj - y * n;
         const float wy = (dj - (d.m - 0.5f)) / (float)(n * n);
-        acc += (gst[stat_at(d, a, 0, l, x, y)] - gst[stat_at(d, a, 1, l, x, y)] / (v * v) +
-                gst[stat_at(d, a, 2, l, x, y)] * 12.0f * n * wx +
-                gst[stat_at(d, a, 3, l, x, y)] * 12.0f * n * wy) * inv;
+        const float* p = g0 + (size_t)x * d.yy + y;
+        acc += (p[0] - p[q] * iv2 + p[2 * q] * k12 * wx + p[3 * q] * k12 * wy) * inv;
       }
     }
   }
@@ -407,14 +562,40 @@ size_t render_stats_floats(int ll, int xx, int yy, int zz) {
   return (size_t)12 * ll * xx * yy + (size_t)4 * ll * zz;
 }
 
-static int render_chunks_host(int xx, int yy) {
-  return std::min(std::max((xx * yy + 4095) / 4096, 1), 64);
+// Workgroups per component of the cell kernels: their waves take 16-pixel
+// groups, about 1366 waves a component (4 a SIMD over the three components)
+// where there are as many groups.
+struct CellGrid {
+  int blocks, gpw;
+};
+static CellGrid cell_grid(int xx, int yy) {
+  const int groups = (xx * yy + 15) / 16;
+  const int gpw = (groups + 4 * 342 - 1) / (4 * 342);
+  return {(groups + kRenderWaves * gpw - 1) / (kRenderWaves * gpw), gpw};
 }
 
 size_t render_workspace_bytes(int ll, int xx, int yy, int zz) {
   return align256(sizeof(float) * (size_t)12 * ll * xx * yy) +
-         align256(sizeof(float) * (size_t)2 * render_chunks_host(xx, yy) * 3 * ll * zz) +
-         align256(sizeof(float) * (size_t)2 * 3 * ll * zz);
+         align256(sizeof(double) * (size_t)cell_grid(xx, yy).blocks * 6 * ll * zz) +
+         align256(sizeof(double) * (size_t)6 * ll * zz);
+}
+
+// Calls f(LL, C) with the layers a cell kernel is built for (the fewest that
+// hold ll: unused ones have share 0) and its cells a lane.  Up to 4 layers
+// two cells a lane where zz > 64; more layers keep one (registers).
+template <typename F>
+static void cell_variant(int ll, int zz, F&& f) {
+  const bool two = zz > 64;
+  auto pick = [&](auto LL) {
+    if (two) f(LL, std::integral_constant<int, 2>());
+    else f(LL, std::integral_constant<int, 1>());
+  };
+  if (ll == 1) pick(std::integral_constant<int, 1>());
+  else if (ll == 2) pick(std::integral_constant<int, 2>());
+  else if (ll == 3) pick(std::integral_constant<int, 3>());
+  else if (ll == 4) pick(std::integral_constant<int, 4>());
+  else if (ll <= 8) f(std::integral_constant<int, 8>(), std::integral_constant<int, 1>());
+  else f(std::integral_constant<int, 16>(), std::integral_constant<int, 1>());
 }
 
 hipError_t render_forward(int ll, int m, int xx, int yy, int zz, int simple, const float* layers,
@@ -426,8 +607,12 @@ hipError_t render_forward(int ll, int m, int xx, int yy, int zz, int simple, con
                      layers, stats);
   hipLaunchKernelGGL(k_render_shares, dim3(blocks_for(2LL * ll * zz)), dim3(256), 0, s, d, pos,
                      gs, ge, tab);
-  hipLaunchKernelGGL(k_render_combine, dim3(blocks_for(3LL * xx * yy * zz)), dim3(256), 0, s, d,
-                     stats, tab, eps);
+  const CellGrid G = cell_grid(xx, yy);
+  cell_variant(ll, zz, [&](auto LL, auto C) {
+    for (int z0 = 0; z0 < zz; z0 += 64 * C.value)
+      hipLaunchKernelGGL((k_render_combine<LL.value, C.value>), dim3(G.blocks, 3),
+                         dim3(64 * kRenderWaves), 0, s, d, stats, tab, eps, G.gpw, z0);
+  });
   return hipGetLastError();
 }
 
@@ -437,20 +622,28 @@ hipError_t render_backward(int ll, int m, int xx, int yy, int zz, int simple, co
                            char* ws, hipStream_t s) {
   const RenderDims d{ll, m, xx, yy, zz, simple};
   const float* tab = stats + (size_t)12 * ll * xx * yy;
+  const CellGrid G = cell_grid(xx, yy);
   float* gst = (float*)ws;
-  float* part = (float*)(ws + align256(sizeof(float) * (size_t)12 * ll * xx * yy));
-  float* gus = (float*)((char*)part + align256(sizeof(float) * (size_t)2 *
-                                               render_chunks_host(xx, yy) * 3 * ll * zz));
-  hipLaunchKernelGGL(k_render_bwd_stats, dim3(blocks_for(3LL * xx * yy)), dim3(256), 0, s, d,
-                     stats, tab, g_eps, gst);
-  hipLaunchKernelGGL(k_render_bwd_layers, dim3(blocks_for((long long)ll * 4 * m * m * xx * yy)),
-                     dim3(256), 0, s, d, layers, gst, g_layers);
-  if (ll > 1 && g_pos) {
-    hipLaunchKernelGGL(k_render_bwd_share, dim3(zz, 3, render_chunks_host(xx, yy)), dim3(256),
-                       0, s, d, stats, tab, g_eps, part);
-    hipLaunchKernelGGL(k_render_sum_parts, dim3(blocks_for(6LL * ll * zz)), dim3(256), 0, s, d,
-                       part, gus);
-    hipLaunchKernelGGL(k_render_bwd_pos, dim3(1), dim3(64), 0, s, d, pos, gs, ge, gus, g_pos);
+  double* part = (double*)(ws + align256(sizeof(float) * (size_t)12 * ll * xx * yy));
+  double* gus = (double*)((char*)part + align256(sizeof(double) * (size_t)G.blocks * 6 * ll * zz));
+  const bool want_pos = ll > 1 && g_pos;
+  cell_variant(ll, zz, [&](auto LL, auto C) {
+    for (int z0 = 0; z0 < zz; z0 += 64 * C.value)
+      hipLaunchKernelGGL((k_render_bwd_cells<LL.value, C.value>), dim3(G.blocks, 3),
+                         dim3(64 * kRenderWaves), 0, s, d, stats, tab, g_eps, gst,
+                         want_pos ? part : (double*)nullptr, G.gpw, z0, z0 > 0);
+  });
+  // ll SX SY < 2^29 (the arrays' bound of the C ABI); a row takes at least
+  // one workgroup.
+  const int SX = 2 * m * xx, SY = 2 * m * yy;
+  hipLaunchKernelGGL(k_render_bwd_layers, dim3((unsigned)ll * SX * ((SY + 255) / 256)), dim3(256),
+                     0, s, d, layers, gst, g_layers);
+  if (want_pos) {
+    const int n = 6 * ll * zz;
+    hipLaunchKernelGGL(k_render_sum_parts, dim3((n + 63) / 64), dim3(64 * kSumWaves), 0, s, n,
+                       G.blocks, part, gus);
+    hipLaunchKernelGGL(k_render_bwd_pos, dim3(ll - 1), dim3(256), 0, s, d, pos, gs, ge, gus,
+                       g_pos);
   }
   return hipGetLastError();
 }

@@ -192,3 +192,33 @@ def test_render_kernel_gradient(gpu, pos, m, simple):
   assert np.linalg.norm(got - ref) <= 1e-5 * np.linalg.norm(ref)
   if pos:
     np.testing.assert_allclose(pg.grad.cpu().numpy(), pc.grad.numpy(), rtol=1e-4, atol=1e-5)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ll,xx,yy,zz", [(1, 1, 1, 1), (2, 3, 5, 63), (3, 4, 4, 64), (4, 3, 11, 65),
+                                         (3, 5, 13, 128), (2, 2, 9, 129), (5, 7, 7, 66),
+                                         (8, 3, 6, 70), (9, 2, 3, 64), (16, 3, 3, 130)])
+def test_render_kernel_sizes(gpu, ll, xx, yy, zz):
+  """Forward and reverse at the edges of the cell kernels' ranges (64 or 128
+  cells a wave, 16 pixels a group, the layer counts they are built for),
+  against the float32 torch restatement on the CPU, which rounds the layers'
+  shares of a cell (differences of z positions) as the kernels do.  Twice the
+  bounds of the float64 comparisons above: both sides round.  Layers with a
+  slope everywhere and interfaces apart: where a cell's gradient vanishes, the
+  average's direction, and with it the derivative, is rounding noise."""
+  rng = np.random.default_rng(17 * ll + zz)
+  m = 2
+  i, j = np.arange(2 * m * xx)[:, None], np.arange(2 * m * yy)[None, :]
+  layers = np.stack([2 + 3 * (k % 3) + 0.1 * i + 0.07 * j for k in range(ll)])
+  layers += rng.uniform(-0.01, 0.01, layers.shape)
+  pos = np.arange(1, ll) * zz / ll + 0.3
+  g = torch.tensor(rng.standard_normal((3, xx, yy, zz)), dtype=torch.float32)
+  res = []
+  for dev in (gpu, torch.device("cpu")):
+    L = torch.tensor(layers, dtype=torch.float32, device=dev, requires_grad=True)
+    p = torch.tensor(pos, dtype=torch.float32, device=dev, requires_grad=True)
+    out = E.render(L, p, *(t.to(dev) for t in zgrid(zz, torch.float32)), m)
+    (out * g.to(dev)).sum().backward()
+    res.append([v.detach().cpu().numpy() for v in (out, L.grad) + ((p.grad,) if ll > 1 else ())])
+  for got, ref, tol in zip(*res, (2e-5, 2e-5, 2e-4)):
+    assert np.linalg.norm(got - ref) <= tol * np.linalg.norm(ref)
