@@ -169,3 +169,46 @@ def test_gpu_kernel_matches_torch_iteration(gpu, xx, yy, mm, ww):
   gram = torch.einsum("wrk,wrl->wkl", q.double(), q.double())
   eye = torch.eye(mm, dtype=torch.float64, device=gpu).expand(ww, mm, mm)
   assert float(torch.max(torch.abs(gram - eye))) <= 1e-5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("xx,yy,mm,ww", [(32, 32, 2, 1), (41, 25, 2, 2), (5, 700, 1, 1),
+                                         (3, 1024, 3, 1), (131, 61, 6, 1), (129, 127, 2, 3),
+                                         (64, 17, 4, 5), (1, 40, 1, 2)])
+def test_gpu_tile_kernel_edges(gpu, xx, yy, mm, ww):
+  """The register-resident kernel at the edges of its plan: 1024 cells (the
+  last on one workgroup) and 1025, one row a workgroup, a short last
+  workgroup, its most modes, several frequencies stopping together and apart.
+  The bounds are those of the comparison above."""
+  rng = np.random.default_rng(xx * yy + mm)
+  eps = torch.tensor(1 + 11 * rng.random((3, xx, yy)), dtype=torch.float32, device=gpu)
+  omega = torch.tensor(2 * np.pi / (30 + 5 * rng.random(ww)), dtype=torch.float32, device=gpu)
+  x0 = M._random((ww, 2, xx, yy, mm), gpu, seed=7)
+  shift = torch.full((ww,), 8.0, device=gpu)
+  print(f"case {(xx, yy, mm, ww)}", flush=True)
+  w0, _, e0, i0 = M._subspace_iteration(M._operator(eps, omega, shift), x0, 30, 0.0)
+  w1, x1, e1, i1 = M._subspace_iteration_hip(eps, omega, shift, x0, 30, 0.0)
+  assert i0 == i1 == 30
+  scale = float(torch.max(torch.abs(w0)))
+  assert float(torch.max(torch.abs(w1 - w0))) <= 2e-5 * scale
+  assert float(torch.max(torch.abs(e1 - e0))) <= 2e-4 * scale + 1e-3 * float(torch.max(e0))
+  q = x1.reshape(ww, -1, mm).double().transpose(1, 2).contiguous()
+  gram = q @ q.transpose(1, 2).contiguous()
+  assert float(torch.max(torch.abs(gram - torch.eye(mm, dtype=torch.float64, device=gpu)))) <= 1e-5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("xx,yy", [(30, 20), (90, 70)])
+def test_gpu_tile_kernel_nearly_dependent_start(gpu, xx, yy):
+  """Start vectors 1e-5 apart need the second orthogonalisation pass: after
+  one iteration the basis is orthonormal to float32 rounding all the same."""
+  eps = 1 + 11 * torch.rand((3, xx, yy), device=gpu,
+                            generator=torch.Generator(device=gpu).manual_seed(3))
+  omega = torch.tensor([0.2], device=gpu)
+  a, b = (M._random((1, 2, xx, yy, 1), gpu, seed=s) for s in (1, 2))
+  x0 = torch.cat([a, a + 1e-5 * b], dim=-1)
+  _, x, _, _ = M._subspace_iteration_hip(eps, omega, torch.tensor([8.0], device=gpu), x0, 1, 0.0)
+  q = x.reshape(-1, 2).double()
+  gram = torch.stack([torch.stack([torch.sum(q[:, i] * q[:, j]) for j in range(2)])
+                      for i in range(2)]).cpu()
+  assert float(torch.max(torch.abs(gram - torch.eye(2, dtype=torch.float64)))) <= 1e-5
