@@ -13,6 +13,7 @@
 #include <vector>
 
 #include "fdtd_common.h"
+#include "resident.h"
 
 namespace {
 
@@ -292,6 +293,36 @@ hipError_t run_steps(const pjz::Geom& g, const pjz_fdtd_problem& p, const float*
   return pjz::run_reference(g, p, mask, src, win, ws, L, r, s);
 }
 
+// A resident run costs about 0.1 ms once (the words, the state) and saves 10 us
+// a step or more.
+constexpr int kResidentMinSteps = 16;
+
+// The resident stepper's tiling for a call, or rx = 0 where steps are launched
+// one by one: another kernel or tiling was asked for, the domain is too large,
+// or the call is recorded into a graph, which a cooperative launch might not
+// be.
+pjz::ResPlan resident_for(const pjz::Geom& g, const pjz_fdtd_problem& p, hipStream_t s) {
+  const pjz::ResPlan none{};
+  if (p.kernel != PJZ_FDTD_KERNEL_AUTO || p.tile_x != 0 || p.tile_y != 0 ||
+      pjz::steps_of(p) < kResidentMinSteps)
+    return none;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  int dev = 0, cus = 0, coop = 0, lds = 0;
+  if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone ||
+      hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+      hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev) != hipSuccess ||
+      hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess ||
+      !coop || (size_t)lds < pjz::kResLds)
+    return none;
+  return pjz::resident_plan(g, p.src_axis, cus);
+}
+
+// Clears the exchange words (once a call: its runs use rising numbers).
+hipError_t clear_words(const pjz::ResPlan& plan, const pjz::Layout& L, char* ws, hipStream_t s) {
+  return pjz::launch_zero((float*)(ws + L.E1), plan.words() * 2, s);
+}
+
 // Checkpoint k holds E, H, the psi_H pair and the psi_E pair of the state that
 // lives in ping-pong set `cur`.
 struct StateParts {
@@ -324,6 +355,12 @@ hipError_t copy_state(const pjz::Geom& g, const pjz::Layout& L, char* ws, int cu
     off += sizes[i];
   }
   return hipSuccess;
+}
+
+// Checkpoint k as a state in place.
+pjz::ResState ckpt_state(const pjz::Geom& g, const pjz::Layout& L, char* ws, int k) {
+  float* c = (float*)(ws + L.ckpt + pjz::ckpt_stride(L) * (size_t)k);
+  return {c, c + 3 * (size_t)g.N, c + 6 * (size_t)g.N};
 }
 
 hipError_t save_state(const pjz::Geom& g, const pjz::Layout& L, char* ws, int cur, int k,
@@ -556,22 +593,31 @@ int pjz_fdtd_forward(const pjz_fdtd_problem* p, const float* epsilon,
     return fail(PJZ_FDTD_EINVAL, "workspace must be 256-byte aligned");
   hipStream_t s = (hipStream_t)stream;
   char* ws = (char*)workspace;
-  // Clear E0, H0 (contiguous) and psi; build cb and the z table.
+  // cb and the z table.
   hipError_t e = pjz::launch_prepare(g, *p, epsilon, absorption_mask, pml_kappa, pml_sigma,
                                      pml_alpha, (float*)(ws + L.cb), (float*)(ws + L.zt), s);
   if (e != hipSuccess) return hip_fail(e, "prepare");
+  pjz::Src src{p->src_axis, p->src_pos, p->src_quad, source_field, source_waveform};
+  pjz::OutWin win{p->x0, p->y0, p->z0, p->ex, p->ey, p->ez, out};
+  const int nsteps = pjz::steps_of(*p);
+  const pjz::ResPlan plan = resident_for(g, *p, s);
+  if (plan.rx > 0) {
+    // The whole run in one launch, its checkpoints written on the way.
+    e = clear_words(plan, L, ws, s);
+    pjz::ResRun r{0, nsteps, {}, {}, nullptr, nullptr, L.S1, 0};
+    if (L.nck > 0) r.ckpt = ckpt_state(g, L, ws, 0).E;
+    if (e == hipSuccess) e = pjz::run_resident(g, *p, absorption_mask, src, win, ws, L, plan, r, s);
+    return e == hipSuccess ? PJZ_FDTD_OK : hip_fail(e, "resident launch");
+  }
   e = pjz::launch_zero((float*)(ws + L.E0), (L.E1 - L.E0) / sizeof(float), s);
   if (e == hipSuccess && g.NP > 0)
     e = pjz::launch_zero((float*)(ws + L.psi), (L.zt - L.psi) / sizeof(float), s);
   if (e != hipSuccess) return hip_fail(e, "clear state");
-  pjz::Src src{p->src_axis, p->src_pos, p->src_quad, source_field, source_waveform};
   Tuned tuned;
   if (p->kernel == PJZ_FDTD_KERNEL_AUTOTUNE && !tuned_choice(*p, &tuned)) {
     e = autotune(g, *p, absorption_mask, src, ws, L, s);
     if (e != hipSuccess) return hip_fail(e, "autotune");
   }
-  pjz::OutWin win{p->x0, p->y0, p->z0, p->ex, p->ey, p->ez, out};
-  const int nsteps = pjz::steps_of(*p);
   int cur = 0;
   if (L.nck > 0) {
     // Checkpoint the state before steps 0, S, 2S, ... for pjz_fdtd_backward.
@@ -934,12 +980,24 @@ int pjz_fdtd_backward(const pjz_fdtd_problem* p, const float* epsilon,
   auto is_out = [&](int n) {
     return n >= p->out_start && n < p->out_stop && (n - p->out_start) % p->out_step == 0;
   };
+  const pjz::ResPlan plan = resident_for(g, *p, s);
+  unsigned tags = 0;  // exchange numbers used
+  if (plan.rx > 0) e = clear_words(plan, L, ws, s);
+  if (e != hipSuccess) return hip_fail(e, "backward set-up");
+  // Steps [b, end) of the resident stepper from checkpoint slot k.
+  auto resident = [&](int k, int b, int end, pjz::ResState out, float* capture, float* ckpt,
+                      int every) {
+    const pjz::ResRun r{b, end, ckpt_state(g, L, ws, k), out, capture, ckpt, every, tags};
+    tags += pjz::resident_tags(end - b);
+    return pjz::run_resident(g, *p, absorption_mask, src, nowin, ws, L, plan, r, s);
+  };
   // Steps [b, end) from the state in checkpoint slot k: recompute them
   // capturing D^n = E^n - E^(n+1), then reverse them.
   auto reverse_segment = [&](int k, int b, int end) {
     int cur = 0;
-    hipError_t e = restore_state(g, L, ws, k, s);
-    if (e == hipSuccess)
+    hipError_t e = plan.rx > 0 ? resident(k, b, end, {}, seg, nullptr, 1)
+                               : restore_state(g, L, ws, k, s);
+    if (e == hipSuccess && plan.rx == 0)
       e = run_steps(g, *p, absorption_mask, src, nowin, ws, L, b, end, &cur, seg, s);
     for (int n = end - 1; n >= b && e == hipSuccess;) {
       if (is_out(n))
@@ -972,6 +1030,18 @@ int pjz_fdtd_backward(const pjz_fdtd_problem* p, const float* epsilon,
     }
     // Two levels: recompute the S1 segment from its checkpoint keeping the
     // state every S steps (slots nck + j), then reverse its sub-segments.
+    if (plan.rx > 0) {
+      const int nsub = (e1 - b1 + L.S - 1) / L.S;
+      const int last = b1 + (nsub - 1) * L.S;
+      // Slots nck .. nck + nsub - 1; the first is slot k itself.
+      if (nsub > 1)
+        e = resident(k, b1, last, ckpt_state(g, L, ws, L.nck + nsub - 1), nullptr,
+                     ckpt_state(g, L, ws, L.nck).E, L.S);
+      for (int j = nsub - 1; j >= 0 && e == hipSuccess; --j)
+        e = reverse_segment(j == 0 ? k : L.nck + j, b1 + j * L.S,
+                            j == nsub - 1 ? e1 : b1 + (j + 1) * L.S);
+      continue;
+    }
     int cur = 0;
     e = restore_state(g, L, ws, k, s);
     int nsub = 0;

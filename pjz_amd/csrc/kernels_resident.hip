@@ -1,0 +1,778 @@
+// Resident stepper: a whole run of steps in one launch, the fields in
+// registers.
+//
+// What bounds the streaming steppers on domains of up to a few million cells
+// is not bytes: a launch of a 64^3 domain takes 26 us for two steps of 9 MB
+// (8-13 planes in sequence, two barriers each, 36-64 workgroups), and a
+// 128x128x64 step of 38 MB 15 us.  The chip's registers (128 MB) hold such a
+// domain.  Here a workgroup owns a tile of z columns for the whole run: E, H
+// (and, up to 20 cells a lane, cb) live in registers, RX x RY columns a wave
+// and CPL cells of a column a lane, so x neighbours and most y neighbours are
+// other registers of the same lane and z neighbours a DPP move; the CPML psi
+// live in LDS.
+//
+// Edges: after a half step a wave passes its edge columns (the low edges of
+// E, the high edges of H) to the next wave through LDS or, at the tile's
+// border, to the next workgroup as self-numbered 8-byte words (resident.h).
+// The columns that need no neighbour's edge are computed first, while the
+// words travel: a step costs the larger of its arithmetic and two exchange
+// latencies (about 1 us each).  A word is rewritten only after its reader
+// has posted the answer that the writer waits for (E of step n + 1 at an edge
+// needs H of step n + 1 there, which the neighbour posts after it read E of
+// step n), so one set of words is enough.  Every workgroup is resident
+// (cooperative launch) and posts before it waits for the answer, so every
+// wait ends.
+//
+// Measured, us a step, two-step kernel (the default before) against this:
+// 64^3 13.4 -> 2.9 (both exchange latencies), 128x128x64 14.3 -> 5.2,
+// 160x160x64 20.4 -> 6.9 (16 cells a lane: arithmetic), 190x200x50 25.1 ->
+// 11.1, 150x140x96 29.0 -> 13.8, 301x187x45 45.0 -> 19.3, 180x150x128 37.2 ->
+// 18.4 (20-30 cells a lane: cb from the caches).
+//
+// The arithmetic of a cell is that of the two-step kernel (stream2_parts.h),
+// in its order of rounding: results equal that kernel's bit for bit.
+// Cells past the domain's end in x, y and z have cb = 0 and start from zero,
+// so they stay zero and need no bounds checks.
+#include <algorithm>
+
+#include "resident.h"
+
+namespace pjz {
+
+struct ResArgs {
+  const float* Ein;  // state before step `begin`: E, H (3N each), psi (4P); null: zeros
+  const float* Hin;
+  const float* psiin;
+  float* Eout;       // state after the last step (or null)
+  float* Hout;
+  float* psiout;
+  const float* cb;
+  const float* zt;
+  const float* mask;
+  const float* sfield;
+  const float* swave;
+  float* out;        // snapshots (or null)
+  float* cap;        // E^n - E^(n+1) at cap + (n - begin) * 3N (CAP kernels)
+  float* ckpt;       // states before steps begin, begin + every, ... (or null)
+  rword_t* words;
+  long long ckpt_stride;  // floats
+  int every;
+  int X, Y, Z, lo, hi, NP, N, P;
+  int saxis, spos, squad;
+  float dt;
+  int begin, end;
+  unsigned tag0;     // exchange numbers tag0 + 1 .. tag0 + 2 (end - begin) + 1
+  int wx, wy, ntx, nty;
+  int alias;
+  int wx0, wy0, wz0, wex, wey, wez, ostart, ostop, ostep;
+};
+
+// The columns of a wave in the order they are computed: first those that need
+// no other wave's edge.  E needs the low neighbours; H, mirrored, the high.
+template <int RX, int RY>
+struct ColOrder {
+  static constexpr int inner = (RX - 1) * (RY - 1);
+  static constexpr int x(int k) {
+    return k < inner ? 1 + k / (RY > 1 ? RY - 1 : 1) : (k - inner < RX ? k - inner : 0);
+  }
+  static constexpr int y(int k) {
+    return k < inner ? 1 + k % (RY > 1 ? RY - 1 : 1) : (k - inner < RX ? 0 : k - inner - RX + 1);
+  }
+};
+
+template <int CPL>
+__device__ __forceinline__ void lds_put(float* p, const float (&v)[CPL]) {
+  if constexpr (CPL == 2) *reinterpret_cast<f32x2*>(p) = f32x2{v[0], v[1]};
+  else p[0] = v[0];
+}
+template <int CPL>
+__device__ __forceinline__ void lds_get(float (&v)[CPL], const float* p) {
+  if constexpr (CPL == 2) {
+    const f32x2 t = *reinterpret_cast<const f32x2*>(p);
+    v[0] = t.x;
+    v[1] = t.y;
+  } else {
+    v[0] = p[0];
+  }
+}
+
+// Registers: 6 a cell for E and H, 3 more for cb where that still fits; past
+// it cb (12 of the 60 bytes a streaming step moves a cell) is read from the
+// caches each step, two columns ahead.
+template <int CPL, int RX, int RY>
+constexpr bool res_keeps_cb() { return CPL * RX * RY <= 16; }
+
+template <int CPL, int RX, int RY, bool CAP>
+__global__ __launch_bounds__(kResThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void
+k_resident(ResArgs a) {
+  constexpr int C = RX * RY;
+  constexpr bool CBR = res_keeps_cb<CPL, RX, RY>();
+  constexpr int ED = 2 * 64 * CPL;  // floats (or words) of an edge column
+  using Order = ColOrder<RX, RY>;
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int WX = a.wx, WY = a.wy;
+  // Quotients of uniform values are computed on the vector unit: back to
+  // scalar registers, or all that follows from them takes vector registers.
+  const int wx = __builtin_amdgcn_readfirstlane(w % WX);
+  const int wy = __builtin_amdgcn_readfirstlane(w / WX);
+  const int TX = RX * WX, TY = RY * WY;
+  const int X = a.X, Y = a.Y, Z = a.Z, N = a.N, P = a.P, NP = a.NP;
+  const int nt = a.ntx * a.nty;
+  // Consecutive workgroups go round-robin over the 8 XCDs; neighbouring tiles
+  // go to one XCD where the count allows it.
+  int tile = blockIdx.x;
+  if ((nt & 7) == 0) tile = (tile & 7) * (nt >> 3) + (tile >> 3);
+  const int bx = __builtin_amdgcn_readfirstlane(tile / a.nty);
+  const int by = __builtin_amdgcn_readfirstlane(tile % a.nty);
+  const int x0 = bx * TX + wx * RX, y0 = by * TY + wy * RY;
+  const int zb = lane * CPL;
+  const float dt = a.dt;
+
+  // LDS: psi as (column, H or E pair, PML cell, 2) and, per column, a zero pair
+  // for the lanes outside the PML (so every lane's address steps alike);
+  // absorber values and source of the tile; edge buffers.
+  extern __shared__ float lds[];
+  float* const psi = lds;
+  const int PS = NP * 4 + 2;
+  f32x4* const sig = reinterpret_cast<f32x4*>(psi + ((TX * TY * PS + 3) & ~3));
+  float* const srcl = reinterpret_cast<float*>(sig + TX * TY);
+  const int nsrc = a.saxis == 0 ? TY * ED : a.saxis == 1 ? TX * ED : TX * TY * 4;
+  float* const edgeE = srcl + nsrc;
+  const int nedge = (WX * TY + WY * TX) * ED;
+  float* const edgeH = a.alias ? edgeE : edgeE + nedge;
+  // Edge slot s of a direction lies between waves s - 1 and s.  E is read
+  // from slot w + 1 and written to slot w, H read from w and written to w + 1;
+  // slots 1 .. WX (E) and 0 .. WX - 1 (H) exist, the outer one holding the
+  // neighbouring workgroup's edge.
+  // (Float offsets, uniform: the lane's address is made where it is used.)
+  const int eoff = (int)(edgeE - lds), hoff = (int)(edgeH - lds);
+  const int sx = (wx * TY + wy * RY) * ED, sy = (WX * TY + wy * TX + wx * RX) * ED;
+  const int exr = eoff + sx, exw = eoff + sx - TY * ED;  // exw if wx > 0
+  const int eyr = eoff + sy, eyw = eoff + sy - TX * ED;  // eyw if wy > 0
+  const int hxr = hoff + sx, hxw = hoff + sx + TY * ED;  // hxw if wx < WX - 1
+  const int hyr = hoff + sy, hyw = hoff + sy + TX * ED;  // hyw if wy < WY - 1
+  auto slot = [&](int off) { return lds + opaque_s(off) + zb; };
+  // A tile's words: E low x (TY columns), E low y (TX), H high x, H high y.
+  const size_t tw = (size_t)2 * (TX + TY) * ED;
+  rword_t* const mine = a.words + (size_t)tile * tw;
+  const int ox = wy * RY * ED, oy = TY * ED + wx * RX * ED, oh = (TX + TY) * ED;
+  const bool xlo = wx == 0 && bx > 0, xhi = wx == WX - 1 && bx + 1 < a.ntx;
+  const bool ylo = wy == 0 && by > 0, yhi = wy == WY - 1 && by + 1 < a.nty;
+  // Of the neighbours' words: E from +x and +y, H from -x and -y (as offsets
+  // from this tile's).
+  const int fx = (int)(a.nty * tw), fy = (int)tw;
+
+  // Per-z coefficients and psi addresses.
+  float ikE[CPL], bE[CPL], cE[CPL], ikH[CPL], bH[CPL], cH[CPL];
+  bool pml[CPL];
+  int pH[CPL], pE[CPL];  // bytes from a column's block
+#pragma unroll
+  for (int c = 0; c < CPL; ++c) {
+    const int z = min(zb + c, Z - 1);
+    ikE[c] = a.zt[IKE * Z + z];
+    bE[c] = a.zt[BE * Z + z];
+    cE[c] = a.zt[CE * Z + z];
+    ikH[c] = a.zt[IKH * Z + z];
+    bH[c] = a.zt[BH * Z + z];
+    cH[c] = a.zt[CH * Z + z];
+    pml[c] = (zb + c < Z) && (zb + c < a.lo || zb + c >= Z - a.hi);
+    const int pidx = zb + c < a.lo ? zb + c : zb + c - (Z - a.hi) + a.lo;
+    pH[c] = 4 * (pml[c] ? pidx * 2 : NP * 4);
+    pE[c] = 4 * (pml[c] ? NP * 2 + pidx * 2 : NP * 4);
+  }
+
+  auto colx = [&](int i) { return x0 + i; };
+  auto coly = [&](int r) { return y0 + r; };
+  auto valid = [&](int i, int r) { return opaque_s(colx(i)) < X && coly(r) < Y; };
+  auto offset = [&](int i, int r) { return (opaque_s(colx(i)) * Y + coly(r)) * Z; };
+  auto load_state = [&](float (&v)[3][CPL], const float* p, int i, int r) {
+    const bool ok = valid(i, r);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+#pragma unroll
+      for (int c = 0; c < CPL; ++c)
+        v[k][c] = ok && zb + c < Z ? to_global(p)[k * N + offset(i, r) + zb + c] : 0.0f;
+  };
+
+  float e[RX][RY][3][CPL], h[RX][RY][3][CPL], cbr[CBR ? RX : 1][CBR ? RY : 1][3][CPL];
+#pragma unroll
+  for (int i = 0; i < RX; ++i)
+#pragma unroll
+    for (int r = 0; r < RY; ++r) {
+      if (a.Ein) {
+        load_state(e[i][r], a.Ein, i, r);
+        load_state(h[i][r], a.Hin, i, r);
+      } else {
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+#pragma unroll
+          for (int c = 0; c < CPL; ++c) e[i][r][k][c] = h[i][r][k][c] = 0.0f;
+      }
+      if constexpr (CBR) load_state(cbr[i][r], a.cb, i, r);
+    }
+  // psi, absorber and source of the tile into LDS.  Column t there is column
+  // t % C of wave t / C.
+  auto tile_x = [&](int t) { return bx * TX + (t / C) % WX * RX + t % C / RY; };
+  auto tile_y = [&](int t) { return by * TY + (t / C) / WX * RY + t % C % RY; };
+  for (int q = threadIdx.x; q < TX * TY * PS; q += kResThreads) {
+    const int t = q / PS, m = q - t * PS;
+    const int pair = m >= NP * 2, pi = (m - pair * NP * 2) >> 1, comp = pair * 2 + (m & 1);
+    const int x = tile_x(t), y = tile_y(t);
+    psi[q] = a.Ein && m < NP * 4 && x < X && y < Y ? a.psiin[comp * P + (x * Y + y) * NP + pi]
+                                                   : 0.0f;
+  }
+  for (int t = threadIdx.x; t < TX * TY; t += kResThreads) {
+    const int x = tile_x(t), y = tile_y(t);
+    f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (x < X && y < Y) {
+      const int m = x * Y + y, XY = X * Y;
+      s = f32x4{a.mask[m], a.mask[XY + m], a.mask[2 * XY + m], 0.0f};
+    }
+    sig[t] = s;
+  }
+  if (a.saxis < 2) {
+    // (row or column, component, z): the plane's field.
+    const int len = a.saxis == 0 ? Y : X, first = a.saxis == 0 ? by * TY : bx * TX;
+    for (int q = threadIdx.x; q < nsrc; q += kResThreads) {
+      const int t = q / ED, k = (q / (ED / 2)) & 1, z = q % (ED / 2);
+      const int j = first + t;
+      srcl[q] = j < len && z < Z ? a.sfield[((size_t)k * len + j) * Z + z] : 0.0f;
+    }
+  } else {
+    for (int q = threadIdx.x; q < nsrc; q += kResThreads) {
+      const int t = q >> 2, k = q & 3;
+      const int x = tile_x(t), y = tile_y(t);
+      srcl[q] = x < X && y < Y && k < 2 * a.squad ? a.sfield[(size_t)k * X * Y + x * Y + y] : 0.0f;
+    }
+  }
+  bool dead = false;
+
+  // A column's two edge values: to LDS, or as words.
+  auto put_edge = [&](float* p, int k, const float (&u)[CPL], const float (&v)[CPL]) {
+    lds_put<CPL>(p + k * ED, u);
+    lds_put<CPL>(p + k * ED + ED / 2, v);
+  };
+  auto post = [&](rword_t* p, int off, unsigned tag, const float (&u)[CPL],
+                  const float (&v)[CPL]) {
+    rword_t* const q = edge_word(p, off, lane);
+#pragma unroll
+    for (int c = 0; c < CPL; ++c) {
+      post_edge(q + 64 * c, tag, u[c]);
+      post_edge(q + ED / 2 + 64 * c, tag, v[c]);
+    }
+  };
+  // Passes the wave's low edges of E on: through LDS within the workgroup,
+  // as words to its neighbours.
+  auto pass_E = [&](unsigned tag) {
+    // Ey, Ez at the low x edge; Ex, Ez at the low y edge.
+    if (wx > 0) {
+#pragma unroll
+      for (int r = 0; r < RY; ++r) put_edge(slot(exw), r, e[0][r][1], e[0][r][2]);
+    } else if (xlo) {
+#pragma unroll
+      for (int r = 0; r < RY; ++r) post(mine, ox + r * ED, tag, e[0][r][1], e[0][r][2]);
+    }
+    if (wy > 0) {
+#pragma unroll
+      for (int i = 0; i < RX; ++i) put_edge(slot(eyw), i, e[i][0][0], e[i][0][2]);
+    } else if (ylo) {
+#pragma unroll
+      for (int i = 0; i < RX; ++i) post(mine, oy + i * ED, tag, e[i][0][0], e[i][0][2]);
+    }
+  };
+  auto pass_H = [&](unsigned tag) {
+    // Hy, Hz at the high x edge; Hx, Hz at the high y edge.
+    if (wx < WX - 1) {
+#pragma unroll
+      for (int r = 0; r < RY; ++r) put_edge(slot(hxw), r, h[RX - 1][r][1], h[RX - 1][r][2]);
+    } else if (xhi) {
+#pragma unroll
+      for (int r = 0; r < RY; ++r)
+        post(mine, oh + ox + r * ED, tag, h[RX - 1][r][1], h[RX - 1][r][2]);
+    }
+    if (wy < WY - 1) {
+#pragma unroll
+      for (int i = 0; i < RX; ++i) put_edge(slot(hyw), i, h[i][RY - 1][0], h[i][RY - 1][2]);
+    } else if (yhi) {
+#pragma unroll
+      for (int i = 0; i < RX; ++i)
+        post(mine, oh + oy + i * ED, tag, h[i][RY - 1][0], h[i][RY - 1][2]);
+    }
+  };
+  // The outer slots of a wave at the tile's border: the neighbour's edge, or
+  // zeros past the domain.  K columns at a time (the registers of the words).
+  auto take = [&](auto cnt, float* dst, rword_t* base, int off, bool there, unsigned tag) {
+    constexpr int n = decltype(cnt)::value;
+    constexpr int K = CPL == 1 ? 4 : 2;  // columns a poll: 16 registers of words
+#pragma unroll
+    for (int k0 = 0; k0 < n; k0 += K) {
+      constexpr int NW = 2 * CPL;
+      float v[K * NW];
+      if (!there) {
+#pragma unroll
+        for (int q = 0; q < K * NW; ++q) v[q] = 0.0f;
+      } else if (k0 + K <= n) {
+        wait_edges<K * NW>(v, edge_word(base, off + k0 * ED, lane), tag, dead);
+      } else {
+        float u[(n % K ? n % K : K) * NW];
+        wait_edges<(n % K ? n % K : K) * NW>(u, edge_word(base, off + k0 * ED, lane), tag, dead);
+#pragma unroll
+        for (int q = 0; q < (n % K) * NW; ++q) v[q] = u[q];
+      }
+#pragma unroll
+      for (int k = 0; k < K && k0 + k < n; ++k)
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          float t[CPL];
+#pragma unroll
+          for (int c = 0; c < CPL; ++c) t[c] = v[k * NW + q * CPL + c];
+          lds_put<CPL>(dst + (k0 + k) * ED + q * (ED / 2), t);
+        }
+    }
+  };
+  using NX = std::integral_constant<int, RX>;
+  using NY = std::integral_constant<int, RY>;
+
+  __syncthreads();
+  pass_E(a.tag0 + 1);
+
+  // A column's psi pairs (pair 0: H, 1: E), read a column ahead of their use.
+  auto psi_at = [&](int c, int pair, int i, int r) {
+    const int b = (pair ? pE[c] : pH[c]) + opaque_s((w * C + i * RY + r) * PS * 4);
+    return reinterpret_cast<f32x2*>(reinterpret_cast<char*>(lds) + b);
+  };
+  auto load_psi = [&](f32x2 (&v)[CPL], int pair, int i, int r) {
+#pragma unroll
+    for (int c = 0; c < CPL; ++c) v[c] = *psi_at(c, pair, i, r);
+  };
+
+  // H half step of the wave's columns.
+  auto h_phase = [&](unsigned tag) {
+    f32x2 nps[CPL];
+    load_psi(nps, 0, RX - 1 - Order::x(0), RY - 1 - Order::y(0));
+    static_for<C>([&](auto kk) __attribute__((always_inline)) {
+      constexpr int k = decltype(kk)::value;
+      if (k == Order::inner) {
+        // Every wave's E edges are in LDS; the neighbours' on their way.
+        lds_barrier();
+        if (wx == WX - 1) take(NY(), slot(exr), mine, fx + ox, xhi, tag);
+        if (wy == WY - 1) take(NX(), slot(eyr), mine, fy + oy, yhi, tag);
+      }
+      constexpr int i = RX - 1 - Order::x(k), r = RY - 1 - Order::y(k);
+      f32x2 ps[CPL];
+#pragma unroll
+      for (int c = 0; c < CPL; ++c) ps[c] = nps[c];
+      float e1[2][CPL], eup[2][CPL];  // Ey, Ez at x + 1; Ex, Ez at y + 1
+      if (i < RX - 1) {
+#pragma unroll
+        for (int c = 0; c < CPL; ++c) {
+          e1[0][c] = e[i + 1 < RX ? i + 1 : 0][r][1][c];
+          e1[1][c] = e[i + 1 < RX ? i + 1 : 0][r][2][c];
+        }
+      } else {
+        const float* q = slot(exr) + r * ED;
+        lds_get<CPL>(e1[0], q);
+        lds_get<CPL>(e1[1], q + ED / 2);
+      }
+      if (r < RY - 1) {
+#pragma unroll
+        for (int c = 0; c < CPL; ++c) {
+          eup[0][c] = e[i][r + 1 < RY ? r + 1 : 0][0][c];
+          eup[1][c] = e[i][r + 1 < RY ? r + 1 : 0][2][c];
+        }
+      } else {
+        const float* q = slot(eyr) + i * ED;
+        lds_get<CPL>(eup[0], q);
+        lds_get<CPL>(eup[1], q + ED / 2);
+      }
+      const float exn = lane_next(e[i][r][0][0]), eyn = lane_next(e[i][r][1][0]);
+      float tEy[CPL], tEx[CPL];
+#pragma unroll
+      for (int c = 0; c < CPL; ++c) {
+        const float dzEy = (c + 1 < CPL ? e[i][r][1][c + 1 < CPL ? c + 1 : 0] : eyn) - e[i][r][1][c];
+        const float dzEx = (c + 1 < CPL ? e[i][r][0][c + 1 < CPL ? c + 1 : 0] : exn) - e[i][r][0][c];
+        const float p0 = pml[c] ? bH[c] * ps[c].x + cH[c] * dzEy : 0.0f;
+        const float p1 = pml[c] ? bH[c] * ps[c].y + cH[c] * dzEx : 0.0f;
+        *psi_at(c, 0, i, r) = f32x2{p0, p1};
+        tEy[c] = ikH[c] * dzEy + p0;
+        tEx[c] = ikH[c] * dzEx + p1;
+      }
+      // Here, not before this column's own wait for its psi.
+      __builtin_amdgcn_sched_barrier(0);
+      if (k + 1 < C)
+        load_psi(nps, 0, RX - 1 - Order::x(k + 1 < C ? k + 1 : 0),
+                 RY - 1 - Order::y(k + 1 < C ? k + 1 : 0));
+#pragma unroll
+      for (int c = 0; c < CPL; ++c) {
+        h[i][r][0][c] = h[i][r][0][c] - dt * ((eup[1][c] - e[i][r][2][c]) - tEy[c]);
+        h[i][r][1][c] = h[i][r][1][c] - dt * (tEx[c] - (e1[1][c] - e[i][r][2][c]));
+        h[i][r][2][c] = h[i][r][2][c] -
+                        dt * ((e1[0][c] - e[i][r][1][c]) - (eup[0][c] - e[i][r][0][c]));
+#pragma unroll
+        for (int q = 0; q < 3; ++q) pin(h[i][r][q][c]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    if (a.alias) lds_barrier();  // every wave has read E's edges
+    pass_H(tag);
+  };
+
+  // cb of a column from memory, from inside the domain (the selects that make
+  // it zero outside stand at its use: here they would wait for the loads).
+  int zc[CPL];
+#pragma unroll
+  for (int c = 0; c < CPL; ++c) zc[c] = 4 * min(zb + c, Z - 1);
+  auto load_cb = [&](float (&v)[3][CPL], int i, int r) {
+    const int x = min(opaque_s(colx(i)), X - 1), y = min(coly(r), Y - 1);
+    const char* const p = reinterpret_cast<const char*>(a.cb + (x * Y + y) * Z);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+#pragma unroll
+      for (int c = 0; c < CPL; ++c)
+        v[k][c] = *reinterpret_cast<gcfloat*>(
+            to_global(reinterpret_cast<const float*>(p + 4 * (size_t)N * k + (unsigned)opaque_v(zc[c]))));
+  };
+
+  // Of the columns in E's order: those inside the domain, those with a source.
+  int valid_mask = 0, src_mask = 0;
+#pragma unroll
+  for (int k = 0; k < C; ++k) {
+    const int x = colx(Order::x(k)), y = coly(Order::y(k)), at = a.saxis == 0 ? x : y;
+    valid_mask |= (x < X && y < Y ? 1 : 0) << k;
+    src_mask |= (a.saxis == 2 || at == a.spos || at == a.spos - 1 ? 1 : 0) << k;
+  }
+
+  // E half step.
+  auto e_phase = [&](int n, unsigned tag, float w0, float w1) {
+    // Columns of cb in flight, by the registers that are left.
+    constexpr int AHEAD = C * CPL <= 20 ? 6 / CPL : C * CPL <= 25 ? 4 / CPL : C * CPL <= 30 ? 2 : 1;
+    float cbq[AHEAD][3][CPL];
+    f32x2 nps[CPL];
+    const f32x4* const sg0 = sig + w * C;
+    f32x4 nsg = sg0[Order::x(0) * RY + Order::y(0)];
+    load_psi(nps, 1, Order::x(0), Order::y(0));
+    if constexpr (!CBR) {
+#pragma unroll
+      for (int k = 0; k < AHEAD && k < C; ++k) load_cb(cbq[k], Order::x(k), Order::y(k));
+    }
+    static_for<C>([&](auto kk) __attribute__((always_inline)) {
+      constexpr int k = decltype(kk)::value;
+      if (k == Order::inner) {
+        lds_barrier();
+        if (wx == 0) take(NY(), slot(hxr), mine, oh + ox - fx, xlo, tag);
+        if (wy == 0) take(NX(), slot(hyr), mine, oh + oy - fy, ylo, tag);
+      }
+      constexpr int i = Order::x(k), r = Order::y(k);
+      const f32x4 sg = nsg;
+      f32x2 ps[CPL];
+#pragma unroll
+      for (int c = 0; c < CPL; ++c) ps[c] = nps[c];
+      float cb[3][CPL];
+#pragma unroll
+      for (int q = 0; q < 3; ++q)
+#pragma unroll
+        for (int c = 0; c < CPL; ++c)
+          cb[q][c] = CBR ? cbr[CBR ? i : 0][CBR ? r : 0][q][c]
+                         : ((opaque_s(valid_mask) >> k) & 1) && zb + c < Z ? cbq[k % AHEAD][q][c]
+                                                                           : 0.0f;
+      if constexpr (!CBR) {
+        if (k + AHEAD < C)
+          load_cb(cbq[k % AHEAD], Order::x(k + AHEAD < C ? k + AHEAD : 0),
+                  Order::y(k + AHEAD < C ? k + AHEAD : 0));
+      }
+      float hm[2][CPL], hdn[2][CPL];  // Hy, Hz at x - 1; Hx, Hz at y - 1
+      if (i > 0) {
+#pragma unroll
+        for (int c = 0; c < CPL; ++c) {
+          hm[0][c] = h[i > 0 ? i - 1 : 0][r][1][c];
+          hm[1][c] = h[i > 0 ? i - 1 : 0][r][2][c];
+        }
+      } else {
+        const float* q = slot(hxr) + r * ED;
+        lds_get<CPL>(hm[0], q);
+        lds_get<CPL>(hm[1], q + ED / 2);
+      }
+      if (r > 0) {
+#pragma unroll
+        for (int c = 0; c < CPL; ++c) {
+          hdn[0][c] = h[i][r > 0 ? r - 1 : 0][0][c];
+          hdn[1][c] = h[i][r > 0 ? r - 1 : 0][2][c];
+        }
+      } else {
+        const float* q = slot(hyr) + i * ED;
+        lds_get<CPL>(hdn[0], q);
+        lds_get<CPL>(hdn[1], q + ED / 2);
+      }
+      const float hxn = lane_prev(h[i][r][0][CPL - 1]), hyn = lane_prev(h[i][r][1][CPL - 1]);
+      float cx[CPL], cy[CPL], cz[CPL];
+#pragma unroll
+      for (int c = 0; c < CPL; ++c) {
+        const float dzHy = h[i][r][1][c] - (c > 0 ? h[i][r][1][c > 0 ? c - 1 : 0] : hyn);
+        const float dzHx = h[i][r][0][c] - (c > 0 ? h[i][r][0][c > 0 ? c - 1 : 0] : hxn);
+        const float p0 = pml[c] ? bE[c] * ps[c].x + cE[c] * dzHy : 0.0f;
+        const float p1 = pml[c] ? bE[c] * ps[c].y + cE[c] * dzHx : 0.0f;
+        *psi_at(c, 1, i, r) = f32x2{p0, p1};
+        const float tHy = ikE[c] * dzHy + p0;
+        const float tHx = ikE[c] * dzHx + p1;
+        cx[c] = (h[i][r][2][c] - hdn[1][c]) - tHy;
+        cy[c] = tHx - (h[i][r][2][c] - hm[1][c]);
+        cz[c] = (h[i][r][1][c] - hm[0][c]) - (h[i][r][0][c] - hdn[0][c]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if (k + 1 < C) {
+        const int i1 = Order::x(k + 1 < C ? k + 1 : 0), r1 = Order::y(k + 1 < C ? k + 1 : 0);
+        load_psi(nps, 1, i1, r1);
+        nsg = sg0[i1 * RY + r1];
+      }
+      // J as in add_source2: two components, to the axes that they belong to.
+      if ((opaque_s(src_mask) >> k) & 1) {
+        float ju[CPL], jv[CPL];
+        if (a.saxis < 2) {
+          const float wv = (a.saxis == 0 ? colx(i) : coly(r)) == a.spos ? w0 : w1;
+          const float* s = srcl + opaque_s((a.saxis == 0 ? wy * RY + r : wx * RX + i) * ED) + zb;
+#pragma unroll
+          for (int c = 0; c < CPL; ++c) {
+            ju[c] = s[c] * wv;
+            jv[c] = s[ED / 2 + c] * wv;
+          }
+        } else {
+          const f32x4 s = reinterpret_cast<const f32x4*>(srcl)[opaque_s(w * C) + i * RY + r];
+          float jx = s.x * w0, jy = s.y * w0;
+          if (a.squad > 1) {
+            jx += s.z * w1;
+            jy += s.w * w1;
+          }
+#pragma unroll
+          for (int c = 0; c < CPL; ++c) {
+            ju[c] = zb + c == a.spos ? jx : 0.0f;
+            jv[c] = zb + c == a.spos ? jy : 0.0f;
+          }
+        }
+#pragma unroll
+        for (int c = 0; c < CPL; ++c) {
+          cx[c] += a.saxis == 0 ? 0.0f : ju[c];
+          cy[c] += a.saxis == 0 ? ju[c] : (a.saxis == 1 ? 0.0f : jv[c]);
+          cz[c] += a.saxis == 2 ? 0.0f : jv[c];
+        }
+      }
+      float d[3][CPL];
+#pragma unroll
+      for (int c = 0; c < CPL; ++c) {
+        const float o0 = e[i][r][0][c], o1 = e[i][r][1][c], o2 = e[i][r][2][c];
+        // The streaming kernels' rounding: cb K rounded, then one fma.
+        e[i][r][0][c] = __builtin_fmaf(o0, 1.0f - sg.x * cb[0][c], cb[0][c] * cx[c]);
+        e[i][r][1][c] = __builtin_fmaf(o1, 1.0f - sg.y * cb[1][c], cb[1][c] * cy[c]);
+        e[i][r][2][c] = __builtin_fmaf(o2, 1.0f - sg.z * cb[2][c], cb[2][c] * cz[c]);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) pin(e[i][r][q][c]);
+        if constexpr (CAP) {
+          d[0][c] = o0 - e[i][r][0][c];
+          d[1][c] = o1 - e[i][r][1][c];
+          d[2][c] = o2 - e[i][r][2][c];
+        }
+      }
+      if constexpr (CAP) {
+        if (valid(i, r)) {
+          gfloat* q = to_global(a.cap) + (size_t)(n - a.begin) * 3 * N + offset(i, r) + zb;
+#pragma unroll
+          for (int m = 0; m < 3; ++m)
+#pragma unroll
+            for (int c = 0; c < CPL; ++c)
+              if (zb + c < Z) __builtin_nontemporal_store(d[m][c], q + m * N + c);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    if (a.alias) lds_barrier();
+    pass_E(tag + 1);
+  };
+
+  // The state in registers and LDS to E, H (3N each) and psi (4P).
+  auto store_state = [&](float* E, float* H, float* ps) {
+#pragma unroll
+    for (int i = 0; i < RX; ++i)
+#pragma unroll
+      for (int r = 0; r < RY; ++r)
+        if (valid(i, r)) {
+          const int o = offset(i, r) + zb;
+#pragma unroll
+          for (int k = 0; k < 3; ++k)
+#pragma unroll
+            for (int c = 0; c < CPL; ++c)
+              if (zb + c < Z) {
+                to_global(E)[k * N + o + c] = e[i][r][k][c];
+                to_global(H)[k * N + o + c] = h[i][r][k][c];
+              }
+        }
+    for (int q = lane; q < RX * RY * NP * 4; q += 64) {  // own columns: no barrier
+      const int t = q / (NP * 4), m = q - t * NP * 4;
+      const int i = t / RY, r = t - i * RY;
+      const int pair = m / (NP * 2), pi = (m - pair * NP * 2) >> 1, comp = pair * 2 + (m & 1);
+      if (colx(i) < X && coly(r) < Y)
+        to_global(ps)[comp * P + (colx(i) * Y + coly(r)) * NP + pi] =
+            psi[(w * C + t) * PS + m];
+    }
+  };
+
+  float w0 = uniform_load(a.swave, 2 * a.begin), w1 = uniform_load(a.swave, 2 * a.begin + 1);
+  int to_ckpt = a.ckpt ? 0 : -1;
+  for (int n = a.begin; n < a.end; ++n) {
+    const unsigned tag = a.tag0 + 1 + (n - a.begin);
+    if (to_ckpt == 0) {
+      float* q = a.ckpt + (long long)((n - a.begin) / a.every) * a.ckpt_stride;
+      store_state(q, q + 3 * (size_t)N, q + 6 * (size_t)N);
+      to_ckpt = a.every;
+    }
+    --to_ckpt;
+    h_phase(tag);
+    const int m = min(n + 1, a.end - 1);  // the next step's waveform row
+    const float u0 = uniform_load(a.swave, 2 * m), u1 = uniform_load(a.swave, 2 * m + 1);
+    e_phase(n, tag, w0, w1);
+    w0 = u0;
+    w1 = u1;
+    if (dead) e[0][0][0][0] = e[0][0][1][0] = e[0][0][2][0] = __builtin_nanf("");
+    if (a.out && n >= a.ostart && n < a.ostop && (n - a.ostart) % a.ostep == 0) {
+      const int slot = (n - a.ostart) / a.ostep;
+#pragma unroll
+      for (int i = 0; i < RX; ++i)
+#pragma unroll
+        for (int r = 0; r < RY; ++r) {
+          const int x = opaque_s(colx(i)) - a.wx0, y = coly(r) - a.wy0;
+          if (x >= 0 && x < a.wex && y >= 0 && y < a.wey) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+              gfloat* q = to_global(a.out) +
+                          ((((long long)slot * 3 + k) * a.wex + x) * a.wey + y) * (long long)a.wez;
+#pragma unroll
+              for (int c = 0; c < CPL; ++c) {
+                const int z = zb + c - a.wz0;
+                if (z >= 0 && z < a.wez) q[z] = e[i][r][k][c];
+              }
+            }
+          }
+        }
+    }
+  }
+  if (a.Eout) store_state(a.Eout, a.Hout, a.psiout);
+}
+
+// ------------------------------------------------------------------ host side
+
+namespace {
+
+// The kernels: columns a wave.
+struct ResShape {
+  int cpl, rx, ry;
+};
+#define PJZ_RES_SHAPES(F)                                                                   \
+  F(1, 2, 1) F(1, 2, 2) F(1, 3, 2) F(1, 4, 2) F(1, 4, 3) F(1, 4, 4) F(1, 5, 4) F(1, 5, 5)   \
+  F(1, 6, 5) F(1, 8, 4)                                                                     \
+  F(2, 1, 1) F(2, 2, 1) F(2, 2, 2) F(2, 3, 2) F(2, 4, 2) F(2, 5, 2) F(2, 4, 3) F(2, 5, 3)   \
+  F(2, 4, 4)
+constexpr ResShape kShapes[] = {
+#define PJZ_RES_ROW(c, x, y) {c, x, y},
+    PJZ_RES_SHAPES(PJZ_RES_ROW)
+#undef PJZ_RES_ROW
+};
+
+size_t res_lds(const Geom& g, int saxis, int cpl, int tx, int ty, int wx, int wy, bool alias) {
+  const size_t ed = 2 * 64 * cpl;
+  const size_t nsrc = saxis == 0 ? ty * ed : saxis == 1 ? tx * ed : (size_t)tx * ty * 4;
+  const size_t edge = (size_t)(wx * ty + wy * tx) * ed;
+  const size_t psi = ((size_t)tx * ty * (g.NP * 4 + 2) + 3) & ~(size_t)3;
+  return sizeof(float) * (psi + (size_t)tx * ty * 4 + nsrc + edge * (alias ? 1 : 2));
+}
+
+}  // namespace
+
+ResPlan resident_plan(const Geom& g, int saxis, int cus) {
+  ResPlan best{};
+  if (g.Z > 128) return best;
+  const int cpl = g.Z <= 64 ? 1 : 2;
+  // Cost of a step: the columns a wave computes, one after the other.
+  int cost = 0;
+  for (const ResShape& s : kShapes) {
+    if (s.cpl != cpl) continue;
+    for (int wx = 1; wx <= kResWaves; wx *= 2) {
+      ResPlan p{s.cpl, s.rx, s.ry, wx, kResWaves / wx, 0, 0, false, 0};
+      p.ntx = (g.X + p.tx() - 1) / p.tx();
+      p.nty = (g.Y + p.ty() - 1) / p.ty();
+      if ((long long)p.ntx * p.nty > cus) continue;
+      p.lds = res_lds(g, saxis, cpl, p.tx(), p.ty(), p.wx, p.wy, false);
+      if (p.lds > kResLds) {
+        p.alias = true;
+        p.lds = res_lds(g, saxis, cpl, p.tx(), p.ty(), p.wx, p.wy, true);
+        if (p.lds > kResLds) continue;
+      }
+      // More than half of a compute unit's LDS: one workgroup each.
+      p.lds = std::max(p.lds, kResLds / 2 + 1024);
+      // The words take the place of the second set of E and H.
+      if (p.words() * sizeof(rword_t) > 2 * align256(sizeof(float) * 3 * (size_t)g.N)) continue;
+      const int c = 64 * s.rx * s.ry + 2 * (s.rx + s.ry) + (p.alias ? 8 : 0) + p.tx() + p.ty();
+      if (!best.rx || c < cost) {
+        best = p;
+        cost = c;
+      }
+    }
+  }
+  return best;
+}
+
+template <int CPL, int RX, int RY, bool CAP>
+static hipError_t launch_resident(ResArgs& a, const ResPlan& p, hipStream_t s) {
+  const void* k = reinterpret_cast<const void*>(&k_resident<CPL, RX, RY, CAP>);
+  hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)p.lds);
+  if (e != hipSuccess) return e;
+  void* args[] = {&a};
+  return hipLaunchCooperativeKernel(k, dim3(p.tiles()), dim3(kResThreads), args, (unsigned)p.lds,
+                                    s);
+}
+
+hipError_t run_resident(const Geom& g, const pjz_fdtd_problem& p, const float* mask,
+                        const Src& src, const OutWin& win, char* ws, const Layout& L,
+                        const ResPlan& plan, const ResRun& r, hipStream_t s) {
+  ResArgs a;
+  a.Ein = r.in.E;
+  a.Hin = r.in.H;
+  a.psiin = r.in.psi;
+  a.Eout = r.out.E;
+  a.Hout = r.out.H;
+  a.psiout = r.out.psi;
+  a.cb = (const float*)(ws + L.cb);
+  a.zt = (const float*)(ws + L.zt);
+  a.mask = mask;
+  a.sfield = src.field;
+  a.swave = src.wave;
+  a.out = win.out;
+  a.cap = r.capture;
+  a.ckpt = r.ckpt;
+  a.ckpt_stride = (long long)(ckpt_stride(L) / sizeof(float));
+  a.every = r.every;
+  a.words = (rword_t*)(ws + L.E1);
+  a.X = g.X; a.Y = g.Y; a.Z = g.Z; a.lo = g.lo; a.hi = g.hi; a.NP = g.NP;
+  a.N = (int)g.N;
+  a.P = g.X * g.Y * g.NP;
+  a.saxis = src.axis; a.spos = src.pos; a.squad = src.quad;
+  a.dt = p.dt;
+  a.begin = r.begin;
+  a.end = r.end;
+  a.tag0 = r.tag0;
+  a.wx = plan.wx;
+  a.wy = plan.wy;
+  a.ntx = plan.ntx;
+  a.nty = plan.nty;
+  a.alias = plan.alias;
+  a.wx0 = win.x0; a.wy0 = win.y0; a.wz0 = win.z0;
+  a.wex = win.ex; a.wey = win.ey; a.wez = win.ez;
+  a.ostart = p.out_start; a.ostop = p.out_stop; a.ostep = p.out_step;
+#define PJZ_RES_LAUNCH(c, x, y)                                               \
+  if (plan.cpl == c && plan.rx == x && plan.ry == y)                          \
+    return r.capture ? launch_resident<c, x, y, true>(a, plan, s)             \
+                     : launch_resident<c, x, y, false>(a, plan, s);
+  PJZ_RES_SHAPES(PJZ_RES_LAUNCH)
+#undef PJZ_RES_LAUNCH
+  return hipErrorInvalidValue;
+}
+
+}  // namespace pjz
