@@ -303,7 +303,7 @@ constexpr int kResidentMinSteps = 16;
 // be.
 pjz::ResPlan resident_for(const pjz::Geom& g, const pjz_fdtd_problem& p, hipStream_t s) {
   const pjz::ResPlan none{};
-  if (p.kernel != PJZ_FDTD_KERNEL_AUTO || p.tile_x != 0 || p.tile_y != 0 ||
+  if (p.kernel != PJZ_FDTD_KERNEL_AUTO || p.tile_x != 0 || p.tile_y != 0 || p.graph_steps != 0 ||
       pjz::steps_of(p) < kResidentMinSteps)
     return none;
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
@@ -372,6 +372,128 @@ hipError_t save_state(const pjz::Geom& g, const pjz::Layout& L, char* ws, int cu
 hipError_t restore_state(const pjz::Geom& g, const pjz::Layout& L, char* ws, int k,
                          hipStream_t s) {
   return copy_state(g, L, ws, 0, k, false, s);
+}
+
+// A forward call's steps by the resident stepper: the whole run in one launch,
+// its checkpoints written on the way.
+hipError_t forward_resident(const pjz::Geom& g, const pjz_fdtd_problem& p, const float* mask,
+                            const pjz::Src& src, const pjz::OutWin& win, char* ws,
+                            const pjz::Layout& L, const pjz::ResPlan& plan, hipStream_t s) {
+  hipError_t e = clear_words(plan, L, ws, s);
+  if (e != hipSuccess) return e;
+  pjz::ResRun r{0, pjz::steps_of(p), {}, {}, nullptr, nullptr, L.S1, 0};
+  if (L.nck > 0) r.ckpt = ckpt_state(g, L, ws, 0).E;
+  return pjz::run_resident(g, p, mask, src, win, ws, L, plan, r, s);
+}
+
+// Every step of a backward call reversed, segment by segment: cb, the cleared
+// adjoint state and the forward's checkpoints are in the workspace, the sum G
+// is left there.
+hipError_t backward_steps(const pjz::Geom& g, const pjz_fdtd_problem& p,
+                          const float* absorption_mask, const pjz::Src& src,
+                          const float* grad_out, char* ws, const pjz::Layout& L,
+                          pjz::ResPlan plan, hipStream_t s) {
+  const int nsteps = pjz::steps_of(p);
+  const long long f3 = 3 * g.N;
+  // The reference kernel choice also selects the cell-by-cell reverse step.
+  const bool stream_adj =
+      p.kernel != PJZ_FDTD_KERNEL_REFERENCE && pjz::adjoint_stream_supported(g);
+  // Two reversed steps per launch unless the one-step kernels were asked for.
+  const bool stream2_adj = stream_adj && p.kernel != PJZ_FDTD_KERNEL_STREAM &&
+                           pjz::adjoint_stream2_supported(g);
+  pjz::OutWin nowin{p.x0, p.y0, p.z0, p.ex, p.ey, p.ez, nullptr};
+  float* seg = (float*)(ws + L.seg);
+  const long long gstride = 3LL * p.ex * p.ey * p.ez;
+  int acur = 0;  // adjoint set holding the current cotangents
+  auto is_out = [&](int n) {
+    return n >= p.out_start && n < p.out_stop && (n - p.out_start) % p.out_step == 0;
+  };
+  if (!pjz::resident_captures(plan)) plan = {};
+  const bool resident_adj = plan.rx > 0 && pjz::adjoint_resident_supported(plan);
+  unsigned tags = 0;  // exchange numbers used
+  hipError_t e = hipSuccess;
+  if (plan.rx > 0) e = clear_words(plan, L, ws, s);
+  if (e != hipSuccess) return e;
+  // Steps [b, end) of the resident stepper from checkpoint slot k.
+  auto resident = [&](int k, int b, int end, pjz::ResState out, float* capture, float* ckpt,
+                      int every) {
+    const pjz::ResRun r{b, end, ckpt_state(g, L, ws, k), out, capture, ckpt, every, tags};
+    tags += pjz::resident_tags(end - b);
+    return pjz::run_resident(g, p, absorption_mask, src, nowin, ws, L, plan, r, s);
+  };
+  // Steps [b, end) from the state in checkpoint slot k: recompute them
+  // capturing D^n = E^n - E^(n+1), then reverse them.
+  auto reverse_segment = [&](int k, int b, int end) {
+    int cur = 0;
+    hipError_t e = plan.rx > 0 ? resident(k, b, end, {}, seg, nullptr, 1)
+                               : restore_state(g, L, ws, k, s);
+    if (e == hipSuccess && plan.rx == 0)
+      e = run_steps(g, p, absorption_mask, src, nowin, ws, L, b, end, &cur, seg, s);
+    if (e == hipSuccess && resident_adj) {
+      e = pjz::run_adjoint_resident(g, p, absorption_mask, ws, L, plan, seg, grad_out, b, end,
+                                    tags, s);
+      tags += pjz::resident_tags(end - b);
+      return e;
+    }
+    for (int n = end - 1; n >= b && e == hipSuccess;) {
+      if (is_out(n))
+        e = pjz::launch_inject(g, p, (float*)(ws + L.lE_[acur]),
+                               grad_out + gstride * ((n - p.out_start) / p.out_step), s);
+      if (e != hipSuccess) break;
+      if (stream2_adj && n - 1 >= b && !is_out(n - 1)) {
+        // Steps n and n-1 in one launch (no cotangent enters between them).
+        e = pjz::launch_adjoint_stream2(g, p, absorption_mask, ws, L, seg + (n - b) * f3,
+                                        seg + (n - 1 - b) * f3, acur, s);
+        acur = 1 - acur;
+        n -= 2;
+      } else if (stream_adj) {
+        e = pjz::launch_adjoint_stream(g, p, absorption_mask, ws, L, seg + (n - b) * f3, acur,
+                                       s);
+        acur = 1 - acur;
+        --n;
+      } else {
+        e = pjz::launch_adjoint_step(g, p, absorption_mask, ws, L, seg + (n - b) * f3, acur, s);
+        --n;
+      }
+    }
+    return e;
+  };
+  for (int k = L.nck - 1; k >= 0 && e == hipSuccess; --k) {
+    const int b1 = k * L.S1, e1 = b1 + L.S1 < nsteps ? b1 + L.S1 : nsteps;
+    if (L.nfine == 0) {
+      e = reverse_segment(k, b1, e1);
+      continue;
+    }
+    // Two levels: recompute the S1 segment from its checkpoint keeping the
+    // state every S steps (slots nck + j), then reverse its sub-segments.
+    if (plan.rx > 0) {
+      const int nsub = (e1 - b1 + L.S - 1) / L.S;
+      const int last = b1 + (nsub - 1) * L.S;
+      // Slots nck .. nck + nsub - 1; the first is slot k itself.
+      if (nsub > 1)
+        e = resident(k, b1, last, ckpt_state(g, L, ws, L.nck + nsub - 1), nullptr,
+                     ckpt_state(g, L, ws, L.nck).E, L.S);
+      for (int j = nsub - 1; j >= 0 && e == hipSuccess; --j)
+        e = reverse_segment(j == 0 ? k : L.nck + j, b1 + j * L.S,
+                            j == nsub - 1 ? e1 : b1 + (j + 1) * L.S);
+      continue;
+    }
+    int cur = 0;
+    e = restore_state(g, L, ws, k, s);
+    int nsub = 0;
+    for (int b = b1; b < e1 && e == hipSuccess; b += L.S, ++nsub) {
+      e = save_state(g, L, ws, cur, L.nck + nsub, s);
+      const int end = b + L.S < e1 ? b + L.S : e1;
+      // The last sub-segment's steps are recomputed again below.
+      if (e == hipSuccess && end < e1)
+        e = run_steps(g, p, absorption_mask, src, nowin, ws, L, b, end, &cur, nullptr, s);
+    }
+    for (int j = nsub - 1; j >= 0 && e == hipSuccess; --j) {
+      const int b = b1 + j * L.S, end = b + L.S < e1 ? b + L.S : e1;
+      e = reverse_segment(L.nck + j, b, end);
+    }
+  }
+  return e;
 }
 
 }  // namespace
@@ -602,11 +724,7 @@ int pjz_fdtd_forward(const pjz_fdtd_problem* p, const float* epsilon,
   const int nsteps = pjz::steps_of(*p);
   const pjz::ResPlan plan = resident_for(g, *p, s);
   if (plan.rx > 0) {
-    // The whole run in one launch, its checkpoints written on the way.
-    e = clear_words(plan, L, ws, s);
-    pjz::ResRun r{0, nsteps, {}, {}, nullptr, nullptr, L.S1, 0};
-    if (L.nck > 0) r.ckpt = ckpt_state(g, L, ws, 0).E;
-    if (e == hipSuccess) e = pjz::run_resident(g, *p, absorption_mask, src, win, ws, L, plan, r, s);
+    e = forward_resident(g, *p, absorption_mask, src, win, ws, L, plan, s);
     return e == hipSuccess ? PJZ_FDTD_OK : hip_fail(e, "resident launch");
   }
   e = pjz::launch_zero((float*)(ws + L.E0), (L.E1 - L.E0) / sizeof(float), s);
@@ -667,9 +785,9 @@ int pjz_fdtd_forward_noalloc(const pjz_fdtd_problem* p, const float* epsilon,
 
 namespace {
 
-int max_steps(const pjz_fdtd_problem* probs, int n) {
+int max_steps(const std::vector<pjz::BatchItem>& items) {
   int m = 0;
-  for (int i = 0; i < n; ++i) m = std::max(m, pjz::steps_of(probs[i]));
+  for (const pjz::BatchItem& it : items) m = std::max(m, pjz::steps_of(*it.p));
   return m;
 }
 
@@ -771,6 +889,33 @@ int batch_setup(const pjz_fdtd_problem* probs, int n, const BatchPlanHost& bp,
   return PJZ_FDTD_OK;
 }
 
+// The simulations of a batch that run by themselves, one after the other, on
+// the resident stepper (their tilings, rx = 0 for the others, which share the
+// batched launches).  A resident step takes about 2.5 us and 0.3 us for every
+// cell a lane, twice that where cb comes from memory (past 16 cells); a
+// simulation's share of a batched step is its cells at 90 per ns, and no
+// batched step is shorter than 12 us.
+std::vector<pjz::ResPlan> batch_resident(const pjz_fdtd_problem* probs, int n, hipStream_t s) {
+  std::vector<pjz::ResPlan> plans(n);
+  double all_res = 0, all_batch = 0;
+  bool fit = true;
+  auto res_us = [](const pjz::ResPlan& p) {
+    const int c = p.cpl * p.rx * p.ry;
+    return 2.5 + (c <= 16 ? 0.3 : 0.6) * c;
+  };
+  auto share_us = [](const pjz_fdtd_problem& q) { return (double)geom_of(q).N / 90e3; };
+  for (int i = 0; i < n; ++i) {
+    plans[i] = resident_for(geom_of(probs[i]), probs[i], s);
+    fit = fit && plans[i].rx > 0;
+    if (plans[i].rx > 0) all_res += res_us(plans[i]);
+    all_batch += share_us(probs[i]);
+  }
+  if (fit && all_res <= std::max(12.0, all_batch)) return plans;
+  for (int i = 0; i < n; ++i)
+    if (plans[i].rx > 0 && res_us(plans[i]) > share_us(probs[i])) plans[i] = {};
+  return plans;
+}
+
 }  // namespace
 
 extern "C" {
@@ -799,20 +944,32 @@ int pjz_fdtd_batch_forward(const pjz_fdtd_problem* probs, int n, const float* co
                    source_field, source_waveform, out, workspace, workspace_bytes, false, s, items);
   if (rc) return rc;
   char* base = (char*)workspace;
-  pjz::Batch2Plan plan;
-  hipError_t e = pjz::batch2_prepare(items.data(), n, base + bp.meta_off, plan, s, bp.S == 0);
-  if (e == hipSuccess && bp.S == 0) e = pjz::batch2_forward(plan, s);
-  // With checkpoints: before the pairs of segment k, save the state of step
-  // k*S (buffer set (k*S/2) & 1) of every simulation that reaches it.
-  for (int k = 0; bp.S > 0 && e == hipSuccess && k * bp.S < 2 * plan.npairs; ++k) {
-    const int b = k * bp.S;
-    for (int i = 0; i < n && e == hipSuccess; ++i)
-      if (k < bp.Ls[i].nck)
-        e = copy_state(items[i].g, bp.Ls[i], items[i].ws, (b / 2) & 1, k, true, s);
-    if (e == hipSuccess) e = pjz::batch2_pairs(plan, b / 2, (b + bp.S) / 2, s);
+  const std::vector<pjz::ResPlan> res = batch_resident(probs, n, s);
+  std::vector<pjz::BatchItem> rest;  // of the batched launches
+  hipError_t e = hipSuccess;
+  for (int i = 0; i < n && e == hipSuccess; ++i) {
+    const pjz::BatchItem& it = items[i];
+    if (res[i].rx > 0)
+      e = forward_resident(it.g, *it.p, it.mask, it.src, it.win, it.ws, *it.L, res[i], s);
+    else
+      rest.push_back(it);
   }
-  const hipError_t r = pjz::batch2_release(plan, s);
-  if (e == hipSuccess) e = r;
+  if (e == hipSuccess && !rest.empty()) {
+    pjz::Batch2Plan plan;
+    e = pjz::batch2_prepare(rest.data(), (int)rest.size(), base + bp.meta_off, plan, s, bp.S == 0);
+    if (e == hipSuccess && bp.S == 0) e = pjz::batch2_forward(plan, s);
+    // With checkpoints: before the pairs of segment k, save the state of step
+    // k*S (buffer set (k*S/2) & 1) of every simulation that reaches it.
+    for (int k = 0; bp.S > 0 && e == hipSuccess && k * bp.S < 2 * plan.npairs; ++k) {
+      const int b = k * bp.S;
+      for (const pjz::BatchItem& it : rest)
+        if (e == hipSuccess && k < it.L->nck)
+          e = copy_state(it.g, *it.L, it.ws, (b / 2) & 1, k, true, s);
+      if (e == hipSuccess) e = pjz::batch2_pairs(plan, b / 2, (b + bp.S) / 2, s);
+    }
+    const hipError_t r = pjz::batch2_release(plan, s);
+    if (e == hipSuccess) e = r;
+  }
   if (e != hipSuccess) return hip_fail(e, "batch launch");
   return PJZ_FDTD_OK;
 }
@@ -841,91 +998,107 @@ int pjz_fdtd_batch_backward(const pjz_fdtd_problem* probs, int n, const float* c
                    items);
   if (rc) return rc;
   char* base = (char*)workspace;
-  const int last_seg = (std::max(1, max_steps(probs, n)) - 1) / bp.S;
-  auto seg_end = [&](int k) {
-    int end = k * bp.S;
-    for (int i = 0; i < n; ++i)
-      if (k < bp.Ls[i].nck) end = std::max(end, std::min((k + 1) * bp.S, pjz::steps_of(probs[i])));
-    return end;
-  };
-  auto is_out = [&](int i, int m) {
-    const pjz_fdtd_problem& q = probs[i];
-    return m < pjz::steps_of(q) && m >= q.out_start && m < q.out_stop &&
-           (m - q.out_start) % q.out_step == 0;
-  };
-  // The reverse schedule, fixed up front: launches of one or two reversed
-  // steps in decreasing step order, segment by segment.  A pair (m, m-1) is
-  // used unless a snapshot cotangent enters some simulation at m-1 or some
-  // simulation's first reversed step is m-1.  lstart[i]: the launch a
-  // simulation joins at (its adjoint set is (launch - lstart) & 1).
-  struct RevLaunch {
-    int m, b;
-    bool two;
-  };
-  std::vector<RevLaunch> sched;
-  std::vector<int> lstart(n, 0);
-  std::vector<bool> joined(n, false);
-  for (int k = last_seg; k >= 0; --k) {
-    const int b = k * bp.S;
-    for (int m = seg_end(k) - 1; m >= b;) {
-      bool two = m - 1 >= b;
-      for (int i = 0; i < n && two; ++i)
-        if (pjz::steps_of(probs[i]) == m || is_out(i, m - 1)) two = false;
-      for (int i = 0; i < n; ++i)
-        if (!joined[i] && m < pjz::steps_of(probs[i])) {
-          joined[i] = true;
-          lstart[i] = (int)sched.size();
-        }
-      sched.push_back({m, b, two});
-      m -= two ? 2 : 1;
+  const std::vector<pjz::ResPlan> res = batch_resident(probs, n, s);
+  std::vector<pjz::BatchItem> rest;  // of the batched launches, their cotangents
+  std::vector<const float*> gout;
+  hipError_t e = hipSuccess;
+  for (int i = 0; i < n && e == hipSuccess; ++i) {
+    const pjz::BatchItem& it = items[i];
+    if (res[i].rx > 0 && bp.Ls[i].nck > 0) {
+      e = backward_steps(it.g, *it.p, it.mask, it.src, grad_out[i], it.ws, *it.L, res[i], s);
+    } else {
+      rest.push_back(it);
+      gout.push_back(grad_out[i]);
     }
   }
-  pjz::Batch2Plan plan;
-  pjz::AdjBatchPlan aplan;
-  pjz::Adj2BatchPlan a2plan;
-  hipError_t e = pjz::batch2_prepare(items.data(), n, base + bp.meta_off, plan, s);
-  if (e == hipSuccess)
-    e = pjz::adjoint_batch_prepare(items.data(), n, bp.S, lstart.data(), base + bp.adj_off, aplan,
-                                   s);
-  if (e == hipSuccess)
-    e = pjz::adjoint2_batch_prepare(items.data(), n, bp.S, lstart.data(), base + bp.adj2_off,
-                                    a2plan, s);
-  size_t L = 0;
-  for (int k = last_seg; k >= 0 && e == hipSuccess; --k) {
-    const int b = k * bp.S;
-    // Recompute segment k of every simulation that reaches it from its
-    // checkpoint, capturing D^n = E^n - E^(n+1) (slot n - b).
-    for (int i = 0; i < n && e == hipSuccess; ++i) {
-      const pjz::Layout& Li = bp.Ls[i];
-      if (k >= Li.nck) continue;
-      e = copy_state(items[i].g, Li, items[i].ws, (b / 2) & 1, k, false, s);
-    }
-    if (e == hipSuccess) e = pjz::batch2_capture_from(plan, b, s);
-    if (e == hipSuccess) e = pjz::batch2_pairs(plan, b / 2, (seg_end(k) + 1) / 2, s);
-    if (e == hipSuccess) e = pjz::adjoint_batch_begin_segment(aplan, s);
-    if (e == hipSuccess) e = pjz::adjoint2_batch_begin_segment(a2plan, s);
-    for (; L < sched.size() && sched[L].b == b && e == hipSuccess; ++L) {
-      const int m = sched[L].m;
-      for (int i = 0; i < n && e == hipSuccess; ++i) {
-        if (!is_out(i, m)) continue;
-        const pjz_fdtd_problem& q = probs[i];
-        const long long gstride = 3LL * q.ex * q.ey * q.ez;
-        e = pjz::launch_inject(items[i].g, q,
-                               (float*)(items[i].ws + bp.Ls[i].lE_[((int)L - lstart[i]) & 1]),
-                               grad_out[i] + gstride * ((m - q.out_start) / q.out_step), s);
+  const int nr = (int)rest.size();
+  if (e == hipSuccess && nr > 0) {
+    const int last_seg = (std::max(1, max_steps(rest)) - 1) / bp.S;
+    auto seg_end = [&](int k) {
+      int end = k * bp.S;
+      for (const pjz::BatchItem& it : rest)
+        if (k < it.L->nck) end = std::max(end, std::min((k + 1) * bp.S, pjz::steps_of(*it.p)));
+      return end;
+    };
+    auto is_out = [&](int i, int m) {
+      const pjz_fdtd_problem& q = *rest[i].p;
+      return m < pjz::steps_of(q) && m >= q.out_start && m < q.out_stop &&
+             (m - q.out_start) % q.out_step == 0;
+    };
+    // The reverse schedule, fixed up front: launches of one or two reversed
+    // steps in decreasing step order, segment by segment.  A pair (m, m-1) is
+    // used unless a snapshot cotangent enters some simulation at m-1 or some
+    // simulation's first reversed step is m-1.  lstart[i]: the launch a
+    // simulation joins at (its adjoint set is (launch - lstart) & 1).
+    struct RevLaunch {
+      int m, b;
+      bool two;
+    };
+    std::vector<RevLaunch> sched;
+    std::vector<int> lstart(nr, 0);
+    std::vector<bool> joined(nr, false);
+    for (int k = last_seg; k >= 0; --k) {
+      const int b = k * bp.S;
+      for (int m = seg_end(k) - 1; m >= b;) {
+        bool two = m - 1 >= b;
+        for (int i = 0; i < nr && two; ++i)
+          if (pjz::steps_of(*rest[i].p) == m || is_out(i, m - 1)) two = false;
+        for (int i = 0; i < nr; ++i)
+          if (!joined[i] && m < pjz::steps_of(*rest[i].p)) {
+            joined[i] = true;
+            lstart[i] = (int)sched.size();
+          }
+        sched.push_back({m, b, two});
+        m -= two ? 2 : 1;
       }
-      if (e != hipSuccess) break;
-      e = sched[L].two ? pjz::launch_adjoint2_batch_step(a2plan, (int)L, m, b, s)
-                       : pjz::launch_adjoint_batch_step(aplan, (int)L, m, b, s);
     }
+    pjz::Batch2Plan plan;
+    pjz::AdjBatchPlan aplan;
+    pjz::Adj2BatchPlan a2plan;
+    e = pjz::batch2_prepare(rest.data(), nr, base + bp.meta_off, plan, s);
+    if (e == hipSuccess)
+      e = pjz::adjoint_batch_prepare(rest.data(), nr, bp.S, lstart.data(), base + bp.adj_off, aplan,
+                                     s);
+    if (e == hipSuccess)
+      e = pjz::adjoint2_batch_prepare(rest.data(), nr, bp.S, lstart.data(), base + bp.adj2_off,
+                                      a2plan, s);
+    size_t L = 0;
+    for (int k = last_seg; k >= 0 && e == hipSuccess; --k) {
+      const int b = k * bp.S;
+      // Recompute segment k of every simulation that reaches it from its
+      // checkpoint, capturing D^n = E^n - E^(n+1) (slot n - b).
+      for (int i = 0; i < nr && e == hipSuccess; ++i) {
+        const pjz::Layout& Li = *rest[i].L;
+        if (k >= Li.nck) continue;
+        e = copy_state(rest[i].g, Li, rest[i].ws, (b / 2) & 1, k, false, s);
+      }
+      if (e == hipSuccess) e = pjz::batch2_capture_from(plan, b, s);
+      if (e == hipSuccess) e = pjz::batch2_pairs(plan, b / 2, (seg_end(k) + 1) / 2, s);
+      if (e == hipSuccess) e = pjz::adjoint_batch_begin_segment(aplan, s);
+      if (e == hipSuccess) e = pjz::adjoint2_batch_begin_segment(a2plan, s);
+      for (; L < sched.size() && sched[L].b == b && e == hipSuccess; ++L) {
+        const int m = sched[L].m;
+        for (int i = 0; i < nr && e == hipSuccess; ++i) {
+          if (!is_out(i, m)) continue;
+          const pjz_fdtd_problem& q = *rest[i].p;
+          const long long gstride = 3LL * q.ex * q.ey * q.ez;
+          e = pjz::launch_inject(rest[i].g, q,
+                                 (float*)(rest[i].ws + (*rest[i].L).lE_[((int)L - lstart[i]) & 1]),
+                                 gout[i] + gstride * ((m - q.out_start) / q.out_step), s);
+        }
+        if (e != hipSuccess) break;
+        e = sched[L].two ? pjz::launch_adjoint2_batch_step(a2plan, (int)L, m, b, s)
+                         : pjz::launch_adjoint_batch_step(aplan, (int)L, m, b, s);
+      }
+    }
+    const hipError_t r = pjz::batch2_release(plan, s);
+    if (e == hipSuccess) e = r;
   }
   for (int i = 0; i < n && e == hipSuccess; ++i)
     e = bp.Ls[i].nck == 0  // no steps: nothing depends on epsilon
             ? pjz::launch_zero(grad_eps[i], 3 * (size_t)probs[i].ex * probs[i].ey * probs[i].ez, s)
             : pjz::launch_grad_eps(items[i].g, probs[i], epsilon[i], absorption_mask[i],
                                    items[i].ws, bp.Ls[i], grad_eps[i], s);
-  const hipError_t r = pjz::batch2_release(plan, s);
-  if (e == hipSuccess) e = r;
   if (e != hipSuccess) return hip_fail(e, "batch backward launch");
   return PJZ_FDTD_OK;
 }
@@ -951,11 +1124,8 @@ int pjz_fdtd_backward(const pjz_fdtd_problem* p, const float* epsilon,
     return fail(PJZ_FDTD_EINVAL, "workspace must be 256-byte aligned");
   hipStream_t s = (hipStream_t)stream;
   char* ws = (char*)workspace;
-  const long long f3 = 3 * g.N;
-  const size_t P = (size_t)g.X * g.Y * (size_t)(g.NP > 0 ? g.NP : 1);
-  const int nsteps = pjz::steps_of(*p);
   hipError_t e = hipSuccess;
-  if (nsteps == 0) {
+  if (pjz::steps_of(*p) == 0) {
     e = pjz::launch_zero(grad_eps, 3 * (size_t)p->ex * p->ey * p->ez, s);
     return e == hipSuccess ? PJZ_FDTD_OK : hip_fail(e, "zero grad");
   }
@@ -965,98 +1135,8 @@ int pjz_fdtd_backward(const pjz_fdtd_problem* p, const float* epsilon,
   if (e == hipSuccess)
     e = pjz::launch_zero((float*)(ws + L.lE_[0]), (L.total - L.lE_[0]) / 4, s);
   if (e != hipSuccess) return hip_fail(e, "backward set-up");
-  // The reference kernel choice also selects the cell-by-cell reverse step.
-  const bool stream_adj =
-      p->kernel != PJZ_FDTD_KERNEL_REFERENCE && pjz::adjoint_stream_supported(g);
-  // Two reversed steps per launch unless the one-step kernels were asked for.
-  const bool stream2_adj = stream_adj && p->kernel != PJZ_FDTD_KERNEL_STREAM &&
-                           pjz::adjoint_stream2_supported(g);
   pjz::Src src{p->src_axis, p->src_pos, p->src_quad, source_field, source_waveform};
-  pjz::OutWin nowin{p->x0, p->y0, p->z0, p->ex, p->ey, p->ez, nullptr};
-  float* seg = (float*)(ws + L.seg);
-  const long long gstride = 3LL * p->ex * p->ey * p->ez;
-  int acur = 0;  // adjoint set holding the current cotangents
-  (void)P;
-  auto is_out = [&](int n) {
-    return n >= p->out_start && n < p->out_stop && (n - p->out_start) % p->out_step == 0;
-  };
-  const pjz::ResPlan plan = resident_for(g, *p, s);
-  unsigned tags = 0;  // exchange numbers used
-  if (plan.rx > 0) e = clear_words(plan, L, ws, s);
-  if (e != hipSuccess) return hip_fail(e, "backward set-up");
-  // Steps [b, end) of the resident stepper from checkpoint slot k.
-  auto resident = [&](int k, int b, int end, pjz::ResState out, float* capture, float* ckpt,
-                      int every) {
-    const pjz::ResRun r{b, end, ckpt_state(g, L, ws, k), out, capture, ckpt, every, tags};
-    tags += pjz::resident_tags(end - b);
-    return pjz::run_resident(g, *p, absorption_mask, src, nowin, ws, L, plan, r, s);
-  };
-  // Steps [b, end) from the state in checkpoint slot k: recompute them
-  // capturing D^n = E^n - E^(n+1), then reverse them.
-  auto reverse_segment = [&](int k, int b, int end) {
-    int cur = 0;
-    hipError_t e = plan.rx > 0 ? resident(k, b, end, {}, seg, nullptr, 1)
-                               : restore_state(g, L, ws, k, s);
-    if (e == hipSuccess && plan.rx == 0)
-      e = run_steps(g, *p, absorption_mask, src, nowin, ws, L, b, end, &cur, seg, s);
-    for (int n = end - 1; n >= b && e == hipSuccess;) {
-      if (is_out(n))
-        e = pjz::launch_inject(g, *p, (float*)(ws + L.lE_[acur]),
-                               grad_out + gstride * ((n - p->out_start) / p->out_step), s);
-      if (e != hipSuccess) break;
-      if (stream2_adj && n - 1 >= b && !is_out(n - 1)) {
-        // Steps n and n-1 in one launch (no cotangent enters between them).
-        e = pjz::launch_adjoint_stream2(g, *p, absorption_mask, ws, L, seg + (n - b) * f3,
-                                        seg + (n - 1 - b) * f3, acur, s);
-        acur = 1 - acur;
-        n -= 2;
-      } else if (stream_adj) {
-        e = pjz::launch_adjoint_stream(g, *p, absorption_mask, ws, L, seg + (n - b) * f3, acur,
-                                       s);
-        acur = 1 - acur;
-        --n;
-      } else {
-        e = pjz::launch_adjoint_step(g, *p, absorption_mask, ws, L, seg + (n - b) * f3, acur, s);
-        --n;
-      }
-    }
-    return e;
-  };
-  for (int k = L.nck - 1; k >= 0 && e == hipSuccess; --k) {
-    const int b1 = k * L.S1, e1 = b1 + L.S1 < nsteps ? b1 + L.S1 : nsteps;
-    if (L.nfine == 0) {
-      e = reverse_segment(k, b1, e1);
-      continue;
-    }
-    // Two levels: recompute the S1 segment from its checkpoint keeping the
-    // state every S steps (slots nck + j), then reverse its sub-segments.
-    if (plan.rx > 0) {
-      const int nsub = (e1 - b1 + L.S - 1) / L.S;
-      const int last = b1 + (nsub - 1) * L.S;
-      // Slots nck .. nck + nsub - 1; the first is slot k itself.
-      if (nsub > 1)
-        e = resident(k, b1, last, ckpt_state(g, L, ws, L.nck + nsub - 1), nullptr,
-                     ckpt_state(g, L, ws, L.nck).E, L.S);
-      for (int j = nsub - 1; j >= 0 && e == hipSuccess; --j)
-        e = reverse_segment(j == 0 ? k : L.nck + j, b1 + j * L.S,
-                            j == nsub - 1 ? e1 : b1 + (j + 1) * L.S);
-      continue;
-    }
-    int cur = 0;
-    e = restore_state(g, L, ws, k, s);
-    int nsub = 0;
-    for (int b = b1; b < e1 && e == hipSuccess; b += L.S, ++nsub) {
-      e = save_state(g, L, ws, cur, L.nck + nsub, s);
-      const int end = b + L.S < e1 ? b + L.S : e1;
-      // The last sub-segment's steps are recomputed again below.
-      if (e == hipSuccess && end < e1)
-        e = run_steps(g, *p, absorption_mask, src, nowin, ws, L, b, end, &cur, nullptr, s);
-    }
-    for (int j = nsub - 1; j >= 0 && e == hipSuccess; --j) {
-      const int b = b1 + j * L.S, end = b + L.S < e1 ? b + L.S : e1;
-      e = reverse_segment(L.nck + j, b, end);
-    }
-  }
+  e = backward_steps(g, *p, absorption_mask, src, grad_out, ws, L, resident_for(g, *p, s), s);
   if (e == hipSuccess)
     e = pjz::launch_grad_eps(g, *p, epsilon, absorption_mask, ws, L, grad_eps, s);
   if (e != hipSuccess) return hip_fail(e, "backward launch");

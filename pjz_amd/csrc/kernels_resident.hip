@@ -54,47 +54,15 @@ struct ResArgs {
   float* out;        // snapshots (or null)
   float* cap;        // E^n - E^(n+1) at cap + (n - begin) * 3N (CAP kernels)
   float* ckpt;       // states before steps begin, begin + every, ... (or null)
-  rword_t* words;
   long long ckpt_stride;  // floats
   int every;
-  int X, Y, Z, lo, hi, NP, N, P;
+  ResTileArgs t;
   int saxis, spos, squad;
   float dt;
   int begin, end;
   unsigned tag0;     // exchange numbers tag0 + 1 .. tag0 + 2 (end - begin) + 1
-  int wx, wy, ntx, nty;
-  int alias;
   int wx0, wy0, wz0, wex, wey, wez, ostart, ostop, ostep;
 };
-
-// The columns of a wave in the order they are computed: first those that need
-// no other wave's edge.  E needs the low neighbours; H, mirrored, the high.
-template <int RX, int RY>
-struct ColOrder {
-  static constexpr int inner = (RX - 1) * (RY - 1);
-  static constexpr int x(int k) {
-    return k < inner ? 1 + k / (RY > 1 ? RY - 1 : 1) : (k - inner < RX ? k - inner : 0);
-  }
-  static constexpr int y(int k) {
-    return k < inner ? 1 + k % (RY > 1 ? RY - 1 : 1) : (k - inner < RX ? 0 : k - inner - RX + 1);
-  }
-};
-
-template <int CPL>
-__device__ __forceinline__ void lds_put(float* p, const float (&v)[CPL]) {
-  if constexpr (CPL == 2) *reinterpret_cast<f32x2*>(p) = f32x2{v[0], v[1]};
-  else p[0] = v[0];
-}
-template <int CPL>
-__device__ __forceinline__ void lds_get(float (&v)[CPL], const float* p) {
-  if constexpr (CPL == 2) {
-    const f32x2 t = *reinterpret_cast<const f32x2*>(p);
-    v[0] = t.x;
-    v[1] = t.y;
-  } else {
-    v[0] = p[0];
-  }
-}
 
 // Registers: 6 a cell for E and H, 3 more for cb where that still fits; past
 // it cb (12 of the 60 bytes a streaming step moves a cell) is read from the
@@ -105,63 +73,18 @@ constexpr bool res_keeps_cb() { return CPL * RX * RY <= 16; }
 template <int CPL, int RX, int RY, bool CAP>
 __global__ __launch_bounds__(kResThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 k_resident(ResArgs a) {
-  constexpr int C = RX * RY;
-  constexpr bool CBR = res_keeps_cb<CPL, RX, RY>();
-  constexpr int ED = 2 * 64 * CPL;  // floats (or words) of an edge column
+  using Tile = ResTile<CPL, RX, RY>;
   using Order = ColOrder<RX, RY>;
-  const int lane = threadIdx.x & 63;
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int WX = a.wx, WY = a.wy;
-  // Quotients of uniform values are computed on the vector unit: back to
-  // scalar registers, or all that follows from them takes vector registers.
-  const int wx = __builtin_amdgcn_readfirstlane(w % WX);
-  const int wy = __builtin_amdgcn_readfirstlane(w / WX);
-  const int TX = RX * WX, TY = RY * WY;
-  const int X = a.X, Y = a.Y, Z = a.Z, N = a.N, P = a.P, NP = a.NP;
-  const int nt = a.ntx * a.nty;
-  // Consecutive workgroups go round-robin over the 8 XCDs; neighbouring tiles
-  // go to one XCD where the count allows it.
-  int tile = blockIdx.x;
-  if ((nt & 7) == 0) tile = (tile & 7) * (nt >> 3) + (tile >> 3);
-  const int bx = __builtin_amdgcn_readfirstlane(tile / a.nty);
-  const int by = __builtin_amdgcn_readfirstlane(tile % a.nty);
-  const int x0 = bx * TX + wx * RX, y0 = by * TY + wy * RY;
-  const int zb = lane * CPL;
-  const float dt = a.dt;
-
-  // LDS: psi as (column, H or E pair, PML cell, 2) and, per column, a zero pair
-  // for the lanes outside the PML (so every lane's address steps alike);
-  // absorber values and source of the tile; edge buffers.
+  constexpr int C = Tile::C, ED = Tile::ED;
+  constexpr bool CBR = res_keeps_cb<CPL, RX, RY>();
   extern __shared__ float lds[];
-  float* const psi = lds;
-  const int PS = NP * 4 + 2;
-  f32x4* const sig = reinterpret_cast<f32x4*>(psi + ((TX * TY * PS + 3) & ~3));
-  float* const srcl = reinterpret_cast<float*>(sig + TX * TY);
-  const int nsrc = a.saxis == 0 ? TY * ED : a.saxis == 1 ? TX * ED : TX * TY * 4;
-  float* const edgeE = srcl + nsrc;
-  const int nedge = (WX * TY + WY * TX) * ED;
-  float* const edgeH = a.alias ? edgeE : edgeE + nedge;
-  // Edge slot s of a direction lies between waves s - 1 and s.  E is read
-  // from slot w + 1 and written to slot w, H read from w and written to w + 1;
-  // slots 1 .. WX (E) and 0 .. WX - 1 (H) exist, the outer one holding the
-  // neighbouring workgroup's edge.
-  // (Float offsets, uniform: the lane's address is made where it is used.)
-  const int eoff = (int)(edgeE - lds), hoff = (int)(edgeH - lds);
-  const int sx = (wx * TY + wy * RY) * ED, sy = (WX * TY + wy * TX + wx * RX) * ED;
-  const int exr = eoff + sx, exw = eoff + sx - TY * ED;  // exw if wx > 0
-  const int eyr = eoff + sy, eyw = eoff + sy - TX * ED;  // eyw if wy > 0
-  const int hxr = hoff + sx, hxw = hoff + sx + TY * ED;  // hxw if wx < WX - 1
-  const int hyr = hoff + sy, hyw = hoff + sy + TX * ED;  // hyw if wy < WY - 1
-  auto slot = [&](int off) { return lds + opaque_s(off) + zb; };
-  // A tile's words: E low x (TY columns), E low y (TX), H high x, H high y.
-  const size_t tw = (size_t)2 * (TX + TY) * ED;
-  rword_t* const mine = a.words + (size_t)tile * tw;
-  const int ox = wy * RY * ED, oy = TY * ED + wx * RX * ED, oh = (TX + TY) * ED;
-  const bool xlo = wx == 0 && bx > 0, xhi = wx == WX - 1 && bx + 1 < a.ntx;
-  const bool ylo = wy == 0 && by > 0, yhi = wy == WY - 1 && by + 1 < a.nty;
-  // Of the neighbours' words: E from +x and +y, H from -x and -y (as offsets
-  // from this tile's).
-  const int fx = (int)(a.nty * tw), fy = (int)tw;
+  Tile T(a.t, lds);
+  const int X = a.t.X, Y = a.t.Y, Z = a.t.Z, N = a.t.N, P = a.t.P, NP = a.t.NP;
+  const int zb = T.zb;
+  const float dt = a.dt;
+  const int nsrc = a.saxis == 0 ? T.TY * ED : a.saxis == 1 ? T.TX * ED : T.TX * T.TY * 4;
+  float* const srcl = T.own();
+  T.edges(nsrc);
 
   // Per-z coefficients and psi addresses.
   float ikE[CPL], bE[CPL], cE[CPL], ikH[CPL], bH[CPL], cH[CPL];
@@ -176,24 +99,11 @@ k_resident(ResArgs a) {
     ikH[c] = a.zt[IKH * Z + z];
     bH[c] = a.zt[BH * Z + z];
     cH[c] = a.zt[CH * Z + z];
-    pml[c] = (zb + c < Z) && (zb + c < a.lo || zb + c >= Z - a.hi);
-    const int pidx = zb + c < a.lo ? zb + c : zb + c - (Z - a.hi) + a.lo;
+    pml[c] = (zb + c < Z) && (zb + c < a.t.lo || zb + c >= Z - a.t.hi);
+    const int pidx = zb + c < a.t.lo ? zb + c : zb + c - (Z - a.t.hi) + a.t.lo;
     pH[c] = 4 * (pml[c] ? pidx * 2 : NP * 4);
     pE[c] = 4 * (pml[c] ? NP * 2 + pidx * 2 : NP * 4);
   }
-
-  auto colx = [&](int i) { return x0 + i; };
-  auto coly = [&](int r) { return y0 + r; };
-  auto valid = [&](int i, int r) { return opaque_s(colx(i)) < X && coly(r) < Y; };
-  auto offset = [&](int i, int r) { return (opaque_s(colx(i)) * Y + coly(r)) * Z; };
-  auto load_state = [&](float (&v)[3][CPL], const float* p, int i, int r) {
-    const bool ok = valid(i, r);
-#pragma unroll
-    for (int k = 0; k < 3; ++k)
-#pragma unroll
-      for (int c = 0; c < CPL; ++c)
-        v[k][c] = ok && zb + c < Z ? to_global(p)[k * N + offset(i, r) + zb + c] : 0.0f;
-  };
 
   float e[RX][RY][3][CPL], h[RX][RY][3][CPL], cbr[CBR ? RX : 1][CBR ? RY : 1][3][CPL];
 #pragma unroll
@@ -201,39 +111,20 @@ k_resident(ResArgs a) {
 #pragma unroll
     for (int r = 0; r < RY; ++r) {
       if (a.Ein) {
-        load_state(e[i][r], a.Ein, i, r);
-        load_state(h[i][r], a.Hin, i, r);
+        T.load(e[i][r], a.Ein, N, i, r);
+        T.load(h[i][r], a.Hin, N, i, r);
       } else {
 #pragma unroll
         for (int k = 0; k < 3; ++k)
 #pragma unroll
           for (int c = 0; c < CPL; ++c) e[i][r][k][c] = h[i][r][k][c] = 0.0f;
       }
-      if constexpr (CBR) load_state(cbr[i][r], a.cb, i, r);
+      if constexpr (CBR) T.load(cbr[i][r], a.cb, N, i, r);
     }
-  // psi, absorber and source of the tile into LDS.  Column t there is column
-  // t % C of wave t / C.
-  auto tile_x = [&](int t) { return bx * TX + (t / C) % WX * RX + t % C / RY; };
-  auto tile_y = [&](int t) { return by * TY + (t / C) / WX * RY + t % C % RY; };
-  for (int q = threadIdx.x; q < TX * TY * PS; q += kResThreads) {
-    const int t = q / PS, m = q - t * PS;
-    const int pair = m >= NP * 2, pi = (m - pair * NP * 2) >> 1, comp = pair * 2 + (m & 1);
-    const int x = tile_x(t), y = tile_y(t);
-    psi[q] = a.Ein && m < NP * 4 && x < X && y < Y ? a.psiin[comp * P + (x * Y + y) * NP + pi]
-                                                   : 0.0f;
-  }
-  for (int t = threadIdx.x; t < TX * TY; t += kResThreads) {
-    const int x = tile_x(t), y = tile_y(t);
-    f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (x < X && y < Y) {
-      const int m = x * Y + y, XY = X * Y;
-      s = f32x4{a.mask[m], a.mask[XY + m], a.mask[2 * XY + m], 0.0f};
-    }
-    sig[t] = s;
-  }
+  T.fill(a.psiin, a.psiin ? a.psiin + 2 * (size_t)P : nullptr, P, a.mask);
   if (a.saxis < 2) {
     // (row or column, component, z): the plane's field.
-    const int len = a.saxis == 0 ? Y : X, first = a.saxis == 0 ? by * TY : bx * TX;
+    const int len = a.saxis == 0 ? Y : X, first = a.saxis == 0 ? T.by * T.TY : T.bx * T.TX;
     for (int q = threadIdx.x; q < nsrc; q += kResThreads) {
       const int t = q / ED, k = (q / (ED / 2)) & 1, z = q % (ED / 2);
       const int j = first + t;
@@ -242,105 +133,18 @@ k_resident(ResArgs a) {
   } else {
     for (int q = threadIdx.x; q < nsrc; q += kResThreads) {
       const int t = q >> 2, k = q & 3;
-      const int x = tile_x(t), y = tile_y(t);
+      const int x = T.tile_x(t), y = T.tile_y(t);
       srcl[q] = x < X && y < Y && k < 2 * a.squad ? a.sfield[(size_t)k * X * Y + x * Y + y] : 0.0f;
     }
   }
   bool dead = false;
 
-  // A column's two edge values: to LDS, or as words.
-  auto put_edge = [&](float* p, int k, const float (&u)[CPL], const float (&v)[CPL]) {
-    lds_put<CPL>(p + k * ED, u);
-    lds_put<CPL>(p + k * ED + ED / 2, v);
-  };
-  auto post = [&](rword_t* p, int off, unsigned tag, const float (&u)[CPL],
-                  const float (&v)[CPL]) {
-    rword_t* const q = edge_word(p, off, lane);
-#pragma unroll
-    for (int c = 0; c < CPL; ++c) {
-      post_edge(q + 64 * c, tag, u[c]);
-      post_edge(q + ED / 2 + 64 * c, tag, v[c]);
-    }
-  };
-  // Passes the wave's low edges of E on: through LDS within the workgroup,
-  // as words to its neighbours.
-  auto pass_E = [&](unsigned tag) {
-    // Ey, Ez at the low x edge; Ex, Ez at the low y edge.
-    if (wx > 0) {
-#pragma unroll
-      for (int r = 0; r < RY; ++r) put_edge(slot(exw), r, e[0][r][1], e[0][r][2]);
-    } else if (xlo) {
-#pragma unroll
-      for (int r = 0; r < RY; ++r) post(mine, ox + r * ED, tag, e[0][r][1], e[0][r][2]);
-    }
-    if (wy > 0) {
-#pragma unroll
-      for (int i = 0; i < RX; ++i) put_edge(slot(eyw), i, e[i][0][0], e[i][0][2]);
-    } else if (ylo) {
-#pragma unroll
-      for (int i = 0; i < RX; ++i) post(mine, oy + i * ED, tag, e[i][0][0], e[i][0][2]);
-    }
-  };
-  auto pass_H = [&](unsigned tag) {
-    // Hy, Hz at the high x edge; Hx, Hz at the high y edge.
-    if (wx < WX - 1) {
-#pragma unroll
-      for (int r = 0; r < RY; ++r) put_edge(slot(hxw), r, h[RX - 1][r][1], h[RX - 1][r][2]);
-    } else if (xhi) {
-#pragma unroll
-      for (int r = 0; r < RY; ++r)
-        post(mine, oh + ox + r * ED, tag, h[RX - 1][r][1], h[RX - 1][r][2]);
-    }
-    if (wy < WY - 1) {
-#pragma unroll
-      for (int i = 0; i < RX; ++i) put_edge(slot(hyw), i, h[i][RY - 1][0], h[i][RY - 1][2]);
-    } else if (yhi) {
-#pragma unroll
-      for (int i = 0; i < RX; ++i)
-        post(mine, oh + oy + i * ED, tag, h[i][RY - 1][0], h[i][RY - 1][2]);
-    }
-  };
-  // The outer slots of a wave at the tile's border: the neighbour's edge, or
-  // zeros past the domain.  K columns at a time (the registers of the words).
-  auto take = [&](auto cnt, float* dst, rword_t* base, int off, bool there, unsigned tag) {
-    constexpr int n = decltype(cnt)::value;
-    constexpr int K = CPL == 1 ? 4 : 2;  // columns a poll: 16 registers of words
-#pragma unroll
-    for (int k0 = 0; k0 < n; k0 += K) {
-      constexpr int NW = 2 * CPL;
-      float v[K * NW];
-      if (!there) {
-#pragma unroll
-        for (int q = 0; q < K * NW; ++q) v[q] = 0.0f;
-      } else if (k0 + K <= n) {
-        wait_edges<K * NW>(v, edge_word(base, off + k0 * ED, lane), tag, dead);
-      } else {
-        float u[(n % K ? n % K : K) * NW];
-        wait_edges<(n % K ? n % K : K) * NW>(u, edge_word(base, off + k0 * ED, lane), tag, dead);
-#pragma unroll
-        for (int q = 0; q < (n % K) * NW; ++q) v[q] = u[q];
-      }
-#pragma unroll
-      for (int k = 0; k < K && k0 + k < n; ++k)
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-          float t[CPL];
-#pragma unroll
-          for (int c = 0; c < CPL; ++c) t[c] = v[k * NW + q * CPL + c];
-          lds_put<CPL>(dst + (k0 + k) * ED + q * (ED / 2), t);
-        }
-    }
-  };
-  using NX = std::integral_constant<int, RX>;
-  using NY = std::integral_constant<int, RY>;
-
   __syncthreads();
-  pass_E(a.tag0 + 1);
+  T.pass_low(a.tag0 + 1, e);
 
   // A column's psi pairs (pair 0: H, 1: E), read a column ahead of their use.
   auto psi_at = [&](int c, int pair, int i, int r) {
-    const int b = (pair ? pE[c] : pH[c]) + opaque_s((w * C + i * RY + r) * PS * 4);
-    return reinterpret_cast<f32x2*>(reinterpret_cast<char*>(lds) + b);
+    return T.psi_at(pair ? pE[c] : pH[c], i, r);
   };
   auto load_psi = [&](f32x2 (&v)[CPL], int pair, int i, int r) {
 #pragma unroll
@@ -353,12 +157,7 @@ k_resident(ResArgs a) {
     load_psi(nps, 0, RX - 1 - Order::x(0), RY - 1 - Order::y(0));
     static_for<C>([&](auto kk) __attribute__((always_inline)) {
       constexpr int k = decltype(kk)::value;
-      if (k == Order::inner) {
-        // Every wave's E edges are in LDS; the neighbours' on their way.
-        lds_barrier();
-        if (wx == WX - 1) take(NY(), slot(exr), mine, fx + ox, xhi, tag);
-        if (wy == WY - 1) take(NX(), slot(eyr), mine, fy + oy, yhi, tag);
-      }
+      if (k == Order::inner) T.take_low(tag, dead);
       constexpr int i = RX - 1 - Order::x(k), r = RY - 1 - Order::y(k);
       f32x2 ps[CPL];
 #pragma unroll
@@ -371,7 +170,7 @@ k_resident(ResArgs a) {
           e1[1][c] = e[i + 1 < RX ? i + 1 : 0][r][2][c];
         }
       } else {
-        const float* q = slot(exr) + r * ED;
+        const float* q = T.low_x() + r * ED;
         lds_get<CPL>(e1[0], q);
         lds_get<CPL>(e1[1], q + ED / 2);
       }
@@ -382,7 +181,7 @@ k_resident(ResArgs a) {
           eup[1][c] = e[i][r + 1 < RY ? r + 1 : 0][2][c];
         }
       } else {
-        const float* q = slot(eyr) + i * ED;
+        const float* q = T.low_y() + i * ED;
         lds_get<CPL>(eup[0], q);
         lds_get<CPL>(eup[1], q + ED / 2);
       }
@@ -414,8 +213,8 @@ k_resident(ResArgs a) {
       }
       __builtin_amdgcn_sched_barrier(0);
     });
-    if (a.alias) lds_barrier();  // every wave has read E's edges
-    pass_H(tag);
+    T.edges_read();
+    T.pass_high(tag, h);
   };
 
   // cb of a column from memory, from inside the domain (the selects that make
@@ -424,7 +223,7 @@ k_resident(ResArgs a) {
 #pragma unroll
   for (int c = 0; c < CPL; ++c) zc[c] = 4 * min(zb + c, Z - 1);
   auto load_cb = [&](float (&v)[3][CPL], int i, int r) {
-    const int x = min(opaque_s(colx(i)), X - 1), y = min(coly(r), Y - 1);
+    const int x = min(opaque_s(T.colx(i)), X - 1), y = min(T.coly(r), Y - 1);
     const char* const p = reinterpret_cast<const char*>(a.cb + (x * Y + y) * Z);
 #pragma unroll
     for (int k = 0; k < 3; ++k)
@@ -438,7 +237,7 @@ k_resident(ResArgs a) {
   int valid_mask = 0, src_mask = 0;
 #pragma unroll
   for (int k = 0; k < C; ++k) {
-    const int x = colx(Order::x(k)), y = coly(Order::y(k)), at = a.saxis == 0 ? x : y;
+    const int x = T.colx(Order::x(k)), y = T.coly(Order::y(k)), at = a.saxis == 0 ? x : y;
     valid_mask |= (x < X && y < Y ? 1 : 0) << k;
     src_mask |= (a.saxis == 2 || at == a.spos || at == a.spos - 1 ? 1 : 0) << k;
   }
@@ -449,7 +248,7 @@ k_resident(ResArgs a) {
     constexpr int AHEAD = C * CPL <= 20 ? 6 / CPL : C * CPL <= 25 ? 4 / CPL : C * CPL <= 30 ? 2 : 1;
     float cbq[AHEAD][3][CPL];
     f32x2 nps[CPL];
-    const f32x4* const sg0 = sig + w * C;
+    const f32x4* const sg0 = T.sig() + T.w * C;
     f32x4 nsg = sg0[Order::x(0) * RY + Order::y(0)];
     load_psi(nps, 1, Order::x(0), Order::y(0));
     if constexpr (!CBR) {
@@ -458,11 +257,7 @@ k_resident(ResArgs a) {
     }
     static_for<C>([&](auto kk) __attribute__((always_inline)) {
       constexpr int k = decltype(kk)::value;
-      if (k == Order::inner) {
-        lds_barrier();
-        if (wx == 0) take(NY(), slot(hxr), mine, oh + ox - fx, xlo, tag);
-        if (wy == 0) take(NX(), slot(hyr), mine, oh + oy - fy, ylo, tag);
-      }
+      if (k == Order::inner) T.take_high(tag, dead);
       constexpr int i = Order::x(k), r = Order::y(k);
       const f32x4 sg = nsg;
       f32x2 ps[CPL];
@@ -489,7 +284,7 @@ k_resident(ResArgs a) {
           hm[1][c] = h[i > 0 ? i - 1 : 0][r][2][c];
         }
       } else {
-        const float* q = slot(hxr) + r * ED;
+        const float* q = T.high_x() + r * ED;
         lds_get<CPL>(hm[0], q);
         lds_get<CPL>(hm[1], q + ED / 2);
       }
@@ -500,7 +295,7 @@ k_resident(ResArgs a) {
           hdn[1][c] = h[i][r > 0 ? r - 1 : 0][2][c];
         }
       } else {
-        const float* q = slot(hyr) + i * ED;
+        const float* q = T.high_y() + i * ED;
         lds_get<CPL>(hdn[0], q);
         lds_get<CPL>(hdn[1], q + ED / 2);
       }
@@ -529,15 +324,15 @@ k_resident(ResArgs a) {
       if ((opaque_s(src_mask) >> k) & 1) {
         float ju[CPL], jv[CPL];
         if (a.saxis < 2) {
-          const float wv = (a.saxis == 0 ? colx(i) : coly(r)) == a.spos ? w0 : w1;
-          const float* s = srcl + opaque_s((a.saxis == 0 ? wy * RY + r : wx * RX + i) * ED) + zb;
+          const float wv = (a.saxis == 0 ? T.colx(i) : T.coly(r)) == a.spos ? w0 : w1;
+          const float* s = srcl + opaque_s((a.saxis == 0 ? T.wy * RY + r : T.wx * RX + i) * ED) + zb;
 #pragma unroll
           for (int c = 0; c < CPL; ++c) {
             ju[c] = s[c] * wv;
             jv[c] = s[ED / 2 + c] * wv;
           }
         } else {
-          const f32x4 s = reinterpret_cast<const f32x4*>(srcl)[opaque_s(w * C) + i * RY + r];
+          const f32x4 s = reinterpret_cast<const f32x4*>(srcl)[opaque_s(T.w * C) + i * RY + r];
           float jx = s.x * w0, jy = s.y * w0;
           if (a.squad > 1) {
             jx += s.z * w1;
@@ -573,8 +368,8 @@ k_resident(ResArgs a) {
         }
       }
       if constexpr (CAP) {
-        if (valid(i, r)) {
-          gfloat* q = to_global(a.cap) + (size_t)(n - a.begin) * 3 * N + offset(i, r) + zb;
+        if (T.valid(i, r)) {
+          gfloat* q = to_global(a.cap) + (size_t)(n - a.begin) * 3 * N + T.offset(i, r) + zb;
 #pragma unroll
           for (int m = 0; m < 3; ++m)
 #pragma unroll
@@ -584,8 +379,8 @@ k_resident(ResArgs a) {
       }
       __builtin_amdgcn_sched_barrier(0);
     });
-    if (a.alias) lds_barrier();
-    pass_E(tag + 1);
+    T.edges_read();
+    T.pass_low(tag + 1, e);
   };
 
   // The state in registers and LDS to E, H (3N each) and psi (4P).
@@ -594,25 +389,11 @@ k_resident(ResArgs a) {
     for (int i = 0; i < RX; ++i)
 #pragma unroll
       for (int r = 0; r < RY; ++r)
-        if (valid(i, r)) {
-          const int o = offset(i, r) + zb;
-#pragma unroll
-          for (int k = 0; k < 3; ++k)
-#pragma unroll
-            for (int c = 0; c < CPL; ++c)
-              if (zb + c < Z) {
-                to_global(E)[k * N + o + c] = e[i][r][k][c];
-                to_global(H)[k * N + o + c] = h[i][r][k][c];
-              }
+        if (T.valid(i, r)) {
+          T.store(E, e[i][r], N, i, r);
+          T.store(H, h[i][r], N, i, r);
         }
-    for (int q = lane; q < RX * RY * NP * 4; q += 64) {  // own columns: no barrier
-      const int t = q / (NP * 4), m = q - t * NP * 4;
-      const int i = t / RY, r = t - i * RY;
-      const int pair = m / (NP * 2), pi = (m - pair * NP * 2) >> 1, comp = pair * 2 + (m & 1);
-      if (colx(i) < X && coly(r) < Y)
-        to_global(ps)[comp * P + (colx(i) * Y + coly(r)) * NP + pi] =
-            psi[(w * C + t) * PS + m];
-    }
+    T.store_psi(ps, ps + 2 * (size_t)P, P);
   };
 
   float w0 = uniform_load(a.swave, 2 * a.begin), w1 = uniform_load(a.swave, 2 * a.begin + 1);
@@ -638,7 +419,7 @@ k_resident(ResArgs a) {
       for (int i = 0; i < RX; ++i)
 #pragma unroll
         for (int r = 0; r < RY; ++r) {
-          const int x = opaque_s(colx(i)) - a.wx0, y = coly(r) - a.wy0;
+          const int x = opaque_s(T.colx(i)) - a.wx0, y = T.coly(r) - a.wy0;
           if (x >= 0 && x < a.wex && y >= 0 && y < a.wey) {
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
@@ -749,20 +530,12 @@ hipError_t run_resident(const Geom& g, const pjz_fdtd_problem& p, const float* m
   a.ckpt = r.ckpt;
   a.ckpt_stride = (long long)(ckpt_stride(L) / sizeof(float));
   a.every = r.every;
-  a.words = (rword_t*)(ws + L.E1);
-  a.X = g.X; a.Y = g.Y; a.Z = g.Z; a.lo = g.lo; a.hi = g.hi; a.NP = g.NP;
-  a.N = (int)g.N;
-  a.P = g.X * g.Y * g.NP;
+  a.t = tile_args(g, plan, (rword_t*)(ws + L.E1));
   a.saxis = src.axis; a.spos = src.pos; a.squad = src.quad;
   a.dt = p.dt;
   a.begin = r.begin;
   a.end = r.end;
   a.tag0 = r.tag0;
-  a.wx = plan.wx;
-  a.wy = plan.wy;
-  a.ntx = plan.ntx;
-  a.nty = plan.nty;
-  a.alias = plan.alias;
   a.wx0 = win.x0; a.wy0 = win.y0; a.wz0 = win.z0;
   a.wex = win.ex; a.wey = win.ey; a.wez = win.ez;
   a.ostart = p.out_start; a.ostop = p.out_stop; a.ostep = p.out_step;

@@ -80,6 +80,35 @@ __device__ __forceinline__ void wait_edges(float (&v)[NW], const rword_t* p, uns
   for (int k = 0; k < NW; ++k) v[k] = __uint_as_float((unsigned)w[k]);
 }
 
+template <int CPL>
+__device__ __forceinline__ void lds_put(float* p, const float (&v)[CPL]) {
+  if constexpr (CPL == 2) *reinterpret_cast<f32x2*>(p) = f32x2{v[0], v[1]};
+  else p[0] = v[0];
+}
+template <int CPL>
+__device__ __forceinline__ void lds_get(float (&v)[CPL], const float* p) {
+  if constexpr (CPL == 2) {
+    const f32x2 t = *reinterpret_cast<const f32x2*>(p);
+    v[0] = t.x;
+    v[1] = t.y;
+  } else {
+    v[0] = p[0];
+  }
+}
+
+// The columns of a wave in the order they are computed: first those that need
+// no other wave's edge.  E needs the low neighbours; H, mirrored, the high.
+template <int RX, int RY>
+struct ColOrder {
+  static constexpr int inner = (RX - 1) * (RY - 1);
+  static constexpr int x(int k) {
+    return k < inner ? 1 + k / (RY > 1 ? RY - 1 : 1) : (k - inner < RX ? k - inner : 0);
+  }
+  static constexpr int y(int k) {
+    return k < inner ? 1 + k % (RY > 1 ? RY - 1 : 1) : (k - inner < RX ? 0 : k - inner - RX + 1);
+  }
+};
+
 constexpr int kResWaves = 8;  // two waves a SIMD, 256 registers a lane each
 constexpr int kResThreads = 64 * kResWaves;
 constexpr size_t kResLds = 160 << 10;
@@ -98,6 +127,286 @@ struct ResPlan {
   // Words of a tile's edges: E and H, 2 components of tx + ty columns.
   size_t words() const { return (size_t)tiles() * 4 * (tx() + ty()) * 64 * cpl; }
 };
+
+// A workgroup's tile as one of its waves sees it: where its columns lie, and
+// the passing of edges.  Low edges are those of E (lK in the reverse run),
+// which the waves below and to the left read; high edges those of H.  At x
+// edges components 1 and 2 are passed, at y edges 0 and 2.
+struct ResTileArgs {
+  int X, Y, Z, N, P, lo, hi, NP;
+  int wx, wy, ntx, nty, alias;
+  rword_t* words;
+};
+
+template <int CPL, int RX, int RY>
+struct ResTile {
+  static constexpr int C = RX * RY;
+  static constexpr int ED = 2 * 64 * CPL;  // floats (or words) of an edge column
+  int lane, w, wx, wy, WX, WY, TX, TY, bx, by, x0, y0, zb, X, Y, Z, NP, PS;
+  float* lds;
+  int er, hr, sx, sy;  // see edges()
+  rword_t* mine;
+  int ox, oy, oh, fx, fy;
+  bool xlo, xhi, ylo, yhi;
+  bool alias;
+
+  __device__ __forceinline__ ResTile(const ResTileArgs& a, float* lds_) {
+    lane = threadIdx.x & 63;
+    w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    WX = a.wx;
+    WY = a.wy;
+    // Quotients of uniform values are computed on the vector unit: back to
+    // scalar registers, or all that follows from them takes vector registers.
+    wx = __builtin_amdgcn_readfirstlane(w % WX);
+    wy = __builtin_amdgcn_readfirstlane(w / WX);
+    TX = RX * WX;
+    TY = RY * WY;
+    X = a.X;
+    Y = a.Y;
+    Z = a.Z;
+    NP = a.NP;
+    const int nt = a.ntx * a.nty;
+    // Consecutive workgroups go round-robin over the 8 XCDs; neighbouring
+    // tiles go to one XCD where the count allows it.
+    int tile = blockIdx.x;
+    if ((nt & 7) == 0) tile = (tile & 7) * (nt >> 3) + (tile >> 3);
+    bx = __builtin_amdgcn_readfirstlane(tile / a.nty);
+    by = __builtin_amdgcn_readfirstlane(tile % a.nty);
+    x0 = bx * TX + wx * RX;
+    y0 = by * TY + wy * RY;
+    zb = lane * CPL;
+    lds = lds_;
+    PS = NP * 4 + 2;
+    alias = a.alias;
+    // A tile's words: low x edge (TY columns), low y (TX), high x, high y.
+    // Of the neighbours' (as offsets from this tile's): the low edges from +x
+    // and +y, the high ones from -x and -y.
+    const size_t tw = (size_t)2 * (TX + TY) * ED;
+    mine = a.words + (size_t)tile * tw;
+    ox = wy * RY * ED;
+    oy = TY * ED + wx * RX * ED;
+    oh = (TX + TY) * ED;
+    fx = (int)(a.nty * tw);
+    fy = (int)tw;
+    xlo = wx == 0 && bx > 0;
+    xhi = wx == WX - 1 && bx + 1 < a.ntx;
+    ylo = wy == 0 && by > 0;
+    yhi = wy == WY - 1 && by + 1 < a.nty;
+  }
+
+  // LDS: psi as (column, pair, PML cell, 2) and, per column, a zero pair for
+  // the lanes outside the PML (so every lane's address steps alike); absorber
+  // values; `more` floats of the kernel's own; edge buffers.
+  __device__ __forceinline__ f32x4* sig() const {
+    return reinterpret_cast<f32x4*>(lds + ((TX * TY * PS + 3) & ~3));
+  }
+  __device__ __forceinline__ float* own() const {
+    return reinterpret_cast<float*>(sig() + TX * TY);
+  }
+  // Edge slot s of a direction lies between waves s - 1 and s.  Low edges are
+  // read from slot w + 1 and written to slot w, high ones read from w and
+  // written to w + 1; slots 1 .. WX (low) and 0 .. WX - 1 (high) exist, the
+  // outer one holding the neighbouring workgroup's edge.  (Float offsets,
+  // uniform: the lane's address is made where it is used.)
+  __device__ __forceinline__ void edges(int more) {
+    const int eoff = (int)(own() - lds) + more;
+    const int hoff = eoff + (alias ? 0 : (WX * TY + WY * TX) * ED);
+    sx = (wx * TY + wy * RY) * ED;
+    sy = (WX * TY + wy * TX + wx * RX) * ED;
+    er = eoff;
+    hr = hoff;
+  }
+  __device__ __forceinline__ float* slot(int off) const { return lds + opaque_s(off) + zb; }
+  __device__ __forceinline__ float* low_x() const { return slot(er + sx); }
+  __device__ __forceinline__ float* low_y() const { return slot(er + sy); }
+  __device__ __forceinline__ float* high_x() const { return slot(hr + sx); }
+  __device__ __forceinline__ float* high_y() const { return slot(hr + sy); }
+
+  __device__ __forceinline__ int colx(int i) const { return x0 + i; }
+  __device__ __forceinline__ int coly(int r) const { return y0 + r; }
+  __device__ __forceinline__ bool valid(int i, int r) const {
+    return opaque_s(colx(i)) < X && coly(r) < Y;
+  }
+  __device__ __forceinline__ int offset(int i, int r) const {
+    return (opaque_s(colx(i)) * Y + coly(r)) * Z;
+  }
+  // Column t of the tile's psi and absorber blocks: column t % C of wave t / C.
+  __device__ __forceinline__ int tile_x(int t) const {
+    return bx * TX + (t / C) % WX * RX + t % C / RY;
+  }
+  __device__ __forceinline__ int tile_y(int t) const {
+    return by * TY + (t / C) / WX * RY + t % C % RY;
+  }
+
+  // Three components of a column from arrays N apart.
+  __device__ __forceinline__ void load(float (&v)[3][CPL], const float* p, int N, int i,
+                                       int r) const {
+    const bool ok = valid(i, r);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+#pragma unroll
+      for (int c = 0; c < CPL; ++c)
+        v[k][c] = ok && zb + c < Z ? to_global(p)[k * N + offset(i, r) + zb + c] : 0.0f;
+  }
+  __device__ __forceinline__ void store(float* p, const float (&v)[3][CPL], int N, int i,
+                                        int r) const {
+    const int o = offset(i, r) + zb;
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+#pragma unroll
+      for (int c = 0; c < CPL; ++c)
+        if (zb + c < Z) to_global(p)[k * N + o + c] = v[k][c];
+  }
+  // The tile's psi (a pair of arrays P apart each) and absorber to LDS.
+  __device__ __forceinline__ void fill(const float* psi0, const float* psi1, int P,
+                                       const float* mask) const {
+    for (int q = threadIdx.x; q < TX * TY * PS; q += kResThreads) {
+      const int t = q / PS, m = q - t * PS;
+      const int pair = m >= NP * 2, pi = (m - pair * NP * 2) >> 1;
+      const int x = tile_x(t), y = tile_y(t);
+      const float* p = pair ? psi1 : psi0;
+      lds[q] = p && m < NP * 4 && x < X && y < Y ? p[(m & 1) * P + (x * Y + y) * NP + pi] : 0.0f;
+    }
+    for (int t = threadIdx.x; t < TX * TY; t += kResThreads) {
+      const int x = tile_x(t), y = tile_y(t);
+      f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};
+      if (x < X && y < Y) {
+        const int m = x * Y + y, XY = X * Y;
+        s = f32x4{mask[m], mask[XY + m], mask[2 * XY + m], 0.0f};
+      }
+      sig()[t] = s;
+    }
+  }
+  // The wave's own psi back to memory (no barrier: nobody else's).
+  __device__ __forceinline__ void store_psi(float* psi0, float* psi1, int P) const {
+    for (int q = lane; q < C * NP * 4; q += 64) {
+      const int t = q / (NP * 4), m = q - t * NP * 4;
+      const int x = x0 + t / RY, y = y0 + t % RY;
+      const int pair = m >= NP * 2, pi = (m - pair * NP * 2) >> 1;
+      if (x < X && y < Y)
+        to_global(pair ? psi1 : psi0)[(m & 1) * P + (x * Y + y) * NP + pi] =
+            lds[(w * C + t) * PS + m];
+    }
+  }
+  // A column's psi pair, from the lane's address in a column's block.
+  __device__ __forceinline__ f32x2* psi_at(int lane_bytes, int i, int r) const {
+    const int b = lane_bytes + opaque_s((w * C + i * RY + r) * PS * 4);
+    return reinterpret_cast<f32x2*>(reinterpret_cast<char*>(lds) + b);
+  }
+
+  // A column's two edge values: to LDS, or as words.
+  __device__ __forceinline__ void put_edge(float* p, int k, const float (&u)[CPL],
+                                           const float (&v)[CPL]) const {
+    lds_put<CPL>(p + k * ED, u);
+    lds_put<CPL>(p + k * ED + ED / 2, v);
+  }
+  __device__ __forceinline__ void post(int off, unsigned tag, const float (&u)[CPL],
+                                       const float (&v)[CPL]) const {
+    rword_t* const q = edge_word(mine, off, lane);
+#pragma unroll
+    for (int c = 0; c < CPL; ++c) {
+      post_edge(q + 64 * c, tag, u[c]);
+      post_edge(q + ED / 2 + 64 * c, tag, v[c]);
+    }
+  }
+  // Passes the wave's edges on: through LDS within the workgroup, as words to
+  // its neighbours.
+  __device__ __forceinline__ void pass_low(unsigned tag, const float (&e)[RX][RY][3][CPL]) const {
+    if (wx > 0) {
+#pragma unroll
+      for (int r = 0; r < RY; ++r) put_edge(slot(er + sx - TY * ED), r, e[0][r][1], e[0][r][2]);
+    } else if (xlo) {
+#pragma unroll
+      for (int r = 0; r < RY; ++r) post(ox + r * ED, tag, e[0][r][1], e[0][r][2]);
+    }
+    if (wy > 0) {
+#pragma unroll
+      for (int i = 0; i < RX; ++i) put_edge(slot(er + sy - TX * ED), i, e[i][0][0], e[i][0][2]);
+    } else if (ylo) {
+#pragma unroll
+      for (int i = 0; i < RX; ++i) post(oy + i * ED, tag, e[i][0][0], e[i][0][2]);
+    }
+  }
+  __device__ __forceinline__ void pass_high(unsigned tag, const float (&h)[RX][RY][3][CPL]) const {
+    if (wx < WX - 1) {
+#pragma unroll
+      for (int r = 0; r < RY; ++r)
+        put_edge(slot(hr + sx + TY * ED), r, h[RX - 1][r][1], h[RX - 1][r][2]);
+    } else if (xhi) {
+#pragma unroll
+      for (int r = 0; r < RY; ++r)
+        post(oh + ox + r * ED, tag, h[RX - 1][r][1], h[RX - 1][r][2]);
+    }
+    if (wy < WY - 1) {
+#pragma unroll
+      for (int i = 0; i < RX; ++i)
+        put_edge(slot(hr + sy + TX * ED), i, h[i][RY - 1][0], h[i][RY - 1][2]);
+    } else if (yhi) {
+#pragma unroll
+      for (int i = 0; i < RX; ++i)
+        post(oh + oy + i * ED, tag, h[i][RY - 1][0], h[i][RY - 1][2]);
+    }
+  }
+  // n columns of a border wave's outer slot: the neighbour's edge, or zeros
+  // past the domain.  K columns at a time (the registers of the words).
+  template <int n>
+  __device__ __forceinline__ void take(float* dst, int off, bool there, unsigned tag,
+                                       bool& dead) const {
+    constexpr int K = CPL == 1 ? 4 : 2, NW = 2 * CPL;
+#pragma unroll
+    for (int k0 = 0; k0 < n; k0 += K) {
+      float v[K * NW];
+      if (!there) {
+#pragma unroll
+        for (int q = 0; q < K * NW; ++q) v[q] = 0.0f;
+      } else if (k0 + K <= n) {
+        wait_edges<K * NW>(v, edge_word(mine, off + k0 * ED, lane), tag, dead);
+      } else {
+        constexpr int rest = n % K ? n % K : K;
+        float u[rest * NW];
+        wait_edges<rest * NW>(u, edge_word(mine, off + k0 * ED, lane), tag, dead);
+#pragma unroll
+        for (int q = 0; q < rest * NW; ++q) v[q] = u[q];
+      }
+#pragma unroll
+      for (int k = 0; k < K && k0 + k < n; ++k)
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          float t[CPL];
+#pragma unroll
+          for (int c = 0; c < CPL; ++c) t[c] = v[k * NW + q * CPL + c];
+          lds_put<CPL>(dst + (k0 + k) * ED + q * (ED / 2), t);
+        }
+    }
+  }
+  // Once every wave of the workgroup has passed its edges: those of the
+  // neighbouring workgroups.
+  __device__ __forceinline__ void take_low(unsigned tag, bool& dead) const {
+    lds_barrier();
+    if (wx == WX - 1) take<RY>(low_x(), fx + ox, xhi, tag, dead);
+    if (wy == WY - 1) take<RX>(low_y(), fy + oy, yhi, tag, dead);
+  }
+  __device__ __forceinline__ void take_high(unsigned tag, bool& dead) const {
+    lds_barrier();
+    if (wx == 0) take<RY>(high_x(), oh + ox - fx, xlo, tag, dead);
+    if (wy == 0) take<RX>(high_y(), oh + oy - fy, ylo, tag, dead);
+  }
+  // With one set of edge buffers: before it is written again.
+  __device__ __forceinline__ void edges_read() const {
+    if (alias) lds_barrier();
+  }
+};
+
+inline ResTileArgs tile_args(const Geom& g, const ResPlan& p, rword_t* words) {
+  ResTileArgs a;
+  a.X = g.X; a.Y = g.Y; a.Z = g.Z; a.lo = g.lo; a.hi = g.hi; a.NP = g.NP;
+  a.N = (int)g.N;
+  a.P = g.X * g.Y * g.NP;
+  a.wx = p.wx; a.wy = p.wy; a.ntx = p.ntx; a.nty = p.nty;
+  a.alias = p.alias;
+  a.words = words;
+  return a;
+}
 
 // A state in memory: E and H (3N floats each) and the four psi components.
 struct ResState {
@@ -119,10 +428,26 @@ inline unsigned resident_tags(int n) { return (unsigned)n + 1; }
 // The tiling for a domain on `cus` compute units (rx = 0: it does not fit).
 ResPlan resident_plan(const Geom& g, int saxis, int cus);
 
+// Whether a tiling's kernel that also writes each step's change of E is worth
+// its while: past 25 cells a lane, two a column, it spills (the one-step
+// change takes 6 more registers a column).
+inline bool resident_captures(const ResPlan& p) {
+  return p.rx > 0 && (p.cpl == 1 || p.cpl * p.rx * p.ry <= 25);
+}
+
 // The words (at L.E1, cleared before a call's first run) and the state it is
 // given in memory are the caller's to prepare.
 hipError_t run_resident(const Geom& g, const pjz_fdtd_problem& p, const float* mask,
                         const Src& src, const OutWin& win, char* ws, const Layout& L,
                         const ResPlan& plan, const ResRun& r, hipStream_t s);
+
+// Reversed steps end - 1 down to begin in one launch, from and to adjoint set
+// 0: D = E^n - E^(n+1) of the steps from `begin` on, gout the snapshots'
+// cotangents.  Uses resident_tags(end - begin) exchange numbers.
+bool adjoint_resident_supported(const ResPlan& p);
+hipError_t run_adjoint_resident(const Geom& g, const pjz_fdtd_problem& p, const float* mask,
+                                char* ws, const Layout& L, const ResPlan& plan, const float* D,
+                                const float* gout, int begin, int end, unsigned tag0,
+                                hipStream_t s);
 
 }  // namespace pjz

@@ -85,3 +85,38 @@ def test_gradient_of_a_large_tiling():
   got, _ = G.gpu_grad(eps, kw, g, ckpt_every=9)
   ref, _ = G.gpu_grad(eps, kw, g, ckpt_every=9, kernel="stream2")
   assert G.rel_l2(got, ref) <= 1e-5
+
+
+# Reverse tilings: cb, G and D in registers (2-8 cells a lane), cb from memory
+# (12), cb and G from memory (16).
+@pytest.mark.parametrize("axis,X,Y,Z", [(0, 64, 62, 33), (1, 83, 90, 20), (2, 110, 107, 24),
+                                        (0, 128, 120, 30), (1, 157, 149, 25), (2, 177, 180, 24),
+                                        (0, 60, 61, 66), (1, 90, 88, 70), (2, 111, 107, 68),
+                                        (0, 128, 126, 66)])
+def test_every_reverse_tiling_matches_two_step_kernels(axis, X, Y, Z):
+  print(f"case {X}x{Y}x{Z} axis {axis}", flush=True)
+  eps, kw, g = G.problem(axis, seed=X, X=X, Y=Y, Z=Z, tt=40)
+  got, _ = G.gpu_grad(eps, kw, g, ckpt_every=11)
+  ref, _ = G.gpu_grad(eps, kw, g, ckpt_every=11, kernel="stream2")
+  assert G.rel_l2(got, ref) <= 1e-5
+
+
+def test_batch_of_resident_and_streamed_simulations():
+  """Each simulation of a batch that mixes both: fields and gradients equal
+  its own call's on the two-step kernels."""
+  cases = [G.problem(axis, seed=axis, X=X, Y=Y, Z=Z, tt=tt)
+           for axis, X, Y, Z, tt in [(0, 130, 120, 64, 40), (1, 30, 40, 64, 41),
+                                     (2, 230, 210, 128, 40), (0, 100, 120, 96, 46)]]
+  eps = [torch.tensor(e, device="cuda", requires_grad=True) for e, _, _ in cases]
+  calls = [dict(kw, epsilon=e, launch_params=dict(ckpt_every=12))
+           for e, (_, kw, _) in zip(eps, cases)]
+  outs = F.fdtdz_batch(calls)
+  sum((o * torch.as_tensor(g, device="cuda")).sum() for o, (_, _, g) in zip(outs, cases)).backward()
+  torch.cuda.synchronize()
+  plain = F.fdtdz_batch([dict(c, epsilon=c["epsilon"].detach()) for c in calls])
+  for e, o, q, (e0, kw, g) in zip(eps, outs, plain, cases):
+    ref, out = G.gpu_grad(e0, kw, g, ckpt_every=12, kernel="stream2")
+    print(tuple(e.shape), flush=True)
+    assert G.rel_l2(o.detach().cpu().numpy(), out) <= 1e-6
+    assert G.rel_l2(q.cpu().numpy(), out) <= 1e-6
+    assert G.rel_l2(e.grad.cpu().numpy(), ref) <= 1e-5
