@@ -251,6 +251,18 @@ k_resident(ResArgs a) {
     const f32x4* const sg0 = T.sig() + T.w * C;
     f32x4 nsg = sg0[Order::x(0) * RY + Order::y(0)];
     load_psi(nps, 1, Order::x(0), Order::y(0));
+    // A z-plane source: J of every column of the wave, column t on lane t (read
+    // in the columns themselves, each would wait for LDS).
+    float jxs = 0.0f, jys = 0.0f;
+    if (a.saxis == 2) {
+      const f32x4 s = reinterpret_cast<const f32x4*>(srcl)[T.w * C + min(T.lane, C - 1)];
+      jxs = s.x * w0;
+      jys = s.y * w0;
+      if (a.squad > 1) {
+        jxs += s.z * w1;
+        jys += s.w * w1;
+      }
+    }
     if constexpr (!CBR) {
 #pragma unroll
       for (int k = 0; k < AHEAD && k < C; ++k) load_cb(cbq[k], Order::x(k), Order::y(k));
@@ -332,12 +344,7 @@ k_resident(ResArgs a) {
             jv[c] = s[ED / 2 + c] * wv;
           }
         } else {
-          const f32x4 s = reinterpret_cast<const f32x4*>(srcl)[opaque_s(T.w * C) + i * RY + r];
-          float jx = s.x * w0, jy = s.y * w0;
-          if (a.squad > 1) {
-            jx += s.z * w1;
-            jy += s.w * w1;
-          }
+          const float jx = read_lane(jxs, i * RY + r), jy = read_lane(jys, i * RY + r);
 #pragma unroll
           for (int c = 0; c < CPL; ++c) {
             ju[c] = zb + c == a.spos ? jx : 0.0f;

@@ -32,6 +32,10 @@ __device__ __forceinline__ int opaque_s(int v) {
 // updates of all columns past the next branch, with their inputs live.
 __device__ __forceinline__ void pin(float& v) { asm volatile("" : "+v"(v)); }
 
+__device__ __forceinline__ float read_lane(float v, int l) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
+}
+
 // f(0), .. f(N - 1) with constant arguments (past the size at which the
 // compiler unrolls a loop over register arrays).
 template <class F, int... K>
