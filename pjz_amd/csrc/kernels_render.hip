@@ -11,10 +11,12 @@
 //                               the cell and its z moment (:47-61, 75-87)
 //             k_render_combine  per (component, x, y, z): the moments mixed
 //                               by the shares into 1 / (p aoi + (1 - p) /
-//                               avg) or the plain average (:63-99)
+//                               avg) or the plain average (:63-99);
+//                               k_render_combine_cells past 4 layers
 //   backward: k_render_bwd_cells   dL/dstats, summed over z, and dL/d(z share,
 //                                  z-moment share), summed over the pixels of
-//                                  a workgroup, in one pass over the cells
+//                                  a workgroup, in one pass over the cells;
+//                                  k_render_bwd_all_cells past 4 layers
 //             k_render_sum_parts   the workgroups' share sums added
 //             k_render_bwd_pos     dL/d(interface positions)
 //             k_render_bwd_layers  dL/d(layer sub-pixels), gathered through
@@ -133,8 +135,8 @@ static_assert(kRenderMaxLayers == PJZ_FDTD_RENDER_MAX_LAYERS, "layer bound of th
 
 // The moment along the component's own axis (selected, not indexed: an array
 // here goes to scratch memory).
-__device__ inline float own_moment(const Mix& r, int a) {
-  return a == 0 ? r.g0 : (a == 1 ? r.g1 : r.g2);
+__device__ __forceinline__ float own_moment(float g0, float g1, float g2, int a) {
+  return a == 0 ? g0 : (a == 1 ? g1 : g2);
 }
 
 // Finishes a cell from its mixed sums (:89-99).
@@ -145,7 +147,8 @@ __device__ inline void mix_finish(Mix& r, int simple, int a) {
     return;
   }
   const float T = r.g0 * r.g0 + r.g1 * r.g1 + r.g2 * r.g2;
-  const float ga = own_moment(r, a);
+  const float g0 = r.g0, g1 = r.g1, g2 = r.g2;
+  const float ga = own_moment(g0, g1, g2, a);
   r.pii = ga * ga / (T == 0.0f ? 1.0f : T);  // (:92-95)
   r.iT = T == 0.0f ? 0.0f : 1.0f / T;
   r.iA = 1.0f / r.A;
@@ -157,7 +160,7 @@ struct MixGrad {
   float gA, gB, gG[3];
 };
 
-__device__ inline MixGrad mix_grad(int simple, const Mix& r, int a, float g) {
+__device__ __forceinline__ MixGrad mix_grad(int simple, const Mix& r, int a, float g) {
   MixGrad t;
   if (simple) {
     t.gA = g;
@@ -171,14 +174,16 @@ __device__ inline MixGrad mix_grad(int simple, const Mix& r, int a, float g) {
   t.gA = gD * (1.0f - r.pii) * (-r.iA * r.iA);
   t.gB = gD * r.pii;
   const float gp = gD * (r.B - r.iA) * (2.0f * r.iT);
-  const float ga = own_moment(r, a);
+  const float g0 = r.g0, g1 = r.g1, g2 = r.g2;
+  const float ga = own_moment(g0, g1, g2, a);
   t.gG[0] = gp * ((a == 0 ? ga : 0.0f) - r.pii * r.g0);
   t.gG[1] = gp * ((a == 1 ? ga : 0.0f) - r.pii * r.g1);
   t.gG[2] = gp * ((a == 2 ? ga : 0.0f) - r.pii * r.g2);
   return t;
 }
 
-// The cell kernels (k_render_combine, k_render_bwd_cells): a wave walks over
+// The cell kernels of more than 4 layers (k_render_combine_cells,
+// k_render_bwd_all_cells; fewer go by classes, below): a wave walks over
 // pixels of one component with its lanes on z, so the output (or its
 // cotangent) is read and written in whole rows of zz floats and the layers'
 // shares of the lane's cells stay in registers.  The 4 LL moments of 16
@@ -251,8 +256,134 @@ __device__ inline GroupRange wave_groups(int np, int gpw) {
   return {min(wave * gpw, n), min(wave * gpw + gpw, n)};
 }
 
+// Up to 4 layers, the cell kernels work by classes of cells.  Along z, a pixel's
+// cells that no interface touches have one of LL share vectors (by how many
+// interfaces lie below them), so their value and its derivatives are those of
+// (pixel, class): a wave evaluates 16 pixels x 4 classes at once, one on each
+// lane, instead of every cell.  A cell that an interface touches, ends included
+// (where the clip's derivative is a half), is a class of its own.  What is left
+// per cell is its read or write.  384 x 384 x 128 cells, 3 layers: combine
+// 135 us (bound by three divisions a cell) -> 46 (226 MB written), reverse 315 -> 94.
+constexpr int kPure = 4;  // classes of untouched cells, the first of a wave's list
+
+template <int C>
+struct Classes {
+  int at[C];  // class of the lane's cells
+  int nsp;    // cells with a class of their own
+};
+
+// Classes of the cells z0 + 64 c + lane; list[k] becomes a cell of class k, or
+// -1.  Called by whole workgroups, a list a wave.
+template <int C>
+__device__ __forceinline__ Classes<C> cell_classes(const RenderDims& d, const float* __restrict__ pos,
+                                          const float* __restrict__ gsa,
+                                          const float* __restrict__ gea, int col, int z0, int lane,
+                                          int* list) {
+  Classes<C> K;
+  K.nsp = 0;
+  for (int k = lane; k < kPure + 64 * C; k += 64) list[k] = -1;
+  __syncthreads();
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    const int z = z0 + 64 * c + lane, zc = min(z, d.zz - 1);
+    const float gs = gsa[2 * zc + col], ge = gea[2 * zc + col];
+    bool own = !(ge > gs);
+    int below = 0;
+    for (int l = 0; l + 1 < d.ll; ++l) {
+      own |= !(pos[l] < gs || pos[l] > ge);
+      below += pos[l] < gs ? 1 : 0;
+    }
+    own &= z < d.zz;
+    const unsigned long long m = __ballot(own);
+    const int before = __popcll(m & ((1ull << lane) - 1));
+    K.at[c] = own ? kPure + K.nsp + before : below;
+    K.nsp += __popcll(m);
+    if (z < d.zz) list[K.at[c]] = z;
+  }
+  __syncthreads();
+  return K;
+}
+
+// Shares of cell z (clamped to the stack) of component a.
+template <int LL>
+struct CellShares {
+  float u[LL], uz[LL];
+};
+template <int LL>
+__device__ __forceinline__ CellShares<LL> cell_shares(const RenderDims& d, const float* tab, int a, int z) {
+  CellShares<LL> S;
+#pragma unroll
+  for (int l = 0; l < LL; ++l) {
+    const float* sh = share_at(d, tab, a, min(l, d.ll - 1), max(z, 0));
+    S.u[l] = l < d.ll ? sh[0] : 0.0f;
+    S.uz[l] = l < d.ll ? sh[1] : 0.0f;
+  }
+  return S;
+}
+
+template <int LL>
+__device__ __forceinline__ Mix class_mix(const float (&m)[LL][4], const CellShares<LL>& S,
+                                         int simple, int a) {
+  float A = 0.0f, B = 0.0f, g0 = 0.0f, g1 = 0.0f, g2 = 0.0f;
+#pragma unroll
+  for (int l = 0; l < LL; ++l) {
+    A += m[l][0] * S.u[l];
+    B += m[l][1] * S.u[l];
+    g0 += m[l][2] * S.u[l];
+    g1 += m[l][3] * S.u[l];
+    g2 += m[l][0] * S.uz[l];
+  }
+  Mix r{A, B, g0, g1, g2, A, 0.0f, 0.0f, 0.0f};
+  mix_finish(r, simple, a);
+  return r;
+}
+
 template <int LL, int C>
 __global__ __launch_bounds__(64 * kRenderWaves) void k_render_combine(
+    RenderDims d, const float* __restrict__ st, const float* __restrict__ tab,
+    const float* __restrict__ pos, const float* __restrict__ gsa, const float* __restrict__ gea,
+    float* __restrict__ eps, int gpw, int z0) {
+  __shared__ int lists[kRenderWaves][kPure + 64 * C];
+  __shared__ __align__(16) float values[kRenderWaves][(kPure + 64 * C) * 16];  // (class, pixel)
+  const int a = blockIdx.y, lane = threadIdx.x & 63, np = d.xx * d.yy;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const Classes<C> K = cell_classes<C>(d, pos, gsa, gea, a == 2 ? 1 : 0, z0, lane, lists[w]);
+  const GroupRange R = wave_groups(np, gpw);
+  const CellShares<LL> pure = cell_shares<LL>(d, tab, a, lists[w][lane >> 4]);
+  float* const val = values[w];
+  for (int g = R.g0; g < R.g1; ++g) {
+    float m[LL][4];
+    load_moments(m, d, st, a, 16 * g, np, lane);
+    val[lane] = class_mix<LL>(m, pure, d.simple, a).out;
+    for (int k = 0; k < K.nsp; k += 4) {
+      const int z = k + (lane >> 4) < K.nsp ? lists[w][kPure + k + (lane >> 4)] : 0;
+      val[(kPure + k) * 16 + lane] =
+          class_mix<LL>(m, cell_shares<LL>(d, tab, a, z), d.simple, a).out;
+    }
+    // The wave's own values: its LDS operations are in order.
+    __builtin_amdgcn_wave_barrier();
+    const int n = min(16, np - 16 * g);
+    float* row = eps + ((size_t)a * np + 16 * g) * d.zz + z0 + lane;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      if (z0 + 64 * c + lane >= d.zz) continue;
+      const float4* v = reinterpret_cast<const float4*>(val + K.at[c] * 16);
+#pragma unroll
+      for (int i = 0; i < 16; i += 4) {
+        const float4 t = v[i / 4];
+        const float o[4] = {t.x, t.y, t.z, t.w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (i + j < n)
+            __builtin_nontemporal_store(o[j], row + (size_t)(i + j) * d.zz + 64 * c);
+      }
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
+template <int LL, int C>
+__global__ __launch_bounds__(64 * kRenderWaves) void k_render_combine_cells(
     RenderDims d, const float* __restrict__ st, const float* __restrict__ tab,
     float* __restrict__ eps, int gpw, int z0) {
   const int a = blockIdx.y, lane = threadIdx.x & 63, np = d.xx * d.yy;
@@ -324,7 +455,7 @@ __device__ inline float sum4(float v0, float v1, float v2, float v3) {
 //    registers (in double once per 16 pixels), over the workgroup in LDS and
 //    written to part[((blockIdx.x * 3 + a) * 2 + w) * ll * zz + l * zz + z].
 template <int LL, int C>
-__global__ __launch_bounds__(64 * kRenderWaves) void k_render_bwd_cells(
+__global__ __launch_bounds__(64 * kRenderWaves) void k_render_bwd_all_cells(
     RenderDims d, const float* __restrict__ st, const float* __restrict__ tab,
     const float* __restrict__ geps, float* __restrict__ gst, double* __restrict__ part, int gpw,
     int z0, int add) {
@@ -424,6 +555,128 @@ __global__ __launch_bounds__(64 * kRenderWaves) void k_render_bwd_cells(
         }
         __syncthreads();
       }
+}
+
+// A row's 16 lanes summed, in each of them.
+__device__ inline float row_sum(float s) {
+  s = row_ror_add<8>(s);
+  s = row_ror_add<4>(s);
+  s = row_ror_add<2>(s);
+  return row_ror_add<1>(s);
+}
+
+// Both reductions of the reverse pass by classes (outputs as
+// k_render_bwd_all_cells').  A pixel's cotangents are summed over the cells of
+// each untouched class (sum4) and taken cell by cell for the others; every
+// cotangent of the mixed sums is linear in them, so the rest is done once a
+// (pixel, class).  dL/du and dL/duz are formed for the touched cells only: the
+// positions' gradient takes no other.
+template <int LL, int C>
+__global__ __launch_bounds__(64 * kRenderWaves) void k_render_bwd_cells(
+    RenderDims d, const float* __restrict__ st, const float* __restrict__ tab,
+    const float* __restrict__ pos, const float* __restrict__ gsa, const float* __restrict__ gea,
+    const float* __restrict__ geps, float* __restrict__ gst, double* __restrict__ part, int gpw,
+    int z0, int add) {
+  static_assert(LL <= kPure, "one class a row of lanes");
+  __shared__ int lists[kRenderWaves][kPure + 64 * C];
+  __shared__ float touched[kRenderWaves][64 * C * 16];         // cotangents (cell, pixel)
+  __shared__ double acc[kRenderWaves][64 * C][2 * LL];  // dL/du, dL/duz of touched cells
+  const int a = blockIdx.y, lane = threadIdx.x & 63, np = d.xx * d.yy;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const Classes<C> K = cell_classes<C>(d, pos, gsa, gea, a == 2 ? 1 : 0, z0, lane, lists[w]);
+  for (int q = lane; q < K.nsp * 2 * LL; q += 64) acc[w][q / (2 * LL)][q % (2 * LL)] = 0.0;
+  __syncthreads();
+  const GroupRange R = wave_groups(np, gpw);
+  // Class, then moment, held by this lane's row (sum4's order).
+  const int row = lane >> 4, qrow = row == 1 ? 2 : (row == 2 ? 1 : row);
+  const CellShares<LL> pure = cell_shares<LL>(d, tab, a, lists[w][qrow]);
+  for (int g = R.g0; g < R.g1; ++g) {
+    float m[LL][4], gv[16][C];
+    load_moments(m, d, st, a, 16 * g, np, lane);
+    const int n = min(16, np - 16 * g);
+    const float* grow = geps + ((size_t)a * np + 16 * g) * d.zz + z0 + lane;
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+#pragma unroll
+      for (int c = 0; c < C; ++c)
+        gv[i][c] = i < n && z0 + 64 * c + lane < d.zz
+                       ? __builtin_nontemporal_load(grow + (size_t)i * d.zz + 64 * c)
+                       : 0.0f;
+    float keep = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+#pragma unroll
+        for (int k = 0; k < LL; ++k) v[k] += K.at[c] == k ? gv[i][c] : 0.0f;
+        if (K.at[c] >= kPure) touched[w][(K.at[c] - kPure) * 16 + i] = gv[i][c];
+      }
+      const float s = sum4(v[0], v[1], v[2], v[3]);
+      keep = (lane & 15) == i ? s : keep;
+    }
+    __builtin_amdgcn_wave_barrier();
+    float v[LL][4];
+    {
+      const Mix r = class_mix<LL>(m, pure, d.simple, a);
+      const MixGrad k = mix_grad(d.simple, r, a, keep);
+#pragma unroll
+      for (int l = 0; l < LL; ++l) {
+        v[l][0] = k.gA * pure.u[l] + k.gG[2] * pure.uz[l];
+        v[l][1] = k.gB * pure.u[l];
+        v[l][2] = k.gG[0] * pure.u[l];
+        v[l][3] = k.gG[1] * pure.u[l];
+      }
+    }
+    for (int t = 0; t < K.nsp; t += 4) {
+      const int e = t + (lane >> 4);
+      const bool in = e < K.nsp;
+      const CellShares<LL> S = cell_shares<LL>(d, tab, a, in ? lists[w][kPure + e] : 0);
+      const Mix r = class_mix<LL>(m, S, d.simple, a);
+      const MixGrad k =
+          mix_grad(d.simple, r, a, in ? touched[w][(in ? e : 0) * 16 + (lane & 15)] : 0.0f);
+#pragma unroll
+      for (int l = 0; l < LL; ++l) {
+        if (in) {
+          v[l][0] += k.gA * S.u[l] + k.gG[2] * S.uz[l];
+          v[l][1] += k.gB * S.u[l];
+          v[l][2] += k.gG[0] * S.u[l];
+          v[l][3] += k.gG[1] * S.u[l];
+        }
+        const float fu = row_sum(k.gA * m[l][0] + k.gB * m[l][1] + k.gG[0] * m[l][2] +
+                                 k.gG[1] * m[l][3]);
+        const float fuz = row_sum(k.gG[2] * m[l][0]);
+        if (in && (lane & 15) == 0) {
+          acc[w][e][2 * l] += fu;
+          acc[w][e][2 * l + 1] += fuz;
+        }
+      }
+    }
+#pragma unroll
+    for (int l = 0; l < LL; ++l) {
+      // Summed over the classes (rows); row r then holds moment qrow.
+      const float sum = swap_add16(swap_add32(v[l][0], v[l][1]), swap_add32(v[l][2], v[l][3]));
+      if (l < d.ll && (lane & 15) < n) {
+        float* o = gst + (((size_t)a * 4 + qrow) * d.ll + l) * np + 16 * g + (lane & 15);
+        *o = add ? *o + sum : sum;
+      }
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+  if (!part) return;
+  __syncthreads();
+  // Entries shared out over the waves.
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    const int z = z0 + 64 * c + lane;
+    for (int q = w; q < 2 * d.ll; q += kRenderWaves) {
+      double t = 0.0;
+      if (K.at[c] >= kPure)
+        for (int j = 0; j < kRenderWaves; ++j) t += acc[j][K.at[c] - kPure][q];
+      if (z < d.zz)
+        part[((((size_t)blockIdx.x * 3 + a) * 2 + (q & 1)) * d.ll + (q >> 1)) * d.zz + z] = t;
+    }
+  }
 }
 
 // d clip(v, lo, hi) / dv with torch's (and jax's) halves at ties.
@@ -581,8 +834,9 @@ size_t render_workspace_bytes(int ll, int xx, int yy, int zz) {
 }
 
 // Calls f(LL, C) with the layers a cell kernel is built for (the fewest that
-// hold ll: unused ones have share 0) and its cells a lane.  Up to 4 layers
-// two cells a lane where zz > 64; more layers keep one (registers).
+// hold ll: unused ones have share 0) and its cells a lane.  Up to 4 layers go
+// by classes, up to 3 with two cells a lane where zz > 64 (4: LDS); more take
+// every cell.
 template <typename F>
 static void cell_variant(int ll, int zz, F&& f) {
   const bool two = zz > 64;
@@ -593,7 +847,7 @@ static void cell_variant(int ll, int zz, F&& f) {
   if (ll == 1) pick(std::integral_constant<int, 1>());
   else if (ll == 2) pick(std::integral_constant<int, 2>());
   else if (ll == 3) pick(std::integral_constant<int, 3>());
-  else if (ll == 4) pick(std::integral_constant<int, 4>());
+  else if (ll == 4) f(std::integral_constant<int, 4>(), std::integral_constant<int, 1>());
   else if (ll <= 8) f(std::integral_constant<int, 8>(), std::integral_constant<int, 1>());
   else f(std::integral_constant<int, 16>(), std::integral_constant<int, 1>());
 }
@@ -609,9 +863,15 @@ hipError_t render_forward(int ll, int m, int xx, int yy, int zz, int simple, con
                      gs, ge, tab);
   const CellGrid G = cell_grid(xx, yy);
   cell_variant(ll, zz, [&](auto LL, auto C) {
-    for (int z0 = 0; z0 < zz; z0 += 64 * C.value)
-      hipLaunchKernelGGL((k_render_combine<LL.value, C.value>), dim3(G.blocks, 3),
-                         dim3(64 * kRenderWaves), 0, s, d, stats, tab, eps, G.gpw, z0);
+    for (int z0 = 0; z0 < zz; z0 += 64 * C.value) {
+      if constexpr (LL.value <= kPure)
+        hipLaunchKernelGGL((k_render_combine<LL.value, C.value>), dim3(G.blocks, 3),
+                           dim3(64 * kRenderWaves), 0, s, d, stats, tab, pos, gs, ge, eps, G.gpw,
+                           z0);
+      else
+        hipLaunchKernelGGL((k_render_combine_cells<LL.value, C.value>), dim3(G.blocks, 3),
+                           dim3(64 * kRenderWaves), 0, s, d, stats, tab, eps, G.gpw, z0);
+    }
   });
   return hipGetLastError();
 }
@@ -628,10 +888,17 @@ hipError_t render_backward(int ll, int m, int xx, int yy, int zz, int simple, co
   double* gus = (double*)((char*)part + align256(sizeof(double) * (size_t)G.blocks * 6 * ll * zz));
   const bool want_pos = ll > 1 && g_pos;
   cell_variant(ll, zz, [&](auto LL, auto C) {
-    for (int z0 = 0; z0 < zz; z0 += 64 * C.value)
-      hipLaunchKernelGGL((k_render_bwd_cells<LL.value, C.value>), dim3(G.blocks, 3),
-                         dim3(64 * kRenderWaves), 0, s, d, stats, tab, g_eps, gst,
-                         want_pos ? part : (double*)nullptr, G.gpw, z0, z0 > 0);
+    for (int z0 = 0; z0 < zz; z0 += 64 * C.value) {
+      double* const parts = want_pos ? part : nullptr;
+      if constexpr (LL.value <= kPure)
+        hipLaunchKernelGGL((k_render_bwd_cells<LL.value, C.value>), dim3(G.blocks, 3),
+                           dim3(64 * kRenderWaves), 0, s, d, stats, tab, pos, gs, ge, g_eps, gst,
+                           parts, G.gpw, z0, z0 > 0);
+      else
+        hipLaunchKernelGGL((k_render_bwd_all_cells<LL.value, C.value>), dim3(G.blocks, 3),
+                           dim3(64 * kRenderWaves), 0, s, d, stats, tab, g_eps, gst, parts, G.gpw,
+                           z0, z0 > 0);
+    }
   });
   // ll SX SY < 2^29 (the arrays' bound of the C ABI); a row takes at least
   // one workgroup.

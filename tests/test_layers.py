@@ -222,3 +222,27 @@ def test_render_kernel_sizes(gpu, ll, xx, yy, zz):
     res.append([v.detach().cpu().numpy() for v in (out, L.grad) + ((p.grad,) if ll > 1 else ())])
   for got, ref, tol in zip(*res, (2e-5, 2e-5, 2e-4)):
     assert np.linalg.norm(got - ref) <= tol * np.linalg.norm(ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("zz", [7, 70, 131])
+@pytest.mark.parametrize("pos", [[2.2, 2.6, 2.9], [3.0, 3.0, 5.5], [-4.0, 2.3, 900.0],
+                                 [1.5, 1.5], [6.4, 1.2], [3.0]])
+def test_render_kernel_interface_orders(gpu, pos, zz):
+  """The classes of cells the kernels work by: several interfaces in a cell or
+  at one place, on cell bounds of both grids, outside the stack, out of
+  order.  Against the float32 torch restatement on the CPU, bounds as above."""
+  rng = np.random.default_rng(zz + len(pos))
+  ll, xx, yy, m = len(pos) + 1, 5, 7, 1
+  i, j = np.arange(2 * m * xx)[:, None], np.arange(2 * m * yy)[None, :]
+  layers = np.stack([2 + 3 * (k % 3) + 0.1 * i + 0.07 * j for k in range(ll)])
+  g = torch.tensor(rng.standard_normal((3, xx, yy, zz)), dtype=torch.float32)
+  res = []
+  for dev in (gpu, torch.device("cpu")):
+    L = torch.tensor(layers, dtype=torch.float32, device=dev, requires_grad=True)
+    p = torch.tensor(pos, dtype=torch.float32, device=dev, requires_grad=True)
+    out = E.render(L, p, *(t.to(dev) for t in zgrid(zz, torch.float32)), m)
+    (out * g.to(dev)).sum().backward()
+    res.append([v.detach().cpu().numpy() for v in (out, L.grad, p.grad)])
+  for got, ref, tol in zip(*res, (2e-5, 2e-5, 2e-4)):
+    assert np.linalg.norm(got - ref) <= tol * np.linalg.norm(ref)
