@@ -263,6 +263,63 @@ int auto_kernel(const pjz::Geom& g) {
   return g.Z <= 256 ? PJZ_FDTD_KERNEL_STREAM : PJZ_FDTD_KERNEL_REFERENCE;
 }
 
+// Compute units the resident stepper may take for a problem, or 0: another
+// kernel or tiling was asked for, or the run is a few steps (a resident run
+// costs about 0.1 ms once, the words and the state, and saves 10 us a step or
+// more).
+constexpr int kResidentMinSteps = 16;
+int resident_cus(const pjz_fdtd_problem& p) {
+  if (p.kernel != PJZ_FDTD_KERNEL_AUTO || p.tile_x != 0 || p.tile_y != 0 || p.graph_steps != 0 ||
+      pjz::steps_of(p) < kResidentMinSteps)
+    return 0;
+  int dev = 0, cus = 0, coop = 0, lds = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+      hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev) != hipSuccess ||
+      hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess ||
+      !coop || (size_t)lds < pjz::kResLds)
+    return 0;
+  return cus;
+}
+// A call recorded into a graph launches step by step: a cooperative launch
+// might not be recordable.
+bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone;
+}
+
+// The resident stepper's tiling for a call, or rx = 0: as above, or the domain
+// is too large.
+pjz::ResPlan resident_for(const pjz::Geom& g, const pjz_fdtd_problem& p, hipStream_t s) {
+  const int cus = capturing(s) ? 0 : resident_cus(p);
+  return cus > 0 ? pjz::resident_plan(g, p.src_axis, cus) : pjz::ResPlan{};
+}
+
+// Its slabs for a larger domain (n = 0: none); `capture`: for steps whose
+// changes of E are written.
+pjz::SlabPlan slabs_for(const pjz::Geom& g, const pjz_fdtd_problem& p, hipStream_t s,
+                        bool capture) {
+  const int cus = capturing(s) ? 0 : resident_cus(p);
+  if (cus <= 0) return {};
+  const pjz::SlabPlan plan = pjz::slab_plan(g, p.src_axis, cus);
+  return capture && !pjz::resident_captures(plan.tile) ? pjz::SlabPlan{} : plan;
+}
+
+// Workspace bytes past the layout's own for a run in slabs (the words), so that
+// a smaller workspace still runs the streaming steppers.
+size_t slab_bytes(const pjz::Geom& g, const pjz_fdtd_problem& p) {
+  const int cus = resident_cus(p);
+  if (cus <= 0 || pjz::resident_plan(g, p.src_axis, cus).rx > 0) return 0;
+  return pjz::slab_words(pjz::slab_plan(g, p.src_axis, cus)) * sizeof(pjz::rword_t);
+}
+// The layout of a call whose workspace has `bytes` bytes.
+pjz::Layout layout_in(const pjz::Geom& g, const pjz_fdtd_problem& p, size_t bytes) {
+  pjz::Layout L = pjz::make_layout(g, p);
+  const size_t more = slab_bytes(g, p);
+  if (more > 0 && bytes >= pjz::align256(L.total) + more) L.words = pjz::align256(L.total);
+  return L;
+}
+
 // Steps [b, end) with the kernel the problem selects (AUTO: auto_kernel;
 // AUTOTUNE: the cached choice for the shape, else AUTO).
 hipError_t run_steps(const pjz::Geom& g, const pjz_fdtd_problem& p, const float* mask,
@@ -281,8 +338,16 @@ hipError_t run_steps(const pjz::Geom& g, const pjz_fdtd_problem& p, const float*
     }
     kernel = PJZ_FDTD_KERNEL_AUTO;
   }
-  if (kernel == PJZ_FDTD_KERNEL_AUTO) kernel = auto_kernel(g);
   pjz::StepRange r{b, end, cur, capture};
+  if (kernel == PJZ_FDTD_KERNEL_AUTO) {
+    if (L.words > 0 && end - b >= kResidentMinSteps) {
+      const pjz::SlabPlan slabs = slabs_for(g, p, s, capture != nullptr);
+      if (slabs.n > 0)
+        return pjz::run_slabs(g, p, mask, src, win, ws, L, slabs, (pjz::rword_t*)(ws + L.words), r,
+                              s);
+    }
+    kernel = auto_kernel(g);
+  }
   if (kernel == PJZ_FDTD_KERNEL_STREAM2)
     return pjz::run_stream2(g, p, mask, src, win, ws, L, r, s);
   if (kernel == PJZ_FDTD_KERNEL_STREAM3)
@@ -291,31 +356,6 @@ hipError_t run_steps(const pjz::Geom& g, const pjz_fdtd_problem& p, const float*
     return pjz::run_stream_deep(g, p, mask, src, win, ws, L, r, 4, s);
   if (kernel == PJZ_FDTD_KERNEL_STREAM) return pjz::run_stream(g, p, mask, src, win, ws, L, r, s);
   return pjz::run_reference(g, p, mask, src, win, ws, L, r, s);
-}
-
-// A resident run costs about 0.1 ms once (the words, the state) and saves 10 us
-// a step or more.
-constexpr int kResidentMinSteps = 16;
-
-// The resident stepper's tiling for a call, or rx = 0 where steps are launched
-// one by one: another kernel or tiling was asked for, the domain is too large,
-// or the call is recorded into a graph, which a cooperative launch might not
-// be.
-pjz::ResPlan resident_for(const pjz::Geom& g, const pjz_fdtd_problem& p, hipStream_t s) {
-  const pjz::ResPlan none{};
-  if (p.kernel != PJZ_FDTD_KERNEL_AUTO || p.tile_x != 0 || p.tile_y != 0 || p.graph_steps != 0 ||
-      pjz::steps_of(p) < kResidentMinSteps)
-    return none;
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  int dev = 0, cus = 0, coop = 0, lds = 0;
-  if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone ||
-      hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-      hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev) != hipSuccess ||
-      hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess ||
-      !coop || (size_t)lds < pjz::kResLds)
-    return none;
-  return pjz::resident_plan(g, p.src_axis, cus);
 }
 
 // Clears the exchange words (once a call: its runs use rising numbers).
@@ -374,16 +414,32 @@ hipError_t restore_state(const pjz::Geom& g, const pjz::Layout& L, char* ws, int
   return copy_state(g, L, ws, 0, k, false, s);
 }
 
-// A forward call's steps by the resident stepper: the whole run in one launch,
-// its checkpoints written on the way.
-hipError_t forward_resident(const pjz::Geom& g, const pjz_fdtd_problem& p, const float* mask,
-                            const pjz::Src& src, const pjz::OutWin& win, char* ws,
-                            const pjz::Layout& L, const pjz::ResPlan& plan, hipStream_t s) {
-  hipError_t e = clear_words(plan, L, ws, s);
-  if (e != hipSuccess) return e;
-  pjz::ResRun r{0, pjz::steps_of(p), {}, {}, nullptr, nullptr, L.S1, 0};
-  if (L.nck > 0) r.ckpt = ckpt_state(g, L, ws, 0).E;
-  return pjz::run_resident(g, p, mask, src, win, ws, L, plan, r, s);
+// Every step of a forward call: cb is in the workspace, where its checkpoints
+// (the states before steps 0, S, 2S, ...) are left for the backward.
+hipError_t forward_steps(const pjz::Geom& g, const pjz_fdtd_problem& p, const float* mask,
+                         const pjz::Src& src, const pjz::OutWin& win, char* ws,
+                         const pjz::Layout& L, hipStream_t s) {
+  const int nsteps = pjz::steps_of(p);
+  const pjz::ResPlan plan = resident_for(g, p, s);
+  if (plan.rx > 0) {
+    // The whole run in one launch, its checkpoints written on the way.
+    hipError_t e = clear_words(plan, L, ws, s);
+    if (e != hipSuccess) return e;
+    pjz::ResRun r{0, nsteps, {}, {}, nullptr, nullptr, L.S1, 0};
+    if (L.nck > 0) r.ckpt = ckpt_state(g, L, ws, 0).E;
+    return pjz::run_resident(g, p, mask, src, win, ws, L, plan, r, s);
+  }
+  // Clears E0, H0 (contiguous) and psi.
+  hipError_t e = clear_state(g, L, ws, s);
+  int cur = 0;
+  if (L.nck == 0 && e == hipSuccess)
+    e = run_steps(g, p, mask, src, win, ws, L, 0, nsteps, &cur, nullptr, s);
+  for (int k = 0; k < L.nck && e == hipSuccess; ++k) {
+    const int b = k * L.S1, end = b + L.S1 < nsteps ? b + L.S1 : nsteps;
+    e = save_state(g, L, ws, cur, k, s);
+    if (e == hipSuccess) e = run_steps(g, p, mask, src, win, ws, L, b, end, &cur, nullptr, s);
+  }
+  return e;
 }
 
 // Every step of a backward call reversed, segment by segment: cb, the cleared
@@ -392,7 +448,7 @@ hipError_t forward_resident(const pjz::Geom& g, const pjz_fdtd_problem& p, const
 hipError_t backward_steps(const pjz::Geom& g, const pjz_fdtd_problem& p,
                           const float* absorption_mask, const pjz::Src& src,
                           const float* grad_out, char* ws, const pjz::Layout& L,
-                          pjz::ResPlan plan, hipStream_t s) {
+                          hipStream_t s) {
   const int nsteps = pjz::steps_of(p);
   const long long f3 = 3 * g.N;
   // The reference kernel choice also selects the cell-by-cell reverse step.
@@ -408,6 +464,7 @@ hipError_t backward_steps(const pjz::Geom& g, const pjz_fdtd_problem& p,
   auto is_out = [&](int n) {
     return n >= p.out_start && n < p.out_stop && (n - p.out_start) % p.out_step == 0;
   };
+  pjz::ResPlan plan = resident_for(g, p, s);
   if (!pjz::resident_captures(plan)) plan = {};
   const bool resident_adj = plan.rx > 0 && pjz::adjoint_resident_supported(plan);
   unsigned tags = 0;  // exchange numbers used
@@ -691,7 +748,9 @@ int pjz_fdtd_workspace_bytes(const pjz_fdtd_problem* p, size_t* bytes) {
   int rc = check(p);
   if (rc) return rc;
   if (!bytes) return fail(PJZ_FDTD_EINVAL, "bytes is NULL");
-  *bytes = pjz::make_layout(geom_of(*p), *p).total;
+  const size_t total = pjz::make_layout(geom_of(*p), *p).total;
+  const size_t more = slab_bytes(geom_of(*p), *p);
+  *bytes = more > 0 ? pjz::align256(total) + more : total;
   return PJZ_FDTD_OK;
 }
 
@@ -708,7 +767,7 @@ int pjz_fdtd_forward(const pjz_fdtd_problem* p, const float* epsilon,
       !source_waveform || !out || !workspace)
     return fail(PJZ_FDTD_EINVAL, "a required pointer argument is NULL");
   pjz::Geom g = geom_of(*p);
-  pjz::Layout L = pjz::make_layout(g, *p);
+  pjz::Layout L = layout_in(g, *p, workspace_bytes);
   if (workspace_bytes < L.total)
     return fail(PJZ_FDTD_ESPACE, "workspace of %zu bytes, %zu needed", workspace_bytes, L.total);
   if (((uintptr_t)workspace & 255) != 0)
@@ -721,33 +780,12 @@ int pjz_fdtd_forward(const pjz_fdtd_problem* p, const float* epsilon,
   if (e != hipSuccess) return hip_fail(e, "prepare");
   pjz::Src src{p->src_axis, p->src_pos, p->src_quad, source_field, source_waveform};
   pjz::OutWin win{p->x0, p->y0, p->z0, p->ex, p->ey, p->ez, out};
-  const int nsteps = pjz::steps_of(*p);
-  const pjz::ResPlan plan = resident_for(g, *p, s);
-  if (plan.rx > 0) {
-    e = forward_resident(g, *p, absorption_mask, src, win, ws, L, plan, s);
-    return e == hipSuccess ? PJZ_FDTD_OK : hip_fail(e, "resident launch");
-  }
-  e = pjz::launch_zero((float*)(ws + L.E0), (L.E1 - L.E0) / sizeof(float), s);
-  if (e == hipSuccess && g.NP > 0)
-    e = pjz::launch_zero((float*)(ws + L.psi), (L.zt - L.psi) / sizeof(float), s);
-  if (e != hipSuccess) return hip_fail(e, "clear state");
   Tuned tuned;
   if (p->kernel == PJZ_FDTD_KERNEL_AUTOTUNE && !tuned_choice(*p, &tuned)) {
     e = autotune(g, *p, absorption_mask, src, ws, L, s);
     if (e != hipSuccess) return hip_fail(e, "autotune");
   }
-  int cur = 0;
-  if (L.nck > 0) {
-    // Checkpoint the state before steps 0, S, 2S, ... for pjz_fdtd_backward.
-    for (int k = 0; k < L.nck && e == hipSuccess; ++k) {
-      const int b = k * L.S1, end = b + L.S1 < nsteps ? b + L.S1 : nsteps;
-      e = save_state(g, L, ws, cur, k, s);
-      if (e == hipSuccess) e = run_steps(g, *p, absorption_mask, src, win, ws, L, b, end, &cur,
-                                         nullptr, s);
-    }
-  } else {
-    e = run_steps(g, *p, absorption_mask, src, win, ws, L, 0, nsteps, &cur, nullptr, s);
-  }
+  e = forward_steps(g, *p, absorption_mask, src, win, ws, L, s);
   if (e != hipSuccess) return hip_fail(e, "step launch");
   return PJZ_FDTD_OK;
 }
@@ -829,7 +867,9 @@ int batch_plan(const pjz_fdtd_problem* probs, int n, BatchPlanHost& bp) {
                   g.Z);
     bp.Ls[i] = pjz::make_layout(g, probs[i]);
     bp.offs[i] = off;
-    off += pjz::align256(bp.Ls[i].total);
+    const size_t more = slab_bytes(g, probs[i]);
+    if (more > 0) bp.Ls[i].words = pjz::align256(bp.Ls[i].total);
+    off += pjz::align256(bp.Ls[i].total) + pjz::align256(more);
   }
   bp.meta_off = off;
   std::vector<pjz::BatchItem> items(n);
@@ -890,30 +930,34 @@ int batch_setup(const pjz_fdtd_problem* probs, int n, const BatchPlanHost& bp,
 }
 
 // The simulations of a batch that run by themselves, one after the other, on
-// the resident stepper (their tilings, rx = 0 for the others, which share the
-// batched launches).  A resident step takes about 2.5 us and 0.3 us for every
-// cell a lane, twice that where cb comes from memory (past 16 cells); a
-// simulation's share of a batched step is its cells at 90 per ns, and no
-// batched step is shorter than 12 us.
-std::vector<pjz::ResPlan> batch_resident(const pjz_fdtd_problem* probs, int n, hipStream_t s) {
-  std::vector<pjz::ResPlan> plans(n);
+// the resident stepper; the others share the batched launches.  A resident
+// step takes about 2.5 us and 0.3 us for every cell a lane, twice that where
+// cb comes from memory (past 16 cells); a simulation's share of a batched step
+// is its cells at 90 per ns, and no batched step is shorter than 12 us.  Slabs
+// are taken where they beat that rate anyway (slab_plan).
+std::vector<bool> batch_alone(const std::vector<pjz::BatchItem>& items, bool capture,
+                              hipStream_t s) {
+  const size_t n = items.size();
+  std::vector<bool> alone(n, false);
+  std::vector<double> us(n, 0.0);
   double all_res = 0, all_batch = 0;
   bool fit = true;
-  auto res_us = [](const pjz::ResPlan& p) {
+  auto share_us = [](const pjz::BatchItem& it) { return (double)it.g.N / 90e3; };
+  for (size_t i = 0; i < n; ++i) {
+    const pjz::ResPlan p = resident_for(items[i].g, *items[i].p, s);
     const int c = p.cpl * p.rx * p.ry;
-    return 2.5 + (c <= 16 ? 0.3 : 0.6) * c;
-  };
-  auto share_us = [](const pjz_fdtd_problem& q) { return (double)geom_of(q).N / 90e3; };
-  for (int i = 0; i < n; ++i) {
-    plans[i] = resident_for(geom_of(probs[i]), probs[i], s);
-    fit = fit && plans[i].rx > 0;
-    if (plans[i].rx > 0) all_res += res_us(plans[i]);
-    all_batch += share_us(probs[i]);
+    if (p.rx > 0) us[i] = 2.5 + (c <= 16 ? 0.3 : 0.6) * c;
+    else fit = false;
+    all_res += us[i];
+    all_batch += share_us(items[i]);
   }
-  if (fit && all_res <= std::max(12.0, all_batch)) return plans;
-  for (int i = 0; i < n; ++i)
-    if (plans[i].rx > 0 && res_us(plans[i]) > share_us(probs[i])) plans[i] = {};
-  return plans;
+  const bool all = fit && all_res <= std::max(12.0, all_batch);
+  for (size_t i = 0; i < n; ++i) {
+    if (us[i] > 0) alone[i] = all || us[i] <= share_us(items[i]);
+    else if (items[i].L->words > 0)
+      alone[i] = slabs_for(items[i].g, *items[i].p, s, capture).n > 0;
+  }
+  return alone;
 }
 
 }  // namespace
@@ -944,13 +988,13 @@ int pjz_fdtd_batch_forward(const pjz_fdtd_problem* probs, int n, const float* co
                    source_field, source_waveform, out, workspace, workspace_bytes, false, s, items);
   if (rc) return rc;
   char* base = (char*)workspace;
-  const std::vector<pjz::ResPlan> res = batch_resident(probs, n, s);
+  const std::vector<bool> alone = batch_alone(items, false, s);
   std::vector<pjz::BatchItem> rest;  // of the batched launches
   hipError_t e = hipSuccess;
   for (int i = 0; i < n && e == hipSuccess; ++i) {
     const pjz::BatchItem& it = items[i];
-    if (res[i].rx > 0)
-      e = forward_resident(it.g, *it.p, it.mask, it.src, it.win, it.ws, *it.L, res[i], s);
+    if (alone[i])
+      e = forward_steps(it.g, *it.p, it.mask, it.src, it.win, it.ws, *it.L, s);
     else
       rest.push_back(it);
   }
@@ -998,14 +1042,14 @@ int pjz_fdtd_batch_backward(const pjz_fdtd_problem* probs, int n, const float* c
                    items);
   if (rc) return rc;
   char* base = (char*)workspace;
-  const std::vector<pjz::ResPlan> res = batch_resident(probs, n, s);
+  const std::vector<bool> alone = batch_alone(items, true, s);
   std::vector<pjz::BatchItem> rest;  // of the batched launches, their cotangents
   std::vector<const float*> gout;
   hipError_t e = hipSuccess;
   for (int i = 0; i < n && e == hipSuccess; ++i) {
     const pjz::BatchItem& it = items[i];
-    if (res[i].rx > 0 && bp.Ls[i].nck > 0) {
-      e = backward_steps(it.g, *it.p, it.mask, it.src, grad_out[i], it.ws, *it.L, res[i], s);
+    if (alone[i] && bp.Ls[i].nck > 0) {
+      e = backward_steps(it.g, *it.p, it.mask, it.src, grad_out[i], it.ws, *it.L, s);
     } else {
       rest.push_back(it);
       gout.push_back(grad_out[i]);
@@ -1117,7 +1161,7 @@ int pjz_fdtd_backward(const pjz_fdtd_problem* p, const float* epsilon,
       !source_waveform || !grad_out || !grad_eps || !workspace)
     return fail(PJZ_FDTD_EINVAL, "a required pointer argument is NULL");
   pjz::Geom g = geom_of(*p);
-  pjz::Layout L = pjz::make_layout(g, *p);
+  pjz::Layout L = layout_in(g, *p, workspace_bytes);
   if (workspace_bytes < L.total)
     return fail(PJZ_FDTD_ESPACE, "workspace of %zu bytes, %zu needed", workspace_bytes, L.total);
   if (((uintptr_t)workspace & 255) != 0)
@@ -1136,7 +1180,7 @@ int pjz_fdtd_backward(const pjz_fdtd_problem* p, const float* epsilon,
     e = pjz::launch_zero((float*)(ws + L.lE_[0]), (L.total - L.lE_[0]) / 4, s);
   if (e != hipSuccess) return hip_fail(e, "backward set-up");
   pjz::Src src{p->src_axis, p->src_pos, p->src_quad, source_field, source_waveform};
-  e = backward_steps(g, *p, absorption_mask, src, grad_out, ws, L, resident_for(g, *p, s), s);
+  e = backward_steps(g, *p, absorption_mask, src, grad_out, ws, L, s);
   if (e == hipSuccess)
     e = pjz::launch_grad_eps(g, *p, epsilon, absorption_mask, ws, L, grad_eps, s);
   if (e != hipSuccess) return hip_fail(e, "backward launch");

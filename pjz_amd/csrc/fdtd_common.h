@@ -62,6 +62,8 @@ struct Layout {
   // of one S1 segment in slots nck .. nck+nfine-1.  One level: S1 = S,
   // nfine = 0.
   int S1, nfine;
+  // Exchange words of a run in slabs, past `total`; 0: the workspace has none.
+  size_t words = 0;
   size_t ckpt_floats;  // E (3N) + H (3N) + psi_H pair (2P) + psi_E pair (2P)
 };
 

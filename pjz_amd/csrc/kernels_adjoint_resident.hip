@@ -89,7 +89,7 @@ k_adj_resident(AdjResArgs a) {
   int valid_mask = 0;  // columns (in lE's order) inside the domain
 #pragma unroll
   for (int k = 0; k < C; ++k)
-    valid_mask |= (T.colx(Order::x(k)) < T.X && T.coly(Order::y(k)) < T.Y ? 1 : 0) << k;
+    valid_mask |= (T.colx(Order::x(k)) < T.xe && T.coly(Order::y(k)) < T.Y ? 1 : 0) << k;
   auto is_out = [&](int n) {
     return n >= a.ostart && n < a.ostop && (n - a.ostart) % a.ostep == 0;
   };
@@ -111,6 +111,8 @@ k_adj_resident(AdjResArgs a) {
     }
   };
 
+  T.fill(a.lu, a.lp, P, a.mask);
+  __builtin_amdgcn_sched_barrier(0);
   float le[RX][RY][3][CPL], lk[RX][RY][3][CPL], lh[RX][RY][3][CPL];
   float cbr[CBR ? RX : 1][CBR ? RY : 1][3][CPL], gr[GR ? RX : 1][GR ? RY : 1][3][CPL];
 #pragma unroll
@@ -131,7 +133,6 @@ k_adj_resident(AdjResArgs a) {
           if constexpr (CBR) cbr[CBR ? i : 0][CBR ? r : 0][k][c] = cb[k][c];
         }
     }
-  T.fill(a.lu, a.lp, P, a.mask);
   bool dead = false;
   __syncthreads();
   T.pass_low(a.tag0 + 1, lk);

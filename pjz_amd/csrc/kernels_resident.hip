@@ -105,6 +105,8 @@ k_resident(ResArgs a) {
     pE[c] = 4 * (pml[c] ? NP * 2 + pidx * 2 : NP * 4);
   }
 
+  T.fill(a.psiin, a.psiin ? a.psiin + 2 * (size_t)P : nullptr, P, a.mask);
+  __builtin_amdgcn_sched_barrier(0);
   float e[RX][RY][3][CPL], h[RX][RY][3][CPL], cbr[CBR ? RX : 1][CBR ? RY : 1][3][CPL];
 #pragma unroll
   for (int i = 0; i < RX; ++i)
@@ -121,10 +123,9 @@ k_resident(ResArgs a) {
       }
       if constexpr (CBR) T.load(cbr[i][r], a.cb, N, i, r);
     }
-  T.fill(a.psiin, a.psiin ? a.psiin + 2 * (size_t)P : nullptr, P, a.mask);
   if (a.saxis < 2) {
     // (row or column, component, z): the plane's field.
-    const int len = a.saxis == 0 ? Y : X, first = a.saxis == 0 ? T.by * T.TY : T.bx * T.TX;
+    const int len = a.saxis == 0 ? Y : X, first = a.saxis == 0 ? T.by * T.TY : T.xs;
     for (int q = threadIdx.x; q < nsrc; q += kResThreads) {
       const int t = q / ED, k = (q / (ED / 2)) & 1, z = q % (ED / 2);
       const int j = first + t;
@@ -134,7 +135,7 @@ k_resident(ResArgs a) {
     for (int q = threadIdx.x; q < nsrc; q += kResThreads) {
       const int t = q >> 2, k = q & 3;
       const int x = T.tile_x(t), y = T.tile_y(t);
-      srcl[q] = x < X && y < Y && k < 2 * a.squad ? a.sfield[(size_t)k * X * Y + x * Y + y] : 0.0f;
+      srcl[q] = x < T.xe && y < Y && k < 2 * a.squad ? a.sfield[(size_t)k * X * Y + x * Y + y] : 0.0f;
     }
   }
   bool dead = false;
@@ -218,19 +219,20 @@ k_resident(ResArgs a) {
   };
 
   // cb of a column from memory, from inside the domain (the selects that make
-  // it zero outside stand at its use: here they would wait for the loads).
-  int zc[CPL];
-#pragma unroll
-  for (int c = 0; c < CPL; ++c) zc[c] = 4 * min(zb + c, Z - 1);
+  // it zero outside stand at its use: here they would wait for the loads).  A
+  // lane's two cells come in one load; past the end of an odd row it reads the
+  // next row's first cell or, at the end of cb, the psi that follow it.
+  const int zc = 4 * min(zb, Z - 1);
   auto load_cb = [&](float (&v)[3][CPL], int i, int r) {
     const int x = min(opaque_s(T.colx(i)), X - 1), y = min(T.coly(r), Y - 1);
     const char* const p = reinterpret_cast<const char*>(a.cb + (x * Y + y) * Z);
+    const unsigned at = (unsigned)opaque_v(zc);
 #pragma unroll
-    for (int k = 0; k < 3; ++k)
+    for (int k = 0; k < 3; ++k) {
+      gcfloat* const q = to_global(reinterpret_cast<const float*>(p + 4 * (size_t)N * k + at));
 #pragma unroll
-      for (int c = 0; c < CPL; ++c)
-        v[k][c] = *reinterpret_cast<gcfloat*>(
-            to_global(reinterpret_cast<const float*>(p + 4 * (size_t)N * k + (unsigned)opaque_v(zc[c]))));
+      for (int c = 0; c < CPL; ++c) v[k][c] = q[c];
+    }
   };
 
   // Of the columns in E's order: those inside the domain, those with a source.
@@ -238,7 +240,7 @@ k_resident(ResArgs a) {
 #pragma unroll
   for (int k = 0; k < C; ++k) {
     const int x = T.colx(Order::x(k)), y = T.coly(Order::y(k)), at = a.saxis == 0 ? x : y;
-    valid_mask |= (x < X && y < Y ? 1 : 0) << k;
+    valid_mask |= (x < T.xe && y < Y ? 1 : 0) << k;
     src_mask |= (a.saxis == 2 || at == a.spos || at == a.spos - 1 ? 1 : 0) << k;
   }
 
@@ -375,7 +377,7 @@ k_resident(ResArgs a) {
         }
       }
       if constexpr (CAP) {
-        if (T.valid(i, r)) {
+        if (T.owned(i, r)) {
           gfloat* q = to_global(a.cap) + (size_t)(n - a.begin) * 3 * N + T.offset(i, r) + zb;
 #pragma unroll
           for (int m = 0; m < 3; ++m)
@@ -396,7 +398,7 @@ k_resident(ResArgs a) {
     for (int i = 0; i < RX; ++i)
 #pragma unroll
       for (int r = 0; r < RY; ++r)
-        if (T.valid(i, r)) {
+        if (T.owned(i, r)) {
           T.store(E, e[i][r], N, i, r);
           T.store(H, h[i][r], N, i, r);
         }
@@ -427,7 +429,7 @@ k_resident(ResArgs a) {
 #pragma unroll
         for (int r = 0; r < RY; ++r) {
           const int x = opaque_s(T.colx(i)) - a.wx0, y = T.coly(r) - a.wy0;
-          if (x >= 0 && x < a.wex && y >= 0 && y < a.wey) {
+          if (x >= 0 && x < a.wex && y >= 0 && y < a.wey && T.owned(i, r)) {
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
               gfloat* q = to_global(a.out) +
@@ -474,7 +476,8 @@ size_t res_lds(const Geom& g, int saxis, int cpl, int tx, int ty, int wx, int wy
 
 }  // namespace
 
-ResPlan resident_plan(const Geom& g, int saxis, int cus) {
+// The best tiling of X x Y columns whose words take at most `room` bytes.
+static ResPlan best_tiling(const Geom& g, int X, int saxis, int cus, size_t room) {
   ResPlan best{};
   if (g.Z > 128) return best;
   const int cpl = g.Z <= 64 ? 1 : 2;
@@ -484,7 +487,7 @@ ResPlan resident_plan(const Geom& g, int saxis, int cus) {
     if (s.cpl != cpl) continue;
     for (int wx = 1; wx <= kResWaves; wx *= 2) {
       ResPlan p{s.cpl, s.rx, s.ry, wx, kResWaves / wx, 0, 0, false, 0};
-      p.ntx = (g.X + p.tx() - 1) / p.tx();
+      p.ntx = (X + p.tx() - 1) / p.tx();
       p.nty = (g.Y + p.ty() - 1) / p.ty();
       if ((long long)p.ntx * p.nty > cus) continue;
       p.lds = res_lds(g, saxis, cpl, p.tx(), p.ty(), p.wx, p.wy, false);
@@ -495,8 +498,7 @@ ResPlan resident_plan(const Geom& g, int saxis, int cus) {
       }
       // More than half of a compute unit's LDS: one workgroup each.
       p.lds = std::max(p.lds, kResLds / 2 + 1024);
-      // The words take the place of the second set of E and H.
-      if (p.words() * sizeof(rword_t) > 2 * align256(sizeof(float) * 3 * (size_t)g.N)) continue;
+      if (p.words() * sizeof(rword_t) > room) continue;
       const int c = 64 * s.rx * s.ry + 2 * (s.rx + s.ry) + (p.alias ? 8 : 0) + p.tx() + p.ty();
       if (!best.rx || c < cost) {
         best = p;
@@ -505,6 +507,84 @@ ResPlan resident_plan(const Geom& g, int saxis, int cus) {
     }
   }
   return best;
+}
+
+ResPlan resident_plan(const Geom& g, int saxis, int cus) {
+  // The words take the place of the second set of E and H.
+  return best_tiling(g, g.X, saxis, cus, 2 * align256(sizeof(float) * 3 * (size_t)g.N));
+}
+
+// A resident step of a tiling, us, by its cells a lane, from the measurements
+// at the head of this file: past 16 cells cb comes from memory, two cells a
+// lane past 30 spill.
+static double step_us(const ResPlan& p) {
+  const int c = p.cpl * p.rx * p.ry;
+  return c <= 16 ? 2.5 + 0.3 * c : p.cpl == 2 && c > 30 ? 21.0 : 1.0 + 0.53 * c;
+}
+
+// Slabs cost their ghost columns, and every `steps` steps a launch each (35 us
+// with the start of its waves) and one pass over the state.  Taken where that
+// is estimated below 0.85 of the streaming steppers' rate, measured as 80-90
+// cells/ns at zz = 96, 94-113 at 128 and 110 at 64 (by the lanes in
+// use).  Measured, us a step: 220x200x96 48.9 -> 39.3, 260x196x96 55.0 -> 39.3,
+// 300x300x64 52.2 -> 31.3, 256x341x64 52.0 -> 35.3, 128x341x128 59.2 -> 42.7,
+// 512x512x64 148 -> 118; 256x256x128 in three slabs 75.7 against 74.5, which
+// this estimate leaves alone.
+SlabPlan slab_plan(const Geom& g, int saxis, int cus) {
+  SlabPlan best{};
+  if (g.Z > 128) return best;
+  const double cells = (double)g.N;
+  double cost = 0.85 * cells / (g.Z <= 64 ? 110e3 / 64 * g.Z : 0.85e3 * g.Z);
+  const double pass = cells * (60.0 + 32.0 * g.NP / g.Z) / 4.5e6;  // us
+  for (int n = 2; n <= 6; ++n) {
+    const int own = (g.X + n - 1) / n;
+    for (int k = 6; k <= 20; k += 2) {
+      if (own < 2 * k) break;
+      // The widest slab: an inner one where there are any.
+      const ResPlan t = best_tiling(g, own + (n > 2 ? 2 : 1) * k, saxis, cus, (size_t)1 << 30);
+      if (!t.rx) break;
+      const double c = n * step_us(t) + (n * 35.0 + pass) / k;
+      if (c < cost) {
+        cost = c;
+        best = {t, n, k};
+      }
+    }
+  }
+  return best;
+}
+
+hipError_t run_slabs(const Geom& g, const pjz_fdtd_problem& p, const float* mask, const Src& src,
+                     const OutWin& win, char* ws, const Layout& L, const SlabPlan& plan,
+                     rword_t* words, const StepRange& r, hipStream_t s) {
+  hipError_t e = launch_zero((float*)words, slab_words(plan) * 2, s);
+  float* psi = (float*)(ws + L.psi);
+  const size_t P4 = (size_t)PSI_SET * g.X * g.Y * g.NP;
+  auto state = [&](int set) {
+    return ResState{(float*)(ws + (set ? L.E1 : L.E0)), (float*)(ws + (set ? L.H1 : L.H0)),
+                    psi + set * P4};
+  };
+  const int own = (g.X + plan.n - 1) / plan.n;
+  unsigned tags = 0;
+  for (int b = r.begin; b < r.end && e == hipSuccess; b += plan.steps) {
+    const int end = std::min(b + plan.steps, r.end);
+    for (int i = 0; i < plan.n && e == hipSuccess; ++i) {
+      ResRun q{b, end, state(*r.cur), state(1 - *r.cur), nullptr, nullptr, 1, tags};
+      if (r.capture) q.capture = r.capture + (size_t)(b - r.begin) * 3 * g.N;
+      q.words = words;
+      q.own0 = i * own;
+      q.own1 = std::min(q.own0 + own, g.X);
+      q.xs = std::max(q.own0 - plan.steps, 0);
+      q.xe = std::min(q.own1 + plan.steps, g.X);
+      if (q.own0 >= q.own1) continue;
+      tags += resident_tags(end - b);
+      // The tiling of the widest slab, as many of its tiles as this one takes.
+      ResPlan t = plan.tile;
+      t.ntx = (q.xe - q.xs + t.tx() - 1) / t.tx();
+      e = run_resident(g, p, mask, src, win, ws, L, t, q, s);
+    }
+    *r.cur = 1 - *r.cur;
+  }
+  return e;
 }
 
 template <int CPL, int RX, int RY, bool CAP>
@@ -537,7 +617,13 @@ hipError_t run_resident(const Geom& g, const pjz_fdtd_problem& p, const float* m
   a.ckpt = r.ckpt;
   a.ckpt_stride = (long long)(ckpt_stride(L) / sizeof(float));
   a.every = r.every;
-  a.t = tile_args(g, plan, (rword_t*)(ws + L.E1));
+  a.t = tile_args(g, plan, r.words ? r.words : (rword_t*)(ws + L.E1));
+  if (r.xe > 0) {
+    a.t.xs = r.xs;
+    a.t.xe = r.xe;
+    a.t.own0 = r.own0;
+    a.t.own1 = r.own1;
+  }
   a.saxis = src.axis; a.spos = src.pos; a.squad = src.quad;
   a.dt = p.dt;
   a.begin = r.begin;

@@ -136,8 +136,12 @@ struct ResPlan {
 // the passing of edges.  Low edges are those of E (lK in the reverse run),
 // which the waves below and to the left read; high edges those of H.  At x
 // edges components 1 and 2 are passed, at y edges 0 and 2.
+//
+// A run may cover a slab of x only: columns [xs, xe), of which it writes (state,
+// snapshots, changes of E) its own, [own0, own1).
 struct ResTileArgs {
   int X, Y, Z, N, P, lo, hi, NP;
+  int xs, xe, own0, own1;
   int wx, wy, ntx, nty, alias;
   rword_t* words;
 };
@@ -146,12 +150,12 @@ template <int CPL, int RX, int RY>
 struct ResTile {
   static constexpr int C = RX * RY;
   static constexpr int ED = 2 * 64 * CPL;  // floats (or words) of an edge column
-  int lane, w, wx, wy, WX, WY, TX, TY, bx, by, x0, y0, zb, X, Y, Z, NP, PS;
+  int lane, w, wx, wy, WX, WY, TX, TY, bx, by, xs, xe, own0, own1, x0, y0, zb, X, Y, Z, NP, PS;
   float* lds;
   int er, hr, sx, sy;  // see edges()
   rword_t* mine;
   int ox, oy, oh, fx, fy;
-  bool xlo, xhi, ylo, yhi;
+  bool bxlo, bxhi, bylo, byhi, xlo, xhi, ylo, yhi;
   bool alias;
 
   __device__ __forceinline__ ResTile(const ResTileArgs& a, float* lds_) {
@@ -176,7 +180,11 @@ struct ResTile {
     if ((nt & 7) == 0) tile = (tile & 7) * (nt >> 3) + (tile >> 3);
     bx = __builtin_amdgcn_readfirstlane(tile / a.nty);
     by = __builtin_amdgcn_readfirstlane(tile % a.nty);
-    x0 = bx * TX + wx * RX;
+    xs = a.xs + bx * TX;
+    xe = a.xe;
+    own0 = a.own0;
+    own1 = a.own1;
+    x0 = xs + wx * RX;
     y0 = by * TY + wy * RY;
     zb = lane * CPL;
     lds = lds_;
@@ -192,10 +200,14 @@ struct ResTile {
     oh = (TX + TY) * ED;
     fx = (int)(a.nty * tw);
     fy = (int)tw;
-    xlo = wx == 0 && bx > 0;
-    xhi = wx == WX - 1 && bx + 1 < a.ntx;
-    ylo = wy == 0 && by > 0;
-    yhi = wy == WY - 1 && by + 1 < a.nty;
+    bxlo = bx > 0;
+    bxhi = bx + 1 < a.ntx;
+    bylo = by > 0;
+    byhi = by + 1 < a.nty;
+    xlo = wx == 0 && bxlo;
+    xhi = wx == WX - 1 && bxhi;
+    ylo = wy == 0 && bylo;
+    yhi = wy == WY - 1 && byhi;
   }
 
   // LDS: psi as (column, pair, PML cell, 2) and, per column, a zero pair for
@@ -229,14 +241,18 @@ struct ResTile {
   __device__ __forceinline__ int colx(int i) const { return x0 + i; }
   __device__ __forceinline__ int coly(int r) const { return y0 + r; }
   __device__ __forceinline__ bool valid(int i, int r) const {
-    return opaque_s(colx(i)) < X && coly(r) < Y;
+    return opaque_s(colx(i)) < xe && opaque_s(coly(r)) < Y;
+  }
+  __device__ __forceinline__ bool owned(int i, int r) const {
+    const int x = opaque_s(colx(i));
+    return x >= own0 && x < own1 && opaque_s(coly(r)) < Y;
   }
   __device__ __forceinline__ int offset(int i, int r) const {
     return (opaque_s(colx(i)) * Y + coly(r)) * Z;
   }
   // Column t of the tile's psi and absorber blocks: column t % C of wave t / C.
   __device__ __forceinline__ int tile_x(int t) const {
-    return bx * TX + (t / C) % WX * RX + t % C / RY;
+    return xs + (t / C) % WX * RX + t % C / RY;
   }
   __device__ __forceinline__ int tile_y(int t) const {
     return by * TY + (t / C) / WX * RY + t % C % RY;
@@ -261,20 +277,39 @@ struct ResTile {
       for (int c = 0; c < CPL; ++c)
         if (zb + c < Z) to_global(p)[k * N + o + c] = v[k][c];
   }
-  // The tile's psi (a pair of arrays P apart each) and absorber to LDS.
+  // A psi block's entry m = lane + 64 j: where it lies in the arrays.
+  __device__ __forceinline__ int psi_entry(int m, int P, bool& second) const {
+    second = m >= NP * 2;
+    return (m & 1) * P + ((m - (second ? NP * 2 : 0)) >> 1);
+  }
+  // The wave's psi (a pair of arrays P apart each; null: zeros) and the tile's
+  // absorber to LDS.  All of a wave's columns are requested at once: entry by
+  // entry over the tile, the loads' latencies added up to 40 us a launch.
   __device__ __forceinline__ void fill(const float* psi0, const float* psi1, int P,
                                        const float* mask) const {
-    for (int q = threadIdx.x; q < TX * TY * PS; q += kResThreads) {
-      const int t = q / PS, m = q - t * PS;
-      const int pair = m >= NP * 2, pi = (m - pair * NP * 2) >> 1;
-      const int x = tile_x(t), y = tile_y(t);
-      const float* p = pair ? psi1 : psi0;
-      lds[q] = p && m < NP * 4 && x < X && y < Y ? p[(m & 1) * P + (x * Y + y) * NP + pi] : 0.0f;
+    for (int j = 0; 64 * j < NP * 4; ++j) {
+      const int m = min(lane + 64 * j, NP * 4 - 1);
+      bool second;
+      const int at = psi_entry(m, P, second);
+      const float* const p = second ? psi1 : psi0;
+      float v[C];
+      static_for<C>([&](auto kk) __attribute__((always_inline)) {
+        constexpr int k = decltype(kk)::value, i = k / RY, r = k % RY;
+        v[k] = psi0 && valid(i, r) ? to_global(p)[at + (opaque_s(colx(i)) * Y + coly(r)) * NP]
+                                   : 0.0f;
+        // (Bounds the scalar registers that the columns' addresses take.)
+        if constexpr (k % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+      });
+      static_for<C>([&](auto kk) __attribute__((always_inline)) {
+        constexpr int k = decltype(kk)::value;
+        lds[(w * C + k) * PS + m] = v[k];
+      });
     }
+    if (lane < 2 * C) lds[(w * C + (lane >> 1)) * PS + NP * 4 + (lane & 1)] = 0.0f;
     for (int t = threadIdx.x; t < TX * TY; t += kResThreads) {
       const int x = tile_x(t), y = tile_y(t);
       f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};
-      if (x < X && y < Y) {
+      if (x < xe && y < Y) {
         const int m = x * Y + y, XY = X * Y;
         s = f32x4{mask[m], mask[XY + m], mask[2 * XY + m], 0.0f};
       }
@@ -283,13 +318,18 @@ struct ResTile {
   }
   // The wave's own psi back to memory (no barrier: nobody else's).
   __device__ __forceinline__ void store_psi(float* psi0, float* psi1, int P) const {
-    for (int q = lane; q < C * NP * 4; q += 64) {
-      const int t = q / (NP * 4), m = q - t * NP * 4;
-      const int x = x0 + t / RY, y = y0 + t % RY;
-      const int pair = m >= NP * 2, pi = (m - pair * NP * 2) >> 1;
-      if (x < X && y < Y)
-        to_global(pair ? psi1 : psi0)[(m & 1) * P + (x * Y + y) * NP + pi] =
-            lds[(w * C + t) * PS + m];
+    for (int j = 0; 64 * j < NP * 4; ++j) {
+      const int m = lane + 64 * j;
+      if (m >= NP * 4) break;
+      bool second;
+      const int at = psi_entry(m, P, second);
+      float* const p = second ? psi1 : psi0;
+      static_for<C>([&](auto kk) __attribute__((always_inline)) {
+        constexpr int k = decltype(kk)::value, i = k / RY, r = k % RY;
+        if (owned(i, r))
+          to_global(p)[at + (opaque_s(colx(i)) * Y + coly(r)) * NP] = lds[(w * C + k) * PS + m];
+        __builtin_amdgcn_sched_barrier(0);
+      });
     }
   }
   // A column's psi pair, from the lane's address in a column's block.
@@ -351,12 +391,48 @@ struct ResTile {
         post(oh + oy + i * ED, tag, h[i][RY - 1][0], h[i][RY - 1][2]);
     }
   }
+  // The words p[0], p[64], .. of K columns once they carry `tag`; columns with
+  // no such neighbour are zeros.
+  template <int K>
+  __device__ __forceinline__ void wait(const int (&at)[K], const int (&dst)[K],
+                                       const bool (&there)[K], unsigned tag, bool& dead) const {
+    constexpr int NW = 2 * CPL;
+    rword_t v[K * NW];
+    for (int polls = 0;; ++polls) {
+      bool ok = true;
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        const rword_t* const p = edge_word(mine, there[k] ? at[k] : 0, lane);
+#pragma unroll
+        for (int c = 0; c < NW; ++c)
+          v[k * NW + c] =
+              __hip_atomic_load(p + 64 * c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+#pragma unroll
+      for (int k = 0; k < K; ++k)
+#pragma unroll
+        for (int c = 0; c < NW; ++c)
+          ok &= (unsigned)(v[k * NW + c] >> 32) == tag || !there[k];
+      if (__all(ok) || dead) break;
+      dead = polls >= kMaxPolls;
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        float t[CPL];
+#pragma unroll
+        for (int c = 0; c < CPL; ++c)
+          t[c] = there[k] ? __uint_as_float((unsigned)v[k * NW + q * CPL + c]) : 0.0f;
+        lds_put<CPL>(slot(dst[k]) + q * (ED / 2), t);
+      }
+  }
   // n columns of a border wave's outer slot: the neighbour's edge, or zeros
   // past the domain.  K columns at a time (the registers of the words).
   template <int n>
-  __device__ __forceinline__ void take(float* dst, int off, bool there, unsigned tag,
+  __device__ __forceinline__ void take_own(float* dst, int off, bool there, unsigned tag,
                                        bool& dead) const {
-    constexpr int K = CPL == 1 ? 4 : 2, NW = 2 * CPL;
+    constexpr int K = kCols, NW = 2 * CPL;
 #pragma unroll
     for (int k0 = 0; k0 < n; k0 += K) {
       float v[K * NW];
@@ -383,17 +459,54 @@ struct ResTile {
         }
     }
   }
-  // Once every wave of the workgroup has passed its edges: those of the
-  // neighbouring workgroups.
+  // The tile's TY + TX columns shared out over its waves.
+  __device__ __forceinline__ void take_shared(int lds_x, int lds_y, int word_x, int word_y,
+                                              bool there_x, bool there_y, unsigned tag,
+                                              bool& dead) const {
+    for (int k0 = 0; w + kResWaves * k0 < TX + TY; k0 += kCols) {
+      int at[kCols], dst[kCols];
+      bool there[kCols];
+#pragma unroll
+      for (int k = 0; k < kCols; ++k) {
+        int q = w + kResWaves * (k0 + k);
+        if (q >= TX + TY) q = w + kResWaves * k0;  // (again)
+        const bool x = q < TY;
+        at[k] = x ? word_x + q * ED : word_y + (q - TY) * ED;
+        dst[k] = x ? lds_x + q * ED : lds_y + (q - TY) * ED;
+        there[k] = x ? there_x : there_y;
+      }
+      wait<kCols>(at, dst, there, tag, dead);
+    }
+  }
+  // The neighbouring workgroups' edges into the outer slots (zeros past the
+  // domain); after these every edge that the wave's columns need is in LDS.
+  // Every poll is a trip to memory in the step's critical path (0.8 us).  Up to
+  // 20 cells a lane the border waves wait for their own columns, in one or two
+  // polls an edge; beyond, all waves share the tile's columns (150x140x96: 14.3
+  // -> 12.6 us a step; 64^3, where one poll is enough, 2.9 with its own
+  // columns, 3.6 shared).
+  static constexpr int kCols = CPL == 1 ? 4 : 2;  // columns a poll: 16 registers
+  static constexpr bool kShared = C * CPL > 20;
   __device__ __forceinline__ void take_low(unsigned tag, bool& dead) const {
-    lds_barrier();
-    if (wx == WX - 1) take<RY>(low_x(), fx + ox, xhi, tag, dead);
-    if (wy == WY - 1) take<RX>(low_y(), fy + oy, yhi, tag, dead);
+    if constexpr (kShared) {
+      take_shared(er + (WX - 1) * TY * ED, er + (WX * TY + (WY - 1) * TX) * ED, fx, fy + TY * ED,
+                  bxhi, byhi, tag, dead);
+      lds_barrier();
+    } else {
+      lds_barrier();
+      if (wx == WX - 1) take_own<RY>(low_x(), fx + ox, bxhi, tag, dead);
+      if (wy == WY - 1) take_own<RX>(low_y(), fy + oy, byhi, tag, dead);
+    }
   }
   __device__ __forceinline__ void take_high(unsigned tag, bool& dead) const {
-    lds_barrier();
-    if (wx == 0) take<RY>(high_x(), oh + ox - fx, xlo, tag, dead);
-    if (wy == 0) take<RX>(high_y(), oh + oy - fy, ylo, tag, dead);
+    if constexpr (kShared) {
+      take_shared(hr, hr + WX * TY * ED, oh - fx, oh - fy + TY * ED, bxlo, bylo, tag, dead);
+      lds_barrier();
+    } else {
+      lds_barrier();
+      if (wx == 0) take_own<RY>(high_x(), oh + ox - fx, bxlo, tag, dead);
+      if (wy == 0) take_own<RX>(high_y(), oh + oy - fy, bylo, tag, dead);
+    }
   }
   // With one set of edge buffers: before it is written again.
   __device__ __forceinline__ void edges_read() const {
@@ -403,6 +516,8 @@ struct ResTile {
 
 inline ResTileArgs tile_args(const Geom& g, const ResPlan& p, rword_t* words) {
   ResTileArgs a;
+  a.xs = a.own0 = 0;
+  a.xe = a.own1 = g.X;
   a.X = g.X; a.Y = g.Y; a.Z = g.Z; a.lo = g.lo; a.hi = g.hi; a.NP = g.NP;
   a.N = (int)g.N;
   a.P = g.X * g.Y * g.NP;
@@ -417,7 +532,8 @@ struct ResState {
   float *E, *H, *psi;
 };
 
-// Steps [begin, end) in one launch.
+// Steps [begin, end) in one launch, on columns [xs, xe) of x, of which [own0,
+// own1) are written (xe = 0: the whole domain).
 struct ResRun {
   int begin, end;
   ResState in, out;   // out.E = null: the last state is not stored
@@ -425,12 +541,30 @@ struct ResRun {
   float* ckpt;        // states before steps begin, begin + every, ... (or null)
   int every;
   unsigned tag0;      // exchange numbers used before (the words start from 0)
+  rword_t* words = nullptr;  // null: at L.E1
+  int xs = 0, xe = 0, own0 = 0, own1 = 0;
 };
 // Exchange numbers a run of n steps uses.
 inline unsigned resident_tags(int n) { return (unsigned)n + 1; }
 
 // The tiling for a domain on `cus` compute units (rx = 0: it does not fit).
 ResPlan resident_plan(const Geom& g, int saxis, int cus);
+
+// A domain that does not fit as a whole, in `n` slabs of x run one after the
+// other, `steps` at a time: each with that many columns more on its inner
+// sides, whose outermost is wrong after one step, the next after two, ...
+// (n = 0: none worth it; tile: of the widest slab).
+struct SlabPlan {
+  ResPlan tile;
+  int n, steps;
+};
+SlabPlan slab_plan(const Geom& g, int saxis, int cus);
+// Steps r of a domain in slabs, from buffer set *r.cur to the one it is set
+// to; words: slab_words() of them.
+inline size_t slab_words(const SlabPlan& p) { return p.n > 0 ? p.tile.words() : 0; }
+hipError_t run_slabs(const Geom& g, const pjz_fdtd_problem& p, const float* mask, const Src& src,
+                     const OutWin& win, char* ws, const Layout& L, const SlabPlan& plan,
+                     rword_t* words, const StepRange& r, hipStream_t s);
 
 // Whether a tiling's kernel that also writes each step's change of E is worth
 // its while: past 25 cells a lane, two a column, it spills (the one-step

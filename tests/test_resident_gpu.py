@@ -120,3 +120,46 @@ def test_batch_of_resident_and_streamed_simulations():
     assert G.rel_l2(o.detach().cpu().numpy(), out) <= 1e-6
     assert G.rel_l2(q.cpu().numpy(), out) <= 1e-6
     assert G.rel_l2(e.grad.cpu().numpy(), ref) <= 1e-5
+
+
+# Larger domains in slabs of x (two to five), each with ghost columns that a
+# block of steps uses up: snapshots inside a block and after it, runs that end
+# inside one, every source axis, ragged last slabs.
+@pytest.mark.parametrize("axis,X,Y,Z,steps", [(0, 260, 196, 96, 50), (1, 200, 190, 96, 37),
+                                              (2, 223, 201, 96, 45), (0, 300, 301, 64, 53),
+                                              (2, 401, 300, 45, 41), (0, 129, 341, 128, 40),
+                                              (1, 256, 341, 50, 64), (0, 500, 81, 99, 40)])
+def test_slabs_match_streaming_kernels(axis, X, Y, Z, steps):
+  print(f"case {X}x{Y}x{Z} axis {axis}", flush=True)
+  kw = T.random_problem(axis, X=X, Y=Y, Z=Z, tt=steps, seed=X, widths=(6, 5))
+  kw["output_steps"] = (steps - 23, steps, 2)
+  if axis == 0:
+    kw["source_position"] = 2 * (X // 4)  # in the slabs' ghost columns
+  kernel = "stream2" if Z <= 64 or Z % 2 == 0 else "stream"
+  assert T.rel_l2(run(kw), run(kw, kernel)) <= 1e-6
+
+
+@pytest.mark.parametrize("launch", [dict(ckpt_every=20), dict(ckpt_every=44, ckpt_inner=18)])
+def test_slab_gradient_matches_streaming_kernels(launch):
+  eps, kw, g = G.problem(0, seed=9, X=260, Y=196, Z=96, tt=60)
+  got, _ = G.gpu_grad(eps, kw, g, **launch)
+  ref, _ = G.gpu_grad(eps, kw, g, kernel="stream2", **launch)
+  assert G.rel_l2(got, ref) <= 1e-5
+
+
+def test_batch_with_slabs():
+  """As test_batch_of_resident_and_streamed_simulations, with domains in slabs."""
+  cases = [G.problem(axis, seed=axis, X=X, Y=Y, Z=Z, tt=tt)
+           for axis, X, Y, Z, tt in [(0, 260, 196, 96, 40), (1, 30, 40, 64, 41),
+                                     (2, 300, 300, 64, 40)]]
+  eps = [torch.tensor(e, device="cuda", requires_grad=True) for e, _, _ in cases]
+  calls = [dict(kw, epsilon=e, launch_params=dict(ckpt_every=18))
+           for e, (_, kw, _) in zip(eps, cases)]
+  outs = F.fdtdz_batch(calls)
+  sum((o * torch.as_tensor(g, device="cuda")).sum() for o, (_, _, g) in zip(outs, cases)).backward()
+  plain = F.fdtdz_batch([dict(c, epsilon=c["epsilon"].detach()) for c in calls])
+  for e, o, q, (e0, kw, g) in zip(eps, outs, plain, cases):
+    ref, out = G.gpu_grad(e0, kw, g, ckpt_every=18, kernel="stream2")
+    assert G.rel_l2(o.detach().cpu().numpy(), out) <= 1e-6
+    assert G.rel_l2(q.cpu().numpy(), out) <= 1e-6
+    assert G.rel_l2(e.grad.cpu().numpy(), ref) <= 1e-5
