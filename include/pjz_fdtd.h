@@ -124,10 +124,10 @@ PJZ_FDTD_API int pjz_fdtd_forward(const pjz_fdtd_problem* p, const float* epsilo
  * Forward simulation without a workspace argument, for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid allocation).  No counterpart in pjz or fdtdz: the
- * library-owned variant of pjz_fdtd_forward (same arguments, results and
- * kernels).  The workspace is a library array of PJZ_FDTD_NOALLOC_MAX_BYTES
+ * library-owned variant of pjz_fdtd_forward (same arguments and results, on
+ * the kernels that are launched step by step).  The workspace is a library array of PJZ_FDTD_NOALLOC_MAX_BYTES
  * per GPU, held until the process ends; a problem whose workspace
- * (pjz_fdtd_workspace_bytes) exceeds it returns PJZ_FDTD_ESPACE, and
+ * (pjz_fdtd_workspace_bytes of those kernels) exceeds it returns PJZ_FDTD_ESPACE, and
  * ckpt_every must be 0.  The call allocates nothing and launches only fill,
  * set-up and stepper kernels (an AUTOTUNE kernel id uses a cached choice
  * for the shape, else the default kernel, instead of tuning).  Every call on
@@ -164,8 +164,9 @@ PJZ_FDTD_API int pjz_fdtd_batch_forward(const pjz_fdtd_problem* probs, int n,
 /*
  * Batched gradient: pjz_fdtd_backward for every simulation of a preceding
  * pjz_fdtd_batch_forward call with ckpt_every > 0 (same problems, arrays and
- * workspace).  Segments are recomputed by the batched two-step kernel and
- * every reverse step is one launch pair for the whole batch.  grad_out and
+ * workspace).  Simulations that the resident kernels take run one by one; for
+ * the others segments are recomputed by the batched two-step kernel and every
+ * reverse step is one launch pair for all of them.  grad_out and
  * grad_eps are HOST arrays of n device pointers.  No counterpart in pjz (see
  * pjz_fdtd_backward).
  */
@@ -279,9 +280,11 @@ PJZ_FDTD_API int pjz_fdtd_render_backward(int32_t ll, int32_t m, int32_t xx, int
                                           size_t workspace_bytes, void* stream);
 
 /*
- * Diagnostic: the stepper (PJZ_FDTD_KERNEL_REFERENCE .. STREAM4) a forward
- * call with this problem runs on the current device: AUTO and AUTOTUNE
- * resolved (AUTOTUNE to its cached choice, or AUTO before the first call).
+ * Diagnostic: the stepper (PJZ_FDTD_KERNEL_REFERENCE .. STREAM4) that a
+ * forward call with this problem launches step by step on the current device:
+ * AUTO and AUTOTUNE resolved (AUTOTUNE to its cached choice, or AUTO before
+ * the first call).  AUTO calls whose domain fits the GPU's registers, whole or
+ * in a few slabs, run the resident stepper instead, with the same results.
  * No counterpart in pjz: bench.py reports it beside the kernel's timings.
  */
 PJZ_FDTD_API int pjz_fdtd_stepper(const pjz_fdtd_problem* p, int32_t* kernel);

@@ -815,6 +815,9 @@ int pjz_fdtd_forward_noalloc(const pjz_fdtd_problem* p, const float* epsilon,
   pjz_fdtd_problem q = *p;
   Tuned t;
   if (q.kernel == PJZ_FDTD_KERNEL_AUTOTUNE && !tuned_choice(q, &t)) q.kernel = PJZ_FDTD_KERNEL_AUTO;
+  // Concurrent calls may share the array (and then get wrong results); workgroups
+  // that wait for one another's words must not.
+  if (q.kernel == PJZ_FDTD_KERNEL_AUTO) q.kernel = auto_kernel(geom_of(q));
   return pjz_fdtd_forward(&q, epsilon, absorption_mask, pml_kappa, pml_sigma, pml_alpha,
                           source_field, source_waveform, out, ws, kScratchBytes, stream);
 }

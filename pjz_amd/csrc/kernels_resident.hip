@@ -25,9 +25,9 @@
 //
 // Measured, us a step, two-step kernel (the default before) against this:
 // 64^3 13.4 -> 2.9 (both exchange latencies), 128x128x64 14.3 -> 5.2,
-// 160x160x64 20.4 -> 6.9 (16 cells a lane: arithmetic), 190x200x50 25.1 ->
-// 11.1, 150x140x96 29.0 -> 13.8, 301x187x45 45.0 -> 19.3, 180x150x128 37.2 ->
-// 18.4 (20-30 cells a lane: cb from the caches).
+// 160x160x64 20.4 -> 7.0 (16 cells a lane: arithmetic), 190x200x50 25.1 ->
+// 10.8, 150x140x96 29.0 -> 12.6, 301x187x45 45.0 -> 17.6, 180x150x128 37.2 ->
+// 16.8 (20-30 cells a lane: arithmetic of two waves a SIMD, cb from the caches).
 //
 // The arithmetic of a cell is that of the two-step kernel (stream2_parts.h),
 // in its order of rounding: results equal that kernel's bit for bit.
@@ -138,7 +138,6 @@ k_resident(ResArgs a) {
       srcl[q] = x < T.xe && y < Y && k < 2 * a.squad ? a.sfield[(size_t)k * X * Y + x * Y + y] : 0.0f;
     }
   }
-  bool dead = false;
 
   __syncthreads();
   T.pass_low(a.tag0 + 1, e);
@@ -158,7 +157,7 @@ k_resident(ResArgs a) {
     load_psi(nps, 0, RX - 1 - Order::x(0), RY - 1 - Order::y(0));
     static_for<C>([&](auto kk) __attribute__((always_inline)) {
       constexpr int k = decltype(kk)::value;
-      if (k == Order::inner) T.take_low(tag, dead);
+      if (k == Order::inner) T.take_low(tag);
       constexpr int i = RX - 1 - Order::x(k), r = RY - 1 - Order::y(k);
       f32x2 ps[CPL];
 #pragma unroll
@@ -271,7 +270,7 @@ k_resident(ResArgs a) {
     }
     static_for<C>([&](auto kk) __attribute__((always_inline)) {
       constexpr int k = decltype(kk)::value;
-      if (k == Order::inner) T.take_high(tag, dead);
+      if (k == Order::inner) T.take_high(tag);
       constexpr int i = Order::x(k), r = Order::y(k);
       const f32x4 sg = nsg;
       f32x2 ps[CPL];
@@ -421,7 +420,13 @@ k_resident(ResArgs a) {
     e_phase(n, tag, w0, w1);
     w0 = u0;
     w1 = u1;
-    if (dead) e[0][0][0][0] = e[0][0][1][0] = e[0][0][2][0] = __builtin_nanf("");
+    // Never taken (every >= 0).  Without a write the compiler cannot rule out
+    // here, the capturing kernels keep both versions of a step's fields live:
+    // 157 spilled registers instead of 13 at 30 cells a lane.
+    if constexpr (CAP) {
+      if (__builtin_expect(a.every < 0, 0))
+        e[0][0][0][0] = e[0][0][1][0] = e[0][0][2][0] = 0.0f;
+    }
     if (a.out && n >= a.ostart && n < a.ostop && (n - a.ostart) % a.ostep == 0) {
       const int slot = (n - a.ostart) / a.ostep;
 #pragma unroll

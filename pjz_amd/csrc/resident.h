@@ -60,26 +60,22 @@ __device__ __forceinline__ void post_edge(rword_t* p, unsigned tag, float v) {
                      __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// The words p[0], p[64], .. p[64 (NW - 1)] once all carry `tag`.  A peer posts
-// within microseconds, so a wait of seconds means that the words were
-// overwritten (two calls that share one workspace): the wave then sets `dead`,
-// waits no more and its fields become NaN.
-constexpr int kMaxPolls = 1 << 22;
-
+// The words p[0], p[64], .. p[64 (NW - 1)] once all carry `tag`.  Every
+// workgroup of the launch is resident at some time (cooperative launch) and
+// posts before it waits for the answer, so the wait ends; it is not bounded,
+// as other streams' kernels may hold back some of the workgroups for long.
 template <int NW>
-__device__ __forceinline__ void wait_edges(float (&v)[NW], const rword_t* p, unsigned tag,
-                                           bool& dead) {
+__device__ __forceinline__ void wait_edges(float (&v)[NW], const rword_t* p, unsigned tag) {
   rword_t w[NW];
-  for (int polls = 0;; ++polls) {
-    bool ok = true;
+  bool ok;
+  do {
+    ok = true;
 #pragma unroll
     for (int k = 0; k < NW; ++k)
       w[k] = __hip_atomic_load(p + 64 * k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
     for (int k = 0; k < NW; ++k) ok &= (unsigned)(w[k] >> 32) == tag;
-    if (__all(ok) || dead) break;
-    dead = polls >= kMaxPolls;
-  }
+  } while (!__all(ok));
 #pragma unroll
   for (int k = 0; k < NW; ++k) v[k] = __uint_as_float((unsigned)w[k]);
 }
@@ -395,11 +391,12 @@ struct ResTile {
   // no such neighbour are zeros.
   template <int K>
   __device__ __forceinline__ void wait(const int (&at)[K], const int (&dst)[K],
-                                       const bool (&there)[K], unsigned tag, bool& dead) const {
+                                       const bool (&there)[K], unsigned tag) const {
     constexpr int NW = 2 * CPL;
     rword_t v[K * NW];
-    for (int polls = 0;; ++polls) {
-      bool ok = true;
+    bool ok;
+    do {
+      ok = true;
 #pragma unroll
       for (int k = 0; k < K; ++k) {
         const rword_t* const p = edge_word(mine, there[k] ? at[k] : 0, lane);
@@ -413,9 +410,7 @@ struct ResTile {
 #pragma unroll
         for (int c = 0; c < NW; ++c)
           ok &= (unsigned)(v[k * NW + c] >> 32) == tag || !there[k];
-      if (__all(ok) || dead) break;
-      dead = polls >= kMaxPolls;
-    }
+    } while (!__all(ok));
 #pragma unroll
     for (int k = 0; k < K; ++k)
 #pragma unroll
@@ -430,8 +425,7 @@ struct ResTile {
   // n columns of a border wave's outer slot: the neighbour's edge, or zeros
   // past the domain.  K columns at a time (the registers of the words).
   template <int n>
-  __device__ __forceinline__ void take_own(float* dst, int off, bool there, unsigned tag,
-                                       bool& dead) const {
+  __device__ __forceinline__ void take_own(float* dst, int off, bool there, unsigned tag) const {
     constexpr int K = kCols, NW = 2 * CPL;
 #pragma unroll
     for (int k0 = 0; k0 < n; k0 += K) {
@@ -440,11 +434,11 @@ struct ResTile {
 #pragma unroll
         for (int q = 0; q < K * NW; ++q) v[q] = 0.0f;
       } else if (k0 + K <= n) {
-        wait_edges<K * NW>(v, edge_word(mine, off + k0 * ED, lane), tag, dead);
+        wait_edges<K * NW>(v, edge_word(mine, off + k0 * ED, lane), tag);
       } else {
         constexpr int rest = n % K ? n % K : K;
         float u[rest * NW];
-        wait_edges<rest * NW>(u, edge_word(mine, off + k0 * ED, lane), tag, dead);
+        wait_edges<rest * NW>(u, edge_word(mine, off + k0 * ED, lane), tag);
 #pragma unroll
         for (int q = 0; q < rest * NW; ++q) v[q] = u[q];
       }
@@ -461,8 +455,7 @@ struct ResTile {
   }
   // The tile's TY + TX columns shared out over its waves.
   __device__ __forceinline__ void take_shared(int lds_x, int lds_y, int word_x, int word_y,
-                                              bool there_x, bool there_y, unsigned tag,
-                                              bool& dead) const {
+                                              bool there_x, bool there_y, unsigned tag) const {
     for (int k0 = 0; w + kResWaves * k0 < TX + TY; k0 += kCols) {
       int at[kCols], dst[kCols];
       bool there[kCols];
@@ -475,7 +468,7 @@ struct ResTile {
         dst[k] = x ? lds_x + q * ED : lds_y + (q - TY) * ED;
         there[k] = x ? there_x : there_y;
       }
-      wait<kCols>(at, dst, there, tag, dead);
+      wait<kCols>(at, dst, there, tag);
     }
   }
   // The neighbouring workgroups' edges into the outer slots (zeros past the
@@ -487,25 +480,25 @@ struct ResTile {
   // columns, 3.6 shared).
   static constexpr int kCols = CPL == 1 ? 4 : 2;  // columns a poll: 16 registers
   static constexpr bool kShared = C * CPL > 20;
-  __device__ __forceinline__ void take_low(unsigned tag, bool& dead) const {
+  __device__ __forceinline__ void take_low(unsigned tag) const {
     if constexpr (kShared) {
       take_shared(er + (WX - 1) * TY * ED, er + (WX * TY + (WY - 1) * TX) * ED, fx, fy + TY * ED,
-                  bxhi, byhi, tag, dead);
+                  bxhi, byhi, tag);
       lds_barrier();
     } else {
       lds_barrier();
-      if (wx == WX - 1) take_own<RY>(low_x(), fx + ox, bxhi, tag, dead);
-      if (wy == WY - 1) take_own<RX>(low_y(), fy + oy, byhi, tag, dead);
+      if (wx == WX - 1) take_own<RY>(low_x(), fx + ox, bxhi, tag);
+      if (wy == WY - 1) take_own<RX>(low_y(), fy + oy, byhi, tag);
     }
   }
-  __device__ __forceinline__ void take_high(unsigned tag, bool& dead) const {
+  __device__ __forceinline__ void take_high(unsigned tag) const {
     if constexpr (kShared) {
-      take_shared(hr, hr + WX * TY * ED, oh - fx, oh - fy + TY * ED, bxlo, bylo, tag, dead);
+      take_shared(hr, hr + WX * TY * ED, oh - fx, oh - fy + TY * ED, bxlo, bylo, tag);
       lds_barrier();
     } else {
       lds_barrier();
-      if (wx == 0) take_own<RY>(high_x(), oh + ox - fx, bxlo, tag, dead);
-      if (wy == 0) take_own<RX>(high_y(), oh + oy - fy, bylo, tag, dead);
+      if (wx == 0) take_own<RY>(high_x(), oh + ox - fx, bxlo, tag);
+      if (wy == 0) take_own<RX>(high_y(), oh + oy - fy, bylo, tag);
     }
   }
   // With one set of edge buffers: before it is written again.
