@@ -368,6 +368,8 @@ k_adj_resident(AdjResArgs a) {
 
 // ------------------------------------------------------------------ host side
 
+// Up to 16 cells a lane: 20 spill 53 registers, and the gradient of 190x200x50
+// over 200 steps takes 14.5 ms instead of 12.6 with the streaming reverse.
 #define PJZ_ADJ_SHAPES(F)                                                              \
   F(1, 2, 1) F(1, 2, 2) F(1, 3, 2) F(1, 4, 2) F(1, 4, 3) F(1, 4, 4)                     \
   F(2, 1, 1) F(2, 2, 1) F(2, 2, 2) F(2, 3, 2) F(2, 4, 2)
