@@ -25,7 +25,18 @@
  *     message names it), PJZ_FDTD_EHIP (HIP runtime error), PJZ_FDTD_ESPACE
  *     (workspace too small).  pjz_fdtd_last_error() returns the calling
  *     thread's last message.
- *   - Calls are re-entrant; concurrent calls must use distinct workspaces.
+ *   - Calls are re-entrant; concurrent calls must use distinct workspaces, and
+ *     a workspace must not be used by a call while an earlier one on another
+ *     stream still runs in it.
+ *   - By default (PJZ_FDTD_KERNEL_AUTO) a run whose domain fits the GPU's
+ *     registers is one launch whose workgroups wait for one another.  They need
+ *     the GPU's compute units at the same time and words of the workspace that
+ *     nobody else writes.  Where that fails (a workspace in use by two calls,
+ *     another process on the same GPU) the waits end after 20 s and 1 ms a
+ *     step, the outputs hold NaN, and the next call on that GPU that enqueues a
+ *     simulation, or pjz_fdtd_run_status, returns PJZ_FDTD_ESTALL, once.
+ *     PJZ_FDTD_FLAG_STEPWISE or a kernel id other than AUTO runs kernels
+ *     without such waits.
  */
 #ifndef PJZ_FDTD_H_
 #define PJZ_FDTD_H_
@@ -49,6 +60,7 @@ extern "C" {
 #define PJZ_FDTD_EINVAL 1
 #define PJZ_FDTD_EHIP 2
 #define PJZ_FDTD_ESPACE 3
+#define PJZ_FDTD_ESTALL 4
 
 /* Kernel selection (the `launch_params` analogue, field `kernel`). */
 #define PJZ_FDTD_KERNEL_AUTO 0
@@ -60,6 +72,11 @@ extern "C" {
                                     /* stream), later calls reuse the fastest    */
 #define PJZ_FDTD_KERNEL_STREAM3 5   /* three steps per launch (zz <= 64)         */
 #define PJZ_FDTD_KERNEL_STREAM4 6   /* four steps per launch (zz <= 64)          */
+
+/* Flags of a problem. */
+#define PJZ_FDTD_FLAG_REDUCED 1  /* use_reduced_precision (fp32 storage kept)      */
+#define PJZ_FDTD_FLAG_STEPWISE 2 /* AUTO: only kernels launched step by step (for  */
+                                 /* a GPU shared with other processes)            */
 
 /* Problem description: the static arguments of fdtdz(...). */
 typedef struct pjz_fdtd_problem {
@@ -73,7 +90,7 @@ typedef struct pjz_fdtd_problem {
   int32_t tt;            /* rows of source_waveform (tt,2)                       */
   int32_t out_start, out_stop, out_step; /* `output_steps`                       */
   float dt;              /* `dt`                                                 */
-  int32_t flags;         /* bit 0: use_reduced_precision (fp32 storage kept)     */
+  int32_t flags;         /* PJZ_FDTD_FLAG_*                                      */
   int32_t kernel;        /* PJZ_FDTD_KERNEL_*                                    */
   int32_t tile_x, tile_y;/* launch overrides for the stream kernel, 0 = auto     */
                          /* (batches: tile_y 8 or 13 on every zz <= 64 sim    */
@@ -97,6 +114,20 @@ PJZ_FDTD_API int pjz_fdtd_abi_version(void);
 
 /* Last error message of the calling thread ("" if none). */
 PJZ_FDTD_API const char* pjz_fdtd_last_error(void);
+
+/*
+ * PJZ_FDTD_ESTALL, once, if a run on the current GPU has waited in vain since
+ * the last report of one (see the conventions above), else 0.  The run has to
+ * have finished: synchronise first.
+ */
+PJZ_FDTD_API int pjz_fdtd_run_status(void);
+
+/*
+ * Makes later calls of the calling thread take failure paths that tests check:
+ * a mask of PJZ_FDTD_TEST_* (0, the default: none).
+ */
+#define PJZ_FDTD_TEST_STALL 1  /* a workgroup is missing and its peers give up soon */
+PJZ_FDTD_API void pjz_fdtd_test_faults(uint32_t faults);
 
 /* Number of snapshots, len(range(*output_steps)). */
 PJZ_FDTD_API int pjz_fdtd_num_outputs(const pjz_fdtd_problem* p, int32_t* nn);

@@ -12,14 +12,18 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libpjzfdtd.so")
 ABI_VERSION = 1
 
-OK, EINVAL, EHIP, ESPACE = 0, 1, 2, 3
+OK, EINVAL, EHIP, ESPACE, ESTALL = 0, 1, 2, 3, 4
 KERNEL_AUTO, KERNEL_REFERENCE, KERNEL_STREAM, KERNEL_STREAM2, KERNEL_AUTOTUNE = 0, 1, 2, 3, 4
 KERNEL_STREAM3, KERNEL_STREAM4 = 5, 6
+FLAG_REDUCED, FLAG_STEPWISE = 1, 2
+TEST_STALL = 1
 
 # Every entry point include/pjz_fdtd.h declares.
 EXPORTS = (
     "pjz_fdtd_abi_version",
     "pjz_fdtd_last_error",
+    "pjz_fdtd_run_status",
+    "pjz_fdtd_test_faults",
     "pjz_fdtd_num_outputs",
     "pjz_fdtd_workspace_bytes",
     "pjz_fdtd_forward",
@@ -83,6 +87,10 @@ def load():
     lib.pjz_fdtd_abi_version.argtypes = []
     lib.pjz_fdtd_last_error.restype = ctypes.c_char_p
     lib.pjz_fdtd_last_error.argtypes = []
+    lib.pjz_fdtd_run_status.restype = ctypes.c_int
+    lib.pjz_fdtd_run_status.argtypes = []
+    lib.pjz_fdtd_test_faults.restype = None
+    lib.pjz_fdtd_test_faults.argtypes = [ctypes.c_uint32]
     lib.pjz_fdtd_num_outputs.restype = ctypes.c_int
     lib.pjz_fdtd_num_outputs.argtypes = [P, ctypes.POINTER(ctypes.c_int32)]
     lib.pjz_fdtd_workspace_bytes.restype = ctypes.c_int

@@ -7,6 +7,7 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include <atomic>
 #include <map>
 #include <mutex>
 #include <tuple>
@@ -34,6 +35,59 @@ int hip_fail(hipError_t e, const char* where) {
 int count_outputs(const pjz_fdtd_problem& p) {
   if (p.out_stop <= p.out_start) return 0;
   return (p.out_stop - p.out_start + p.out_step - 1) / p.out_step;
+}
+
+// ------------------------------------------------- waits that ended in vain
+// Failure paths under test in the calling thread (PJZ_FDTD_TEST_*).
+thread_local unsigned g_test_faults = 0;
+
+constexpr int kMaxDevices = 64;
+
+// The current GPU's word in which device code reports that a wait ended in
+// vain (waits.h): pinned host memory, one allocation for all GPUs, kept until
+// the process ends.  Null if there is none, or none yet and `allocate` is
+// false.
+unsigned* report_word(bool allocate) {
+  static std::mutex mu;
+  static std::atomic<unsigned*> words{nullptr};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return nullptr;
+  unsigned* w = words.load(std::memory_order_acquire);
+  if (!w && allocate) {
+    std::lock_guard<std::mutex> lock(mu);
+    w = words.load(std::memory_order_acquire);
+    if (!w) {
+      // (Another thread may be recording a graph, which an allocation would
+      // end unless this thread is exempt.)
+      hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+      if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) return nullptr;
+      void* p = nullptr;
+      const hipError_t e =
+          hipHostMalloc(&p, sizeof(unsigned) * kMaxDevices,
+                        hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent);
+      (void)hipThreadExchangeStreamCaptureMode(&mode);
+      if (e != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+      }
+      memset(p, 0, sizeof(unsigned) * kMaxDevices);
+      w = (unsigned*)p;
+      words.store(w, std::memory_order_release);
+    }
+  }
+  return w ? w + dev : nullptr;
+}
+
+// The error of an earlier run on the current GPU that waited in vain, once.
+int stall_reported() {
+  unsigned* const w = report_word(false);
+  if (!w || __atomic_load_n(w, __ATOMIC_ACQUIRE) == 0 ||
+      __atomic_exchange_n(w, 0u, __ATOMIC_ACQ_REL) == 0)
+    return PJZ_FDTD_OK;
+  return fail(PJZ_FDTD_ESTALL,
+              "an earlier run on this GPU gave up waiting for its own workgroups and its results "
+              "are not valid: its workspace was shared with another call, or another process "
+              "holds the GPU (PJZ_FDTD_FLAG_STEPWISE avoids such waits)");
 }
 
 pjz::Geom geom_of(const pjz_fdtd_problem& p);
@@ -148,7 +202,6 @@ hipError_t run_steps(const pjz::Geom& g, const pjz_fdtd_problem& p, const float*
 // per device and kept in g_scratch_ptr.
 constexpr size_t kScratchBytes = PJZ_FDTD_NOALLOC_MAX_BYTES;
 __device__ __align__(256) unsigned char scratch[kScratchBytes];
-constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
 void* g_scratch_ptr[kMaxDevices] = {};
 
@@ -264,13 +317,13 @@ int auto_kernel(const pjz::Geom& g) {
 }
 
 // Compute units the resident stepper may take for a problem, or 0: another
-// kernel or tiling was asked for, or the run is a few steps (a resident run
-// costs about 0.1 ms once, the words and the state, and saves 10 us a step or
-// more).
+// kernel or tiling or step-by-step launches were asked for, or the run is a
+// few steps (a resident run costs about 0.1 ms once, the words and the state,
+// and saves 10 us a step or more).
 constexpr int kResidentMinSteps = 16;
 int resident_cus(const pjz_fdtd_problem& p) {
   if (p.kernel != PJZ_FDTD_KERNEL_AUTO || p.tile_x != 0 || p.tile_y != 0 || p.graph_steps != 0 ||
-      pjz::steps_of(p) < kResidentMinSteps)
+      (p.flags & PJZ_FDTD_FLAG_STEPWISE) || pjz::steps_of(p) < kResidentMinSteps)
     return 0;
   int dev = 0, cus = 0, coop = 0, lds = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
@@ -288,18 +341,29 @@ bool capturing(hipStream_t s) {
   return hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone;
 }
 
+// What a call's resident runs report to, for the workspace `ws`.
+pjz::WaitWords waits_in(const pjz_fdtd_problem& p, const pjz::Layout& L, char* ws) {
+  pjz::WaitWords w;
+  if (resident_cus(p) <= 0) return w;
+  w.stalled = (unsigned*)(ws + L.stalled);
+  w.report = report_word(true);
+  w.no_time = (g_test_faults & PJZ_FDTD_TEST_STALL) != 0;
+  return w;
+}
+
 // The resident stepper's tiling for a call, or rx = 0: as above, or the domain
 // is too large.
-pjz::ResPlan resident_for(const pjz::Geom& g, const pjz_fdtd_problem& p, hipStream_t s) {
-  const int cus = capturing(s) ? 0 : resident_cus(p);
+pjz::ResPlan resident_for(const pjz::Geom& g, const pjz_fdtd_problem& p, const pjz::Layout& L,
+                          hipStream_t s) {
+  const int cus = !L.waits.report || capturing(s) ? 0 : resident_cus(p);
   return cus > 0 ? pjz::resident_plan(g, p.src_axis, cus) : pjz::ResPlan{};
 }
 
 // Its slabs for a larger domain (n = 0: none); `capture`: for steps whose
 // changes of E are written.
-pjz::SlabPlan slabs_for(const pjz::Geom& g, const pjz_fdtd_problem& p, hipStream_t s,
-                        bool capture) {
-  const int cus = capturing(s) ? 0 : resident_cus(p);
+pjz::SlabPlan slabs_for(const pjz::Geom& g, const pjz_fdtd_problem& p, const pjz::Layout& L,
+                        hipStream_t s, bool capture) {
+  const int cus = !L.waits.report || capturing(s) ? 0 : resident_cus(p);
   if (cus <= 0) return {};
   const pjz::SlabPlan plan = pjz::slab_plan(g, p.src_axis, cus);
   return capture && !pjz::resident_captures(plan.tile) ? pjz::SlabPlan{} : plan;
@@ -312,11 +376,12 @@ size_t slab_bytes(const pjz::Geom& g, const pjz_fdtd_problem& p) {
   if (cus <= 0 || pjz::resident_plan(g, p.src_axis, cus).rx > 0) return 0;
   return pjz::slab_words(pjz::slab_plan(g, p.src_axis, cus)) * sizeof(pjz::rword_t);
 }
-// The layout of a call whose workspace has `bytes` bytes.
-pjz::Layout layout_in(const pjz::Geom& g, const pjz_fdtd_problem& p, size_t bytes) {
+// The layout of a call in a workspace `ws` of `bytes` bytes.
+pjz::Layout layout_in(const pjz::Geom& g, const pjz_fdtd_problem& p, void* ws, size_t bytes) {
   pjz::Layout L = pjz::make_layout(g, p);
   const size_t more = slab_bytes(g, p);
   if (more > 0 && bytes >= pjz::align256(L.total) + more) L.words = pjz::align256(L.total);
+  if (bytes >= L.total) L.waits = waits_in(p, L, (char*)ws);
   return L;
 }
 
@@ -341,7 +406,7 @@ hipError_t run_steps(const pjz::Geom& g, const pjz_fdtd_problem& p, const float*
   pjz::StepRange r{b, end, cur, capture};
   if (kernel == PJZ_FDTD_KERNEL_AUTO) {
     if (L.words > 0 && end - b >= kResidentMinSteps) {
-      const pjz::SlabPlan slabs = slabs_for(g, p, s, capture != nullptr);
+      const pjz::SlabPlan slabs = slabs_for(g, p, L, s, capture != nullptr);
       if (slabs.n > 0)
         return pjz::run_slabs(g, p, mask, src, win, ws, L, slabs, (pjz::rword_t*)(ws + L.words), r,
                               s);
@@ -420,7 +485,7 @@ hipError_t forward_steps(const pjz::Geom& g, const pjz_fdtd_problem& p, const fl
                          const pjz::Src& src, const pjz::OutWin& win, char* ws,
                          const pjz::Layout& L, hipStream_t s) {
   const int nsteps = pjz::steps_of(p);
-  const pjz::ResPlan plan = resident_for(g, p, s);
+  const pjz::ResPlan plan = resident_for(g, p, L, s);
   if (plan.rx > 0) {
     // The whole run in one launch, its checkpoints written on the way.
     hipError_t e = clear_words(plan, L, ws, s);
@@ -464,7 +529,7 @@ hipError_t backward_steps(const pjz::Geom& g, const pjz_fdtd_problem& p,
   auto is_out = [&](int n) {
     return n >= p.out_start && n < p.out_stop && (n - p.out_start) % p.out_step == 0;
   };
-  pjz::ResPlan plan = resident_for(g, p, s);
+  pjz::ResPlan plan = resident_for(g, p, L, s);
   if (!pjz::resident_captures(plan)) plan = {};
   const bool resident_adj = plan.rx > 0 && pjz::adjoint_resident_supported(plan);
   unsigned tags = 0;  // exchange numbers used
@@ -736,6 +801,10 @@ int pjz_fdtd_stepper(const pjz_fdtd_problem* p, int32_t* kernel) {
   return PJZ_FDTD_OK;
 }
 
+int pjz_fdtd_run_status(void) { return stall_reported(); }
+
+void pjz_fdtd_test_faults(uint32_t faults) { g_test_faults = faults; }
+
 int pjz_fdtd_num_outputs(const pjz_fdtd_problem* p, int32_t* nn) {
   int rc = check(p);
   if (rc) return rc;
@@ -767,16 +836,17 @@ int pjz_fdtd_forward(const pjz_fdtd_problem* p, const float* epsilon,
       !source_waveform || !out || !workspace)
     return fail(PJZ_FDTD_EINVAL, "a required pointer argument is NULL");
   pjz::Geom g = geom_of(*p);
-  pjz::Layout L = layout_in(g, *p, workspace_bytes);
+  pjz::Layout L = layout_in(g, *p, workspace, workspace_bytes);
   if (workspace_bytes < L.total)
     return fail(PJZ_FDTD_ESPACE, "workspace of %zu bytes, %zu needed", workspace_bytes, L.total);
   if (((uintptr_t)workspace & 255) != 0)
     return fail(PJZ_FDTD_EINVAL, "workspace must be 256-byte aligned");
+  if (const int bad = stall_reported()) return bad;
   hipStream_t s = (hipStream_t)stream;
   char* ws = (char*)workspace;
   // cb and the z table.
   hipError_t e = pjz::launch_prepare(g, *p, epsilon, absorption_mask, pml_kappa, pml_sigma,
-                                     pml_alpha, (float*)(ws + L.cb), (float*)(ws + L.zt), s);
+                                     pml_alpha, ws, L, s);
   if (e != hipSuccess) return hip_fail(e, "prepare");
   pjz::Src src{p->src_axis, p->src_pos, p->src_quad, source_field, source_waveform};
   pjz::OutWin win{p->x0, p->y0, p->z0, p->ex, p->ey, p->ez, out};
@@ -912,8 +982,7 @@ int batch_setup(const pjz_fdtd_problem* probs, int n, const BatchPlanHost& bp,
     char* ws = base + bp.offs[i];
     const pjz::Layout& L = bp.Ls[i];
     hipError_t e = pjz::launch_prepare(g, q, epsilon[i], absorption_mask[i], pml_kappa[i],
-                                       pml_sigma[i], pml_alpha[i], (float*)(ws + L.cb),
-                                       (float*)(ws + L.zt), s);
+                                       pml_sigma[i], pml_alpha[i], ws, L, s);
     if (adjoint) {
       // Clear both adjoint sets and G (contiguous from L.lE_[0] to the end).
       if (e == hipSuccess && L.total > L.lE_[0])
@@ -932,6 +1001,13 @@ int batch_setup(const pjz_fdtd_problem* probs, int n, const BatchPlanHost& bp,
   return PJZ_FDTD_OK;
 }
 
+// One word for the waits of all a batch's simulations (the first's): once one
+// has waited in vain, the others do not wait as long again.
+void batch_waits(const std::vector<pjz::BatchItem>& items, BatchPlanHost& bp) {
+  for (size_t i = 0; i < items.size(); ++i)
+    bp.Ls[i].waits = waits_in(*items[i].p, bp.Ls[0], items[0].ws);
+}
+
 // The simulations of a batch that run by themselves, one after the other, on
 // the resident stepper; the others share the batched launches.  A resident
 // step takes about 2.5 us and 0.3 us for every cell a lane, twice that where
@@ -947,7 +1023,7 @@ std::vector<bool> batch_alone(const std::vector<pjz::BatchItem>& items, bool cap
   bool fit = true;
   auto share_us = [](const pjz::BatchItem& it) { return (double)it.g.N / 90e3; };
   for (size_t i = 0; i < n; ++i) {
-    const pjz::ResPlan p = resident_for(items[i].g, *items[i].p, s);
+    const pjz::ResPlan p = resident_for(items[i].g, *items[i].p, *items[i].L, s);
     const int c = p.cpl * p.rx * p.ry;
     if (p.rx > 0) us[i] = 2.5 + (c <= 16 ? 0.3 : 0.6) * c;
     else fit = false;
@@ -958,7 +1034,7 @@ std::vector<bool> batch_alone(const std::vector<pjz::BatchItem>& items, bool cap
   for (size_t i = 0; i < n; ++i) {
     if (us[i] > 0) alone[i] = all || us[i] <= share_us(items[i]);
     else if (items[i].L->words > 0)
-      alone[i] = slabs_for(items[i].g, *items[i].p, s, capture).n > 0;
+      alone[i] = slabs_for(items[i].g, *items[i].p, *items[i].L, s, capture).n > 0;
   }
   return alone;
 }
@@ -985,12 +1061,14 @@ int pjz_fdtd_batch_forward(const pjz_fdtd_problem* probs, int n, const float* co
   BatchPlanHost bp;
   int rc = batch_plan(probs, n, bp);
   if (rc) return rc;
+  if (const int bad = stall_reported()) return bad;
   hipStream_t s = (hipStream_t)stream;
   std::vector<pjz::BatchItem> items;
   rc = batch_setup(probs, n, bp, epsilon, absorption_mask, pml_kappa, pml_sigma, pml_alpha,
                    source_field, source_waveform, out, workspace, workspace_bytes, false, s, items);
   if (rc) return rc;
   char* base = (char*)workspace;
+  batch_waits(items, bp);
   const std::vector<bool> alone = batch_alone(items, false, s);
   std::vector<pjz::BatchItem> rest;  // of the batched launches
   hipError_t e = hipSuccess;
@@ -1038,6 +1116,7 @@ int pjz_fdtd_batch_backward(const pjz_fdtd_problem* probs, int n, const float* c
   for (int i = 0; i < n; ++i)
     if (!grad_out[i] || !grad_eps[i])
       return fail(PJZ_FDTD_EINVAL, "batch item %d: a required pointer is NULL", i);
+  if (const int bad = stall_reported()) return bad;
   hipStream_t s = (hipStream_t)stream;
   std::vector<pjz::BatchItem> items;
   rc = batch_setup(probs, n, bp, epsilon, absorption_mask, pml_kappa, pml_sigma, pml_alpha,
@@ -1045,6 +1124,7 @@ int pjz_fdtd_batch_backward(const pjz_fdtd_problem* probs, int n, const float* c
                    items);
   if (rc) return rc;
   char* base = (char*)workspace;
+  batch_waits(items, bp);
   const std::vector<bool> alone = batch_alone(items, true, s);
   std::vector<pjz::BatchItem> rest;  // of the batched launches, their cotangents
   std::vector<const float*> gout;
@@ -1164,11 +1244,12 @@ int pjz_fdtd_backward(const pjz_fdtd_problem* p, const float* epsilon,
       !source_waveform || !grad_out || !grad_eps || !workspace)
     return fail(PJZ_FDTD_EINVAL, "a required pointer argument is NULL");
   pjz::Geom g = geom_of(*p);
-  pjz::Layout L = layout_in(g, *p, workspace_bytes);
+  pjz::Layout L = layout_in(g, *p, workspace, workspace_bytes);
   if (workspace_bytes < L.total)
     return fail(PJZ_FDTD_ESPACE, "workspace of %zu bytes, %zu needed", workspace_bytes, L.total);
   if (((uintptr_t)workspace & 255) != 0)
     return fail(PJZ_FDTD_EINVAL, "workspace must be 256-byte aligned");
+  if (const int bad = stall_reported()) return bad;
   hipStream_t s = (hipStream_t)stream;
   char* ws = (char*)workspace;
   hipError_t e = hipSuccess;
@@ -1176,8 +1257,8 @@ int pjz_fdtd_backward(const pjz_fdtd_problem* p, const float* epsilon,
     e = pjz::launch_zero(grad_eps, 3 * (size_t)p->ex * p->ey * p->ez, s);
     return e == hipSuccess ? PJZ_FDTD_OK : hip_fail(e, "zero grad");
   }
-  e = pjz::launch_prepare(g, *p, epsilon, absorption_mask, pml_kappa, pml_sigma, pml_alpha,
-                          (float*)(ws + L.cb), (float*)(ws + L.zt), s);
+  e = pjz::launch_prepare(g, *p, epsilon, absorption_mask, pml_kappa, pml_sigma, pml_alpha, ws, L,
+                          s);
   // Clear both adjoint sets and G (contiguous from L.lE_[0] to the end).
   if (e == hipSuccess)
     e = pjz::launch_zero((float*)(ws + L.lE_[0]), (L.total - L.lE_[0]) / 4, s);

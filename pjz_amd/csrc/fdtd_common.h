@@ -44,9 +44,17 @@ struct OutWin {
 };
 
 // Byte offsets of the workspace segments (each 256-byte aligned).
+// Where a call's resident runs say that they waited in vain (waits.h).
+struct WaitWords {
+  unsigned* stalled = nullptr;  // in the workspace, cleared by launch_prepare
+  unsigned* report = nullptr;   // host memory; null: no resident runs
+  bool no_time = false;         // waits in vain end at once (tests)
+};
+
 struct Layout {
   size_t E0, H0, E1, H1, cb, psi, zt;
   size_t rare;        // 256 B of per-call launch data for the two-step kernel
+  size_t stalled;     // its last word (WaitWords)
   // Gradient support (only when ckpt_every > 0):
   size_t ckpt;        // nck checkpoints of ckpt_floats each
   size_t seg;         // (S + 1) x 3N: E^n - E^(n+1) of every step of a segment (+1 spare)
@@ -64,6 +72,7 @@ struct Layout {
   int S1, nfine;
   // Exchange words of a run in slabs, past `total`; 0: the workspace has none.
   size_t words = 0;
+  WaitWords waits;  // of the call's resident runs
   size_t ckpt_floats;  // E (3N) + H (3N) + psi_H pair (2P) + psi_E pair (2P)
 };
 
@@ -91,6 +100,7 @@ inline Layout make_layout(const Geom& g, const pjz_fdtd_problem& p) {
   off += align256(sizeof(float) * PSI_N * P);
   L.zt = off; off += align256(sizeof(float) * ZROWS * (size_t)g.Z);
   L.rare = off; off += 256;
+  L.stalled = L.rare + 248;
   L.S = 0;
   L.nck = 0;
   L.S1 = 0;
@@ -140,7 +150,7 @@ struct StepRange {
 // Launchers implemented in the kernel translation units.
 hipError_t launch_prepare(const Geom& g, const pjz_fdtd_problem& p, const float* eps,
                           const float* mask, const float* kappa, const float* sigma,
-                          const float* alpha, float* cb, float* zt, hipStream_t s);
+                          const float* alpha, char* ws, const Layout& L, hipStream_t s);
 
 // Clears n floats with a fill kernel (no hipMemsetAsync, so the call can sit
 // inside a captured graph).

@@ -113,7 +113,7 @@ k_adj_resident(AdjResArgs a) {
     }
   };
 
-  T.fill(a.lu, a.lp, P, a.mask);
+  T.fill(a.lu, a.lp, P, a.mask, a.t.waits);
   __builtin_amdgcn_sched_barrier(0);
   float le[RX][RY][3][CPL], lk[RX][RY][3][CPL], lh[RX][RY][3][CPL];
   float cbr[CBR ? RX : 1][CBR ? RY : 1][3][CPL], gr[GR ? RX : 1][GR ? RY : 1][3][CPL];
@@ -364,6 +364,11 @@ k_adj_resident(AdjResArgs a) {
         if constexpr (GR) T.store(a.G, gr[GR ? i : 0][GR ? r : 0], N, i, r);
       }
   T.store_psi(a.lu, a.lp, P);
+  if (T.late()) {
+    // A wait in vain: the wave's first column of the gradient is spoiled.
+    if (T.valid(0, 0) && zb < Z) to_global(a.G)[T.offset(0, 0) + zb] = __builtin_nanf("");
+    tell_late(a.t.waits);
+  }
 }
 
 // ------------------------------------------------------------------ host side
@@ -380,8 +385,8 @@ static hipError_t launch_adj_resident(AdjResArgs& a, const ResPlan& p, hipStream
   hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)p.lds);
   if (e != hipSuccess) return e;
   void* args[] = {&a};
-  return hipLaunchCooperativeKernel(k, dim3(p.tiles()), dim3(kResThreads), args, (unsigned)p.lds,
-                                    s);
+  return hipLaunchCooperativeKernel(k, dim3(launched_tiles(a.t)), dim3(kResThreads), args,
+                                    (unsigned)p.lds, s);
 }
 
 bool adjoint_resident_supported(const ResPlan& p) {
@@ -406,7 +411,7 @@ hipError_t run_adjoint_resident(const Geom& g, const pjz_fdtd_problem& p, const 
   a.zt = (const float*)(ws + L.zt);
   a.mask = mask;
   a.gout = gout;
-  a.t = tile_args(g, plan, (rword_t*)(ws + L.E1));
+  a.t = tile_args(g, plan, (rword_t*)(ws + L.E1), wait_args(L.waits, end - begin));
   a.dt = p.dt;
   a.begin = begin;
   a.end = end;

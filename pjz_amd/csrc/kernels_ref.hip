@@ -29,11 +29,12 @@ __global__ void k_prepare_cb(const float* __restrict__ eps, const float* __restr
   cb[idx] = (float)((dt / e) / (1.0 + q));
 }
 
-// Per-z CPML table from the (zz, 2) kappa/sigma/alpha arrays.
+// Per-z CPML table from the (zz, 2) kappa/sigma/alpha arrays; clears `stalled`.
 __global__ void k_prepare_zt(const float* __restrict__ kappa, const float* __restrict__ sigma,
-                             const float* __restrict__ alpha, float* __restrict__ zt, int Z,
-                             double dt) {
+                             const float* __restrict__ alpha, float* __restrict__ zt,
+                             unsigned* __restrict__ stalled, int Z, double dt) {
   int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k == 0) *stalled = 0;
   if (k >= Z) return;
   for (int col = 0; col < 2; ++col) {
     double kap = kappa[2 * k + col], sig = sigma[2 * k + col], alp = alpha[2 * k + col];
@@ -61,11 +62,11 @@ static inline unsigned blocks_for(long long n, int bs) {
 
 hipError_t launch_prepare(const Geom& g, const pjz_fdtd_problem& p, const float* eps,
                           const float* mask, const float* kappa, const float* sigma,
-                          const float* alpha, float* cb, float* zt, hipStream_t s) {
+                          const float* alpha, char* ws, const Layout& L, hipStream_t s) {
   hipLaunchKernelGGL(k_prepare_cb, dim3(blocks_for(3 * g.N, 256)), dim3(256), 0, s, eps, mask,
-                     cb, g, p.x0, p.y0, p.z0, p.ex, p.ey, p.ez, (double)p.dt);
+                     (float*)(ws + L.cb), g, p.x0, p.y0, p.z0, p.ex, p.ey, p.ez, (double)p.dt);
   hipLaunchKernelGGL(k_prepare_zt, dim3(blocks_for(g.Z, 64)), dim3(64), 0, s, kappa, sigma,
-                     alpha, zt, g.Z, (double)p.dt);
+                     alpha, (float*)(ws + L.zt), (unsigned*)(ws + L.stalled), g.Z, (double)p.dt);
   return hipGetLastError();
 }
 

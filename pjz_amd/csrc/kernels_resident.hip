@@ -19,9 +19,10 @@
 // latencies (about 1 us each).  A word is rewritten only after its reader
 // has posted the answer that the writer waits for (E of step n + 1 at an edge
 // needs H of step n + 1 there, which the neighbour posts after it read E of
-// step n), so one set of words is enough.  Every workgroup is resident
-// (cooperative launch) and posts before it waits for the answer, so every
-// wait ends.
+// step n), so one set of words is enough.  All workgroups are on the chip at
+// the same time (cooperative launch, one a compute unit) and post before they
+// wait for the answer, so every wait ends; where that does not hold, by the
+// clock (waits.h).
 //
 // Measured, us a step, two-step kernel (the default before) against this:
 // 64^3 13.4 -> 2.9 (both exchange latencies), 128x128x64 14.3 -> 5.2,
@@ -62,6 +63,12 @@ struct ResArgs {
   int begin, end;
   unsigned tag0;     // exchange numbers tag0 + 1 .. tag0 + 2 (end - begin) + 1
   int wx0, wy0, wz0, wex, wey, wez, ostart, ostop, ostep;
+  __device__ __forceinline__ void split() {
+    apart(Ein, Hin, psiin, Eout, Hout, psiout, cb, zt, mask, sfield, swave, out, cap, ckpt,
+          ckpt_stride, every, saxis, spos, squad, dt, begin, end, tag0, wx0, wy0, wz0, wex, wey,
+          wez, ostart, ostop, ostep);
+    t.split();
+  }
 };
 
 // Registers: 6 a cell for E and H, 3 more for cb where that still fits; past
@@ -73,6 +80,7 @@ constexpr bool res_keeps_cb() { return CPL * RX * RY <= 16; }
 template <int CPL, int RX, int RY, bool CAP>
 __global__ __launch_bounds__(kResThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 k_resident(ResArgs a) {
+  a.split();
   using Tile = ResTile<CPL, RX, RY>;
   using Order = ColOrder<RX, RY>;
   constexpr int C = Tile::C, ED = Tile::ED;
@@ -105,7 +113,7 @@ k_resident(ResArgs a) {
     pE[c] = 4 * (pml[c] ? NP * 2 + pidx * 2 : NP * 4);
   }
 
-  T.fill(a.psiin, a.psiin ? a.psiin + 2 * (size_t)P : nullptr, P, a.mask);
+  T.fill(a.psiin, a.psiin ? a.psiin + 2 * (size_t)P : nullptr, P, a.mask, a.t.waits);
   __builtin_amdgcn_sched_barrier(0);
   float e[RX][RY][3][CPL], h[RX][RY][3][CPL], cbr[CBR ? RX : 1][CBR ? RY : 1][3][CPL];
 #pragma unroll
@@ -450,6 +458,22 @@ k_resident(ResArgs a) {
     }
   }
   if (a.Eout) store_state(a.Eout, a.Hout, a.psiout);
+  if (T.late()) {
+    // A wait in vain: the wave's first column of what it wrote is spoiled.
+    const float nan = __builtin_nanf("");
+    if (T.owned(0, 0) && zb < Z) {
+      const int o = T.offset(0, 0) + zb;
+      if (a.Eout) to_global(a.Eout)[o] = nan;
+      if (CAP) to_global(a.cap)[o] = nan;
+      const int x = T.colx(0) - a.wx0, y = T.coly(0) - a.wy0, z = zb - a.wz0;
+      if (a.out && x >= 0 && x < a.wex && y >= 0 && y < a.wey && z >= 0 && z < a.wez)
+        for (int n = max(a.begin, a.ostart); n < min(a.end, a.ostop); ++n)
+          if ((n - a.ostart) % a.ostep == 0)
+            to_global(a.out)[((((long long)((n - a.ostart) / a.ostep) * 3) * a.wex + x) * a.wey +
+                              y) * (long long)a.wez + z] = nan;
+    }
+    tell_late(a.t.waits);
+  }
 }
 
 // ------------------------------------------------------------------ host side
@@ -598,8 +622,8 @@ static hipError_t launch_resident(ResArgs& a, const ResPlan& p, hipStream_t s) {
   hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)p.lds);
   if (e != hipSuccess) return e;
   void* args[] = {&a};
-  return hipLaunchCooperativeKernel(k, dim3(p.tiles()), dim3(kResThreads), args, (unsigned)p.lds,
-                                    s);
+  return hipLaunchCooperativeKernel(k, dim3(launched_tiles(a.t)), dim3(kResThreads), args,
+                                    (unsigned)p.lds, s);
 }
 
 hipError_t run_resident(const Geom& g, const pjz_fdtd_problem& p, const float* mask,
@@ -622,7 +646,8 @@ hipError_t run_resident(const Geom& g, const pjz_fdtd_problem& p, const float* m
   a.ckpt = r.ckpt;
   a.ckpt_stride = (long long)(ckpt_stride(L) / sizeof(float));
   a.every = r.every;
-  a.t = tile_args(g, plan, r.words ? r.words : (rword_t*)(ws + L.E1));
+  a.t = tile_args(g, plan, r.words ? r.words : (rword_t*)(ws + L.E1),
+                  wait_args(L.waits, r.end - r.begin));
   if (r.xe > 0) {
     a.t.xs = r.xs;
     a.t.xe = r.xe;

@@ -3,10 +3,12 @@
 // compute units and the exchange of edge columns between workgroups.
 #pragma once
 
+#include <algorithm>
 #include <type_traits>
 #include <utility>
 
 #include "stream_common.h"
+#include "waits.h"
 
 namespace pjz {
 
@@ -27,6 +29,30 @@ __device__ __forceinline__ int opaque_s(int v) {
   v = __builtin_amdgcn_readfirstlane(v);
   asm volatile("" : "+s"(v));
   return v;
+}
+// A kernel argument in registers of its own.  Arguments arrive in groups of up
+// to 16 registers; where such a group is spilled, each use of one of its values
+// reloads all of it (k_resident<2,5,3>: 7200 reloaded registers, apart 700;
+// 220x200x96 in slabs, 800 steps: 29.8 -> 26.8 ms).
+template <class T>
+__device__ __forceinline__ void apart(T& v) {
+  if constexpr (std::is_pointer_v<T>) {
+    unsigned long long w;
+    asm volatile("s_mov_b64 %0, %1" : "=s"(w) : "s"(v));
+    // (The compiler knows that an argument points to global memory; of the
+    // copy it is told.)
+    v = (T)(__attribute__((address_space(1))) std::remove_pointer_t<T>*)w;
+  } else {
+    T w;
+    if constexpr (sizeof(T) == 8) asm volatile("s_mov_b64 %0, %1" : "=s"(w) : "s"(v));
+    else asm volatile("s_mov_b32 %0, %1" : "=s"(w) : "s"(v));
+    v = w;
+  }
+}
+template <class T, class... Ts>
+__device__ __forceinline__ void apart(T& v, Ts&... vs) {
+  apart(v);
+  apart(vs...);
 }
 // Pins a result where it is computed: the compiler would otherwise move the
 // updates of all columns past the next branch, with their inputs live.
@@ -58,26 +84,6 @@ __device__ __forceinline__ void post_edge(rword_t* p, unsigned tag, float v) {
   pin(v);
   __hip_atomic_store(p, ((rword_t)tag << 32) | __float_as_uint(v), __ATOMIC_RELAXED,
                      __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// The words p[0], p[64], .. p[64 (NW - 1)] once all carry `tag`.  Every
-// workgroup of the launch is resident at some time (cooperative launch) and
-// posts before it waits for the answer, so the wait ends; it is not bounded,
-// as other streams' kernels may hold back some of the workgroups for long.
-template <int NW>
-__device__ __forceinline__ void wait_edges(float (&v)[NW], const rword_t* p, unsigned tag) {
-  rword_t w[NW];
-  bool ok;
-  do {
-    ok = true;
-#pragma unroll
-    for (int k = 0; k < NW; ++k)
-      w[k] = __hip_atomic_load(p + 64 * k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-#pragma unroll
-    for (int k = 0; k < NW; ++k) ok &= (unsigned)(w[k] >> 32) == tag;
-  } while (!__all(ok));
-#pragma unroll
-  for (int k = 0; k < NW; ++k) v[k] = __uint_as_float((unsigned)w[k]);
 }
 
 template <int CPL>
@@ -140,19 +146,32 @@ struct ResTileArgs {
   int xs, xe, own0, own1;
   int wx, wy, ntx, nty, alias;
   rword_t* words;
+  WaitArgs waits;
+  __device__ __forceinline__ void split() {
+    apart(X, Y, Z, N, P, lo, hi, NP, xs, xe, own0, own1, wx, wy, ntx, nty, alias, words,
+          waits.ticks, waits.stalled, waits.report);
+  }
 };
 
 template <int CPL, int RX, int RY>
 struct ResTile {
   static constexpr int C = RX * RY;
   static constexpr int ED = 2 * 64 * CPL;  // floats (or words) of an edge column
+  // Whether the tile, and in its tile the wave, has a neighbour on a side.  Bits
+  // of one register, tested where they are used: as booleans they took a pair of
+  // scalar registers each, and what that spilled was reloaded lane by lane.
+  enum Place {
+    TILE_XLO = 1, TILE_XHI = 2, TILE_YLO = 4, TILE_YHI = 8,
+    WAVE_XLO = 16, WAVE_XHI = 32, WAVE_YLO = 64, WAVE_YHI = 128,
+    ALIAS = 256  // one set of edge buffers
+  };
+  __device__ __forceinline__ bool is(int p) const { return (opaque_s(place) & p) != 0; }
   int lane, w, wx, wy, WX, WY, TX, TY, bx, by, xs, xe, own0, own1, x0, y0, zb, X, Y, Z, NP, PS;
   float* lds;
   int er, hr, sx, sy;  // see edges()
   rword_t* mine;
   int ox, oy, oh, fx, fy;
-  bool bxlo, bxhi, bylo, byhi, xlo, xhi, ylo, yhi;
-  bool alias;
+  int place;  // bits of Place
 
   __device__ __forceinline__ ResTile(const ResTileArgs& a, float* lds_) {
     lane = threadIdx.x & 63;
@@ -185,7 +204,6 @@ struct ResTile {
     zb = lane * CPL;
     lds = lds_;
     PS = NP * 4 + 2;
-    alias = a.alias;
     // A tile's words: low x edge (TY columns), low y (TX), high x, high y.
     // Of the neighbours' (as offsets from this tile's): the low edges from +x
     // and +y, the high ones from -x and -y.
@@ -196,21 +214,22 @@ struct ResTile {
     oh = (TX + TY) * ED;
     fx = (int)(a.nty * tw);
     fy = (int)tw;
-    bxlo = bx > 0;
-    bxhi = bx + 1 < a.ntx;
-    bylo = by > 0;
-    byhi = by + 1 < a.nty;
-    xlo = wx == 0 && bxlo;
-    xhi = wx == WX - 1 && bxhi;
-    ylo = wy == 0 && bylo;
-    yhi = wy == WY - 1 && byhi;
+    place = __builtin_amdgcn_readfirstlane(
+            (bx > 0 ? TILE_XLO : 0) | (bx + 1 < a.ntx ? TILE_XHI : 0) |
+            (by > 0 ? TILE_YLO : 0) | (by + 1 < a.nty ? TILE_YHI : 0) |
+            (wx > 0 ? WAVE_XLO : 0) | (wx < WX - 1 ? WAVE_XHI : 0) |
+            (wy > 0 ? WAVE_YLO : 0) | (wy < WY - 1 ? WAVE_YHI : 0) | (a.alias ? ALIAS : 0));
   }
 
   // LDS: psi as (column, pair, PML cell, 2) and, per column, a zero pair for
   // the lanes outside the PML (so every lane's address steps alike); absorber
-  // values; `more` floats of the kernel's own; edge buffers.
+  // values and in their fourth place, for the wave's first column, the end of
+  // its waits; `more` floats of the kernel's own; edge buffers.
   __device__ __forceinline__ f32x4* sig() const {
     return reinterpret_cast<f32x4*>(lds + ((TX * TY * PS + 3) & ~3));
+  }
+  __device__ __forceinline__ unsigned* waits() const {
+    return reinterpret_cast<unsigned*>(lds + opaque_s(((TX * TY * PS + 3) & ~3) + w * C * 4 + 3));
   }
   __device__ __forceinline__ float* own() const {
     return reinterpret_cast<float*>(sig() + TX * TY);
@@ -222,7 +241,7 @@ struct ResTile {
   // uniform: the lane's address is made where it is used.)
   __device__ __forceinline__ void edges(int more) {
     const int eoff = (int)(own() - lds) + more;
-    const int hoff = eoff + (alias ? 0 : (WX * TY + WY * TX) * ED);
+    const int hoff = eoff + (is(ALIAS) ? 0 : (WX * TY + WY * TX) * ED);
     sx = (wx * TY + wy * RY) * ED;
     sy = (WX * TY + wy * TX + wx * RX) * ED;
     er = eoff;
@@ -282,7 +301,7 @@ struct ResTile {
   // absorber to LDS.  All of a wave's columns are requested at once: entry by
   // entry over the tile, the loads' latencies added up to 40 us a launch.
   __device__ __forceinline__ void fill(const float* psi0, const float* psi1, int P,
-                                       const float* mask) const {
+                                       const float* mask, const WaitArgs& wa) const {
     for (int j = 0; 64 * j < NP * 4; ++j) {
       const int m = min(lane + 64 * j, NP * 4 - 1);
       bool second;
@@ -302,12 +321,13 @@ struct ResTile {
       });
     }
     if (lane < 2 * C) lds[(w * C + (lane >> 1)) * PS + NP * 4 + (lane & 1)] = 0.0f;
+    const float end = __uint_as_float(wait_end(wa));
     for (int t = threadIdx.x; t < TX * TY; t += kResThreads) {
       const int x = tile_x(t), y = tile_y(t);
-      f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};
+      f32x4 s = {0.0f, 0.0f, 0.0f, end};
       if (x < xe && y < Y) {
         const int m = x * Y + y, XY = X * Y;
-        s = f32x4{mask[m], mask[XY + m], mask[2 * XY + m], 0.0f};
+        s = f32x4{mask[m], mask[XY + m], mask[2 * XY + m], end};
       }
       sig()[t] = s;
     }
@@ -352,51 +372,89 @@ struct ResTile {
   // Passes the wave's edges on: through LDS within the workgroup, as words to
   // its neighbours.
   __device__ __forceinline__ void pass_low(unsigned tag, const float (&e)[RX][RY][3][CPL]) const {
-    if (wx > 0) {
+    if (is(WAVE_XLO)) {
 #pragma unroll
       for (int r = 0; r < RY; ++r) put_edge(slot(er + sx - TY * ED), r, e[0][r][1], e[0][r][2]);
-    } else if (xlo) {
+    } else if (is(TILE_XLO)) {
 #pragma unroll
       for (int r = 0; r < RY; ++r) post(ox + r * ED, tag, e[0][r][1], e[0][r][2]);
     }
-    if (wy > 0) {
+    if (is(WAVE_YLO)) {
 #pragma unroll
       for (int i = 0; i < RX; ++i) put_edge(slot(er + sy - TX * ED), i, e[i][0][0], e[i][0][2]);
-    } else if (ylo) {
+    } else if (is(TILE_YLO)) {
 #pragma unroll
       for (int i = 0; i < RX; ++i) post(oy + i * ED, tag, e[i][0][0], e[i][0][2]);
     }
   }
   __device__ __forceinline__ void pass_high(unsigned tag, const float (&h)[RX][RY][3][CPL]) const {
-    if (wx < WX - 1) {
+    if (is(WAVE_XHI)) {
 #pragma unroll
       for (int r = 0; r < RY; ++r)
         put_edge(slot(hr + sx + TY * ED), r, h[RX - 1][r][1], h[RX - 1][r][2]);
-    } else if (xhi) {
+    } else if (is(TILE_XHI)) {
 #pragma unroll
       for (int r = 0; r < RY; ++r)
         post(oh + ox + r * ED, tag, h[RX - 1][r][1], h[RX - 1][r][2]);
     }
-    if (wy < WY - 1) {
+    if (is(WAVE_YHI)) {
 #pragma unroll
       for (int i = 0; i < RX; ++i)
         put_edge(slot(hr + sy + TX * ED), i, h[i][RY - 1][0], h[i][RY - 1][2]);
-    } else if (yhi) {
+    } else if (is(TILE_YHI)) {
 #pragma unroll
       for (int i = 0; i < RX; ++i)
         post(oh + oy + i * ED, tag, h[i][RY - 1][0], h[i][RY - 1][2]);
     }
   }
-  // The words p[0], p[64], .. of K columns once they carry `tag`; columns with
-  // no such neighbour are zeros.
+  __device__ __forceinline__ bool late() const {
+    return __builtin_amdgcn_readfirstlane(*waits()) == (int)kLate;
+  }
+  // Polls until load() returns 0 (the lanes whose words have not come) or the
+  // wave's waits end.  The first polls are a loop of their own with one exit,
+  // whose count is kept while the loads are on their way: with the clock in the
+  // same loop, what follows the last load cost 0.1 us an exchange (64^3: 2.85 us
+  // a step instead of 2.62).
+  template <class F>
+  __device__ __forceinline__ void poll(F&& load) const {
+    int left = kWaitPolls;
+    unsigned long long missing;
+    do {
+      --left;
+      const unsigned more = ~opaque_s(left >> 31);  // all ones, or 0 at the last
+      missing = load() & ((unsigned long long)more << 32 | more);
+    } while (missing != 0);
+    if (__builtin_expect(left < 0, 0)) {
+      while (load() != 0)
+        if (wait_over(waits())) break;
+    }
+  }
+  // The words p[0], p[64], .. p[64 (NW - 1)] once all carry `tag`, or what is
+  // there when the wave's waits end.
+  template <int NW>
+  __device__ __forceinline__ void wait_edges(float (&v)[NW], const rword_t* p,
+                                             unsigned tag) const {
+    rword_t w[NW];
+    poll([&]() __attribute__((always_inline)) {
+      unsigned other = 0;
+#pragma unroll
+      for (int k = 0; k < NW; ++k)
+        w[k] = __hip_atomic_load(p + 64 * k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+      for (int k = 0; k < NW; ++k) other |= (unsigned)(w[k] >> 32) ^ tag;
+      return __ballot(other != 0);
+    });
+#pragma unroll
+    for (int k = 0; k < NW; ++k) v[k] = __uint_as_float((unsigned)w[k]);
+  }
+  // The same for K columns; columns with no such neighbour are zeros.
   template <int K>
   __device__ __forceinline__ void wait(const int (&at)[K], const int (&dst)[K],
                                        const bool (&there)[K], unsigned tag) const {
     constexpr int NW = 2 * CPL;
     rword_t v[K * NW];
-    bool ok;
-    do {
-      ok = true;
+    poll([&]() __attribute__((always_inline)) {
+      unsigned other = 0;
 #pragma unroll
       for (int k = 0; k < K; ++k) {
         const rword_t* const p = edge_word(mine, there[k] ? at[k] : 0, lane);
@@ -409,8 +467,9 @@ struct ResTile {
       for (int k = 0; k < K; ++k)
 #pragma unroll
         for (int c = 0; c < NW; ++c)
-          ok &= (unsigned)(v[k * NW + c] >> 32) == tag || !there[k];
-    } while (!__all(ok));
+          other |= there[k] ? (unsigned)(v[k * NW + c] >> 32) ^ tag : 0;
+      return __ballot(other != 0);
+    });
 #pragma unroll
     for (int k = 0; k < K; ++k)
 #pragma unroll
@@ -483,32 +542,48 @@ struct ResTile {
   __device__ __forceinline__ void take_low(unsigned tag) const {
     if constexpr (kShared) {
       take_shared(er + (WX - 1) * TY * ED, er + (WX * TY + (WY - 1) * TX) * ED, fx, fy + TY * ED,
-                  bxhi, byhi, tag);
+                  is(TILE_XHI), is(TILE_YHI), tag);
       lds_barrier();
     } else {
       lds_barrier();
-      if (wx == WX - 1) take_own<RY>(low_x(), fx + ox, bxhi, tag);
-      if (wy == WY - 1) take_own<RX>(low_y(), fy + oy, byhi, tag);
+      if (!is(WAVE_XHI)) take_own<RY>(low_x(), fx + ox, is(TILE_XHI), tag);
+      if (!is(WAVE_YHI)) take_own<RX>(low_y(), fy + oy, is(TILE_YHI), tag);
     }
   }
   __device__ __forceinline__ void take_high(unsigned tag) const {
     if constexpr (kShared) {
-      take_shared(hr, hr + WX * TY * ED, oh - fx, oh - fy + TY * ED, bxlo, bylo, tag);
+      take_shared(hr, hr + WX * TY * ED, oh - fx, oh - fy + TY * ED, is(TILE_XLO),
+                  is(TILE_YLO), tag);
       lds_barrier();
     } else {
       lds_barrier();
-      if (wx == 0) take_own<RY>(high_x(), oh + ox - fx, bxlo, tag);
-      if (wy == 0) take_own<RX>(high_y(), oh + oy - fy, bylo, tag);
+      if (!is(WAVE_XLO)) take_own<RY>(high_x(), oh + ox - fx, is(TILE_XLO), tag);
+      if (!is(WAVE_YLO)) take_own<RX>(high_y(), oh + oy - fy, is(TILE_YLO), tag);
     }
   }
   // With one set of edge buffers: before it is written again.
   __device__ __forceinline__ void edges_read() const {
-    if (alias) lds_barrier();
+    if (is(ALIAS)) lds_barrier();
   }
 };
 
-inline ResTileArgs tile_args(const Geom& g, const ResPlan& p, rword_t* words) {
+// The waits of a launch of `steps` steps (at most about 20 us each): 20 s, far
+// more than other streams' kernels hold a workgroup back, and 1 ms a step.
+inline WaitArgs wait_args(const WaitWords& w, int steps) {
+  const double ms = w.no_time ? 0.0 : 20e3 + steps;
+  return {(unsigned)std::min(ms * (100e3 / kWaitTick), 1e9), w.stalled, w.report};
+}
+
+// Workgroups to launch: without the last, a run whose waits have no time (tests)
+// waits for words that nobody posts.
+inline unsigned launched_tiles(const ResTileArgs& a) {
+  const int n = a.ntx * a.nty;
+  return a.waits.ticks == 0 && n > 1 ? n - 1 : n;
+}
+
+inline ResTileArgs tile_args(const Geom& g, const ResPlan& p, rword_t* words, const WaitArgs& w) {
   ResTileArgs a;
+  a.waits = w;
   a.xs = a.own0 = 0;
   a.xe = a.own1 = g.X;
   a.X = g.X; a.Y = g.Y; a.Z = g.Z; a.lo = g.lo; a.hi = g.hi; a.NP = g.NP;

@@ -24,7 +24,7 @@ _KERNELS = {"auto": _lib.KERNEL_AUTO, "reference": _lib.KERNEL_REFERENCE,
             "stream3": _lib.KERNEL_STREAM3, "stream4": _lib.KERNEL_STREAM4,
             "autotune": _lib.KERNEL_AUTOTUNE}
 _LAUNCH_KEYS = {"kernel", "tile_x", "tile_y", "waves_per_simd", "ckpt_every", "ckpt_inner",
-                "memory_budget", "graph_steps"}
+                "memory_budget", "graph_steps", "resident"}
 
 
 def _launch_options(launch_params):
@@ -42,7 +42,10 @@ def _launch_options(launch_params):
   workspace may take; default 90% of the device's free memory.  Without an
   explicit ``ckpt_every``, checkpoints go to two levels when one does not
   fit), ``graph_steps`` (batches: steps per captured and replayed hipGraph
-  chunk, even, <= 128; 0, the default, launches every step pair directly).
+  chunk, even, <= 128; 0, the default, launches every step pair directly),
+  ``resident`` (default True: "auto" runs domains that fit the GPU's registers
+  in launches whose workgroups wait for one another; False, for a GPU that
+  other processes use as well: only kernels that are launched step by step).
   """
   if launch_params is None:
     return {}
@@ -115,7 +118,9 @@ def make_problem(epsilon_shape, dt, source_shape, source_position, mask_shape,
   p.tt = int(tt)
   p.out_start, p.out_stop, p.out_step = (int(v) for v in output_steps)
   p.dt = float(dt)
-  p.flags = 1 if use_reduced_precision else 0
+  p.flags = _lib.FLAG_REDUCED if use_reduced_precision else 0
+  if not opts.get("resident", True):
+    p.flags |= _lib.FLAG_STEPWISE
   p.kernel = _KERNELS[opts.get("kernel", "auto")]
   p.tile_x = int(opts.get("tile_x", 0))
   p.tile_y = int(opts.get("tile_y", 0))
@@ -273,7 +278,9 @@ def fdtdz(epsilon, dt, source_field, source_waveform, source_position,
   Snapshot i is E after time step ``output_steps[0] + i * output_steps[2]``
   over the epsilon window at ``offset``.  Differentiable with respect to
   ``epsilon`` when it is a tensor that requires grad.  Raises ValueError for
-  inconsistent shapes or arguments, RuntimeError for GPU failures.
+  inconsistent shapes or arguments, RuntimeError for GPU failures; a run on
+  this GPU whose workgroups waited for one another in vain (another process
+  holds part of it) is reported by the next call, its own snapshots hold NaN.
   """
   arrays = (epsilon, source_field, source_waveform, absorption_mask,
             pml_kappa, pml_sigma, pml_alpha)

@@ -142,3 +142,13 @@ def test_density_and_render_reject_bad_arguments_before_any_launch():
   assert lib.pjz_fdtd_render_forward(2, 1, 8, 8, 16, 0, p, None, p, p, p, p, None) == _lib.EINVAL
   assert lib.pjz_fdtd_render_backward(2, 1, 8, 8, 16, 0, p, p, p, p, p, p, p, p, p, 16,
                                       None) == _lib.ESPACE
+
+
+def test_step_by_step_option_sets_its_flag():
+  assert _problem().flags & _lib.FLAG_STEPWISE == 0
+  p = _problem(launch_params=dict(resident=False), use_reduced_precision=True)
+  assert p.flags == _lib.FLAG_REDUCED | _lib.FLAG_STEPWISE
+
+
+def test_run_status_without_a_run():
+  assert _lib.load().pjz_fdtd_run_status() == _lib.OK
