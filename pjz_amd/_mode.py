@@ -142,7 +142,9 @@ def _subspace_iteration_hip(epsilon, omega, shift, x, n, tol):
   x = torch.take_along_dim(x, inds[:, None, None, None, :], dim=-1)
   w = torch.take_along_dim(w, inds, dim=-1)
   err = torch.take_along_dim(err, inds, dim=-1)
-  return w, x, err, int(iters.max())
+  most = int(iters.max())
+  _lib.check(lib.pjz_fdtd_run_status(), "mode")
+  return w, x, err, most
 
 
 HIP_MAX_MODES = 10

@@ -658,8 +658,12 @@ int pjz_fdtd_mode_solve(int32_t ww, int32_t xx, int32_t yy, int32_t mm, const fl
   const size_t need = pjz::mode_workspace_floats(ww, xx, yy, mm) * sizeof(float);
   if (workspace_bytes < need)
     return fail(PJZ_FDTD_ESPACE, "mode: workspace of %zu bytes, need %zu", workspace_bytes, need);
+  if (const int bad = stall_reported()) return bad;
+  pjz::WaitWords waits;
+  waits.report = report_word(true);
+  waits.no_time = (g_test_faults & PJZ_FDTD_TEST_STALL) != 0;
   hipError_t e = pjz::launch_mode(ww, xx, yy, mm, epsilon, omega, shift, x, w, err, iters,
-                                  max_iters, tol, (float*)workspace, (hipStream_t)stream);
+                                  max_iters, tol, (float*)workspace, waits, (hipStream_t)stream);
   return e == hipSuccess ? PJZ_FDTD_OK : hip_fail(e, "mode");
 }
 

@@ -174,7 +174,8 @@ constexpr int kModeMaxModes = 10;
 size_t mode_workspace_floats(int ww, int xx, int yy, int mm);
 hipError_t launch_mode(int ww, int xx, int yy, int mm, const float* eps, const float* omega,
                        const float* shift, float* x, float* w, float* err, int* iters,
-                       int max_iters, float tol, float* ws, hipStream_t s);
+                       int max_iters, float tol, float* ws, const WaitWords& waits,
+                       hipStream_t s);
 
 hipError_t run_reference(const Geom& g, const pjz_fdtd_problem& p, const float* mask,
                          const Src& src, const OutWin& win, char* ws, const Layout& L,

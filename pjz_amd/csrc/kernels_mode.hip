@@ -38,6 +38,7 @@
 #include <type_traits>
 
 #include "fdtd_common.h"
+#include "waits.h"
 
 namespace pjz {
 
@@ -553,8 +554,9 @@ __global__ __launch_bounds__(kModeThreads) void k_mode_grid(ModeArgs a) {
 // are waited for, so both travel at once (the other order: 256 x 128 6.7 us an
 // iteration instead of 3.9).  Two sets of words alternate: a
 // workgroup posts exchange s + 2 only after it has everyone's sums of s + 1,
-// which each posts after it has read all of s.  All workgroups are resident
-// (cooperative launch) and post before they wait, so every wait ends.
+// which each posts after it has read all of s.  All workgroups are resident at
+// the same time (cooperative launch) and post before they wait, so every wait
+// ends; where that does not hold, by the clock (waits.h), with NaN for results.
 //
 // Cholesky QR: the Gram matrix is summed in double over float rows, so one
 // pass leaves x orthonormal to the rounding of its floats unless y is close to
@@ -577,23 +579,33 @@ __device__ __forceinline__ void post_word(word_t* p, unsigned tag, unsigned v) {
 __device__ __forceinline__ word_t read_word(const word_t* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ unsigned wait_word(const word_t* p, unsigned tag) {
-  word_t v = read_word(p);
-  while ((unsigned)(v >> 32) != tag) v = read_word(p);
-  return (unsigned)v;
+// Polls until load() finds all its words, or the workgroup's waits end at
+// `*end`; false: they did.
+template <class F>
+__device__ __forceinline__ bool poll_words(unsigned* end, F&& load) {
+  int left = kWaitPolls;
+  bool found;
+  do found = load(); while (!found && --left > 0);
+  while (!found) {
+    if (wait_over(end)) return false;
+    found = load();
+  }
+  return true;
 }
 
 struct TileArgs {
   ModeArgs m;
   word_t* box;   // words of the exchanges, cleared before the launch
   int R, joint;  // rows a workgroup; whether all frequencies stop together
+  WaitArgs waits;
 };
 
 // Words of one exchange set: per frequency and workgroup its first and last
 // row of y (2 x 2 components x YY x MM), then per frequency and sum every
-// workgroup's double in two words, then one stop word a frequency.
+// workgroup's double in two words, then one stop word a frequency; last the
+// word of waits in vain (of the first set).
 struct TileBox {
-  size_t row, sum, go, total;
+  size_t row, sum, go, late, total;
 };
 __host__ __device__ inline TileBox tile_box(int ww, int gpf, int YY, int mm) {
   const size_t nall = 3 * mm + mm * (mm + 1) / 2;
@@ -602,7 +614,8 @@ __host__ __device__ inline TileBox tile_box(int ww, int gpf, int YY, int mm) {
   b.row = 0;
   b.sum = n * 4 * YY * mm;
   b.go = b.sum + n * nall * 2;
-  b.total = b.go + ww;
+  b.late = b.go + ww;
+  b.total = b.late + 1;
   return b;
 }
 
@@ -744,12 +757,15 @@ __device__ __forceinline__ void row_ri_regs(float (&v)[MM], const double (&Ri)[M
   for (int k = 0; k < MM; ++k) v[k] = o[k];
 }
 
-template <int MM, int CPT>
+// EX: workgroups exchange; without, one workgroup a frequency stops by itself
+// (a kernel of its own: with the exchange's code in it, unused, a 30 x 20 call
+// of 1500 iterations took 3.80 ms instead of 3.60).
+template <int MM, int CPT, bool EX>
 __global__ __launch_bounds__(kModeThreads) void k_mode_tile(TileArgs ta) {
   constexpr int NQ = ModeLds<MM>::NQ, NPAIR = ModeLds<MM>::NPAIR, NALL = ModeLds<MM>::NALL;
   constexpr int T = kModeThreads;
   const ModeArgs& a = ta.m;
-  const int XX = a.XX, YY = a.YY, PC = XX * YY, gpf = a.gpf;
+  const int XX = a.XX, YY = a.YY, PC = XX * YY, gpf = EX ? a.gpf : 1;
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
   const int f = blockIdx.x / gpf, part = blockIdx.x - f * gpf;
   const int r0 = part * ta.R, R = min(ta.R, XX - r0);  // own rows r0 .. r0 + R - 1
@@ -763,6 +779,13 @@ __global__ __launch_bounds__(kModeThreads) void k_mode_tile(TileArgs ta) {
   __shared__ double red[kModeWaves][NALL];
   __shared__ double sum[NALL];
   __shared__ int s_go;
+  __shared__ unsigned s_end;  // of the workgroup's waits
+
+  if constexpr (EX) {
+    // (Without time to wait, a test: a workgroup is missing.)
+    if (ta.waits.ticks == 0 && blockIdx.x + 1 == gridDim.x) return;
+    if (t == 0) s_end = wait_end(ta.waits);
+  }
 
   const TileBox tb = tile_box(gridDim.x / gpf, gpf, YY, MM);
   const long long n = 2LL * PC;
@@ -844,9 +867,8 @@ __global__ __launch_bounds__(kModeThreads) void k_mode_tile(TileArgs ta) {
       for (int i = 0; i < NW; ++i) v[i] = 0.0;
       for (int j = lane; j < gpf; j += 64) {
         word_t lo[NW], hi[NW];
-        bool ok;
-        do {
-          ok = true;
+        poll_words(&s_end, [&]() __attribute__((always_inline)) {
+          bool ok = true;
 #pragma unroll
           for (int i = 0; i < NW; ++i) {
             const int q = min(wv + i * kModeWaves, P - 1);
@@ -857,7 +879,8 @@ __global__ __launch_bounds__(kModeThreads) void k_mode_tile(TileArgs ta) {
 #pragma unroll
           for (int i = 0; i < NW; ++i)
             ok &= (unsigned)(lo[i] >> 32) == seq && (unsigned)(hi[i] >> 32) == seq;
-        } while (!ok);
+          return ok;
+        });
 #pragma unroll
         for (int i = 0; i < NW; ++i)
           v[i] += __builtin_bit_cast(double, (hi[i] << 32) | (lo[i] & 0xffffffffu));
@@ -971,19 +994,22 @@ __global__ __launch_bounds__(kModeThreads) void k_mode_tile(TileArgs ta) {
         const word_t* q = rb + ((size_t)((side ? pd * 2 : pu * 2 + 1) * 2 + comp) * YY + j) * MM;
         float* d = (comp ? X1 : X0) + (side ? (R + 1) * rowlen : 0) + j * MM;
         word_t v[MM];
-        bool ok;
-        do {
-          ok = true;
+        poll_words(&s_end, [&]() __attribute__((always_inline)) {
+          bool ok = true;
 #pragma unroll
           for (int k = 0; k < MM; ++k) v[k] = read_word(q + k);
 #pragma unroll
           for (int k = 0; k < MM; ++k) ok &= (unsigned)(v[k] >> 32) == seq;
-        } while (!ok);
+          return ok;
+        });
 #pragma unroll
         for (int k = 0; k < MM; ++k) d[k] = __uint_as_float((unsigned)v[k]);
       }
     }
     collect_sums(std::integral_constant<int, 0>(), std::integral_constant<int, NALL>());
+    // A wait in vain ends the run.  (All waves read the same: none waits again
+    // before the others have come to its next barrier.)
+    if (EX && s_end == kLate) break;
     // The stop test: while the largest residual is above tol, which a NaN ends
     // (the square of the residual against tol's: no square root).
     if (it > 0) {
@@ -995,7 +1021,7 @@ __global__ __launch_bounds__(kModeThreads) void k_mode_tile(TileArgs ta) {
         above |= e2 > (double)a.tol * (double)a.tol;
       }
       go = above && !nan;
-      if (ta.joint && gridDim.x > (unsigned)gpf) {
+      if (EX && ta.joint && gridDim.x > (unsigned)gpf) {
         // All frequencies: one word each, numbered by the iteration.
         const int ww = gridDim.x / gpf;
         word_t* gb = ta.box + (it & 1) * tb.total + tb.go;
@@ -1003,7 +1029,14 @@ __global__ __launch_bounds__(kModeThreads) void k_mode_tile(TileArgs ta) {
         if (t == 0) s_go = 0;
         __syncthreads();
         int got = 0;
-        for (int g = t; g < ww; g += T) got |= wait_word(gb + g, it);
+        for (int g = t; g < ww; g += T) {
+          word_t v;
+          const bool came = poll_words(&s_end, [&]() __attribute__((always_inline)) {
+            v = read_word(gb + g);
+            return (unsigned)(v >> 32) == (unsigned)it;
+          });
+          got |= came ? (int)(unsigned)v : 2;
+        }
         if (got) atomicOr(&s_go, got);
         __syncthreads();
         go = s_go == 1;
@@ -1090,9 +1123,19 @@ __global__ __launch_bounds__(kModeThreads) void k_mode_tile(TileArgs ta) {
       xg[(PC + g) * MM + k] = x[c][1][k];
     }
   }
+  __syncthreads();
+  const bool late = EX && s_end == kLate;
+  if (late) {
+    if (t == 0) {
+      xg[(long long)r0 * rowlen] = __builtin_nanf("");
+      tell_late(ta.waits);
+    }
+  }
   if (part == 0 && t == 0) {
     a.iters[f] = it;
-    if (it > 0) {
+    if (late) {
+      for (int k = 0; k < MM; ++k) a.w[f * MM + k] = a.err[f * MM + k] = __builtin_nanf("");
+    } else if (it > 0) {
       residuals<MM>(sum, a.w + f * MM, a.err + f * MM, true);
     } else {
       for (int k = 0; k < MM; ++k) {
@@ -1171,18 +1214,20 @@ size_t mode_workspace_floats(int ww, int XX, int YY, int mm) {
 // The tile kernel where it applies; *done says whether it was launched.
 template <int MM, int CPT>
 static hipError_t launch_tile(const ModeArgs& a, int ww, TilePlan p, float* ws, hipStream_t s,
-                              bool* done) {
+                              const WaitWords& waits, bool* done) {
   TileArgs ta;
+  ta.waits = {};
   ta.m = a;
   ta.m.gpf = p.gpf;
   ta.R = p.R;
   // Small sections stop frequency by frequency, large ones together.
   ta.joint = (long long)a.XX * a.YY * MM >= kModeJointWork;
   ta.box = reinterpret_cast<word_t*>((reinterpret_cast<uintptr_t>(ws) + 255) & ~uintptr_t(255));
-  const void* kernel = reinterpret_cast<const void*>(&k_mode_tile<MM, CPT>);
+  const void* kernel = reinterpret_cast<const void*>(&k_mode_tile<MM, CPT, true>);
   const size_t lds = tile_lds(p.R, a.YY, MM);
   const bool coop = p.gpf > 1 || (ta.joint && ww > 1);
   if (coop) {
+    if (!waits.report) return hipSuccess;
     // Every workgroup has to be resident at once.  A small section's launch
     // can be recorded into a graph, which a cooperative one might not.
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
@@ -1200,28 +1245,36 @@ static hipError_t launch_tile(const ModeArgs& a, int ww, TilePlan p, float* ws, 
     hipError_t e = launch_zero(reinterpret_cast<float*>(ta.box),
                                4 * tile_box(ww, p.gpf, a.YY, MM).total, s);
     if (e != hipSuccess) return e;
+    // 20 s, as the resident steppers' launches, and 0.1 ms an iteration (of
+    // 2-8 us).
+    const double ms = waits.no_time ? 0.0 : 20e3 + 0.1 * a.max_iters;
+    ta.waits.ticks = (unsigned)std::min(ms * (100e3 / kWaitTick), 1e9);
+    ta.waits.stalled =
+        reinterpret_cast<unsigned*>(ta.box + tile_box(ww, p.gpf, a.YY, MM).late);
+    ta.waits.report = waits.report;
     *done = true;
     void* args[] = {&ta};
     return hipLaunchCooperativeKernel(kernel, dim3(ww * p.gpf), dim3(kModeThreads), args,
                                       (unsigned)lds, s);
   }
   *done = true;
-  hipLaunchKernelGGL((k_mode_tile<MM, CPT>), dim3(ww), dim3(kModeThreads), lds, s, ta);
+  hipLaunchKernelGGL((k_mode_tile<MM, CPT, false>), dim3(ww), dim3(kModeThreads), lds, s, ta);
   return hipGetLastError();
 }
 
 template <int MM>
-static hipError_t launch_mode_mm(ModeArgs a, int ww, float* ws, hipStream_t s) {
+static hipError_t launch_mode_mm(ModeArgs a, int ww, float* ws, const WaitWords& waits,
+                                 hipStream_t s) {
   if constexpr (MM <= kTileMaxModes) {
     const TilePlan p = tile_plan(ww, a.XX, a.YY, MM);
     if (p.R > 0) {
       bool done = false;
       const int cells = p.R * a.YY;
       const hipError_t e =
-          cells <= kModeThreads ? launch_tile<MM, 1>(a, ww, p, ws, s, &done)
+          cells <= kModeThreads ? launch_tile<MM, 1>(a, ww, p, ws, s, waits, &done)
           : cells <= 2 * kModeThreads
-              ? launch_tile<MM, 2>(a, ww, p, ws, s, &done)
-              : launch_tile<MM, tile_max_cells(MM)>(a, ww, p, ws, s, &done);
+              ? launch_tile<MM, 2>(a, ww, p, ws, s, waits, &done)
+              : launch_tile<MM, tile_max_cells(MM)>(a, ww, p, ws, s, waits, &done);
       if (done || e != hipSuccess) return e;
     }
   }
@@ -1238,7 +1291,8 @@ static hipError_t launch_mode_mm(ModeArgs a, int ww, float* ws, hipStream_t s) {
 
 hipError_t launch_mode(int ww, int XX, int YY, int mm, const float* eps, const float* omega,
                        const float* shift, float* x, float* w, float* err, int* iters,
-                       int max_iters, float tol, float* ws, hipStream_t s) {
+                       int max_iters, float tol, float* ws, const WaitWords& waits,
+                       hipStream_t s) {
   ModeArgs a;
   a.XX = XX;
   a.YY = YY;
@@ -1258,16 +1312,16 @@ hipError_t launch_mode(int ww, int XX, int YY, int mm, const float* eps, const f
   a.err = err;
   a.iters = iters;
   switch (mm) {
-    case 1: return launch_mode_mm<1>(a, ww, ws, s);
-    case 2: return launch_mode_mm<2>(a, ww, ws, s);
-    case 3: return launch_mode_mm<3>(a, ww, ws, s);
-    case 4: return launch_mode_mm<4>(a, ww, ws, s);
-    case 5: return launch_mode_mm<5>(a, ww, ws, s);
-    case 6: return launch_mode_mm<6>(a, ww, ws, s);
-    case 7: return launch_mode_mm<7>(a, ww, ws, s);
-    case 8: return launch_mode_mm<8>(a, ww, ws, s);
-    case 9: return launch_mode_mm<9>(a, ww, ws, s);
-    case 10: return launch_mode_mm<10>(a, ww, ws, s);
+    case 1: return launch_mode_mm<1>(a, ww, ws, waits, s);
+    case 2: return launch_mode_mm<2>(a, ww, ws, waits, s);
+    case 3: return launch_mode_mm<3>(a, ww, ws, waits, s);
+    case 4: return launch_mode_mm<4>(a, ww, ws, waits, s);
+    case 5: return launch_mode_mm<5>(a, ww, ws, waits, s);
+    case 6: return launch_mode_mm<6>(a, ww, ws, waits, s);
+    case 7: return launch_mode_mm<7>(a, ww, ws, waits, s);
+    case 8: return launch_mode_mm<8>(a, ww, ws, waits, s);
+    case 9: return launch_mode_mm<9>(a, ww, ws, waits, s);
+    case 10: return launch_mode_mm<10>(a, ww, ws, waits, s);
     default: return hipErrorInvalidValue;
   }
 }

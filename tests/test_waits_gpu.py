@@ -16,6 +16,7 @@ import torch
 
 import test_fdtdz_gpu as T
 from pjz_amd import _lib
+from pjz_amd import _mode as M
 from pjz_amd import fdtdz_torch as F
 
 pytestmark = pytest.mark.gpu
@@ -104,6 +105,24 @@ def test_step_by_step_option_does_not_wait():
       got = F.fdtdz(**kw)
     assert not reported()
     assert torch.equal(got, F.fdtdz(**dict(kw, launch_params=dict(kernel="stream2"))))
+
+
+# Frequencies that stop one by one, and together; of several workgroups each.
+@pytest.mark.parametrize("X,Y,ww,modes", [(64, 48, 1, 2), (64, 48, 3, 1), (128, 96, 2, 2)])
+def test_mode_solve_that_waits_in_vain(X, Y, ww, modes):
+  eps = torch.ones(3, X, Y, device="cuda")
+  eps[:, X // 3:X // 2, Y // 3:Y // 2] = 12.25
+  omega = torch.linspace(0.25, 0.3, ww, device="cuda")
+  gen = torch.Generator().manual_seed(X)
+  x = torch.randn((ww, 2, X, Y, modes), generator=gen).cuda()
+  args = (eps, omega, torch.zeros_like(omega), x, 40, 0.0)
+  want = M._subspace_iteration_hip(*args)
+  with stalled():
+    with pytest.raises(RuntimeError, match="gave up waiting"):
+      M._subspace_iteration_hip(*args)
+  assert not reported()
+  for a, b in zip(M._subspace_iteration_hip(*args)[:3], want):
+    assert torch.equal(a, b) and bool(torch.isfinite(a).all())
 
 
 def test_resident_runs_of_several_streams_and_threads():
