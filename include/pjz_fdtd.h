@@ -322,6 +322,28 @@ PJZ_FDTD_API int pjz_fdtd_render_backward(int32_t ll, int32_t m, int32_t xx, int
 PJZ_FDTD_API int pjz_fdtd_stepper(const pjz_fdtd_problem* p, int32_t* kernel);
 
 /*
+ * Diagnostic: the way a call with this problem takes on the current device and
+ * `stream`, with a workspace of pjz_fdtd_workspace_bytes: a forward call, or
+ * (`backward`) the recompute and the reverse of a gradient.  The batched form
+ * tells it for every simulation of a batch, where `kind` LAUNCHES means that
+ * the simulation shares the batched launches.
+ */
+#define PJZ_FDTD_ROUTE_LAUNCHES 0 /* kernels launched step by step               */
+#define PJZ_FDTD_ROUTE_RESIDENT 1 /* the domain in registers, a launch a run     */
+#define PJZ_FDTD_ROUTE_SLABS 2    /* the domain in slabs of x, each in registers */
+typedef struct pjz_fdtd_route {
+  int32_t kind;        /* PJZ_FDTD_ROUTE_*                                      */
+  int32_t cells;       /* cells of a column a lane (1 or 2), 0: LAUNCHES        */
+  int32_t rx, ry;      /* columns a wave in x and y                             */
+  int32_t slabs, steps;/* SLABS: their count, steps a slab's launch             */
+  int32_t reverse;     /* backward: whether the reverse steps are resident too  */
+} pjz_fdtd_route;
+PJZ_FDTD_API int pjz_fdtd_route_of(const pjz_fdtd_problem* p, int backward, void* stream,
+                                   pjz_fdtd_route* route);
+PJZ_FDTD_API int pjz_fdtd_batch_routes(const pjz_fdtd_problem* probs, int n, int backward,
+                                       void* stream, pjz_fdtd_route* routes);
+
+/*
  * Diagnostic: copies `bytes` (a multiple of 16; both pointers 16-byte
  * aligned) from src to dst on the device with nontemporal loads and stores,
  * stream-ordered.  No counterpart in pjz: bench.py times it on 1 GiB to

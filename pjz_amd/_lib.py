@@ -22,6 +22,8 @@ TEST_STALL = 1
 EXPORTS = (
     "pjz_fdtd_abi_version",
     "pjz_fdtd_last_error",
+    "pjz_fdtd_route_of",
+    "pjz_fdtd_batch_routes",
     "pjz_fdtd_run_status",
     "pjz_fdtd_test_faults",
     "pjz_fdtd_num_outputs",
@@ -64,6 +66,15 @@ class Problem(ctypes.Structure):
   ]
 
 
+class Route(ctypes.Structure):
+  """Mirror of ``pjz_fdtd_route``."""
+  _fields_ = [("kind", ctypes.c_int32), ("cells", ctypes.c_int32), ("rx", ctypes.c_int32),
+              ("ry", ctypes.c_int32), ("slabs", ctypes.c_int32), ("steps", ctypes.c_int32),
+              ("reverse", ctypes.c_int32)]
+
+
+ROUTE_LAUNCHES, ROUTE_RESIDENT, ROUTE_SLABS = 0, 1, 2
+
 _lock = threading.Lock()
 _lib = None
 
@@ -87,6 +98,11 @@ def load():
     lib.pjz_fdtd_abi_version.argtypes = []
     lib.pjz_fdtd_last_error.restype = ctypes.c_char_p
     lib.pjz_fdtd_last_error.argtypes = []
+    R = ctypes.POINTER(Route)
+    lib.pjz_fdtd_route_of.restype = ctypes.c_int
+    lib.pjz_fdtd_route_of.argtypes = [P, ctypes.c_int, vp, R]
+    lib.pjz_fdtd_batch_routes.restype = ctypes.c_int
+    lib.pjz_fdtd_batch_routes.argtypes = [P, ctypes.c_int, ctypes.c_int, vp, R]
     lib.pjz_fdtd_run_status.restype = ctypes.c_int
     lib.pjz_fdtd_run_status.argtypes = []
     lib.pjz_fdtd_test_faults.restype = None
@@ -159,6 +175,23 @@ def stepper(prob):
   k = ctypes.c_int32(0)
   check(load().pjz_fdtd_stepper(ctypes.byref(prob), ctypes.byref(k)), "pjz_fdtd_stepper")
   return k.value
+
+
+def route(prob, backward=False, stream=0):
+  """The :class:`Route` of a single call with ``prob``."""
+  r = Route()
+  check(load().pjz_fdtd_route_of(ctypes.byref(prob), int(backward), ctypes.c_void_p(stream),
+                                 ctypes.byref(r)), "pjz_fdtd_route_of")
+  return r
+
+
+def batch_routes(probs, backward=False, stream=0):
+  """The :class:`Route` of every simulation of a batch (ctypes array of
+  problems)."""
+  r = (Route * len(probs))()
+  check(load().pjz_fdtd_batch_routes(probs, len(probs), int(backward), ctypes.c_void_p(stream), r),
+        "pjz_fdtd_batch_routes")
+  return list(r)
 
 
 def num_outputs(prob):

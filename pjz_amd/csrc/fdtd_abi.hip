@@ -385,6 +385,38 @@ pjz::Layout layout_in(const pjz::Geom& g, const pjz_fdtd_problem& p, void* ws, s
   return L;
 }
 
+// What a call takes of these, for the diagnostic: a forward's steps, or the
+// recompute and the reverse of a gradient.
+pjz_fdtd_route route_of(const pjz::Geom& g, const pjz_fdtd_problem& p, const pjz::Layout& L,
+                        bool backward, hipStream_t s) {
+  pjz_fdtd_route r{};
+  auto tile = [&](int kind, const pjz::ResPlan& t) {
+    r.kind = kind;
+    r.cells = t.cpl;
+    r.rx = t.rx;
+    r.ry = t.ry;
+  };
+  const pjz::ResPlan plan = resident_for(g, p, L, s);
+  if (plan.rx > 0) {
+    if (!backward || pjz::resident_captures(plan)) {
+      tile(PJZ_FDTD_ROUTE_RESIDENT, plan);
+      r.reverse = backward && pjz::adjoint_resident_supported(plan);
+    }
+    return r;
+  }
+  const int nsteps = pjz::steps_of(p);
+  const int run = L.nck == 0 ? nsteps : backward ? L.S : L.S1;
+  if (L.words > 0 && run >= kResidentMinSteps) {
+    const pjz::SlabPlan slabs = slabs_for(g, p, L, s, backward);
+    if (slabs.n > 0) {
+      tile(PJZ_FDTD_ROUTE_SLABS, slabs.tile);
+      r.slabs = slabs.n;
+      r.steps = slabs.steps;
+    }
+  }
+  return r;
+}
+
 // Steps [b, end) with the kernel the problem selects (AUTO: auto_kernel;
 // AUTOTUNE: the cached choice for the shape, else AUTO).
 hipError_t run_steps(const pjz::Geom& g, const pjz_fdtd_problem& p, const float* mask,
@@ -805,6 +837,17 @@ int pjz_fdtd_stepper(const pjz_fdtd_problem* p, int32_t* kernel) {
   return PJZ_FDTD_OK;
 }
 
+int pjz_fdtd_route_of(const pjz_fdtd_problem* p, int backward, void* stream,
+                      pjz_fdtd_route* route) {
+  int rc = check(p);
+  if (rc) return rc;
+  if (!route) return fail(PJZ_FDTD_EINVAL, "route is NULL");
+  const pjz::Geom g = geom_of(*p);
+  const pjz::Layout L = layout_in(g, *p, nullptr, SIZE_MAX);
+  *route = route_of(g, *p, L, backward != 0, (hipStream_t)stream);
+  return PJZ_FDTD_OK;
+}
+
 int pjz_fdtd_run_status(void) { return stall_reported(); }
 
 void pjz_fdtd_test_faults(uint32_t faults) { g_test_faults = faults; }
@@ -1053,6 +1096,24 @@ int pjz_fdtd_batch_workspace_bytes(const pjz_fdtd_problem* probs, int n, size_t*
   if (rc) return rc;
   if (!bytes) return fail(PJZ_FDTD_EINVAL, "bytes is NULL");
   *bytes = bp.total;
+  return PJZ_FDTD_OK;
+}
+
+int pjz_fdtd_batch_routes(const pjz_fdtd_problem* probs, int n, int backward, void* stream,
+                          pjz_fdtd_route* routes) {
+  BatchPlanHost bp;
+  int rc = batch_plan(probs, n, bp);
+  if (rc) return rc;
+  if (!routes) return fail(PJZ_FDTD_EINVAL, "routes is NULL");
+  const hipStream_t s = (hipStream_t)stream;
+  std::vector<pjz::BatchItem> items(n);
+  for (int i = 0; i < n; ++i)
+    items[i] = {geom_of(probs[i]), &probs[i], nullptr, {}, {}, nullptr, &bp.Ls[i], nullptr};
+  batch_waits(items, bp);
+  const std::vector<bool> alone = batch_alone(items, backward != 0, s);
+  for (int i = 0; i < n; ++i)
+    routes[i] = alone[i] ? route_of(items[i].g, probs[i], bp.Ls[i], backward != 0, s)
+                         : pjz_fdtd_route{};
   return PJZ_FDTD_OK;
 }
 

@@ -152,3 +152,17 @@ def test_step_by_step_option_sets_its_flag():
 
 def test_run_status_without_a_run():
   assert _lib.load().pjz_fdtd_run_status() == _lib.OK
+
+
+def test_routes_check_their_problem():
+  bad = _problem()
+  bad.dt = 0.0
+  with pytest.raises(ValueError, match="dt"):
+    _lib.route(bad)
+  with pytest.raises(ValueError, match="batch item 0"):
+    _lib.batch_routes((_lib.Problem * 1)(bad))
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="without a GPU")
+def test_no_resident_route_without_a_gpu():
+  assert _lib.route(_problem()).kind == _lib.ROUTE_LAUNCHES

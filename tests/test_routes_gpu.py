@@ -1,0 +1,107 @@
+"""Which way a call takes (pjz_fdtd_route_of, pjz_fdtd_batch_routes), asserted
+for the domain each kernel is tested on: a change of the dispatch that leaves a
+kernel untested fails here instead of passing on another one.
+
+Forward and reverse tilings that no other file reaches, captured runs in slabs
+of more than one block, and the batched launches of simulations that would run
+resident by default.
+"""
+
+import numpy as np
+import pytest
+import torch
+
+import test_batch_gpu as B
+import test_fdtdz_gpu as T
+import test_grad_gpu as G
+from oracle import c_oracle as C
+from pjz_amd import _lib
+from pjz_amd import fdtdz_torch as F
+
+pytestmark = pytest.mark.gpu
+
+
+def prob_of(kw, eps=None, **launch):
+  shapes = {k: np.shape(v) for k, v in dict(kw, epsilon=kw.get("epsilon", eps)).items()}
+  return F.make_problem(shapes["epsilon"], kw["dt"], shapes["source_field"],
+                        kw["source_position"], shapes["absorption_mask"], shapes["pml_kappa"],
+                        kw["pml_widths"], kw["output_steps"], shapes["source_waveform"][0], False,
+                        launch, kw["offset"])
+
+
+def tiling(r):
+  return (r.cells, r.rx, r.ry)
+
+
+@pytest.mark.parametrize("axis", [0, 1, 2])
+@pytest.mark.parametrize("want,X,Y,Z", [((1, 2, 1), 64, 64, 64), ((1, 2, 2), 88, 88, 64),
+                                        ((2, 1, 1), 40, 40, 128), ((2, 2, 1), 62, 58, 120),
+                                        ((2, 5, 2), 136, 122, 66)])
+def test_forward_tilings(want, X, Y, Z, axis):
+  print(f"case {X}x{Y}x{Z} axis {axis}", flush=True)
+  kw = T.random_problem(axis, X=X, Y=Y, Z=Z, tt=40, seed=X + axis, widths=(6, 5))
+  kw["output_steps"] = (30, 40, 3)
+  r = _lib.route(prob_of(kw))
+  assert r.kind == _lib.ROUTE_RESIDENT and tiling(r) == want
+  step = prob_of(kw, resident=False)
+  assert _lib.route(step).kind == _lib.ROUTE_LAUNCHES
+  got = F.fdtdz(**kw)
+  ref = F.fdtdz(**dict(kw, launch_params=dict(kernel="stream2")))
+  assert torch.equal(got, ref)
+
+
+@pytest.mark.parametrize("axis", [0, 1, 2])
+@pytest.mark.parametrize("want,X,Y,Z", [((1, 2, 1), 64, 64, 64), ((1, 2, 2), 88, 88, 64),
+                                        ((2, 1, 1), 40, 40, 128), ((2, 2, 1), 62, 58, 120)])
+def test_reverse_tilings(want, X, Y, Z, axis):
+  print(f"case {X}x{Y}x{Z} axis {axis}", flush=True)
+  eps, kw, g = G.problem(axis, seed=X, X=X, Y=Y, Z=Z, tt=40)
+  r = _lib.route(prob_of(kw, eps, ckpt_every=11), backward=True)
+  assert r.kind == _lib.ROUTE_RESIDENT and r.reverse == 1 and tiling(r) == want
+  got, _ = G.gpu_grad(eps, kw, g, ckpt_every=11)
+  ref, _ = G.gpu_grad(eps, kw, g, ckpt_every=11, kernel="stream2")
+  assert G.rel_l2(got, ref) <= 1e-5
+
+
+# Recomputes that capture, in slabs: two cells a lane and one, segments of
+# several blocks, and of one and a part.
+@pytest.mark.parametrize("want,X,Y,Z,launch", [
+    ((1, 5, 5), 300, 300, 64, dict(ckpt_every=50)),
+    ((1, 5, 5), 300, 300, 64, dict(ckpt_every=44, ckpt_inner=23)),
+    ((2, 4, 3), 200, 180, 66, dict(ckpt_every=30))])
+def test_slab_gradients_that_capture(want, X, Y, Z, launch):
+  print(f"case {X}x{Y}x{Z} {launch}", flush=True)
+  eps, kw, g = G.problem(0, seed=9, X=X, Y=Y, Z=Z, tt=60)
+  r = _lib.route(prob_of(kw, eps, **launch), backward=True)
+  assert r.kind == _lib.ROUTE_SLABS and tiling(r) == want
+  assert launch.get("ckpt_inner", launch["ckpt_every"]) > r.steps
+  got, _ = G.gpu_grad(eps, kw, g, **launch)
+  ref, _ = G.gpu_grad(eps, kw, g, kernel="stream2", **launch)
+  assert G.rel_l2(got, ref) <= 1e-5
+
+
+def test_three_steps_per_launch_in_batches():
+  """Simulations that run resident by default, in the batched launches: the
+  zz <= 64 class three steps a launch, uneven step counts (remainders 0, 1, 2),
+  snapshots every step at the end."""
+  cases = [(11, 150, 140, 64, 60, 0), (12, 130, 150, 40, 50, 1), (13, 141, 122, 64, 49, 2),
+           (14, 90, 70, 128, 44, 0)]
+  calls = []
+  for c in cases:
+    kw = B.sim(*c)
+    kw["output_steps"] = (c[4] - 7, c[4], 1)
+    calls.append(dict(kw, launch_params=dict(resident=False)))
+  probs, _, _ = F._batch_problems(calls)
+  assert [r.kind for r in _lib.batch_routes(probs)] == [_lib.ROUTE_LAUNCHES] * len(cases)
+  probs, _, _ = F._batch_problems([dict(kw, launch_params=None) for kw in calls])
+  assert all(r.kind == _lib.ROUTE_RESIDENT for r in _lib.batch_routes(probs))
+  outs = F.fdtdz_batch(calls)
+  torch.cuda.synchronize()
+  for case, kw, out in zip(cases, calls, outs):
+    print(f"case {case}", flush=True)
+    got = out.cpu().numpy()
+    ref = C.fdtdz(**kw)
+    assert np.linalg.norm(got - ref) <= 1e-4 * np.linalg.norm(ref), case
+    kernel = "stream3" if case[3] <= 64 else "stream2"
+    want = F.fdtdz(**dict(kw, launch_params=dict(kernel=kernel))).cpu().numpy()
+    assert np.linalg.norm(got - want) <= 1e-6 * np.linalg.norm(want), case
