@@ -128,6 +128,8 @@ PJZ_FDTD_API int pjz_fdtd_run_status(void);
  * a mask of PJZ_FDTD_TEST_* (0, the default: none).
  */
 #define PJZ_FDTD_TEST_STALL 1  /* a workgroup is missing and its peers give up soon */
+#define PJZ_FDTD_TEST_REFUSE 2 /* cooperative launches fail                        */
+#define PJZ_FDTD_TEST_REFUSE_LATER 4 /* all but a call's first fail               */
 PJZ_FDTD_API void pjz_fdtd_test_faults(uint32_t faults);
 
 /* Number of snapshots, len(range(*output_steps)). */

@@ -16,7 +16,7 @@ OK, EINVAL, EHIP, ESPACE, ESTALL = 0, 1, 2, 3, 4
 KERNEL_AUTO, KERNEL_REFERENCE, KERNEL_STREAM, KERNEL_STREAM2, KERNEL_AUTOTUNE = 0, 1, 2, 3, 4
 KERNEL_STREAM3, KERNEL_STREAM4 = 5, 6
 FLAG_REDUCED, FLAG_STEPWISE = 1, 2
-TEST_STALL = 1
+TEST_STALL, TEST_REFUSE, TEST_REFUSE_LATER = 1, 2, 4
 
 # Every entry point include/pjz_fdtd.h declares.
 EXPORTS = (

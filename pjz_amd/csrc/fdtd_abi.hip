@@ -40,6 +40,15 @@ int count_outputs(const pjz_fdtd_problem& p) {
 // ------------------------------------------------- waits that ended in vain
 // Failure paths under test in the calling thread (PJZ_FDTD_TEST_*).
 thread_local unsigned g_test_faults = 0;
+thread_local int g_test_launches = 0;  // cooperative ones that a call has left
+
+void test_faults_of_call(pjz::WaitWords& w) {
+  w.no_time = (g_test_faults & PJZ_FDTD_TEST_STALL) != 0;
+  if (g_test_faults & (PJZ_FDTD_TEST_REFUSE | PJZ_FDTD_TEST_REFUSE_LATER)) {
+    g_test_launches = g_test_faults & PJZ_FDTD_TEST_REFUSE ? 0 : 1;
+    w.launches = &g_test_launches;
+  }
+}
 
 constexpr int kMaxDevices = 64;
 
@@ -347,7 +356,7 @@ pjz::WaitWords waits_in(const pjz_fdtd_problem& p, const pjz::Layout& L, char* w
   if (resident_cus(p) <= 0) return w;
   w.stalled = (unsigned*)(ws + L.stalled);
   w.report = report_word(true);
-  w.no_time = (g_test_faults & PJZ_FDTD_TEST_STALL) != 0;
+  test_faults_of_call(w);
   return w;
 }
 
@@ -439,9 +448,16 @@ hipError_t run_steps(const pjz::Geom& g, const pjz_fdtd_problem& p, const float*
   if (kernel == PJZ_FDTD_KERNEL_AUTO) {
     if (L.words > 0 && end - b >= kResidentMinSteps) {
       const pjz::SlabPlan slabs = slabs_for(g, p, L, s, capture != nullptr);
-      if (slabs.n > 0)
-        return pjz::run_slabs(g, p, mask, src, win, ws, L, slabs, (pjz::rword_t*)(ws + L.words), r,
-                              s);
+      if (slabs.n > 0) {
+        int done = b;
+        if (pjz::run_slabs(g, p, mask, src, win, ws, L, slabs, (pjz::rword_t*)(ws + L.words), r,
+                           &done, s) == hipSuccess)
+          return hipSuccess;
+        // A launch was refused: the rest step by step.
+        (void)hipGetLastError();
+        r.begin = done;
+        if (capture) r.capture = capture + (size_t)(done - b) * 3 * g.N;
+      }
     }
     kernel = auto_kernel(g);
   }
@@ -524,7 +540,10 @@ hipError_t forward_steps(const pjz::Geom& g, const pjz_fdtd_problem& p, const fl
     if (e != hipSuccess) return e;
     pjz::ResRun r{0, nsteps, {}, {}, nullptr, nullptr, L.S1, 0};
     if (L.nck > 0) r.ckpt = ckpt_state(g, L, ws, 0).E;
-    return pjz::run_resident(g, p, mask, src, win, ws, L, plan, r, s);
+    e = pjz::run_resident(g, p, mask, src, win, ws, L, plan, r, s);
+    if (e == hipSuccess) return e;
+    // The launch was refused: step by step.
+    (void)hipGetLastError();
   }
   // Clears E0, H0 (contiguous) and psi.
   hipError_t e = clear_state(g, L, ws, s);
@@ -563,31 +582,43 @@ hipError_t backward_steps(const pjz::Geom& g, const pjz_fdtd_problem& p,
   };
   pjz::ResPlan plan = resident_for(g, p, L, s);
   if (!pjz::resident_captures(plan)) plan = {};
-  const bool resident_adj = plan.rx > 0 && pjz::adjoint_resident_supported(plan);
+  bool resident_adj = plan.rx > 0 && pjz::adjoint_resident_supported(plan);
   unsigned tags = 0;  // exchange numbers used
   hipError_t e = hipSuccess;
   if (plan.rx > 0) e = clear_words(plan, L, ws, s);
   if (e != hipSuccess) return e;
-  // Steps [b, end) of the resident stepper from checkpoint slot k.
+  // Steps [b, end) of the resident stepper from checkpoint slot k; false: not
+  // (any more), from here on all is launched step by step.
   auto resident = [&](int k, int b, int end, pjz::ResState out, float* capture, float* ckpt,
                       int every) {
+    if (plan.rx == 0) return false;
     const pjz::ResRun r{b, end, ckpt_state(g, L, ws, k), out, capture, ckpt, every, tags};
     tags += pjz::resident_tags(end - b);
-    return pjz::run_resident(g, p, absorption_mask, src, nowin, ws, L, plan, r, s);
+    if (pjz::run_resident(g, p, absorption_mask, src, nowin, ws, L, plan, r, s) == hipSuccess)
+      return true;
+    (void)hipGetLastError();
+    plan = {};
+    resident_adj = false;
+    return false;
   };
   // Steps [b, end) from the state in checkpoint slot k: recompute them
   // capturing D^n = E^n - E^(n+1), then reverse them.
   auto reverse_segment = [&](int k, int b, int end) {
     int cur = 0;
-    hipError_t e = plan.rx > 0 ? resident(k, b, end, {}, seg, nullptr, 1)
-                               : restore_state(g, L, ws, k, s);
-    if (e == hipSuccess && plan.rx == 0)
-      e = run_steps(g, p, absorption_mask, src, nowin, ws, L, b, end, &cur, seg, s);
+    hipError_t e = hipSuccess;
+    if (!resident(k, b, end, {}, seg, nullptr, 1)) {
+      e = restore_state(g, L, ws, k, s);
+      if (e == hipSuccess)
+        e = run_steps(g, p, absorption_mask, src, nowin, ws, L, b, end, &cur, seg, s);
+    }
     if (e == hipSuccess && resident_adj) {
-      e = pjz::run_adjoint_resident(g, p, absorption_mask, ws, L, plan, seg, grad_out, b, end,
-                                    tags, s);
-      tags += pjz::resident_tags(end - b);
-      return e;
+      if (pjz::run_adjoint_resident(g, p, absorption_mask, ws, L, plan, seg, grad_out, b, end,
+                                    tags, s) == hipSuccess) {
+        tags += pjz::resident_tags(end - b);
+        return hipSuccess;
+      }
+      (void)hipGetLastError();
+      resident_adj = false;  // (the cotangents are in set 0, as acur says)
     }
     for (int n = end - 1; n >= b && e == hipSuccess;) {
       if (is_out(n))
@@ -620,16 +651,15 @@ hipError_t backward_steps(const pjz::Geom& g, const pjz_fdtd_problem& p,
     }
     // Two levels: recompute the S1 segment from its checkpoint keeping the
     // state every S steps (slots nck + j), then reverse its sub-segments.
-    if (plan.rx > 0) {
-      const int nsub = (e1 - b1 + L.S - 1) / L.S;
-      const int last = b1 + (nsub - 1) * L.S;
-      // Slots nck .. nck + nsub - 1; the first is slot k itself.
-      if (nsub > 1)
-        e = resident(k, b1, last, ckpt_state(g, L, ws, L.nck + nsub - 1), nullptr,
-                     ckpt_state(g, L, ws, L.nck).E, L.S);
-      for (int j = nsub - 1; j >= 0 && e == hipSuccess; --j)
+    const int nres = (e1 - b1 + L.S - 1) / L.S;
+    // Slots nck .. nck + nres - 1; the first is slot k itself.
+    if (plan.rx > 0 &&
+        (nres == 1 || resident(k, b1, b1 + (nres - 1) * L.S,
+                               ckpt_state(g, L, ws, L.nck + nres - 1), nullptr,
+                               ckpt_state(g, L, ws, L.nck).E, L.S))) {
+      for (int j = nres - 1; j >= 0 && e == hipSuccess; --j)
         e = reverse_segment(j == 0 ? k : L.nck + j, b1 + j * L.S,
-                            j == nsub - 1 ? e1 : b1 + (j + 1) * L.S);
+                            j == nres - 1 ? e1 : b1 + (j + 1) * L.S);
       continue;
     }
     int cur = 0;
@@ -693,7 +723,7 @@ int pjz_fdtd_mode_solve(int32_t ww, int32_t xx, int32_t yy, int32_t mm, const fl
   if (const int bad = stall_reported()) return bad;
   pjz::WaitWords waits;
   waits.report = report_word(true);
-  waits.no_time = (g_test_faults & PJZ_FDTD_TEST_STALL) != 0;
+  test_faults_of_call(waits);
   hipError_t e = pjz::launch_mode(ww, xx, yy, mm, epsilon, omega, shift, x, w, err, iters,
                                   max_iters, tol, (float*)workspace, waits, (hipStream_t)stream);
   return e == hipSuccess ? PJZ_FDTD_OK : hip_fail(e, "mode");

@@ -44,11 +44,15 @@ struct OutWin {
 };
 
 // Byte offsets of the workspace segments (each 256-byte aligned).
-// Where a call's resident runs say that they waited in vain (waits.h).
+// Where a call's launches say that they waited in vain (waits.h).
 struct WaitWords {
   unsigned* stalled = nullptr;  // in the workspace, cleared by launch_prepare
   unsigned* report = nullptr;   // host memory; null: no resident runs
   bool no_time = false;         // waits in vain end at once (tests)
+  int* launches = nullptr;      // cooperative ones before they are refused (tests)
+
+  // The next cooperative launch's turn.
+  bool refused() const { return launches && (*launches)-- <= 0; }
 };
 
 struct Layout {

@@ -400,6 +400,7 @@ hipError_t run_adjoint_resident(const Geom& g, const pjz_fdtd_problem& p, const 
                                 char* ws, const Layout& L, const ResPlan& plan, const float* D,
                                 const float* gout, int begin, int end, unsigned tag0,
                                 hipStream_t s) {
+  if (L.waits.refused()) return hipErrorCooperativeLaunchTooLarge;
   AdjResArgs a;
   a.lE = (float*)(ws + L.lE_[0]);
   a.lH = (float*)(ws + L.lH_[0]);

@@ -1211,7 +1211,7 @@ size_t mode_workspace_floats(int ww, int XX, int YY, int mm) {
                   2 * tile_words(ww, XX, YY, mm) + 64);
 }
 
-// The tile kernel where it applies; *done says whether it was launched.
+// The tile kernel where it applies; *done says whether it runs.
 template <int MM, int CPT>
 static hipError_t launch_tile(const ModeArgs& a, int ww, TilePlan p, float* ws, hipStream_t s,
                               const WaitWords& waits, bool* done) {
@@ -1252,10 +1252,14 @@ static hipError_t launch_tile(const ModeArgs& a, int ww, TilePlan p, float* ws, 
     ta.waits.stalled =
         reinterpret_cast<unsigned*>(ta.box + tile_box(ww, p.gpf, a.YY, MM).late);
     ta.waits.report = waits.report;
-    *done = true;
     void* args[] = {&ta};
-    return hipLaunchCooperativeKernel(kernel, dim3(ww * p.gpf), dim3(kModeThreads), args,
-                                      (unsigned)lds, s);
+    e = waits.refused() ? hipErrorCooperativeLaunchTooLarge
+                        : hipLaunchCooperativeKernel(kernel, dim3(ww * p.gpf), dim3(kModeThreads),
+                                                     args, (unsigned)lds, s);
+    // A refused launch leaves it to the other kernels.
+    *done = e == hipSuccess;
+    if (!*done) (void)hipGetLastError();
+    return hipSuccess;
   }
   *done = true;
   hipLaunchKernelGGL((k_mode_tile<MM, CPT, false>), dim3(ww), dim3(kModeThreads), lds, s, ta);

@@ -584,7 +584,7 @@ SlabPlan slab_plan(const Geom& g, int saxis, int cus) {
 
 hipError_t run_slabs(const Geom& g, const pjz_fdtd_problem& p, const float* mask, const Src& src,
                      const OutWin& win, char* ws, const Layout& L, const SlabPlan& plan,
-                     rword_t* words, const StepRange& r, hipStream_t s) {
+                     rword_t* words, const StepRange& r, int* done, hipStream_t s) {
   hipError_t e = launch_zero((float*)words, slab_words(plan) * 2, s);
   float* psi = (float*)(ws + L.psi);
   const size_t P4 = (size_t)PSI_SET * g.X * g.Y * g.NP;
@@ -611,7 +611,9 @@ hipError_t run_slabs(const Geom& g, const pjz_fdtd_problem& p, const float* mask
       t.ntx = (q.xe - q.xs + t.tx() - 1) / t.tx();
       e = run_resident(g, p, mask, src, win, ws, L, t, q, s);
     }
+    if (e != hipSuccess) break;
     *r.cur = 1 - *r.cur;
+    *done = end;
   }
   return e;
 }
@@ -629,6 +631,7 @@ static hipError_t launch_resident(ResArgs& a, const ResPlan& p, hipStream_t s) {
 hipError_t run_resident(const Geom& g, const pjz_fdtd_problem& p, const float* mask,
                         const Src& src, const OutWin& win, char* ws, const Layout& L,
                         const ResPlan& plan, const ResRun& r, hipStream_t s) {
+  if (L.waits.refused()) return hipErrorCooperativeLaunchTooLarge;
   ResArgs a;
   a.Ein = r.in.E;
   a.Hin = r.in.H;

@@ -628,11 +628,12 @@ struct SlabPlan {
 };
 SlabPlan slab_plan(const Geom& g, int saxis, int cus);
 // Steps r of a domain in slabs, from buffer set *r.cur to the one it is set
-// to; words: slab_words() of them.
+// to; words: slab_words() of them.  After an error the set holds the state
+// before step *done (r.begin if untouched).
 inline size_t slab_words(const SlabPlan& p) { return p.n > 0 ? p.tile.words() : 0; }
 hipError_t run_slabs(const Geom& g, const pjz_fdtd_problem& p, const float* mask, const Src& src,
                      const OutWin& win, char* ws, const Layout& L, const SlabPlan& plan,
-                     rword_t* words, const StepRange& r, hipStream_t s);
+                     rword_t* words, const StepRange& r, int* done, hipStream_t s);
 
 // Whether a tiling's kernel that also writes each step's change of E is worth
 // its while: past 25 cells a lane, two a column, it spills (the one-step

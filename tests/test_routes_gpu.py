@@ -16,6 +16,7 @@ import test_fdtdz_gpu as T
 import test_grad_gpu as G
 from oracle import c_oracle as C
 from pjz_amd import _lib
+from pjz_amd import _mode as M
 from pjz_amd import fdtdz_torch as F
 
 pytestmark = pytest.mark.gpu
@@ -105,3 +106,66 @@ def test_three_steps_per_launch_in_batches():
     kernel = "stream3" if case[3] <= 64 else "stream2"
     want = F.fdtdz(**dict(kw, launch_params=dict(kernel=kernel))).cpu().numpy()
     assert np.linalg.norm(got - want) <= 1e-6 * np.linalg.norm(want), case
+
+
+class refused:
+  """Cooperative launches of this thread's calls inside the block are refused:
+  all, or all but a call's first."""
+
+  def __init__(self, later=False):
+    self.fault = _lib.TEST_REFUSE_LATER if later else _lib.TEST_REFUSE
+
+  def __enter__(self):
+    _lib.load().pjz_fdtd_test_faults(self.fault)
+
+  def __exit__(self, *_):
+    _lib.load().pjz_fdtd_test_faults(0)
+
+
+@pytest.mark.parametrize("later", [False, True])
+@pytest.mark.parametrize("X,Y,Z", [(88, 88, 64), (136, 122, 66), (260, 196, 96), (300, 300, 64)])
+def test_refused_launches_step_instead(X, Y, Z, later):
+  """A cooperative launch that the runtime refuses leaves the run, or what is
+  left of it (slabs), to the kernels launched step by step: the same snapshots."""
+  kw = T.random_problem(1, X=X, Y=Y, Z=Z, tt=60, seed=X, widths=(6, 5))
+  kw["output_steps"] = (10, 60, 7)
+  assert _lib.route(prob_of(kw)).kind != _lib.ROUTE_LAUNCHES
+  want = F.fdtdz(**kw)
+  with refused(later):
+    got = F.fdtdz(**kw)
+  assert torch.equal(got, want)
+  with refused(later):
+    outs = F.fdtdz_batch([kw, kw])
+  for o in outs:
+    diff = float(torch.linalg.vector_norm(o - want))
+    assert diff <= 1e-6 * float(torch.linalg.vector_norm(want))
+
+
+@pytest.mark.parametrize("later", [False, True])
+@pytest.mark.parametrize("launch", [dict(ckpt_every=20), dict(ckpt_every=40, ckpt_inner=18)])
+@pytest.mark.parametrize("X,Y,Z", [(88, 88, 64), (124, 136, 66), (300, 300, 64)])
+def test_refused_launches_in_gradients(X, Y, Z, launch, later):
+  """The same for the recompute and the reverse (refused from the first, or
+  from the second launch on: the first segment's reverse)."""
+  eps, kw, g = G.problem(0, seed=9, X=X, Y=Y, Z=Z, tt=60)
+  assert _lib.route(prob_of(kw, eps, **launch), backward=True).kind != _lib.ROUTE_LAUNCHES
+  want, _ = G.gpu_grad(eps, kw, g, **launch)
+  out = F.fdtdz(torch.tensor(eps, device="cuda", requires_grad=True),
+                **dict(kw, launch_params=launch))
+  ctx = out.grad_fn
+  with refused(later):  # (of this thread: autograd's own would not see it)
+    got = F._backward(ctx.prob, ctx.dev, ctx.device, ctx.ws, torch.as_tensor(g, device="cuda"))
+  assert G.rel_l2(got.cpu().numpy(), want) <= 1e-5
+
+
+def test_refused_launches_in_mode_solves():
+  eps = torch.ones(3, 96, 64, device="cuda")
+  eps[:, 30:50, 20:40] = 12.25
+  omega = torch.tensor([0.25, 0.3], device="cuda")
+  x = torch.randn((2, 2, 96, 64, 1), generator=torch.Generator().manual_seed(1)).cuda()
+  args = (eps, omega, torch.zeros_like(omega), x, 40, 0.0)
+  want = M._subspace_iteration_hip(*args)
+  with refused():
+    got = M._subspace_iteration_hip(*args)
+  for a, b in zip(got[:2], want[:2]):
+    torch.testing.assert_close(a, b, rtol=1e-4, atol=1e-5)
