@@ -365,7 +365,8 @@ pjz::WaitWords waits_in(const pjz_fdtd_problem& p, const pjz::Layout& L, char* w
 pjz::ResPlan resident_for(const pjz::Geom& g, const pjz_fdtd_problem& p, const pjz::Layout& L,
                           hipStream_t s) {
   const int cus = !L.waits.report || capturing(s) ? 0 : resident_cus(p);
-  return cus > 0 ? pjz::resident_plan(g, p.src_axis, cus) : pjz::ResPlan{};
+  if (cus <= 0 || !pjz::whole_device(s, cus)) return {};
+  return pjz::resident_plan(g, p.src_axis, cus);
 }
 
 // Its slabs for a larger domain (n = 0: none); `capture`: for steps whose
@@ -373,7 +374,7 @@ pjz::ResPlan resident_for(const pjz::Geom& g, const pjz_fdtd_problem& p, const p
 pjz::SlabPlan slabs_for(const pjz::Geom& g, const pjz_fdtd_problem& p, const pjz::Layout& L,
                         hipStream_t s, bool capture) {
   const int cus = !L.waits.report || capturing(s) ? 0 : resident_cus(p);
-  if (cus <= 0) return {};
+  if (cus <= 0 || !pjz::whole_device(s, cus)) return {};
   const pjz::SlabPlan plan = pjz::slab_plan(g, p.src_axis, cus);
   return capture && !pjz::resident_captures(plan.tile) ? pjz::SlabPlan{} : plan;
 }

@@ -1238,6 +1238,7 @@ static hipError_t launch_tile(const ModeArgs& a, int ww, TilePlan p, float* ws, 
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
         hipDeviceGetAttribute(&ok, hipDeviceAttributeCooperativeLaunch, dev) != hipSuccess || !ok ||
+        !whole_device(s, cus) ||
         hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kModeThreads, lds) !=
             hipSuccess ||
         (long long)p.gpf * ww > (long long)cus * per_cu)

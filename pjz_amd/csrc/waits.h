@@ -5,6 +5,21 @@
 
 namespace pjz {
 
+// Whether a stream's kernels may use all `cus` compute units of its device: a
+// stream can be created with a mask, and workgroups that need them all at the
+// same time have to keep off its others.
+inline bool whole_device(hipStream_t s, int cus) {
+  uint32_t mask[32] = {};
+  if (cus > 32 * 32) return true;
+  if (hipExtStreamGetCUMask(s, (cus + 31) / 32, mask) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  int n = 0;
+  for (uint32_t m : mask) n += __builtin_popcount(m);
+  return n == 0 || n >= cus;
+}
+
 // Workgroups that exchange words wait for one another.  Such a wait ends by
 // itself where all of them are on the chip at the same time and nobody else
 // writes the words.  A cooperative launch arranges the first on a GPU of its

@@ -7,6 +7,8 @@ of more than one block, and the batched launches of simulations that would run
 resident by default.
 """
 
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -169,3 +171,31 @@ def test_refused_launches_in_mode_solves():
     got = M._subspace_iteration_hip(*args)
   for a, b in zip(got[:2], want[:2]):
     torch.testing.assert_close(a, b, rtol=1e-4, atol=1e-5)
+
+
+def test_masked_streams_take_no_launches_that_need_the_whole_gpu():
+  """On a stream whose kernels keep to a part of the compute units, workgroups
+  that wait for one another might not all run at once."""
+  hip = ctypes.CDLL("libamdhip64.so")
+  cus = torch.cuda.get_device_properties(0).multi_processor_count
+  words = (cus + 31) // 32
+  masked = ctypes.c_void_p()
+  half = (ctypes.c_uint32 * words)(*[0x0000FFFF] * words)
+  assert hip.hipExtStreamCreateWithCUMask(ctypes.byref(masked), words, half) == 0
+  try:
+    stream = torch.cuda.ExternalStream(masked.value)
+    plain = torch.cuda.Stream()
+    for X, Y, Z in [(88, 88, 64), (260, 196, 96)]:
+      kw = T.random_problem(1, X=X, Y=Y, Z=Z, tt=40, seed=X, widths=(6, 5))
+      p = prob_of(kw)
+      assert _lib.route(p, stream=masked.value).kind == _lib.ROUTE_LAUNCHES
+      assert _lib.route(p, stream=plain.cuda_stream).kind != _lib.ROUTE_LAUNCHES
+      want = F.fdtdz(**kw)
+      torch.cuda.synchronize()
+      with torch.cuda.stream(stream):
+        got = F.fdtdz(**kw)
+        stream.synchronize()
+      assert torch.equal(got, want)
+  finally:
+    torch.cuda.synchronize()
+    assert hip.hipStreamDestroy(masked) == 0
