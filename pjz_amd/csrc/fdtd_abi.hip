@@ -704,7 +704,7 @@ int pjz_fdtd_mode_workspace_bytes(int32_t ww, int32_t xx, int32_t yy, int32_t mm
   int rc = check_mode(ww, xx, yy, mm);
   if (rc) return rc;
   if (!bytes) return fail(PJZ_FDTD_EINVAL, "mode: bytes is NULL");
-  *bytes = pjz::mode_workspace_floats(ww, xx, yy, mm) * sizeof(float);
+  *bytes = pjz::mode_workspace_floats(ww, xx, yy, mm, true) * sizeof(float);
   return PJZ_FDTD_OK;
 }
 
@@ -718,7 +718,9 @@ int pjz_fdtd_mode_solve(int32_t ww, int32_t xx, int32_t yy, int32_t mm, const fl
     return fail(PJZ_FDTD_EINVAL, "mode: NULL array");
   if (max_iters < 0) return fail(PJZ_FDTD_EINVAL, "mode: max_iters = %d < 0", max_iters);
   if (!(tol >= 0.0f)) return fail(PJZ_FDTD_EINVAL, "mode: tol must be >= 0");
-  const size_t need = pjz::mode_workspace_floats(ww, xx, yy, mm) * sizeof(float);
+  const size_t need = pjz::mode_workspace_floats(ww, xx, yy, mm, false) * sizeof(float);
+  const bool tile =
+      workspace_bytes >= pjz::mode_workspace_floats(ww, xx, yy, mm, true) * sizeof(float);
   if (workspace_bytes < need)
     return fail(PJZ_FDTD_ESPACE, "mode: workspace of %zu bytes, need %zu", workspace_bytes, need);
   if (const int bad = stall_reported()) return bad;
@@ -726,7 +728,8 @@ int pjz_fdtd_mode_solve(int32_t ww, int32_t xx, int32_t yy, int32_t mm, const fl
   waits.report = report_word(true);
   test_faults_of_call(waits);
   hipError_t e = pjz::launch_mode(ww, xx, yy, mm, epsilon, omega, shift, x, w, err, iters,
-                                  max_iters, tol, (float*)workspace, waits, (hipStream_t)stream);
+                                  max_iters, tol, (float*)workspace, tile, waits,
+                                  (hipStream_t)stream);
   return e == hipSuccess ? PJZ_FDTD_OK : hip_fail(e, "mode");
 }
 
@@ -982,18 +985,21 @@ int max_steps(const std::vector<pjz::BatchItem>& items) {
 
 // Workspace plan of a batch: one prepared single-simulation layout per item
 // (with checkpoints and adjoint buffers when ckpt_every > 0), then the batch
-// tables.
+// tables (to `total`), then the words of the simulations in slabs: a workspace
+// without them runs those step by step.
 struct BatchPlanHost {
   std::vector<pjz::Layout> Ls;
-  std::vector<size_t> offs;
-  size_t meta_off = 0, adj_off = 0, adj2_off = 0, total = 0;
+  std::vector<size_t> offs, more;
+  size_t meta_off = 0, adj_off = 0, adj2_off = 0, total = 0, with_words = 0;
   int S = 0;  // common checkpoint spacing, 0 = forward only
 };
 
-int batch_plan(const pjz_fdtd_problem* probs, int n, BatchPlanHost& bp) {
+// For a workspace of `bytes` bytes.
+int batch_plan(const pjz_fdtd_problem* probs, int n, BatchPlanHost& bp, size_t bytes) {
   if (!probs || n < 1) return fail(PJZ_FDTD_EINVAL, "a batch needs at least one problem");
   bp.Ls.resize(n);
   bp.offs.resize(n);
+  bp.more.resize(n);
   bp.S = probs[0].ckpt_every > 0 ? probs[0].ckpt_every : 0;
   size_t off = 0;
   for (int i = 0; i < n; ++i) {
@@ -1018,9 +1024,8 @@ int batch_plan(const pjz_fdtd_problem* probs, int n, BatchPlanHost& bp) {
                   g.Z);
     bp.Ls[i] = pjz::make_layout(g, probs[i]);
     bp.offs[i] = off;
-    const size_t more = slab_bytes(g, probs[i]);
-    if (more > 0) bp.Ls[i].words = pjz::align256(bp.Ls[i].total);
-    off += pjz::align256(bp.Ls[i].total) + pjz::align256(more);
+    bp.more[i] = pjz::align256(slab_bytes(g, probs[i]));
+    off += pjz::align256(bp.Ls[i].total);
   }
   bp.meta_off = off;
   std::vector<pjz::BatchItem> items(n);
@@ -1029,6 +1034,17 @@ int batch_plan(const pjz_fdtd_problem* probs, int n, BatchPlanHost& bp) {
   bp.adj_off = off + pjz::align256(pjz::batch2_meta_bytes(items.data(), n));
   bp.adj2_off = bp.adj_off + (bp.S > 0 ? pjz::align256(pjz::adjoint_batch_meta_bytes(n, bp.S)) : 0);
   bp.total = bp.adj2_off + (bp.S > 0 ? pjz::adjoint2_batch_meta_bytes(n, bp.S) : 0);
+  bp.with_words = bp.total;
+  for (int i = 0; i < n; ++i)
+    if (bp.more[i] > 0) bp.with_words = pjz::align256(bp.with_words) + bp.more[i];
+  if (bytes >= bp.with_words) {
+    size_t at = bp.total;
+    for (int i = 0; i < n; ++i)
+      if (bp.more[i] > 0) {
+        bp.Ls[i].words = pjz::align256(at) - bp.offs[i];
+        at = pjz::align256(at) + bp.more[i];
+      }
+  }
   return PJZ_FDTD_OK;
 }
 
@@ -1123,17 +1139,17 @@ extern "C" {
 
 int pjz_fdtd_batch_workspace_bytes(const pjz_fdtd_problem* probs, int n, size_t* bytes) {
   BatchPlanHost bp;
-  int rc = batch_plan(probs, n, bp);
+  int rc = batch_plan(probs, n, bp, SIZE_MAX);
   if (rc) return rc;
   if (!bytes) return fail(PJZ_FDTD_EINVAL, "bytes is NULL");
-  *bytes = bp.total;
+  *bytes = bp.with_words;
   return PJZ_FDTD_OK;
 }
 
 int pjz_fdtd_batch_routes(const pjz_fdtd_problem* probs, int n, int backward, void* stream,
                           pjz_fdtd_route* routes) {
   BatchPlanHost bp;
-  int rc = batch_plan(probs, n, bp);
+  int rc = batch_plan(probs, n, bp, SIZE_MAX);
   if (rc) return rc;
   if (!routes) return fail(PJZ_FDTD_EINVAL, "routes is NULL");
   const hipStream_t s = (hipStream_t)stream;
@@ -1155,7 +1171,7 @@ int pjz_fdtd_batch_forward(const pjz_fdtd_problem* probs, int n, const float* co
                            const float* const* source_waveform, float* const* out,
                            void* workspace, size_t workspace_bytes, void* stream) {
   BatchPlanHost bp;
-  int rc = batch_plan(probs, n, bp);
+  int rc = batch_plan(probs, n, bp, workspace_bytes);
   if (rc) return rc;
   if (const int bad = stall_reported()) return bad;
   hipStream_t s = (hipStream_t)stream;
@@ -1203,7 +1219,7 @@ int pjz_fdtd_batch_backward(const pjz_fdtd_problem* probs, int n, const float* c
                             float* const* grad_eps, void* workspace, size_t workspace_bytes,
                             void* stream) {
   BatchPlanHost bp;
-  int rc = batch_plan(probs, n, bp);
+  int rc = batch_plan(probs, n, bp, workspace_bytes);
   if (rc) return rc;
   if (bp.S <= 0)
     return fail(PJZ_FDTD_EINVAL,

@@ -175,10 +175,12 @@ int grid_chunk_x(int X, int nty, int slots, int ghost);
 // Waveguide mode solver (kernels_mode.hip): ww frequencies of a (xx, yy)
 // cross-section, 1 <= mm <= kModeMaxModes modes, one workgroup per frequency.
 constexpr int kModeMaxModes = 10;
-size_t mode_workspace_floats(int ww, int xx, int yy, int mm);
+// `tile`: with room for the tile kernel's words, without it (launch_mode) the
+// other kernels run.
+size_t mode_workspace_floats(int ww, int xx, int yy, int mm, bool tile);
 hipError_t launch_mode(int ww, int xx, int yy, int mm, const float* eps, const float* omega,
                        const float* shift, float* x, float* w, float* err, int* iters,
-                       int max_iters, float tol, float* ws, const WaitWords& waits,
+                       int max_iters, float tol, float* ws, bool tile, const WaitWords& waits,
                        hipStream_t s);
 
 hipError_t run_reference(const Geom& g, const pjz_fdtd_problem& p, const float* mask,

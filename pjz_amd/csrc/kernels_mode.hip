@@ -1202,13 +1202,15 @@ static int grid_share(int ww, int XX, int YY) {
   return gpf >= 2 && (long long)gpf * ww <= slots ? gpf : 0;
 }
 
-size_t mode_workspace_floats(int ww, int XX, int YY, int mm) {
+size_t mode_workspace_floats(int ww, int XX, int YY, int mm, bool tile) {
   // y and bc, then (256-byte aligned) the grid kernel's partial sums:
   // kModeMaxShare rows of NQ + NPAIR doubles per frequency.
-  // The tile kernel's exchange words take the same memory.
+  // The tile kernel's exchange words take the same memory, in some sections
+  // more: a workspace without it is left to the other kernels.
   const size_t nall = 3 * (size_t)mm + (size_t)mm * (mm + 1) / 2;
-  return std::max(2 * (size_t)ww * 2 * XX * YY * mm + 64 + (size_t)ww * kModeMaxShare * nall * 2,
-                  2 * tile_words(ww, XX, YY, mm) + 64);
+  const size_t others =
+      2 * (size_t)ww * 2 * XX * YY * mm + 64 + (size_t)ww * kModeMaxShare * nall * 2;
+  return tile ? std::max(others, 2 * tile_words(ww, XX, YY, mm) + 64) : others;
 }
 
 // The tile kernel where it applies; *done says whether it runs.
@@ -1268,11 +1270,11 @@ static hipError_t launch_tile(const ModeArgs& a, int ww, TilePlan p, float* ws, 
 }
 
 template <int MM>
-static hipError_t launch_mode_mm(ModeArgs a, int ww, float* ws, const WaitWords& waits,
+static hipError_t launch_mode_mm(ModeArgs a, int ww, float* ws, bool tile, const WaitWords& waits,
                                  hipStream_t s) {
   if constexpr (MM <= kTileMaxModes) {
     const TilePlan p = tile_plan(ww, a.XX, a.YY, MM);
-    if (p.R > 0) {
+    if (tile && p.R > 0) {
       bool done = false;
       const int cells = p.R * a.YY;
       const hipError_t e =
@@ -1296,7 +1298,7 @@ static hipError_t launch_mode_mm(ModeArgs a, int ww, float* ws, const WaitWords&
 
 hipError_t launch_mode(int ww, int XX, int YY, int mm, const float* eps, const float* omega,
                        const float* shift, float* x, float* w, float* err, int* iters,
-                       int max_iters, float tol, float* ws, const WaitWords& waits,
+                       int max_iters, float tol, float* ws, bool tile, const WaitWords& waits,
                        hipStream_t s) {
   ModeArgs a;
   a.XX = XX;
@@ -1317,16 +1319,16 @@ hipError_t launch_mode(int ww, int XX, int YY, int mm, const float* eps, const f
   a.err = err;
   a.iters = iters;
   switch (mm) {
-    case 1: return launch_mode_mm<1>(a, ww, ws, waits, s);
-    case 2: return launch_mode_mm<2>(a, ww, ws, waits, s);
-    case 3: return launch_mode_mm<3>(a, ww, ws, waits, s);
-    case 4: return launch_mode_mm<4>(a, ww, ws, waits, s);
-    case 5: return launch_mode_mm<5>(a, ww, ws, waits, s);
-    case 6: return launch_mode_mm<6>(a, ww, ws, waits, s);
-    case 7: return launch_mode_mm<7>(a, ww, ws, waits, s);
-    case 8: return launch_mode_mm<8>(a, ww, ws, waits, s);
-    case 9: return launch_mode_mm<9>(a, ww, ws, waits, s);
-    case 10: return launch_mode_mm<10>(a, ww, ws, waits, s);
+    case 1: return launch_mode_mm<1>(a, ww, ws, tile, waits, s);
+    case 2: return launch_mode_mm<2>(a, ww, ws, tile, waits, s);
+    case 3: return launch_mode_mm<3>(a, ww, ws, tile, waits, s);
+    case 4: return launch_mode_mm<4>(a, ww, ws, tile, waits, s);
+    case 5: return launch_mode_mm<5>(a, ww, ws, tile, waits, s);
+    case 6: return launch_mode_mm<6>(a, ww, ws, tile, waits, s);
+    case 7: return launch_mode_mm<7>(a, ww, ws, tile, waits, s);
+    case 8: return launch_mode_mm<8>(a, ww, ws, tile, waits, s);
+    case 9: return launch_mode_mm<9>(a, ww, ws, tile, waits, s);
+    case 10: return launch_mode_mm<10>(a, ww, ws, tile, waits, s);
     default: return hipErrorInvalidValue;
   }
 }

@@ -199,3 +199,74 @@ def test_masked_streams_take_no_launches_that_need_the_whole_gpu():
   finally:
     torch.cuda.synchronize()
     assert hip.hipStreamDestroy(masked) == 0
+
+
+def test_batch_in_a_workspace_without_the_slabs_words():
+  """Sized for the launches alone, a batch's workspace is enough: its
+  simulations in slabs then step as well (single calls: below)."""
+  kws = [T.random_problem(1, X=X, Y=Y, Z=Z, tt=40, seed=X, widths=(6, 5))
+         for X, Y, Z in [(260, 196, 96), (40, 44, 96)]]
+  kws = [dict(kw, output_steps=(20, 40, 7)) for kw in kws]
+  probs, devs, device = F._batch_problems(kws)
+  lean, _, _ = F._batch_problems([dict(kw, launch_params=dict(resident=False)) for kw in kws])
+  small, full = F._batch_workspace_bytes(lean), F._batch_workspace_bytes(probs)
+  assert small < full
+  want = F.fdtdz_batch(kws)
+  outs = [torch.empty_like(o) for o in want]
+  ws = F._Workspace(small, device)
+  col = lambda j: F._ptrs([d[j] for d in devs])
+  rc = _lib.load().pjz_fdtd_batch_forward(
+      probs, len(kws), col(0), col(3), col(4), col(5), col(6), col(1), col(2), F._ptrs(outs), ws.ptr,
+      ctypes.c_size_t(small), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+  _lib.check(rc, "pjz_fdtd_batch_forward")
+  # (35 steps: the odd last one is the one-step kernel's in a single call, the
+  # first of a pair's in a batch.)
+  for a, b in zip(outs, want):
+    diff = float(torch.linalg.vector_norm(a - b))
+    assert diff <= 1e-6 * float(torch.linalg.vector_norm(b))
+  # The single call of the first.
+  p, dev = probs[0], devs[0]
+  small = _lib.workspace_bytes(lean[0])
+  assert small < _lib.workspace_bytes(p)
+  out, ws = torch.empty_like(want[0]), F._Workspace(small, device)
+  rc = _lib.load().pjz_fdtd_forward(
+      ctypes.byref(p), *[F._ptr(dev[j]) for j in (0, 3, 4, 5, 6, 1, 2)], F._ptr(out), ws.ptr,
+      ctypes.c_size_t(small), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+  _lib.check(rc, "pjz_fdtd_forward")
+  diff = float(torch.linalg.vector_norm(out - want[0]))
+  assert diff <= 1e-6 * float(torch.linalg.vector_norm(want[0]))
+
+
+def test_mode_solve_in_a_workspace_without_the_tile_kernels_words():
+  """A section with few long rows, whose exchange takes more room than the
+  other kernels do."""
+  X, Y, modes = 32, 512, 1
+  nall = 3 * modes + modes * (modes + 1) // 2
+  small = 4 * (4 * X * Y * modes + 64 + 32 * nall * 2)
+  full = ctypes.c_size_t()
+  lib = _lib.load()
+  _lib.check(lib.pjz_fdtd_mode_workspace_bytes(1, X, Y, modes, ctypes.byref(full)), "mode")
+  assert small < full.value
+  eps = torch.ones(3, X, Y, device="cuda")
+  eps[:, 10:20, 200:260] = 12.25
+  omega, shift = torch.full((1,), 0.25, device="cuda"), torch.zeros(1, device="cuda")
+  start = torch.randn((1, 2, X, Y, modes), generator=torch.Generator().manual_seed(1)).cuda()
+
+  def solve(nbytes):
+    x, w, err = start.clone(), torch.empty(1, modes, device="cuda"), torch.empty(1, modes,
+                                                                                 device="cuda")
+    iters = torch.empty(1, dtype=torch.int32, device="cuda")
+    ws = torch.empty(nbytes // 4, device="cuda")
+    rc = lib.pjz_fdtd_mode_solve(1, X, Y, modes, *[F._ptr(t) for t in
+                                                  (eps, omega, shift, x, w, err, iters)], 40, 0.0,
+                                 F._ptr(ws), nbytes,
+                                 ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    return rc, w, x
+
+  assert solve(small - 4)[0] == _lib.ESPACE
+  rc, w, x = solve(small)
+  _lib.check(rc, "mode")
+  rc, w1, x1 = solve(full.value)
+  _lib.check(rc, "mode")
+  torch.testing.assert_close(w, w1, rtol=1e-4, atol=1e-5)
+  torch.testing.assert_close(x, x1, rtol=1e-3, atol=1e-4)
