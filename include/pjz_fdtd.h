@@ -327,8 +327,7 @@ PJZ_FDTD_API int pjz_fdtd_stepper(const pjz_fdtd_problem* p, int32_t* kernel);
  * Diagnostic: the way a call with this problem takes on the current device and
  * `stream`, with a workspace of pjz_fdtd_workspace_bytes: a forward call, or
  * (`backward`) the recompute and the reverse of a gradient.  The batched form
- * tells it for every simulation of a batch, where `kind` LAUNCHES means that
- * the simulation shares the batched launches.
+ * tells it for every simulation of a batch.
  */
 #define PJZ_FDTD_ROUTE_LAUNCHES 0 /* kernels launched step by step               */
 #define PJZ_FDTD_ROUTE_RESIDENT 1 /* the domain in registers, a launch a run     */
@@ -339,6 +338,7 @@ typedef struct pjz_fdtd_route {
   int32_t rx, ry;      /* columns a wave in x and y                             */
   int32_t slabs, steps;/* SLABS: their count, steps a slab's launch             */
   int32_t reverse;     /* backward: whether the reverse steps are resident too  */
+  int32_t batched;     /* whether it shares the batched launches                */
 } pjz_fdtd_route;
 PJZ_FDTD_API int pjz_fdtd_route_of(const pjz_fdtd_problem* p, int backward, void* stream,
                                    pjz_fdtd_route* route);

@@ -70,7 +70,7 @@ class Route(ctypes.Structure):
   """Mirror of ``pjz_fdtd_route``."""
   _fields_ = [("kind", ctypes.c_int32), ("cells", ctypes.c_int32), ("rx", ctypes.c_int32),
               ("ry", ctypes.c_int32), ("slabs", ctypes.c_int32), ("steps", ctypes.c_int32),
-              ("reverse", ctypes.c_int32)]
+              ("reverse", ctypes.c_int32), ("batched", ctypes.c_int32)]
 
 
 ROUTE_LAUNCHES, ROUTE_RESIDENT, ROUTE_SLABS = 0, 1, 2

@@ -1103,11 +1103,19 @@ void batch_waits(const std::vector<pjz::BatchItem>& items, BatchPlanHost& bp) {
 }
 
 // The simulations of a batch that run by themselves, one after the other, on
-// the resident stepper; the others share the batched launches.  A resident
-// step takes about 2.5 us and 0.3 us for every cell a lane, twice that where
-// cb comes from memory (past 16 cells); a simulation's share of a batched step
-// is its cells at 90 per ns, and no batched step is shorter than 12 us.  Slabs
-// are taken where they beat that rate anyway (slab_plan).
+// the resident stepper; the others share the batched launches.  A simulation's
+// share of a batched step is its cells at 90 per ns, and no batched step is
+// shorter than 12 us, against resident_step_us.  Slabs are taken where they
+// beat that rate anyway (slab_plan).
+// A gradient's recompute (`capture`) runs alone where it is resident too; its
+// reverse is then faster alone in either form.  Where it is not (two cells a
+// lane past 25), all is launched step by step either way, and from three
+// simulations on the batched launches are as fast or faster.  Measured, the
+// backward of six equal simulations over 100 steps, alone / batched, ms:
+// resident reverse (128x128x64) 11.4 / 20.7, streaming reverse (190x200x50, 20
+// cells a lane) 30.9 / 42.6, (301x187x45, 30) 45.0 / 60.3; recompute not
+// resident (180x150x128) 61.5 / 58.2, and over 150 steps one 15.0 / 17.7, two
+// 30.0 / 30.2, three 44.8 / 43.4.
 std::vector<bool> batch_alone(const std::vector<pjz::BatchItem>& items, bool capture,
                               hipStream_t s) {
   const size_t n = items.size();
@@ -1115,11 +1123,15 @@ std::vector<bool> batch_alone(const std::vector<pjz::BatchItem>& items, bool cap
   std::vector<double> us(n, 0.0);
   double all_res = 0, all_batch = 0;
   bool fit = true;
+  std::vector<size_t> launched;  // resident but for the recompute
   auto share_us = [](const pjz::BatchItem& it) { return (double)it.g.N / 90e3; };
   for (size_t i = 0; i < n; ++i) {
-    const pjz::ResPlan p = resident_for(items[i].g, *items[i].p, *items[i].L, s);
-    const int c = p.cpl * p.rx * p.ry;
-    if (p.rx > 0) us[i] = 2.5 + (c <= 16 ? 0.3 : 0.6) * c;
+    pjz::ResPlan p = resident_for(items[i].g, *items[i].p, *items[i].L, s);
+    if (capture && p.rx > 0 && !pjz::resident_captures(p)) {
+      launched.push_back(i);
+      p = {};
+    }
+    if (p.rx > 0) us[i] = pjz::resident_step_us(p);
     else fit = false;
     all_res += us[i];
     all_batch += share_us(items[i]);
@@ -1130,6 +1142,9 @@ std::vector<bool> batch_alone(const std::vector<pjz::BatchItem>& items, bool cap
     else if (items[i].L->words > 0)
       alone[i] = slabs_for(items[i].g, *items[i].p, *items[i].L, s, capture).n > 0;
   }
+  const size_t together = std::count(alone.begin(), alone.end(), false);
+  if (together <= 2 && together == launched.size())
+    for (size_t i : launched) alone[i] = true;
   return alone;
 }
 
@@ -1158,9 +1173,11 @@ int pjz_fdtd_batch_routes(const pjz_fdtd_problem* probs, int n, int backward, vo
     items[i] = {geom_of(probs[i]), &probs[i], nullptr, {}, {}, nullptr, &bp.Ls[i], nullptr};
   batch_waits(items, bp);
   const std::vector<bool> alone = batch_alone(items, backward != 0, s);
-  for (int i = 0; i < n; ++i)
-    routes[i] = alone[i] ? route_of(items[i].g, probs[i], bp.Ls[i], backward != 0, s)
-                         : pjz_fdtd_route{};
+  for (int i = 0; i < n; ++i) {
+    routes[i] = {};
+    if (alone[i]) routes[i] = route_of(items[i].g, probs[i], bp.Ls[i], backward != 0, s);
+    routes[i].batched = !alone[i];
+  }
   return PJZ_FDTD_OK;
 }
 

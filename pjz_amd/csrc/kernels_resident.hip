@@ -543,10 +543,9 @@ ResPlan resident_plan(const Geom& g, int saxis, int cus) {
   return best_tiling(g, g.X, saxis, cus, 2 * align256(sizeof(float) * 3 * (size_t)g.N));
 }
 
-// A resident step of a tiling, us, by its cells a lane, from the measurements
-// at the head of this file: past 16 cells cb comes from memory, two cells a
-// lane past 30 spill.
-static double step_us(const ResPlan& p) {
+// By the tiling's cells a lane, from the measurements at the head of this file:
+// past 16 cells cb comes from memory, two cells a lane past 30 spill.
+double resident_step_us(const ResPlan& p) {
   const int c = p.cpl * p.rx * p.ry;
   return c <= 16 ? 2.5 + 0.3 * c : p.cpl == 2 && c > 30 ? 21.0 : 1.0 + 0.53 * c;
 }
@@ -572,7 +571,7 @@ SlabPlan slab_plan(const Geom& g, int saxis, int cus) {
       // The widest slab: an inner one where there are any.
       const ResPlan t = best_tiling(g, own + (n > 2 ? 2 : 1) * k, saxis, cus, (size_t)1 << 30);
       if (!t.rx) break;
-      const double c = n * step_us(t) + (n * 35.0 + pass) / k;
+      const double c = n * resident_step_us(t) + (n * 35.0 + pass) / k;
       if (c < cost) {
         cost = c;
         best = {t, n, k};

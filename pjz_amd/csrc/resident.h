@@ -617,6 +617,8 @@ inline unsigned resident_tags(int n) { return (unsigned)n + 1; }
 
 // The tiling for a domain on `cus` compute units (rx = 0: it does not fit).
 ResPlan resident_plan(const Geom& g, int saxis, int cus);
+// What a step of a tiling takes, about, us.
+double resident_step_us(const ResPlan& p);
 
 // A domain that does not fit as a whole, in `n` slabs of x run one after the
 // other, `steps` at a time: each with that many columns more on its inner

@@ -95,9 +95,9 @@ def test_three_steps_per_launch_in_batches():
     kw["output_steps"] = (c[4] - 7, c[4], 1)
     calls.append(dict(kw, launch_params=dict(resident=False)))
   probs, _, _ = F._batch_problems(calls)
-  assert [r.kind for r in _lib.batch_routes(probs)] == [_lib.ROUTE_LAUNCHES] * len(cases)
+  assert all(r.kind == _lib.ROUTE_LAUNCHES and r.batched for r in _lib.batch_routes(probs))
   probs, _, _ = F._batch_problems([dict(kw, launch_params=None) for kw in calls])
-  assert all(r.kind == _lib.ROUTE_RESIDENT for r in _lib.batch_routes(probs))
+  assert all(r.kind == _lib.ROUTE_RESIDENT and not r.batched for r in _lib.batch_routes(probs))
   outs = F.fdtdz_batch(calls)
   torch.cuda.synchronize()
   for case, kw, out in zip(cases, calls, outs):
@@ -270,3 +270,29 @@ def test_mode_solve_in_a_workspace_without_the_tile_kernels_words():
   _lib.check(rc, "mode")
   torch.testing.assert_close(w, w1, rtol=1e-4, atol=1e-5)
   torch.testing.assert_close(x, x1, rtol=1e-3, atol=1e-4)
+
+
+@pytest.mark.parametrize("many", [2, 3])
+def test_batched_gradients_share_launches_unless_their_recompute_is_resident(many):
+  """Forward alone, backward batched, of three simulations whose tiling cannot
+  capture (two cells a lane past 25); alone where there are only two, and where
+  it can, with and without a resident reverse."""
+  cases = [(180, 150, 128), (150, 140, 96), (128, 120, 64)] + [(170, 150, 96)] * (many - 1)
+  probs = [G.problem(0, seed=i, X=X, Y=Y, Z=Z, tt=40) for i, (X, Y, Z) in enumerate(cases)]
+  eps = [torch.tensor(e, device="cuda", requires_grad=True) for e, _, _ in probs]
+  calls = [dict(kw, epsilon=e, launch_params=dict(ckpt_every=12))
+           for e, (_, kw, _) in zip(eps, probs)]
+  ps, _, _ = F._batch_problems(calls)
+  assert [r.kind for r in _lib.batch_routes(ps)] == [_lib.ROUTE_RESIDENT] * len(cases)
+  back = _lib.batch_routes(ps, backward=True)
+  assert [r.kind for r in back[1:3]] == [_lib.ROUTE_RESIDENT] * 2
+  assert [r.reverse for r in back[:3]] == [0, 0, 1]
+  assert [r.batched for r in back] == [many == 3, False, False] + [many == 3] * (many - 1)
+  outs = F.fdtdz_batch(calls)
+  sum((o * torch.as_tensor(g, device="cuda")).sum() for o, (_, _, g) in zip(outs, probs)).backward()
+  torch.cuda.synchronize()
+  for e, o, (e0, kw, g) in zip(eps, outs, probs):
+    print(tuple(e.shape), flush=True)
+    ref, out = G.gpu_grad(e0, kw, g, ckpt_every=12, kernel="stream2")
+    assert G.rel_l2(o.detach().cpu().numpy(), out) <= 1e-6
+    assert G.rel_l2(e.grad.cpu().numpy(), ref) <= 1e-5
