@@ -665,9 +665,11 @@ hipError_t run_resident(const Geom& g, const pjz_fdtd_problem& p, const float* m
   a.wex = win.ex; a.wey = win.ey; a.wez = win.ez;
   a.ostart = p.out_start; a.ostop = p.out_stop; a.ostep = p.out_step;
 #define PJZ_RES_LAUNCH(c, x, y)                                               \
-  if (plan.cpl == c && plan.rx == x && plan.ry == y)                          \
-    return r.capture ? launch_resident<c, x, y, true>(a, plan, s)             \
-                     : launch_resident<c, x, y, false>(a, plan, s);
+  if (plan.cpl == c && plan.rx == x && plan.ry == y) {                        \
+    if (!r.capture) return launch_resident<c, x, y, false>(a, plan, s);       \
+    if constexpr (tiling_captures(c, x, y))                                   \
+      return launch_resident<c, x, y, true>(a, plan, s);                      \
+  }
   PJZ_RES_SHAPES(PJZ_RES_LAUNCH)
 #undef PJZ_RES_LAUNCH
   return hipErrorInvalidValue;

@@ -640,9 +640,10 @@ hipError_t run_slabs(const Geom& g, const pjz_fdtd_problem& p, const float* mask
 // Whether a tiling's kernel that also writes each step's change of E is worth
 // its while: past 25 cells a lane, two a column, it spills (the one-step
 // change takes 6 more registers a column).
-inline bool resident_captures(const ResPlan& p) {
-  return p.rx > 0 && (p.cpl == 1 || p.cpl * p.rx * p.ry <= 25);
+constexpr bool tiling_captures(int cpl, int rx, int ry) {
+  return rx > 0 && (cpl == 1 || cpl * rx * ry <= 25);
 }
+inline bool resident_captures(const ResPlan& p) { return tiling_captures(p.cpl, p.rx, p.ry); }
 
 // The words (at L.E1, cleared before a call's first run) and the state it is
 // given in memory are the caller's to prepare.
