@@ -287,7 +287,10 @@ __device__ __forceinline__ Classes<C> cell_classes(const RenderDims& d, const fl
   for (int c = 0; c < C; ++c) {
     const int z = z0 + 64 * c + lane, zc = min(z, d.zz - 1);
     const float gs = gsa[2 * zc + col], ge = gea[2 * zc + col];
-    bool own = !(ge > gs);
+    // (Cells whose height, or its square in the z moment, is no positive number
+    // have no such share vector: what they are must not become a class's value.)
+    const float dz = ge - gs;
+    bool own = !(dz > 0.0f && dz < INFINITY && dz * dz / 12.0f > 0.0f);
     int below = 0;
     for (int l = 0; l + 1 < d.ll; ++l) {
       own |= !(pos[l] < gs || pos[l] > ge);

@@ -246,3 +246,27 @@ def test_render_kernel_interface_orders(gpu, pos, zz):
     res.append([v.detach().cpu().numpy() for v in (out, L.grad, p.grad)])
   for got, ref, tol in zip(*res, (2e-5, 2e-5, 2e-4)):
     assert np.linalg.norm(got - ref) <= tol * np.linalg.norm(ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("zz", [5, 40, 100])
+@pytest.mark.parametrize("cell,start,end", [(0, -np.inf, 0.5), (-1, None, np.inf), (2, 1.5, 1.5),
+                                            (2, 1.5, 1.5 + 1e-30), (3, 3.0, 2.0)])
+def test_render_kernel_cells_without_a_height(gpu, zz, cell, start, end):
+  """Grid cells of infinite, no, denormal-square or negative height give what the
+  torch restatement gives for them (NaN in most) and leave the cells between the
+  same interfaces alone."""
+  rng = np.random.default_rng(zz)
+  layers = 2 + 3 * rng.random((3, 8, 12))
+  gs, ge = (t.clone() for t in zgrid(zz, torch.float32))
+  if cell == 2 and end == 1.5 + 1e-30:  # a height that only a cell near zero can have
+    gs[cell], ge[cell] = 0.0, 1e-30
+  else:
+    if start is not None:
+      gs[cell] = start
+    ge[cell] = end
+  res = [E.render(torch.tensor(layers, dtype=torch.float32, device=d),
+                  torch.tensor([0.3 * zz, 0.7 * zz], device=d), gs.to(d), ge.to(d), 1).cpu().numpy()
+         for d in (gpu, torch.device("cpu"))]
+  assert np.isnan(res[1]).any() or cell == 3
+  np.testing.assert_allclose(res[0], res[1], rtol=1e-4, atol=0, equal_nan=True)
