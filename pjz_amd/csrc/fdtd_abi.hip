@@ -350,10 +350,12 @@ bool capturing(hipStream_t s) {
   return hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone;
 }
 
-// What a call's resident runs report to, for the workspace `ws`.
-pjz::WaitWords waits_in(const pjz_fdtd_problem& p, const pjz::Layout& L, char* ws) {
+// What a call's resident runs report to, for the workspace `ws`: nothing where
+// none are made.
+pjz::WaitWords waits_in(const pjz_fdtd_problem& p, const pjz::Layout& L, char* ws,
+                        hipStream_t s) {
   pjz::WaitWords w;
-  if (resident_cus(p) <= 0) return w;
+  if (resident_cus(p) <= 0 || capturing(s)) return w;
   w.stalled = (unsigned*)(ws + L.stalled);
   w.report = report_word(true);
   test_faults_of_call(w);
@@ -364,7 +366,7 @@ pjz::WaitWords waits_in(const pjz_fdtd_problem& p, const pjz::Layout& L, char* w
 // is too large.
 pjz::ResPlan resident_for(const pjz::Geom& g, const pjz_fdtd_problem& p, const pjz::Layout& L,
                           hipStream_t s) {
-  const int cus = !L.waits.report || capturing(s) ? 0 : resident_cus(p);
+  const int cus = L.waits.report ? resident_cus(p) : 0;
   if (cus <= 0 || !pjz::whole_device(s, cus)) return {};
   return pjz::resident_plan(g, p.src_axis, cus);
 }
@@ -373,7 +375,7 @@ pjz::ResPlan resident_for(const pjz::Geom& g, const pjz_fdtd_problem& p, const p
 // changes of E are written.
 pjz::SlabPlan slabs_for(const pjz::Geom& g, const pjz_fdtd_problem& p, const pjz::Layout& L,
                         hipStream_t s, bool capture) {
-  const int cus = !L.waits.report || capturing(s) ? 0 : resident_cus(p);
+  const int cus = L.waits.report ? resident_cus(p) : 0;
   if (cus <= 0 || !pjz::whole_device(s, cus)) return {};
   const pjz::SlabPlan plan = pjz::slab_plan(g, p.src_axis, cus);
   return capture && !pjz::resident_captures(plan.tile) ? pjz::SlabPlan{} : plan;
@@ -387,11 +389,12 @@ size_t slab_bytes(const pjz::Geom& g, const pjz_fdtd_problem& p) {
   return pjz::slab_words(pjz::slab_plan(g, p.src_axis, cus)) * sizeof(pjz::rword_t);
 }
 // The layout of a call in a workspace `ws` of `bytes` bytes.
-pjz::Layout layout_in(const pjz::Geom& g, const pjz_fdtd_problem& p, void* ws, size_t bytes) {
+pjz::Layout layout_in(const pjz::Geom& g, const pjz_fdtd_problem& p, void* ws, size_t bytes,
+                      hipStream_t s) {
   pjz::Layout L = pjz::make_layout(g, p);
   const size_t more = slab_bytes(g, p);
   if (more > 0 && bytes >= pjz::align256(L.total) + more) L.words = pjz::align256(L.total);
-  if (bytes >= L.total) L.waits = waits_in(p, L, (char*)ws);
+  if (bytes >= L.total) L.waits = waits_in(p, L, (char*)ws, s);
   return L;
 }
 
@@ -725,7 +728,7 @@ int pjz_fdtd_mode_solve(int32_t ww, int32_t xx, int32_t yy, int32_t mm, const fl
     return fail(PJZ_FDTD_ESPACE, "mode: workspace of %zu bytes, need %zu", workspace_bytes, need);
   if (const int bad = stall_reported()) return bad;
   pjz::WaitWords waits;
-  waits.report = report_word(true);
+  waits.report = report_word(!capturing((hipStream_t)stream));
   test_faults_of_call(waits);
   hipError_t e = pjz::launch_mode(ww, xx, yy, mm, epsilon, omega, shift, x, w, err, iters,
                                   max_iters, tol, (float*)workspace, tile, waits,
@@ -877,7 +880,7 @@ int pjz_fdtd_route_of(const pjz_fdtd_problem* p, int backward, void* stream,
   if (rc) return rc;
   if (!route) return fail(PJZ_FDTD_EINVAL, "route is NULL");
   const pjz::Geom g = geom_of(*p);
-  const pjz::Layout L = layout_in(g, *p, nullptr, SIZE_MAX);
+  const pjz::Layout L = layout_in(g, *p, nullptr, SIZE_MAX, (hipStream_t)stream);
   *route = route_of(g, *p, L, backward != 0, (hipStream_t)stream);
   return PJZ_FDTD_OK;
 }
@@ -917,7 +920,7 @@ int pjz_fdtd_forward(const pjz_fdtd_problem* p, const float* epsilon,
       !source_waveform || !out || !workspace)
     return fail(PJZ_FDTD_EINVAL, "a required pointer argument is NULL");
   pjz::Geom g = geom_of(*p);
-  pjz::Layout L = layout_in(g, *p, workspace, workspace_bytes);
+  pjz::Layout L = layout_in(g, *p, workspace, workspace_bytes, (hipStream_t)stream);
   if (workspace_bytes < L.total)
     return fail(PJZ_FDTD_ESPACE, "workspace of %zu bytes, %zu needed", workspace_bytes, L.total);
   if (((uintptr_t)workspace & 255) != 0)
@@ -1097,9 +1100,9 @@ int batch_setup(const pjz_fdtd_problem* probs, int n, const BatchPlanHost& bp,
 
 // One word for the waits of all a batch's simulations (the first's): once one
 // has waited in vain, the others do not wait as long again.
-void batch_waits(const std::vector<pjz::BatchItem>& items, BatchPlanHost& bp) {
+void batch_waits(const std::vector<pjz::BatchItem>& items, BatchPlanHost& bp, hipStream_t s) {
   for (size_t i = 0; i < items.size(); ++i)
-    bp.Ls[i].waits = waits_in(*items[i].p, bp.Ls[0], items[0].ws);
+    bp.Ls[i].waits = waits_in(*items[i].p, bp.Ls[0], items[0].ws, s);
 }
 
 // The simulations of a batch that run by themselves, one after the other, on
@@ -1171,7 +1174,7 @@ int pjz_fdtd_batch_routes(const pjz_fdtd_problem* probs, int n, int backward, vo
   std::vector<pjz::BatchItem> items(n);
   for (int i = 0; i < n; ++i)
     items[i] = {geom_of(probs[i]), &probs[i], nullptr, {}, {}, nullptr, &bp.Ls[i], nullptr};
-  batch_waits(items, bp);
+  batch_waits(items, bp, s);
   const std::vector<bool> alone = batch_alone(items, backward != 0, s);
   for (int i = 0; i < n; ++i) {
     routes[i] = {};
@@ -1197,7 +1200,7 @@ int pjz_fdtd_batch_forward(const pjz_fdtd_problem* probs, int n, const float* co
                    source_field, source_waveform, out, workspace, workspace_bytes, false, s, items);
   if (rc) return rc;
   char* base = (char*)workspace;
-  batch_waits(items, bp);
+  batch_waits(items, bp, s);
   const std::vector<bool> alone = batch_alone(items, false, s);
   std::vector<pjz::BatchItem> rest;  // of the batched launches
   hipError_t e = hipSuccess;
@@ -1253,7 +1256,7 @@ int pjz_fdtd_batch_backward(const pjz_fdtd_problem* probs, int n, const float* c
                    items);
   if (rc) return rc;
   char* base = (char*)workspace;
-  batch_waits(items, bp);
+  batch_waits(items, bp, s);
   const std::vector<bool> alone = batch_alone(items, true, s);
   std::vector<pjz::BatchItem> rest;  // of the batched launches, their cotangents
   std::vector<const float*> gout;
@@ -1373,7 +1376,7 @@ int pjz_fdtd_backward(const pjz_fdtd_problem* p, const float* epsilon,
       !source_waveform || !grad_out || !grad_eps || !workspace)
     return fail(PJZ_FDTD_EINVAL, "a required pointer argument is NULL");
   pjz::Geom g = geom_of(*p);
-  pjz::Layout L = layout_in(g, *p, workspace, workspace_bytes);
+  pjz::Layout L = layout_in(g, *p, workspace, workspace_bytes, (hipStream_t)stream);
   if (workspace_bytes < L.total)
     return fail(PJZ_FDTD_ESPACE, "workspace of %zu bytes, %zu needed", workspace_bytes, L.total);
   if (((uintptr_t)workspace & 255) != 0)

@@ -296,3 +296,27 @@ def test_batched_gradients_share_launches_unless_their_recompute_is_resident(man
     ref, out = G.gpu_grad(e0, kw, g, ckpt_every=12, kernel="stream2")
     assert G.rel_l2(o.detach().cpu().numpy(), out) <= 1e-6
     assert G.rel_l2(e.grad.cpu().numpy(), ref) <= 1e-5
+
+
+@pytest.mark.parametrize("X,Y,Z", [(64, 64, 64), (260, 196, 96)])
+def test_recorded_calls_are_launched_step_by_step(X, Y, Z):
+  """A call recorded into a graph makes no cooperative launch and allocates no
+  host memory; its replays, with eager runs in between, equal those."""
+  kw = T.random_problem(1, X=X, Y=Y, Z=Z, tt=40, seed=X, widths=(6, 5))
+  prob = prob_of(kw)
+  kw = {k: torch.as_tensor(v, device="cuda") if isinstance(v, np.ndarray) else v
+        for k, v in kw.items()}
+  want = F.fdtdz(**kw)
+  torch.cuda.synchronize()
+  graph = torch.cuda.CUDAGraph()
+  with torch.cuda.graph(graph):
+    route = _lib.route(prob, stream=torch.cuda.current_stream().cuda_stream)
+    out = F.fdtdz(**kw)
+  assert route.kind == _lib.ROUTE_LAUNCHES
+  for _ in range(3):
+    out.zero_()
+    graph.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(out, want)
+    assert torch.equal(F.fdtdz(**kw), want)
+    torch.cuda.synchronize()
