@@ -14,8 +14,9 @@
 // Bound by the exchange's latency on small domains and by arithmetic on
 // larger ones.  The streaming reverse pair it replaces there is bound by
 // latency within a workgroup (7 waves, two barriers a level and plane).
-// 128x128x64: 6.8 us a reversed step; the gradient of 600 steps 17.4 -> 11.8
-// ms.  160x160x64, 200 steps: 15.2 -> 8.4 ms with the resident recompute.
+// 128x128x64: 6.5 us a reversed step; the gradient of 600 steps, with the
+// resident recompute and the streaming reverse 17.4 ms, takes 11.5.
+// 160x160x64, 200 steps: 15.2 ms all streaming, 8.2.
 #include "resident.h"
 
 namespace pjz {

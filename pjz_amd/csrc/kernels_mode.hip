@@ -538,9 +538,9 @@ __global__ __launch_bounds__(kModeThreads) void k_mode_grid(ModeArgs a) {
 // spent 40 us an iteration on 0.5 MB of vectors (five grid barriers, each with
 // a cache write-back, and four dependent passes that each wait for L2), the
 // 30 x 20 strip with 2 modes 7.5 us (three block sums, two Cholesky
-// factorisations on one lane, every pass through L2).  They are now 3.4 us,
-// where the exchange and its waits take about half, and 2.1 us, bound by the
-// instructions of eight waves on one compute unit.  Here the state never
+// factorisations on one lane, every pass through L2).  They are now 3.5 us (of
+// the launch; the exchange and its waits take about half) and 2.0 us, bound by
+// the instructions of eight waves on one compute unit.  Here the state never
 // leaves the compute units: a workgroup owns R rows of the section for the
 // whole run, x, y and the permittivity live in registers (CPT cells a thread),
 // neighbours read x, b and c from LDS, and one exchange an iteration carries
@@ -551,8 +551,8 @@ __global__ __launch_bounds__(kModeThreads) void k_mode_grid(ModeArgs a) {
 // itself whether it has arrived, so there is no flag, fence or grid barrier:
 // one store and one load latency (0.7-1.2 us measured for 4-32 workgroups,
 // against 2-5 us for each grid barrier).  The sums are posted before the rows
-// are waited for, so both travel at once (the other order: 256 x 128 6.7 us an
-// iteration instead of 3.9).  Two sets of words alternate: a
+// are waited for, so both travel at once (with the other order an iteration at
+// 256 x 128 took 1.7 x as long).  Two sets of words alternate: a
 // workgroup posts exchange s + 2 only after it has everyone's sums of s + 1,
 // which each posts after it has read all of s.  All workgroups are resident at
 // the same time (cooperative launch) and post before they wait, so every wait

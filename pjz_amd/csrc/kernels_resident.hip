@@ -6,7 +6,7 @@
 // (8-13 planes in sequence, two barriers each, 36-64 workgroups), and a
 // 128x128x64 step of 38 MB 15 us.  The chip's registers (128 MB) hold such a
 // domain.  Here a workgroup owns a tile of z columns for the whole run: E, H
-// (and, up to 20 cells a lane, cb) live in registers, RX x RY columns a wave
+// (and, up to 16 cells a lane, cb) live in registers, RX x RY columns a wave
 // and CPL cells of a column a lane, so x neighbours and most y neighbours are
 // other registers of the same lane and z neighbours a DPP move; the CPML psi
 // live in LDS.
@@ -25,10 +25,11 @@
 // clock (waits.h).
 //
 // Measured, us a step, two-step kernel (the default before) against this:
-// 64^3 13.4 -> 2.9 (both exchange latencies), 128x128x64 14.3 -> 5.2,
-// 160x160x64 20.4 -> 7.0 (16 cells a lane: arithmetic), 190x200x50 25.1 ->
-// 10.8, 150x140x96 29.0 -> 12.6, 301x187x45 45.0 -> 17.6, 180x150x128 37.2 ->
-// 16.8 (20-30 cells a lane: arithmetic of two waves a SIMD, cb from the caches).
+// 64^3 13.4 -> 2.6 (both exchange latencies: a wave waits 0.74 of its cycles),
+// 128x128x64 14.3 -> 4.8, 160x160x64 20.4 -> 6.8, 190x200x50 25.1 -> 10.4,
+// 150x140x96 29.0 -> 11.4, 301x187x45 45.0 -> 17.0, 180x150x128 37.2 -> 13.8
+// (16-30 cells a lane: the instructions of two waves a SIMD, at 301x187x45
+// vector ones in 0.53 of a SIMD's cycles and any in 0.98; cb from the caches).
 //
 // The arithmetic of a cell is that of the two-step kernel (stream2_parts.h),
 // in its order of rounding: results equal that kernel's bit for bit.
@@ -61,7 +62,7 @@ struct ResArgs {
   int saxis, spos, squad;
   float dt;
   int begin, end;
-  unsigned tag0;     // exchange numbers tag0 + 1 .. tag0 + 2 (end - begin) + 1
+  unsigned tag0;     // exchange numbers tag0 + 1 .. tag0 + (end - begin) + 1
   int wx0, wy0, wz0, wex, wey, wez, ostart, ostop, ostep;
   __device__ __forceinline__ void split() {
     apart(Ein, Hin, psiin, Eout, Hout, psiout, cb, zt, mask, sfield, swave, out, cap, ckpt,
@@ -543,8 +544,10 @@ ResPlan resident_plan(const Geom& g, int saxis, int cus) {
   return best_tiling(g, g.X, saxis, cus, 2 * align256(sizeof(float) * 3 * (size_t)g.N));
 }
 
-// By the tiling's cells a lane, from the measurements at the head of this file:
-// past 16 cells cb comes from memory, two cells a lane past 30 spill.
+// By the tiling's cells a lane, from the measurements at the head of this file
+// (tilings of two cells a lane past 25 were slower when it was fitted: 16.8 at
+// 30 cells, now 13.8): past 16 cells cb comes from memory, two cells a lane past
+// 30 spill.
 double resident_step_us(const ResPlan& p) {
   const int c = p.cpl * p.rx * p.ry;
   return c <= 16 ? 2.5 + 0.3 * c : p.cpl == 2 && c > 30 ? 21.0 : 1.0 + 0.53 * c;
@@ -554,10 +557,11 @@ double resident_step_us(const ResPlan& p) {
 // with the start of its waves) and one pass over the state.  Taken where that
 // is estimated below 0.85 of the streaming steppers' rate, measured as 80-90
 // cells/ns at zz = 96, 94-113 at 128 and 110 at 64 (by the lanes in
-// use).  Measured, us a step: 220x200x96 48.9 -> 39.3, 260x196x96 55.0 -> 39.3,
-// 300x300x64 52.2 -> 31.3, 256x341x64 52.0 -> 35.3, 128x341x128 59.2 -> 42.7,
-// 512x512x64 148 -> 118; 256x256x128 in three slabs 75.7 against 74.5, which
-// this estimate leaves alone.
+// use).  Measured, us a step: 220x200x96 48.9 -> 32.8, 260x196x96 55.0 -> 34.0,
+// 300x300x64 52.2 -> 29.6, 256x341x64 52.0 -> 33.6, 128x341x128 59.2 -> 39.0,
+// 512x512x64 148 -> 110; 256x256x128 in three slabs 75.7 against 74.5 (before
+// kernel arguments had registers of their own), which this estimate leaves
+// alone.
 SlabPlan slab_plan(const Geom& g, int saxis, int cus) {
   SlabPlan best{};
   if (g.Z > 128) return best;

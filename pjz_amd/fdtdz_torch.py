@@ -32,8 +32,9 @@ def _launch_options(launch_params):
 
   Keys: ``kernel`` ("auto" | "reference" | "stream" | "stream2" | "stream3" |
   "stream4" (one, two, three or four steps per pass) | "autotune": the first
-  call per shape times the kernels, depths and tilings, later calls reuse the
-  fastest), ``tile_x``, ``tile_y``,
+  call per shape times the streaming kernels, depths and tilings, later calls
+  reuse the fastest; it does not consider the resident runs of "auto", which on
+  domains that fit are up to five times faster), ``tile_x``, ``tile_y``,
   ``waves_per_simd`` (stream kernel tiling), ``ckpt_every`` (steps between
   checkpoints kept for the gradient; default about sqrt(2 * steps)),
   ``ckpt_inner`` (single calls: steps between the second level of
@@ -492,12 +493,15 @@ def batch_ckpt_every(probs):
 def fdtdz_batch(calls, memory_budget=None):
   """Runs several fdtdz() calls, given as keyword dicts, as one batch.
 
-  All simulations advance together through the batched kernels
-  (``pjz_fdtd_batch_forward``): persistent two-step launches over a work queue
-  of (simulation, tile) items.  Returns the list of snapshot tensors, in the
-  order of ``calls``.  When any ``epsilon`` requires grad, the batch is one
-  ``torch.autograd.Function`` whose backward runs the batched adjoint
-  (``pjz_fdtd_batch_backward``) for every simulation at once.  Every call needs
+  Simulations that fit the GPU's registers, whole or in slabs, run by
+  themselves, one after the other, where that is faster; the others advance
+  together through the batched kernels (``pjz_fdtd_batch_forward``): persistent
+  two-step launches over a work queue of (simulation, tile) items.  A call with
+  ``launch_params`` ``resident=False`` is one of the others.  Returns the list
+  of snapshot tensors, in the order of ``calls``.  When any ``epsilon`` requires
+  grad, the batch is one ``torch.autograd.Function`` whose backward
+  (``pjz_fdtd_batch_backward``) takes the simulations in the same two ways.
+  Every call needs
   zz <= 64 or an even zz <= 128.  Tiles are chosen for the whole batch (x
   chunks and, at zz <= 64, 8 or 13 rows per tile, from a model of the work
   queue); ``launch_params`` ``tile_y`` = 8 or 13 on every zz <= 64 call fixes
