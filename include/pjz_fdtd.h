@@ -32,12 +32,12 @@
  *     registers is one launch whose workgroups wait for one another.  They need
  *     the GPU's compute units at the same time and words of the workspace that
  *     nobody else writes.  Where that fails (a workspace in use by two calls,
- *     another process on the same GPU) the waits end after 20 s and 1 ms a
+ *     another process on the same GPU) the waits end after 60 s and 1 ms a
  *     step, the outputs hold NaN, and the next call on that GPU that enqueues a
  *     simulation or a mode solve, or pjz_fdtd_run_status, returns
  *     PJZ_FDTD_ESTALL, once.  PJZ_FDTD_FLAG_STEPWISE or a kernel id other than
  *     AUTO runs kernels without such waits.  Mode solves of more than one
- *     workgroup wait in the same way (20 s and 0.1 ms an iteration).
+ *     workgroup wait in the same way (60 s and 0.1 ms an iteration).
  */
 #ifndef PJZ_FDTD_H_
 #define PJZ_FDTD_H_

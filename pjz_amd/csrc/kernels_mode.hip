@@ -1249,9 +1249,9 @@ static hipError_t launch_tile(const ModeArgs& a, int ww, TilePlan p, float* ws, 
     hipError_t e = launch_zero(reinterpret_cast<float*>(ta.box),
                                4 * tile_box(ww, p.gpf, a.YY, MM).total, s);
     if (e != hipSuccess) return e;
-    // 20 s, as the resident steppers' launches, and 0.1 ms an iteration (of
+    // 60 s, as the resident steppers' launches, and 0.1 ms an iteration (of
     // 2-8 us).
-    const double ms = waits.no_time ? 0.0 : 20e3 + 0.1 * a.max_iters;
+    const double ms = waits.no_time ? 0.0 : 60e3 + 0.1 * a.max_iters;
     ta.waits.ticks = (unsigned)std::min(ms * (100e3 / kWaitTick), 1e9);
     ta.waits.stalled =
         reinterpret_cast<unsigned*>(ta.box + tile_box(ww, p.gpf, a.YY, MM).late);

@@ -567,10 +567,10 @@ struct ResTile {
   }
 };
 
-// The waits of a launch of `steps` steps (at most about 20 us each): 20 s, far
+// The waits of a launch of `steps` steps (at most about 20 us each): 60 s, far
 // more than other streams' kernels hold a workgroup back, and 1 ms a step.
 inline WaitArgs wait_args(const WaitWords& w, int steps) {
-  const double ms = w.no_time ? 0.0 : 20e3 + steps;
+  const double ms = w.no_time ? 0.0 : 60e3 + steps;
   return {(unsigned)std::min(ms * (100e3 / kWaitTick), 1e9), w.stalled, w.report};
 }
 
