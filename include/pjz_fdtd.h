@@ -18,7 +18,8 @@
  *     z fastest, exactly the layouts pjz passes (shapes below).
  *   - The caller owns all memory.  Scratch (field state, coefficients) comes
  *     in as `workspace`, sized by pjz_fdtd_workspace_bytes().  The library
- *     does not allocate device memory.
+ *     does not allocate device memory (and 256 bytes of pinned host memory
+ *     once, for reports of waits in vain, see below).
  *   - Work is enqueued on `stream` (a hipStream_t, NULL = default stream) and
  *     is stream-ordered; no host synchronisation happens inside the calls.
  *   - Return 0 on success.  Non-zero codes: PJZ_FDTD_EINVAL (bad argument,

@@ -347,7 +347,11 @@ int resident_cus(const pjz_fdtd_problem& p) {
 // might not be recordable.
 bool capturing(hipStream_t s) {
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  return hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &cap) != hipSuccess) {
+    (void)hipGetLastError();  // (not for the next launch to report)
+    return true;
+  }
+  return cap != hipStreamCaptureStatusNone;
 }
 
 // What a call's resident runs report to, for the workspace `ws`: nothing where
